@@ -296,16 +296,33 @@ int lampa_gdr_bwd(const void* q, const void* k, const void* v, const float* g, c
 /* The same gradients in the chunked (WY) form on the matrix cores, the form of the reference's own backward pass
  * (chunk_gated_delta_rule_bwd, models/hattention/gated_delta_rule_ori.py:83-160: chunk_bwd_dv_local chunk_o.py:372,
  * chunk_gated_delta_rule_bwd_dhu chunk_delta_h.py:209, chunk_bwd_dqkwg chunk_o.py:128, prepare_wy_repr_bwd wy_fast.py:27;
- * l2norm_bwd gated_delta_rule_ori.py:205-233): per chunk of 64 tokens the affine map of the state (forwards) and of its
- * gradient (backwards), a scan over the maps in three levels of groups of 8, then every gradient of a chunk from its tiles
- * and the two states. For K = V = 64, HV = H, dtype LAMPA_BF16 / LAMPA_FP16 (LAMPA_ERR_UNSUPPORTED otherwise: use
- * lampa_gdr_bwd); every intermediate operand is rounded to the input type, as in the forward pass, so all gradients
- * carry the rounding of that type. g <= 0 is assumed (the forward's masking of positive exponents is not differentiated).
- * Shapes as for lampa_gdr_bwd. plan: lampa_gdr_bwd_chunk_plan_fill's tables of the sequence boundaries
- * (cu_seqlens_host: int64 [n_seq+1]), the same int32 array in host and in device memory.
- * workspace: lampa_gdr_bwd_chunk_workspace_bytes(plan_host, HV): about 41 KiB per (chunk, head) -- the chunk's record,
- * its two map parts and the state and state gradient it starts from, all in the 16-bit input type, plus the maps and
- * states of the groups -- 0.33 GB for one sequence of 60 000 tokens with 8 heads (lampa_gdr_bwd: 1.9 GB there). */
+ * l2norm_bwd gated_delta_rule_ori.py:205-233), for K = V = 64 and dtype LAMPA_BF16 / LAMPA_FP16 (LAMPA_ERR_UNSUPPORTED
+ * otherwise: use lampa_gdr_bwd); every intermediate operand is rounded to the input type, as in the forward pass, so all
+ * gradients carry the rounding of that type. g <= 0 is assumed (the forward's masking of positive exponents is not
+ * differentiated).
+ *
+ * lampa_gdr_chunk_fwd_train is lampa_gdr_chunk_fwd (the same plan, the same o and ht) and also fills `saved`
+ * (lampa_gdr_train_saved_bytes: about 13.6 KB per chunk and head -- its record and the state in front of it in the 16-bit
+ * input type -- and 8 KB per segment and head). positive_g_host (nullable): an int32 in pinned host memory, zeroed by the
+ * caller, becomes 1 when an entry of g is positive (to be read once the call's kernels have run).
+ * lampa_gdr_bwd_saved computes the gradients from q, k, v and `saved`: the gradient of the state is walked from the last
+ * chunk of every segment to its first, segments in parallel, as the forward pass walks the state. dq and dk have one row
+ * per VALUE head, [tokens, HV, 64]: with grouped value heads the caller sums them over each group. dht, dh0 nullable.
+ * `saved` is only read; workspace: about 24 KB per segment and head. */
+int64_t lampa_gdr_train_saved_bytes(const int32_t* plan_host, int HV);
+int64_t lampa_gdr_train_workspace_bytes(const int32_t* plan_host, int HV);
+int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const void* v, const float* g, const float* beta, void* o,
+                              const float* h0, float* ht, const int32_t* plan_host, const int32_t* plan_dev, int H, int HV,
+                              int K, int V, int dtype, float scale, int l2norm, void* saved, int32_t* positive_g_host,
+                              void* workspace, int64_t workspace_bytes, void* stream);
+int64_t lampa_gdr_bwd_saved_workspace_bytes(const int32_t* plan_host, int HV);
+int lampa_gdr_bwd_saved(const void* q, const void* k, const void* v, const void* saved, const void* dout, const float* dht,
+                        void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, const int32_t* plan_host,
+                        const int32_t* plan_dev, int H, int HV, int K, int V, int dtype, float scale, int l2norm,
+                        void* workspace, int64_t workspace_bytes, void* stream);
+/* Both in one call, from the inputs alone (HV = H). plan: lampa_gdr_bwd_chunk_plan_fill's tables of the sequence boundaries
+ * (cu_seqlens_host: int64 [n_seq+1]; any plan of lampa_gdr_plan_fill* will do), the same int32 array in host and in device
+ * memory. workspace: lampa_gdr_bwd_chunk_workspace_bytes(plan_host, HV): about 25 KiB per (chunk, head). */
 int64_t lampa_gdr_bwd_chunk_plan_size(const int64_t* cu_seqlens_host, int n_seq);
 int lampa_gdr_bwd_chunk_plan_fill(const int64_t* cu_seqlens_host, int n_seq, int32_t* plan_host);
 int64_t lampa_gdr_bwd_chunk_workspace_bytes(const int32_t* plan_host, int HV);

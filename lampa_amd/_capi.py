@@ -66,6 +66,11 @@ _SIGNATURES = {
     "lampa_gdr_bwd_chunk_plan_fill": (_i32, [_vp, _i32, _vp]),
     "lampa_gdr_bwd_chunk_workspace_bytes": (_i64, [_vp, _i32]),
     "lampa_gdr_bwd_chunk": (_i32, [_vp] * 16 + [_i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp, _i64, _vp]),
+    "lampa_gdr_train_saved_bytes": (_i64, [_vp, _i32]),
+    "lampa_gdr_train_workspace_bytes": (_i64, [_vp, _i32]),
+    "lampa_gdr_chunk_fwd_train": (_i32, [_vp] * 10 + [_i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp, _vp, _vp, _i64, _vp]),
+    "lampa_gdr_bwd_saved_workspace_bytes": (_i64, [_vp, _i32]),
+    "lampa_gdr_bwd_saved": (_i32, [_vp] * 14 + [_i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp, _i64, _vp]),
     "lampa_profile_begin": (_i32, []),
     "lampa_profile_end": (_i32, [_i32, _vp, _vp]),
     "lampa_gdr_traffic_probe": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),

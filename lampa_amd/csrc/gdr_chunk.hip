@@ -1,6 +1,7 @@
 // Host side of the chunkwise gated-delta-rule forward: workspace layout, launch sequence and the C entry points.
 // The kernels (and the description of the algorithm) are in gdr_chunk_kernels.h.
 #include "gdr_chunk_kernels.h"
+#include "gdr_train.h"
 #include <atomic>
 #include <mutex>
 
@@ -44,15 +45,23 @@ extern "C" int64_t lampa_gdr_chunk_workspace_bytes(int64_t total_chunks, int64_t
   return gdr_workspace(total_chunks, n_segments, HV, K, V).bytes;
 }
 
-template <typename T, int KT, int VT>
+// Buffers of the training form (gdr_train.h), or none.
+struct GdrKeep {
+  unsigned char *rec, *states, *mt;
+  float* d;
+  int32_t* positive_g;
+};
+
+template <typename T, int KT, int VT, bool KEEP = false>
 static int gdr_chunk_launch(const void* q, const void* k, const void* v, const float* g, const float* beta, void* o,
                             const float* h0, float* ht, const GdrPlanView pv, int n_seq, int chunks, int segs, int max_nseg,
-                            int H, int HV, float scale, int l2norm, unsigned char* ws, hipStream_t s) {
-  const GdrWorkspace w = gdr_workspace(chunks, segs, HV, KT, VT);
-  unsigned char* tf = ws + w.off_t;
+                            int H, int HV, float scale, int l2norm, unsigned char* ws, hipStream_t s,
+                            const GdrKeep kp = GdrKeep{}) {
+  const GdrWorkspace w = gdr_workspace(KEEP ? 0 : chunks, segs, HV, KT, VT);  // (KEEP: the records are kept elsewhere)
+  unsigned char* tf = KEEP ? kp.rec : ws + w.off_t;
   unsigned char* Mc = ws + w.off_m;
   unsigned char* Nc = ws + w.off_n;
-  float* Dc = (float*)(ws + w.off_d);
+  float* Dc = KEEP ? kp.d : (float*)(ws + w.off_d);
   float* Si = (float*)(ws + w.off_sinit);
   constexpr int smem_a = GdrSegSmem<KT, VT, false>::BYTES, smem_b = GdrSegSmem<KT, VT, true>::BYTES;
   constexpr int CWN = KT >= 64 ? 16 : 32;  // chain-wave width of the narrow output pass (K = 32 has none)
@@ -64,9 +73,9 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return LAMPA_ERR_LAUNCH;
   std::unique_lock<std::mutex> hold(attr_lock);
   if (!attr_set[dev]) {
-    if (hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, false>,
+    if (hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_a) != hipSuccess ||
-        hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, true>,
+        hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, true, false, T, 32, KEEP>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_b) != hipSuccess ||
         hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, true, false, T, CWN>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_n) != hipSuccess)
@@ -77,13 +86,13 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
   LAMPA_PROF(s, "start");
   if (chunks > 0) {
     hipLaunchKernelGGL((gdr_local_kernel<T, T, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g, beta,
-                       pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm);
+                       pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, kp.positive_g);
     LAMPA_PROF(s, "gdr_local_kernel");
     if (segs > n_seq) {
-      hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
+      hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
                          (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, Mc, Nc, Dc,
                          (T*)nullptr, (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
-                         (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0);
+                         (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, kp.mt);
       LAMPA_PROF(s, "gdr_segment_kernel<composite>");
     }
   }
@@ -112,15 +121,15 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
     LAMPA_PROF(s, "gdr_scan_kernel");
   }
   const int narrow = gdr_narrow_output.load();
-  if (CWN == 16 && (narrow == 2 || (narrow == 1 && KT + VT > 128)))
+  if (!KEEP && CWN == 16 && (narrow == 2 || (narrow == 1 && KT + VT > 128)))
     hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true, false, T, CWN>), dim3(segs * HV),
                        dim3(64 * GdrSegShape<KT, VT, true, CWN>::WAVES), smem_n, s, (const T*)q, (const T*)k, (const T*)v, g, beta,
                        pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, Nc, Dc, (T*)o, ht, H, HV, scale, l2norm,
-                       (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0);
+                       (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states);
   else
-  hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, true>::WAVES), smem_b, s, (const T*)q,
+  hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true, false, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, true>::WAVES), smem_b, s, (const T*)q,
                      (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, Nc, Dc, (T*)o, ht, H, HV, scale,
-                     l2norm, (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0);
+                     l2norm, (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states);
   LAMPA_PROF(s, "gdr_segment_kernel<output>");
   return lampa_launch_status();
 }
@@ -162,4 +171,56 @@ extern "C" int lampa_gdr_chunk_fwd(const void* q, const void* k, const void* v, 
   }
 #undef GDR_CASE
   return LAMPA_ERR_UNSUPPORTED;
+}
+
+// ---- training form: the same forward, keeping what the backward pass needs (gdr_train.h) --------------------------------
+GdrSaved gdr_saved_layout(int64_t chunks, int64_t segs, int HV) {
+  GdrSaved v;
+  int64_t off = 0;
+  v.off_rec = off;    off += lampa_align_up(chunks * HV * (int64_t)REC_BYTES, 256);
+  v.off_states = off; off += lampa_align_up(chunks * HV * (int64_t)GDR_STATE_BYTES, 256);
+  v.off_mt = off;     off += lampa_align_up(segs * HV * (int64_t)GDR_STATE_BYTES, 256);
+  v.off_d = off;      off += lampa_align_up(segs * HV * 4, 256);
+  v.bytes = off > 0 ? off : 256;
+  return v;
+}
+
+extern "C" int64_t lampa_gdr_train_saved_bytes(const int32_t* plan_host, int HV) {
+  if (!plan_host || HV < 1) return LAMPA_ERR_INVALID;
+  return gdr_saved_layout(plan_host[PLAN_TOTAL_CHUNKS], plan_host[PLAN_N_SEGMENTS], HV).bytes;
+}
+extern "C" int64_t lampa_gdr_train_workspace_bytes(const int32_t* plan_host, int HV) {
+  if (!plan_host || HV < 1) return LAMPA_ERR_INVALID;
+  return gdr_workspace(0, plan_host[PLAN_N_SEGMENTS], HV, 64, 64).bytes;
+}
+
+// As lampa_gdr_chunk_fwd for K = V = 64. saved: lampa_gdr_train_saved_bytes bytes for lampa_gdr_bwd_saved. positive_g_host
+// (nullable): pinned host memory, zeroed by the caller; becomes 1 when an entry of g is positive.
+extern "C" int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const void* v, const float* g, const float* beta,
+                                         void* o, const float* h0, float* ht, const int32_t* plan_host,
+                                         const int32_t* plan_dev, int H, int HV, int K, int V, int dtype, float scale,
+                                         int l2norm, void* saved, int32_t* positive_g_host, void* workspace,
+                                         int64_t workspace_bytes, void* stream) {
+  if (!q || !k || !v || !g || !beta || !o || !plan_host || !plan_dev || !saved) return LAMPA_ERR_INVALID;
+  if (H < 1 || HV < H || HV % H != 0 || l2norm < 0 || l2norm > 2) return LAMPA_ERR_INVALID;
+  if (K != 64 || V != 64 || (dtype != GDR_BF16 && dtype != GDR_FP16)) return LAMPA_ERR_UNSUPPORTED;
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o | (uintptr_t)saved) & 15) return LAMPA_ERR_INVALID;
+  const int n_seq = plan_host[PLAN_N_SEQ], chunks = plan_host[PLAN_TOTAL_CHUNKS], segs = plan_host[PLAN_N_SEGMENTS];
+  if (n_seq < 1 || segs < n_seq) return LAMPA_ERR_INVALID;
+  if (!workspace || workspace_bytes < lampa_gdr_train_workspace_bytes(plan_host, HV)) return LAMPA_ERR_WORKSPACE;
+  const GdrPlanView pv = gdr_plan_view(plan_host, plan_dev);
+  int max_nseg = 0;
+  for (int i = 0; i < n_seq; ++i) max_nseg = plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] > max_nseg ? plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] : max_nseg;
+  const GdrSaved sv = gdr_saved_layout(chunks, segs, HV);
+  unsigned char* sp = (unsigned char*)saved;
+  GdrKeep kp{sp + sv.off_rec, sp + sv.off_states, sp + sv.off_mt, (float*)(sp + sv.off_d), nullptr};
+  if (positive_g_host && hipHostGetDevicePointer((void**)&kp.positive_g, positive_g_host, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    return LAMPA_ERR_INVALID;
+  }
+  if (dtype == GDR_BF16)
+    return gdr_chunk_launch<__bf16, 64, 64, true>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, H, HV, scale,
+                                                  l2norm, (unsigned char*)workspace, (hipStream_t)stream, kp);
+  return gdr_chunk_launch<_Float16, 64, 64, true>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, H, HV, scale,
+                                                  l2norm, (unsigned char*)workspace, (hipStream_t)stream, kp);
 }

@@ -215,7 +215,7 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
                                                           const int32_t* __restrict__ chunk_tok0,
                                                           const int32_t* __restrict__ chunk_len,
                                                           unsigned char* __restrict__ rec, int n_chunks, int H, int HV,
-                                                          int l2norm) {
+                                                          int l2norm, int32_t* positive_g) {
   using X8 = typename OpVec<T>::x8;    // input fragments (the K K^T products run in the input type)
   using O8 = typename OpVec<OT>::x8;   // record elements
   using O2 = typename OpVec<OT>::x2;
@@ -291,7 +291,9 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
   // Fast gating: e^{gamma_i - gamma_j} = E_i / E_j with E = e^{gamma - gamma_ref}, gamma_ref = gamma_last / 2, as long as
   // no exponent can leave the fp32 range (total decay of the chunk above 2^-120) and no g is positive (then every ratio
   // has to go through safe_exp one by one).
-  const bool fast = !__ballot(rg > 0.0f && lane < len) && g_last > -120.0f;
+  const bool rising = __ballot(rg > 0.0f && lane < len) != 0;
+  if (positive_g && rising && lane == 0) *positive_g = 1;  // (for the backward pass, which is defined for g <= 0 only)
+  const bool fast = !rising && g_last > -120.0f;
   const float E = __builtin_amdgcn_exp2f(gcum - 0.5f * g_last), iE = __builtin_amdgcn_exp2f(0.5f * g_last - gcum);
   s_gamma[lane] = gcum;
   s_beta[lane] = bz;
@@ -598,7 +600,10 @@ __device__ __forceinline__ bf16x8 ld_kappa_tr(const __bf16* arr, int stride, int
   return out;
 }
 
-template <typename T, int KT, int VT, bool PASS_B, bool SCALED_K = !PASS_B, typename OT = T, int CW = 32>
+// KEEP (training form, K = V = 64, see gdr_train.h): PASS_A also maps the last segment of a sequence and stores M' once
+// more in the fragment order of its transpose; PASS_B stores the state in front of every chunk -- the operand fragments
+// the chain waves hold anyway, 8 KiB per chunk and head in 1 KiB runs.
+template <typename T, int KT, int VT, bool PASS_B, bool SCALED_K = !PASS_B, typename OT = T, int CW = 32, bool KEEP = false>
 __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
                                   ((SCALED_K || CW == 16) ? GdrSegShape<KT, VT, PASS_B, CW>::WAVES_PER_SIMD : 2))
     gdr_segment_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
@@ -609,7 +614,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
                        unsigned char* __restrict__ Ncomp, float* __restrict__ Dcomp, T* __restrict__ o,
                        float* __restrict__ ht, int H, int HV, float scale, int l2norm,
                        const unsigned char* __restrict__ Mgrp, const unsigned char* __restrict__ Ngrp,
-                       const float* __restrict__ Dgrp, const float* __restrict__ h0, int gmax) {
+                       const float* __restrict__ Dgrp, const float* __restrict__ h0, int gmax,
+                       unsigned char* __restrict__ keep) {
   // OT: the 16-bit type of every MFMA operand (tiles in LDS, T, R, v_new, P, the state as operand, M' of the
   // composites): the input type, so that fp16 inputs run on the fp16 MFMA without losing mantissa bits
   using X8 = typename OpVec<OT>::x8;
@@ -669,7 +675,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   const int hv = gridDim.y > 1 ? blockIdx.y : blockIdx.x % HV;
   const int h = hv / (HV / H);
   const int flags = pv.seg_flags[seg];
-  if (!PASS_B && (flags & SEG_LAST)) return;  // nothing follows the last segment of a sequence
+  if (!PASS_B && !KEEP && (flags & SEG_LAST)) return;  // nothing follows the last segment of a sequence
   const int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg];
   const int c1 = c0 + nc;
   // (the per-chunk tables are separate restrict parameters: read through the view they could alias the kernel's
@@ -1596,6 +1602,11 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
     X8 Sb[KT / 16];
 #pragma unroll
     for (int ks = 0; ks < KT / 16; ++ks) Sb[ks] = acc_to_op<OT>(S[ks / 2], 8 * (ks % 2));
+    if constexpr (KEEP && PASS_B) {
+      unsigned char* st = keep + (((size_t)uniform(c) * HV + hv) * (VT / 32) + vslab) * (KT * 32 * 2);
+#pragma unroll
+      for (int ks = 0; ks < KT / 16; ++ks) op_frag_store<OT>(st, ks, lane, Sb[ks]);
+    }
     lds_fence();
     // batch for stage 2: T fragments and the per-token factors / v tile of stage 1's epilogue
 #pragma unroll
@@ -1776,6 +1787,17 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
             (OT)val;
       }
     if (wave == 0 && lane == 0) Dcomp[(size_t)seg * HV + hv] = dtot;
+    if constexpr (KEEP) {  // accumulator tiles read as A operand are the transpose
+      unsigned char* mt = keep + ((size_t)seg * HV + hv) * (KT * KT * 2);
+#pragma unroll
+      for (int km = 0; km < KT / 32; ++km) {
+        f32x16 m = S[km];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) m[r] -= (32 * km + acc_row(r, hh) == mcol) ? dtot : 0.0f;
+        op_frag_store<OT>(mt, wave * (KT / 16) + 2 * km + 0, lane, acc_to_op<OT>(m, 0));
+        op_frag_store<OT>(mt, wave * (KT / 16) + 2 * km + 1, lane, acc_to_op<OT>(m, 8));
+      }
+    }
   } else {
     // N slab in accumulator order: tile (vslab, km), plane q (registers 4q..4q+3), lane -> 16 bytes
     unsigned char* out = Ncomp + (((size_t)seg * HV + hv) * (VT / 32) + vslab) * (KT * 32 * 4) + late;
@@ -1908,7 +1930,8 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan_kernel(const GdrPlanV
 // Same step code in both modes; loops are branch free with clamped operands and a spare store slot as above.
 enum { SCAN_GROUP = 1, SCAN_LEAF = 2 };
 
-template <typename OT, int KT, int VT, int DEPTH, int MODE>
+// REV (GROUP): the segments of a sequence are taken from the last to the first (the maps of the backward pass).
+template <typename OT, int KT, int VT, int DEPTH, int MODE, bool REV = false>
 __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlanView pv,
                                                                   const unsigned char* __restrict__ Msrc,
                                                                   const unsigned char* __restrict__ Nsrc,
@@ -1932,7 +1955,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
   int item0, nsteps, slot0, lead = 0;  // lead: group-level maps walked before the workgroup's own items (LEAF)
   if (MODE == SCAN_GROUP) {
     if (j >= ngroups - 1) return;  // the composite of a sequence's last group is never needed
-    item0 = seg0 + j * G; nsteps = G - 1; slot0 = 0;
+    item0 = REV ? seg0 + nseg - 1 - j * G : seg0 + j * G; nsteps = G - 1; slot0 = 0;
   } else {
     if (j >= ngroups) return;
     item0 = seg0 + j * G; lead = j; nsteps = lead + min(G, nseg - j * G) - 1; slot0 = item0;
@@ -1958,7 +1981,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
   float rd[DEPTH];
   auto issue = [&](int p, X8* m, f32x4* n, float& d) {
     const bool top = MODE == SCAN_LEAF && p < lead;  // a group composite (read through the *out pointers)
-    const size_t sh = (size_t)(top ? seq * gmax + p : item0 + (p - lead)) * HV + hv;
+    const size_t sh = (size_t)(top ? seq * gmax + p : REV ? item0 - p : item0 + (p - lead)) * HV + hv;
     const X8* M = reinterpret_cast<const X8*>((top ? Mout : Msrc) + sh * M_BYTES);
     const f32x4* N = reinterpret_cast<const f32x4*>((top ? Nout : Nsrc) + (sh * (VT / 32) + nblk) * N_BYTES);
 #pragma unroll

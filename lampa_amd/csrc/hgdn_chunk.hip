@@ -899,7 +899,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   if (chunks == 0) return LAMPA_OK;
   // (the hierarchical kernels keep bf16 operands whatever the input type)
   hipLaunchKernelGGL((gdr_local_kernel<T, __bf16, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g,
-                     beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm);
+                     beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, (int32_t*)nullptr);
   LAMPA_PROF(s, "gdr_local_kernel");
   const bool split = segs > n_seq;
   // The segment composites and their scan depend on T only, like the prep kernel, and are latency bound on a few
@@ -930,7 +930,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
                        dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, cs, (const T*)q, (const T*)k, (const T*)v, g,
                        beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, Mc, Nm, Dc, (T*)nullptr,
                        (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
-                       (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0);
+                       (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, (unsigned char*)nullptr);
     LAMPA_PROF(s, "gdr_segment_kernel<composite>");
     hipLaunchKernelGGL((hgdn_scan_kernel<KT, VT>), dim3(VT / 32, n_seq, HV), dim3(64 * HG_CW), 0, cs, pv, Mc, Nm, Dc, Xi,
                        HV, p);

@@ -6,7 +6,8 @@ defaults, checks and return tuples.  The arithmetic runs in hand-written gfx950 
 C ABI of ``liblampa_amd.so``; there is no Triton, no PyTorch fallback and no CPU path.
 
 Differences that a caller can observe, all additive:
-* ``chunk_gated_delta_rule`` is differentiable (``lampa_gdr_bwd``: fp32, token-serial inside parallel segments);
+* ``chunk_gated_delta_rule`` is differentiable (16-bit inputs and heads up to 64 x 64: the chunked form,
+  ``lampa_gdr_bwd_saved``; everything else ``lampa_gdr_bwd``: fp32, token-serial inside parallel segments);
   ``fused_recurrent_gated_delta_rule``'s backward raises ``NotImplementedError`` as the reference's does;
 * ``allow_fp32=True`` lets ``chunk_gated_delta_rule`` accept float32 q/k/v (the reference rejects them); they
   are evaluated by the token-serial fp32 kernel (long sequences cut into segments that run in parallel);
@@ -313,78 +314,111 @@ def _backward_tables(cu_host, seg_len: int, device):
     return tables
 
 
-# Backward pass in the chunked form on the matrix cores (``lampa_gdr_bwd_chunk``) where it is built: 16-bit inputs,
-# K = V = 64, one value head per q/k head. False sends everything to the fp32 token-serial form (``lampa_gdr_bwd``).
+# Backward pass in the chunked form on the matrix cores (``lampa_gdr_bwd_saved``) where it is built: 16-bit inputs and heads
+# up to 64 x 64. False sends everything to the fp32 token-serial form (``lampa_gdr_bwd``).
 CHUNKED_BACKWARD = True
-
-_backward_plan_cache = {}
-
-
-def _backward_chunk_plan(cu_host, device):
-    """Host + device copies of the chunk tables of ``lampa_gdr_bwd_chunk`` for these sequence boundaries (cached)."""
-    key = (tuple(cu_host), str(device))
-    hit = _backward_plan_cache.get(key)
-    if hit is not None:
-        return hit
-    lib = _capi.lib()
-    cu = (ctypes.c_int64 * len(cu_host))(*cu_host)
-    n_seq = len(cu_host) - 1
-    size = check(lib.lampa_gdr_bwd_chunk_plan_size(cu, n_seq), "lampa_gdr_bwd_chunk_plan_size")
-    host = torch.empty(size, dtype=torch.int32)
-    check(lib.lampa_gdr_bwd_chunk_plan_fill(cu, n_seq, ctypes.c_void_p(host.data_ptr())), "lampa_gdr_bwd_chunk_plan_fill")
-    dev = host.to(device)
-    if len(_backward_plan_cache) > 64:
-        _backward_plan_cache.clear()
-    _backward_plan_cache[key] = (host, dev)
-    return host, dev
-
 
 def _backward_chunk_supported(q, v) -> bool:
     """16-bit inputs with K, V <= 64: smaller heads are zero-padded to 64 x 64 (as in the forward pass: zero columns of
-    q, k and v change neither the function nor the other columns' gradients), and grouped value heads (HV > H) run with
-    q and k repeated per value head, their gradients summed over each group afterwards."""
+    q, k and v change neither the function nor the other columns' gradients)."""
     return (CHUNKED_BACKWARD and q.dtype in (torch.bfloat16, torch.float16) and q.shape[-1] <= 64 and v.shape[-1] <= 64
             and q.data_ptr() % 16 == 0)
 
 
-def _backward_chunk_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, do, dht):
-    """Gradients (dq, dk, dv, dg, dbeta, dh0) through ``lampa_gdr_bwd_chunk`` (built for K = V = 64, HV = H)."""
-    B, T, H, K = q.shape
-    HV, V = v.shape[2], v.shape[3]
-    pad = torch.nn.functional.pad
-    if K < 64:
-        q, k = pad(q, (0, 64 - K)), pad(k, (0, 64 - K))
-    if V < 64:
-        v, do = pad(v, (0, 64 - V)), pad(do, (0, 64 - V))
-    if (K, V) != (64, 64):
-        initial_state = None if initial_state is None else pad(initial_state.to(torch.float32), (0, 64 - V, 0, 64 - K))
-        dht = None if dht is None else pad(dht.to(torch.float32), (0, 64 - V, 0, 64 - K))
-    rep = HV // H
-    if rep > 1:
-        q, k = q.repeat_interleave(rep, dim=2), k.repeat_interleave(rep, dim=2)
-    q, k, v, do = q.contiguous(), k.contiguous(), v.contiguous(), do.contiguous()
+def _pad_last(x, n: int):
+    return x if x is None or x.shape[-1] == n else torch.nn.functional.pad(x, (0, n - x.shape[-1]))
+
+
+def _pad_state(x):
+    """[N, HV, K, V] -> fp32 [N, HV, 64, 64]."""
+    if x is None:
+        return None
+    K, V = x.shape[-2:]
+    x = x.to(torch.float32)
+    return (x if (K, V) == (64, 64) else torch.nn.functional.pad(x, (0, 64 - V, 0, 64 - K))).contiguous()
+
+
+class _Kept:
+    """What the training form of the chunk forward (``lampa_gdr_chunk_fwd_train``) leaves for the backward pass: the plan,
+    the kept buffer (chunk records, states in front of the chunks, transposed segment maps) and the flag for positive
+    entries of g in pinned host memory, valid once ``done`` has passed."""
+    __slots__ = ("plan", "buffer", "flag", "done")
+
+
+def _chunk_train_forward(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm):
+    """The forward for inputs that require gradients: q, k, v padded to 64 x 64 heads -> (o, final state, kept)."""
+    B, T, H, _ = q.shape
+    HV = v.shape[2]
     cu_host = _sequence_bounds(cu_seqlens, B, T)
-    plan_host, plan_dev = _backward_chunk_plan(cu_host, q.device)
-    lib = _capi.lib()
-    ws_bytes = check(lib.lampa_gdr_bwd_chunk_workspace_bytes(ctypes.c_void_p(plan_host.data_ptr()), HV),
-                     "lampa_gdr_bwd_chunk_workspace_bytes")
+    n_seq = len(cu_host) - 1
+    kept = _Kept()
+    kept.plan = _plan(cu_host, q.device, HV, (64, 64))
+    plan_host, plan_dev = kept.plan
+    lib, host_ptr = _capi.lib(), ctypes.c_void_p(plan_host.data_ptr())
+    n_saved = check(lib.lampa_gdr_train_saved_bytes(host_ptr, HV), "lampa_gdr_train_saved_bytes")
+    ws_bytes = check(lib.lampa_gdr_train_workspace_bytes(host_ptr, HV), "lampa_gdr_train_workspace_bytes")
+    kept.buffer = torch.empty(n_saved, dtype=torch.uint8, device=q.device)
+    kept.flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    dg, dbeta = torch.empty_like(g), torch.empty_like(beta)
-    h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
-    dht = None if dht is None else dht.to(torch.float32).contiguous()
-    dh0 = None if h0 is None else torch.empty_like(h0)
-    check(lib.lampa_gdr_bwd_chunk(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(h0), ptr(do), ptr(dht), ptr(dq), ptr(dk),
-                                  ptr(dv), ptr(dg), ptr(dbeta), ptr(dh0), ctypes.c_void_p(plan_host.data_ptr()),
-                                  ptr(plan_dev), HV, HV, 64, 64, _DTYPES[q.dtype], float(scale), l2norm, ptr(ws), ws_bytes,
-                                  stream_of(q)), "lampa_gdr_bwd_chunk")
-    if rep > 1:  # the value heads of a group share their q / k head
-        dq = dq.view(B, T, H, rep, 64).float().sum(3).to(q.dtype)
-        dk = dk.view(B, T, H, rep, 64).float().sum(3).to(k.dtype)
-    if (K, V) != (64, 64):
-        dq, dk, dv = dq[..., :K].contiguous(), dk[..., :K].contiguous(), dv[..., :V].contiguous()
-        dh0 = None if dh0 is None else dh0[..., :K, :V].contiguous()
+    o = torch.empty_like(v)
+    ht = torch.empty((n_seq, HV, 64, 64), dtype=torch.float32, device=q.device) if output_final_state else None
+    h0 = _pad_state(initial_state)
+    check(lib.lampa_gdr_chunk_fwd_train(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(o), ptr(h0), ptr(ht), host_ptr,
+                                        ptr(plan_dev), H, HV, 64, 64, _DTYPES[q.dtype], float(scale), l2norm,
+                                        ptr(kept.buffer), ctypes.c_void_p(kept.flag.data_ptr()), ptr(ws), ws_bytes,
+                                        stream_of(q)), "lampa_gdr_chunk_fwd_train")
+    kept.done = torch.cuda.Event()
+    kept.done.record(torch.cuda.current_stream(q.device))
+    return o, ht, kept
+
+
+def _raise_positive_g():
+    # the forward masks decay ratios with a positive exponent (safe_exp); the gradients here are those of the unmasked
+    # recurrence, which is the same function only for g <= 0
+    raise ValueError("chunk_gated_delta_rule backward: g has positive entries; the gradients are defined for log-decays "
+                     "g <= 0 only (the forward masks decay ratios with positive exponents, the backward pass differentiates "
+                     "the unmasked recurrence)")
+
+
+def _backward_kept_launch(q, k, v, kept, scale, l2norm, do, dht, want_dh0):
+    """Gradients (dq, dk, dv, dg, dbeta, dh0) through ``lampa_gdr_bwd_saved``; q, k, v, do with 64 x 64 heads. dq and dk come
+    back with one row per value head when value heads share q / k heads: summed over each group here."""
+    B, T, H, _ = q.shape
+    HV = v.shape[2]
+    plan_host, plan_dev = kept.plan
+    lib, host_ptr = _capi.lib(), ctypes.c_void_p(plan_host.data_ptr())
+    ws_bytes = check(lib.lampa_gdr_bwd_saved_workspace_bytes(host_ptr, HV), "lampa_gdr_bwd_saved_workspace_bytes")
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+    dq, dk, dv = (torch.empty((B, T, HV, 64), dtype=q.dtype, device=q.device) for _ in range(3))
+    dg, dbeta = (torch.empty((B, T, HV), dtype=torch.float32, device=q.device) for _ in range(2))
+    n_seq = int(plan_host[0])
+    dh0 = torch.empty((n_seq, HV, 64, 64), dtype=torch.float32, device=q.device) if want_dh0 else None
+    check(lib.lampa_gdr_bwd_saved(ptr(q), ptr(k), ptr(v), ptr(kept.buffer), ptr(do), ptr(dht), ptr(dq), ptr(dk), ptr(dv),
+                                  ptr(dg), ptr(dbeta), ptr(dh0), host_ptr, ptr(plan_dev), H, HV, 64, 64, _DTYPES[q.dtype],
+                                  float(scale), l2norm, ptr(ws), ws_bytes, stream_of(q)), "lampa_gdr_bwd_saved")
+    if HV > H:
+        dq = dq.view(B, T, H, HV // H, 64).float().sum(3).to(q.dtype)
+        dk = dk.view(B, T, H, HV // H, 64).float().sum(3).to(k.dtype)
     return dq, dk, dv, dg, dbeta, dh0
+
+
+def _cut_heads(grads, K: int, V: int):
+    """The gradients of padded heads -> the caller's head sizes."""
+    if (K, V) == (64, 64):
+        return grads
+    dq, dk, dv, dg, dbeta, dh0 = grads
+    return (dq[..., :K].contiguous(), dk[..., :K].contiguous(), dv[..., :V].contiguous(), dg, dbeta,
+            None if dh0 is None else dh0[..., :K, :V].contiguous())
+
+
+def _backward_chunk_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, do, dht):
+    """Gradients in the chunked form from the inputs alone: the training form of the forward (its outputs dropped), then the
+    backward pass over what it kept."""
+    K, V = q.shape[-1], v.shape[-1]
+    q, k, v, do = (_pad_last(x, 64).contiguous() for x in (q, k, v, do))
+    _, _, kept = _chunk_train_forward(q, k, v, g, beta, scale, initial_state, False, cu_seqlens, l2norm)
+    return _cut_heads(_backward_kept_launch(q, k, v, kept, scale, l2norm, do, _pad_state(dht), initial_state is not None),
+                      K, V)
 
 
 def _backward_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, do, dht):
@@ -440,12 +474,23 @@ class _GatedDelta(torch.autograd.Function):
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
         ctx.differentiable = differentiable
+        ctx.kept = None
+        ctx.set_materialize_grads(False)
         if differentiable:
+            ctx.scale, ctx.l2norm, ctx.head = scale, l2norm, (q.shape[-1], v.shape[-1])
+            if (any(ctx.needs_input_grad) and launcher is _chunk_launch_any_head and _backward_chunk_supported(q, v)
+                    and q.shape[0] * q.shape[1] > 0):
+                K, V = ctx.head
+                q, k, v = _pad_last(q, 64), _pad_last(k, 64), _pad_last(v, 64)
+                o, ht, ctx.kept = _chunk_train_forward(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
+                                                       l2norm)
+                ctx.save_for_backward(q, k, v, initial_state, ctx.kept.buffer)
+                ctx.kept.buffer = None
+                if (K, V) != (64, 64):
+                    o, ht = o[..., :V].contiguous(), None if ht is None else ht[..., :K, :V].contiguous()
+                return o, ht
             ctx.save_for_backward(q, k, v, g, beta, initial_state, cu_seqlens)
-            ctx.scale, ctx.l2norm = scale, l2norm
-        o, ht = launcher(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm)
-        ctx.o_shape, ctx.o_dtype = o.shape, o.dtype
-        return o, ht
+        return launcher(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm)
 
     @staticmethod
     def backward(ctx, do, dht):
@@ -454,17 +499,24 @@ class _GatedDelta(torch.autograd.Function):
                 "Backward pass is not implemented yet and we do not have plans to implement it "
                 "because we haven't figured out how to compute dg without materializing the full "
                 "hidden states for all time steps.")
-        q, k, v, g, beta, initial_state, cu_seqlens = ctx.saved_tensors
-        if bool((g > 0).any()):
-            # the forward masks decay ratios with a positive exponent (safe_exp); the gradients here are those of the
-            # unmasked recurrence, which is the same function only for g <= 0
-            raise ValueError("chunk_gated_delta_rule backward: g has positive entries; the gradients are defined for "
-                             "log-decays g <= 0 only (the forward masks decay ratios with positive exponents, the "
-                             "backward pass differentiates the unmasked recurrence)")
-        if do is None:
-            do = torch.zeros(ctx.o_shape, dtype=ctx.o_dtype, device=q.device)
-        dq, dk, dv, dg, dbeta, dh0 = _backward_launch(q, k, v, g, beta, ctx.scale, initial_state, cu_seqlens,
-                                                      ctx.l2norm, do.to(v.dtype), dht)
+        if ctx.kept is not None:
+            q, k, v, initial_state, buffer = ctx.saved_tensors
+            kept = _Kept()
+            kept.plan, kept.buffer = ctx.kept.plan, buffer
+            do = torch.zeros_like(v) if do is None else _pad_last(do.to(v.dtype), 64).contiguous()
+            grads = _cut_heads(_backward_kept_launch(q, k, v, kept, ctx.scale, ctx.l2norm, do, _pad_state(dht),
+                                                     initial_state is not None), *ctx.head)
+            # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them
+            ctx.kept.done.synchronize()
+            if int(ctx.kept.flag[0]):
+                _raise_positive_g()
+        else:
+            q, k, v, g, beta, initial_state, cu_seqlens = ctx.saved_tensors
+            if bool((g > 0).any()):
+                _raise_positive_g()
+            do = torch.zeros_like(v) if do is None else do.to(v.dtype)
+            grads = _backward_launch(q, k, v, g, beta, ctx.scale, initial_state, cu_seqlens, ctx.l2norm, do, dht)
+        dq, dk, dv, dg, dbeta, dh0 = grads
         if dh0 is not None:
             dh0 = dh0.to(initial_state.dtype)
         return (None, dq, dk, dv, dg.to(ctx.g_dtype), dbeta.to(ctx.beta_dtype), None, dh0, None, None, None, None)

@@ -249,6 +249,24 @@ def test_chunked_gradients_long_sequence_weak_decay_against_oracle(device):
     _check(got, want, torch.bfloat16, chunked=True)
 
 
+@pytest.mark.parametrize("T,K,V", [(64 * 23, 64, 64), (64 * 24, 64, 64), (64 * 26 + 1, 64, 64), (63, 48, 64), (65, 64, 40)])
+def test_chunked_gradients_one_chunk_per_segment(device, T, K, V, monkeypatch):
+    """Segments of one chunk, so that a sequence has 23 (the walk passes all of them one by one), 24 (groups of 8, no
+    remainder) and 27 segments (groups and a remainder); one partial chunk, and a second chunk of one token; grouped value
+    heads, heads below 64 x 64. The gradients are taken twice from one graph: the kept buffer is only read."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 1)
+    (q, k, v, g, beta, do), gen = _inputs(1, T, 1, 2, K, V, torch.bfloat16, T + K, unit=False, g_scale=0.02)
+    h0 = 0.5 * torch.randn(1, 2, K, V, generator=gen)
+    dht = torch.randn(1, 2, K, V, generator=gen)
+    want = ob.backward_manual(q, k, v, g, beta, do, dht, None, h0, None, og.L2_CHUNK)
+    leaves = [x.to(device).requires_grad_(True) for x in (q, k, v, g, beta, h0)]
+    o, ht = gd.chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], output_final_state=True,
+                                      use_qk_l2norm_in_kernel=True)
+    for _ in range(2):
+        got = torch.autograd.grad((o, ht), leaves, (do.to(device), dht.to(device)), retain_graph=True)
+        _check(got, want, torch.bfloat16, chunked=True)
+
+
 def test_chunked_gradients_at_full_size_against_the_token_serial_form(device, monkeypatch):
     """Config-2 shape (60 000 tokens, 8 heads, K = V = 64, bf16), too long for the float64 loop: the chunked form on the
     MFMA against the fp32 token-serial form, two implementations that share no kernel of the backward pass."""
