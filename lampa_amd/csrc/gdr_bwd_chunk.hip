@@ -17,54 +17,68 @@
 // behind it to the gradient in front of it by G -> M^T G + N', with the M the forward composite pass already made.
 //   forward   (gdr_chunk.hip, training form) leaves the chunks' records, the state in front of every chunk (16-bit operand
 //             fragments) and the transposed M of every segment;
-//   source    gdrb_segment_kernel<false>: every segment's N' (the walk below from a zero gradient, nothing else);
+//   source    gdrb_source_kernel: every segment's N' (the walk below from a zero gradient, nothing else);
 //   group     gdr_scan2_kernel, reversed: composites of groups of 8 segments of long sequences;
-//   walk      gdrb_segment_kernel<true>: a workgroup pushes the gradient behind the sequence through the composites of the
+//   walk      gdrb_walk_kernel: a workgroup pushes the gradient behind the sequence through the composites of the
 //             later segments, then walks its own chunks from the last to the first and writes every gradient of each.
 #include "gdr_chunk_kernels.h"
 #include "gdr_train.h"
 #include <mutex>
 
-#define GB_THREADS 512
 #define GB_LS 72                    // row stride (16-bit elements) of the k, q and dO tiles: 16-byte aligned rows
 #define GB_TS 36                    // row stride of a 32 x 32 block of T
 #define GB_TRI 2048                 // bytes of one 32 x 32 tile in operand fragment order
+#define GB_SOURCE_THREADS 512
+#define GB_WALK_THREADS 768
 
-// LDS of the kernel (bytes). Fragment order of a 64 x 64 tile with rows r and columns c: fragment 4 (c / 32) + r / 16,
-// lane 32 ((r / 4) % 2) + c % 32, element 4 ((r / 8) % 2) + r % 4 -- what a lane holds of an accumulator tile, rounded.
+// One set of a chunk's tiles in LDS (bytes). Fragment order of a 64 x 64 tile with rows r and columns c: fragment
+// 4 (c / 32) + r / 16, lane 32 ((r / 4) % 2) + c % 32, element 4 ((r / 8) % 2) + r % 4 -- what a lane holds of an
+// accumulator tile, rounded.
 template <bool GRADS>
-struct GbSmem {
+struct GbSet {
   static constexpr int TILE = 64 * GB_LS * 2;
-  static constexpr int OFF_K = 0;                           // kh rows; at the end of a chunk the rows of dk
-  static constexpr int OFF_Q = OFF_K + TILE;                // qh rows; at the end of a chunk the rows of dq
+  static constexpr int OFF_K = 0;                           // kh rows
+  static constexpr int OFF_Q = OFF_K + TILE;                // qh rows
   static constexpr int OFF_DO = OFF_Q + TILE;
-  static constexpr int OFF_T = OFF_DO + TILE;               // T11 | T21 | T22; later M (grad A gated), three tiles
-  static constexpr int OFF_P = OFF_T + 3 * 32 * GB_TS * 2;  // P, three tiles; later the waves' partial sums (GbSums)
-  static constexpr int OFF_F = OFF_P + 3 * GB_TRI;
-  static constexpr int OFF_N = OFF_F + 7 * 256;             // N (grad P gated), three tiles
-  static constexpr int OFF_V = OFF_N + (GRADS ? 3 * GB_TRI : 0);  // v as two 64 x 32 tiles, then Vn (fragment order)
-  static constexpr int OFF_S = OFF_V + (GRADS ? 8192 : 0);
-  static constexpr int OFF_G = OFF_S + (GRADS ? 8192 : 0);
-  static constexpr int OFF_X = OFF_G + (GRADS ? 8192 : 0);
-  static constexpr int BYTES = OFF_X + (GRADS ? 8192 : 0);
+  static constexpr int OFF_T = OFF_DO + TILE;               // T11 | T21 | T22
+  static constexpr int OFF_F = OFF_T + 3 * 32 * GB_TS * 2;  // rows of 64 floats: gamma, beta, e^gamma, e^{gamma_L - gamma}, rk, rq
+  static constexpr int OFF_V = OFF_F + 6 * 256;             // v as two 64 x 32 tiles, then Vn (fragment order)
+  static constexpr int OFF_S = OFF_V + (GRADS ? 8192 : 0);  // the state in front of the chunk (fragment order)
+  static constexpr int BYTES = OFF_S + (GRADS ? 8192 : 0);
 };
-static_assert(GbSmem<true>::BYTES <= 81920, "two workgroups per CU");
 
-// The partial sums of a chunk (float offsets into the dead P tiles): every wave writes its own, wave 2 adds them up. (As
-// LDS atomics they took a third of the kernel's LDS cycles.)
+// The partial sums of a chunk (float offsets): every wave writes its own, wave 7 adds them up. (As LDS atomics they took
+// half of the kernel's LDS cycles.)
 struct GbSums {
-  static constexpr int DOTQ = 0;                 // [2][64] products of the rows of dQh / dKh with qh / kh, per half of the columns
-  static constexpr int DOTK = DOTQ + 128;
-  static constexpr int DGAM = DOTK + 128;        // [8 waves][32] d gamma of the wave's tokens 32 (wave % 2) ..
-  static constexpr int TILE_G = DGAM + 256;      // [3 tiles][32] d gamma of the tile's columns i
+  static constexpr int DOTK = 0;                 // [2][64] products of the rows of dKh with kh, per half of the columns
+  static constexpr int DGAM = DOTK + 128;        // [6][32] d gamma: the two dQh waves, then the four dKh waves
+  static constexpr int TILE_G = DGAM + 192;      // [3 tiles][32] d gamma of the tile's columns i
   static constexpr int TILE_C = TILE_G + 96;     // [3 tiles][32] and of its rows j (to be subtracted)
   static constexpr int TILE_B = TILE_C + 96;     // [3 tiles][32] d beta of the columns
-  static constexpr int DBETA = TILE_B + 96;      // [waves 4 .. 7][32] d beta of the wave's tokens
-  static constexpr int XV = DBETA + 128;         // [2][64] X . v per half of the columns
-  static constexpr int GL = XV + 128;            // [waves 4 .. 7][2] the terms of d gamma that belong to the chunk's last row
-  static constexpr int FLOATS = GL + 8;
+  static constexpr int DBETA = TILE_B + 96;      // [four dKh waves][32] d beta of the wave's tokens
+  static constexpr int XV = DBETA + 128;         // [64] X . v
+  static constexpr int GL = XV + 64;             // [5][2] the terms of d gamma that belong to the chunk's last row: dKh waves, wave 7
+  static constexpr int FLOATS = GL + 12;
 };
-static_assert(GbSums::FLOATS * 4 <= 3 * GB_TRI, "partial sums over the P tiles");
+
+// LDS of the walk: two sets of tiles, what the waves exchange inside a chunk, the rows of dq and dk on their way out.
+struct GbWalkSmem {
+  static constexpr int OFF_P = 2 * GbSet<true>::BYTES;  // P, N (grad P gated), M (grad A gated): three 32 x 32 tiles each
+  static constexpr int OFF_N = OFF_P + 3 * GB_TRI;
+  static constexpr int OFF_M = OFF_N + 3 * GB_TRI;
+  static constexpr int OFF_G = OFF_M + 3 * GB_TRI;      // G' (fragment order)
+  static constexpr int OFF_X = OFF_G + 8192;            // X (fragment order)
+  static constexpr int OFF_OQ = OFF_X + 8192;
+  static constexpr int OFF_OK = OFF_OQ + 64 * GB_LS * 2;
+  static constexpr int OFF_SUM = OFF_OK + 64 * GB_LS * 2;
+  static constexpr int BYTES = OFF_SUM + 4 * GbSums::FLOATS;
+};
+static_assert(GbWalkSmem::BYTES <= 163840, "LDS of a CU");
+struct GbSourceSmem {
+  static constexpr int OFF_P = 2 * GbSet<false>::BYTES;
+  static constexpr int BYTES = OFF_P + 3 * GB_TRI;
+};
+static_assert(GbSourceSmem::BYTES <= 81920, "two workgroups per CU");
 
 // Transposing read of a tile in fragment order: operand row / column = tile row r0 + lane % 32, contraction over the tile
 // columns c0 .. c0 + 15; KAPPA: in accumulator slot order, otherwise consecutive (slots of lane half hh: 8 hh ..).
@@ -134,168 +148,552 @@ __device__ __forceinline__ f32x4 gb_rows4(const float* f, int r0, int b4, int hh
   return *reinterpret_cast<const f32x4*>(&f[r0 + 8 * b4 + 4 * hh]);
 }
 
-// The walk of one (segment, head) from its last chunk to its first. Grid segments x heads (long segments first), eight
-// waves. GRADS false: from a zero gradient, writes the segment's N' and nothing else.
-//   waves 0, 1  the gradient of the state, 32 value columns each, in accumulators: dVn -> X -> the next gradient, every
-//               intermediate handed on in registers (accumulator = operand, as in the forward pass)
-//   waves 2, 3  Vn = T B (V - E Kh S) for 32 value columns each
-//   waves 4-6   the three token x token tiles (j tile, i tile) = (0,0), (0,1), (1,1): P, then grad P and grad A with their
-//               gating and their sums over the rows and columns (rows j in the registers, the lane holds i)
-//   waves 0-3 / 4-7  one 32 x 32 tile each of dQh^T / dKh^T (lane = token: per-token factors and row sums are one scalar
-//               or one in-lane sum)
-// The tiles of the next chunk are loaded into registers while this one is worked on.
-// Bound by the latency of a chunk's dependent stages (about 17 700 cycles per chunk, of which 2 000 stage, 10 000 are the
-// four phases between barriers (0) and (4), and 3 900 the rows' normalisation and the stores). The gradients form takes one
-// workgroup per CU (212 registers): two of them with 128 registers spill, and every reload waits for the tiles being
-// prefetched (395 against 256 us at 60 000 tokens x 8 heads). The source form fits 128 and shares a CU (74 us).
-template <typename T, bool GRADS>
-__global__ void __launch_bounds__(GB_THREADS, GRADS ? 2 : 4)
-    gdrb_segment_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
-                        const T* __restrict__ dout, const unsigned char* __restrict__ recs,
-                        const unsigned char* __restrict__ states, const GdrPlanView pv,
-                        const int32_t* __restrict__ chunk_tok0, const int32_t* __restrict__ chunk_len,
-                        const unsigned char* __restrict__ Mt, const float* __restrict__ Dc,
-                        unsigned char* __restrict__ Nr, const unsigned char* __restrict__ Mgrp,
-                        const unsigned char* __restrict__ Ngrp, const float* __restrict__ Dgrp, int gmax,
-                        const float* __restrict__ dht, T* __restrict__ dq, T* __restrict__ dk, T* __restrict__ dv,
-                        float* __restrict__ dg, float* __restrict__ dbeta, float* __restrict__ dh0, int H, int HV,
-                        float scale, int l2norm) {
+// Fragments requested together: passing them through an asm behind all the reads keeps the MFMAs that use them there (an
+// MFMA is no memory access, and left alone the compiler puts each one behind its own read and pays the LDS latency each time).
+template <int N, typename X8>
+__device__ __forceinline__ void gb_pin(X8 (&x)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) asm volatile("" : "+v"(x[j]));
+}
+
+// One 16-bit set of tiles in LDS
+template <typename OT>
+struct GbTiles {
+  OT *k, *q, *dout, *t, *v;
+  unsigned char* s;
+  float *gam, *beta, *eg, *dk, *rk, *rq;
+};
+template <typename OT, bool GRADS>
+__device__ __forceinline__ GbTiles<OT> gb_tiles(unsigned char* smem, int par) {
+  unsigned char* b = smem + par * GbSet<GRADS>::BYTES;
+  GbTiles<OT> t;
+  t.k = reinterpret_cast<OT*>(b + GbSet<GRADS>::OFF_K);
+  t.q = reinterpret_cast<OT*>(b + GbSet<GRADS>::OFF_Q);
+  t.dout = reinterpret_cast<OT*>(b + GbSet<GRADS>::OFF_DO);
+  t.t = reinterpret_cast<OT*>(b + GbSet<GRADS>::OFF_T);
+  t.v = reinterpret_cast<OT*>(b + GbSet<GRADS>::OFF_V);
+  t.s = b + GbSet<GRADS>::OFF_S;
+  t.gam = reinterpret_cast<float*>(b + GbSet<GRADS>::OFF_F);
+  t.beta = t.gam + 64;
+  t.eg = t.gam + 128;
+  t.dk = t.gam + 192;
+  t.rk = t.gam + 256;
+  t.rq = t.gam + 320;
+  return t;
+}
+
+// operand fragments of the row-major tiles: rows in accumulator slot order / in consecutive order, and the transpose
+template <typename OT>
+__device__ __forceinline__ typename OpVec<OT>::x8 gb_rows_k(const OT* buf, int row, int c, int hh) {
+  return op_ld_kappa<OT>(buf, GB_LS, row, c, hh);
+}
+template <typename OT>
+__device__ __forceinline__ typename OpVec<OT>::x8 gb_rows_n(const OT* buf, int row, int c, int hh) {
+  return *reinterpret_cast<const typename OpVec<OT>::x8*>(&buf[row * GB_LS + c + 8 * hh]);
+}
+template <typename OT>
+__device__ __forceinline__ typename OpVec<OT>::x8 gb_cols(const OT* buf, int col0, int row0, int lane) {
+  return op_ld_kappa_tr<OT, false>(buf, GB_LS, col0, row0, lane);
+}
+// a 32 x 32 product over 64 contraction steps, both operands from LDS, all eight fragments requested first
+template <typename OT, typename FA, typename FB>
+__device__ __forceinline__ f32x16 gb_mm(f32x16 acc, FA fa, FB fb) {
+  typename OpVec<OT>::x8 a[4], b[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) { a[ks] = fa(ks); b[ks] = fb(ks); }
+  gb_pin(a);
+  gb_pin(b);
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) acc = mfma32(a[ks], b[ks], acc);
+  return acc;
+}
+// the same over the token steps a triangular tile leaves: lower (first 2 (tt + 1) of 4) or upper (from 2 tt on)
+template <typename OT, bool LOWER, typename FA, typename FB>
+__device__ __forceinline__ f32x16 gb_mm_tri(f32x16 acc, int tt, FA fa, FB fb) {
+  if (tt == (LOWER ? 1 : 0)) return gb_mm<OT>(acc, fa, fb);
+  typename OpVec<OT>::x8 a[2], b[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) { a[x] = fa(LOWER ? x : 2 + x); b[x] = fb(LOWER ? x : 2 + x); }
+  gb_pin(a);
+  gb_pin(b);
+  acc = mfma32(a[0], b[0], acc);
+  return mfma32(a[1], b[1], acc);
+}
+
+// The tile (j tile, i tile) of Q K^T (rows j, column i): scaled and gated it is P^T's operand and grad P's counterpart.
+template <typename OT>
+__device__ __forceinline__ f32x16 gb_pair(const OT* rows, int jt, const OT* colsb, int it, int ln, int hh) {
+  return gb_mm<OT>(zero16(), [&](int ks) { return gb_rows_n<OT>(rows, 32 * jt + ln, 16 * ks, hh); },
+                   [&](int ks) { return gb_rows_n<OT>(colsb, 32 * it + ln, 16 * ks, hh); });
+}
+// e^{gamma_i - gamma_j} of the tile for i >= j + e_min, else 0
+__device__ __forceinline__ f32x16 gb_ratio(const float* gam, int jt, int it, int e_min, int ln, int hh) {
+  const float gi = gam[32 * it + ln];
+  const int lx = ln - 4 * hh - e_min + (jt != it ? 64 : 0);  // (the tile below the diagonal is full)
+  f32x16 out;
+#pragma unroll
+  for (int b4 = 0; b4 < 4; ++b4) {
+    const f32x4 gj = gb_rows4(gam, 32 * jt, b4, hh);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[4 * b4 + e] = __builtin_amdgcn_exp2f(lx >= 8 * b4 + e ? gi - gj[e] : -1e30f);
+  }
+  return out;
+}
+template <typename OT>
+__device__ __forceinline__ void gb_store_tile(unsigned char* tile, const f32x16& x, int lane) {
+  op_frag_store<OT>(tile, 0, lane, acc_to_op<OT>(x, 0));
+  op_frag_store<OT>(tile, 1, lane, acc_to_op<OT>(x, 8));
+}
+
+// The gradient of the state: a wave's 32 value columns (all 64 rows) in accumulators. Every intermediate is handed on in
+// registers: the accumulator tile of one product is the B operand of the next.
+template <typename OT>
+struct GbChain {
+  using X8 = typename OpVec<OT>::x8;
+  f32x16 G[2];  // the gradient behind the chunk
+  f32x16 a[2];  // D Kh G', then dVn, then X
+  X8 Xb[4];     // -beta e^gamma X as operand
+
+  // a = D Kh G'; frags (nullable): G' goes there in fragment order
+  __device__ __forceinline__ void state_rows(const GbTiles<OT>& t, unsigned char* frags, int slab, int lane, int hh, int ln) {
+    X8 Gb[4], fk[8];
+#pragma unroll
+    for (int f = 0; f < 8; ++f) fk[f] = gb_rows_k<OT>(t.k, 32 * (f >> 2) + ln, 16 * (f & 3), hh);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      Gb[ks] = acc_to_op<OT>(G[ks / 2], 8 * (ks % 2));
+      if (frags) op_frag_store<OT>(frags, slab * 4 + ks, lane, Gb[ks]);
+    }
+    gb_pin(fk);
+    a[0] = zero16();
+    a[1] = zero16();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      a[0] = mfma32(fk[ks], Gb[ks], a[0]);
+      a[1] = mfma32(fk[4 + ks], Gb[ks], a[1]);
+    }
+#pragma unroll
+    for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+      for (int b4 = 0; b4 < 4; ++b4) {
+        const f32x4 f = gb_rows4(t.dk, 32 * tm, b4, hh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[tm][4 * b4 + e] *= f[e];
+      }
+  }
+  // dVn = a + P^T dO, X = T^T dVn; X goes to frags (nullable) in fragment order
+  __device__ __forceinline__ void chunk_rows(const GbTiles<OT>& t, const unsigned char* p, unsigned char* frags, int slab,
+                                             int lane, int hh) {
+    {
+      X8 d[4], fp[6];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) d[ks] = gb_cols<OT>(t.dout, 32 * slab, 16 * ks, lane);
+#pragma unroll
+      for (int f = 0; f < 6; ++f) fp[f] = fr_tr<OT, true>(p + (f >> 1) * GB_TRI, 0, 16 * (f & 1), lane);
+      gb_pin(d);
+      gb_pin(fp);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        a[0] = mfma32(fp[ks], d[ks], a[0]);
+        if (ks >= 2) a[1] = mfma32(fp[2 + ks], d[ks], a[1]);
+      }
+    }
+    X8 ft[6];
+#pragma unroll
+    for (int f = 0; f < 6; ++f)
+      ft[f] = op_ld_kappa_tr<OT, false>(t.t + (f >> 1) * 32 * GB_TS, GB_TS, 0, 16 * (f & 1), lane);
+    X8 Rb[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) Rb[ks] = acc_to_op<OT>(a[ks / 2], 8 * (ks % 2));
+    gb_pin(ft);
+    a[0] = zero16();
+    a[1] = zero16();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {  // (blocks T11, T21 | T22)
+      a[0] = mfma32(ft[ks], Rb[ks], a[0]);
+      if (ks >= 2) a[1] = mfma32(ft[2 + ks], Rb[ks], a[1]);
+    }
+#pragma unroll
+    for (int tm = 0; tm < 2; ++tm) {
+      if (frags) {
+        op_frag_store<OT>(frags, slab * 4 + 2 * tm + 0, lane, acc_to_op<OT>(a[tm], 0));
+        op_frag_store<OT>(frags, slab * 4 + 2 * tm + 1, lane, acc_to_op<OT>(a[tm], 8));
+      }
+#pragma unroll
+      for (int b4 = 0; b4 < 4; ++b4) {
+        const f32x4 fb = gb_rows4(t.beta, 32 * tm, b4, hh), fe = gb_rows4(t.eg, 32 * tm, b4, hh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[tm][4 * b4 + e] *= -fb[e] * fe[e];
+      }
+      Xb[2 * tm + 0] = acc_to_op<OT>(a[tm], 0);
+      Xb[2 * tm + 1] = acc_to_op<OT>(a[tm], 8);
+    }
+  }
+  // the gradient in front of the chunk: e^{gamma_L} G' + (scale e^gamma Qh)^T dO - (beta e^gamma Kh)^T X
+  __device__ __forceinline__ void update(const GbTiles<OT>& t, float scale, int slab, int lane, int hh) {
+    const float dec = __builtin_amdgcn_exp2f(t.gam[63]);
+#pragma unroll
+    for (int km = 0; km < 2; ++km)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) G[km][r] *= dec;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      X8 f[8], d[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int ks = 2 * half + x;
+        d[x] = gb_cols<OT>(t.dout, 32 * slab, 16 * ks, lane);
+#pragma unroll
+        for (int km = 0; km < 2; ++km) {
+          f[4 * x + km] = gb_cols<OT>(t.q, 32 * km, 16 * ks, lane);
+          f[4 * x + 2 + km] = gb_cols<OT>(t.k, 32 * km, 16 * ks, lane);
+        }
+      }
+      gb_pin(d);
+      gb_pin(f);
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int ks = 2 * half + x;
+        const f32x4 f0 = *reinterpret_cast<const f32x4*>(&t.eg[16 * ks + 4 * hh]);
+        const f32x4 f1 = *reinterpret_cast<const f32x4*>(&t.eg[16 * ks + 8 + 4 * hh]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          d[x][e] = (OT)((float)d[x][e] * (scale * f0[e]));
+          d[x][4 + e] = (OT)((float)d[x][4 + e] * (scale * f1[e]));
+        }
+#pragma unroll
+        for (int km = 0; km < 2; ++km) {
+          G[km] = mfma32(f[4 * x + 2 + km], Xb[ks], G[km]);
+          G[km] = mfma32(f[4 * x + km], d[x], G[km]);
+        }
+      }
+    }
+  }
+};
+
+// ---- staging of a chunk's tiles: loads into registers a chunk ahead, LDS writes when the other set is free ----------------
+// k, q rows through the l2 normalisation: 256 threads, rows gt / 8 and 32 + gt / 8, 8-column piece gt % 8
+template <typename T>
+struct GbStageKQ {
+  using OT = T;
+  using X8 = typename OpVec<OT>::x8;
+  typename Raw8<T>::type pk[2], pq[2];
+  float prk[2];
+  __device__ __forceinline__ void issue(const T* k, const T* q, const unsigned char* rec, int tok0, int len, int H, int h, int gt) {
+    const float* rk = reinterpret_cast<const float*>(rec + T_BYTES) + 128;
+    const size_t row0 = ((size_t)tok0 * H + h) * 64;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = 32 * u + (gt >> 3), r = min(row, len - 1);
+      const uint32_t at = (uint32_t)(r * H * 64 + 8 * (gt & 7));  // (from the chunk's first row: one register per lane)
+      pk[u] = *reinterpret_cast<const typename Raw8<T>::type*>(k + row0 + at);
+      pq[u] = *reinterpret_cast<const typename Raw8<T>::type*>(q + row0 + at);
+      prk[u] = rk[row];
+    }
+  }
+  __device__ __forceinline__ void stage_k(const GbTiles<OT>& t, int len, int l2norm, int gt) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = 32 * u + (gt >> 3), part = gt & 7;
+      const bool live = row < len;  // (rows past the end of a partial chunk become zero)
+      const float ck = live ? prk[u] : 0.0f;
+      X8 ok;
+      if (l2norm != GDR_L2_NONE) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ok[e] = (OT)((float)pk[u][e] * ck);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ok[e] = live ? (OT)pk[u][e] : (OT)0.0f;
+      }
+      *reinterpret_cast<X8*>(&t.k[row * GB_LS + 8 * part]) = ok;
+    }
+  }
+  __device__ __forceinline__ void stage_q(const GbTiles<OT>& t, int len, int l2norm, int gt) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = 32 * u + (gt >> 3), part = gt & 7;
+      const bool live = row < len;
+      float cq = 1.0f;
+      X8 oq;
+      if (l2norm != GDR_L2_NONE) {
+        float fq[8], ss = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          fq[e] = live ? (float)pq[u][e] : 0.0f;
+          ss = __builtin_fmaf(fq[e], fq[e], ss);
+        }
+        cq = l2_factor(gb_sum8(ss), l2norm);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) oq[e] = (OT)(fq[e] * cq);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) oq[e] = live ? (OT)pq[u][e] : (OT)0.0f;
+      }
+      *reinterpret_cast<X8*>(&t.q[row * GB_LS + 8 * part]) = oq;
+      if (part == 0) t.rq[row] = cq;
+    }
+  }
+};
+// dO rows and T (and v, S): NT threads
+template <typename T, int NT, bool GRADS>
+struct GbStageRest {
   using OT = T;
   using X8 = typename OpVec<OT>::x8;
   using X4 = typename OpVec<OT>::x4;
-  using SM = GbSmem<GRADS>;
+  static constexpr int NR = 512 / NT, NP = NT == 128 ? 3 : 2;  // (the last 32 pieces of T are loaded several times over)
+  typename Raw8<T>::type pd[NR], pv[GRADS ? NR : 1];
+  X8 ps[GRADS ? NR : 1], pt[NP];
+  static __device__ __forceinline__ int t_piece(int u, int bt) { return NT * u + (u == NP - 1 ? (bt & 31) : bt); }
+  static __device__ __forceinline__ int t_off(int p) {
+    int row, pc;
+    const int d = p - 128;
+    tri_piece(d < 0 ? 0 : d < T_DIAG_PIECES ? d : d - T_DIAG_PIECES, row, pc);
+    return d < 0 ? (32 + (p >> 2)) * GB_TS + 8 * (p & 3) : ((d < T_DIAG_PIECES ? 0 : 64) + row) * GB_TS + 8 * pc;
+  }
+  __device__ __forceinline__ void issue(const T* dout, const T* v, const unsigned char* rec, const unsigned char* state, int tok0,
+                                        int len, int HV, int hv, int bt) {
+    const size_t row0 = ((size_t)tok0 * HV + hv) * 64;
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      const int p = bt + NT * u, r = min(p >> 3, len - 1);
+      const uint32_t at = (uint32_t)(r * HV * 64 + 8 * (p & 7));
+      pd[u] = *reinterpret_cast<const typename Raw8<T>::type*>(dout + row0 + at);
+      if constexpr (GRADS) {
+        pv[u] = *reinterpret_cast<const typename Raw8<T>::type*>(v + row0 + at);
+        ps[u] = reinterpret_cast<const X8*>(state)[p];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u) pt[u] = reinterpret_cast<const X8*>(rec)[t_piece(u, bt)];
+  }
+  __device__ __forceinline__ void stage(const GbTiles<OT>& t, int len, int bt) {
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      const int p = bt + NT * u, row = p >> 3, part = p & 7;
+      typename Raw8<T>::type z;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) z[e] = (T)0.0f;
+      const bool live = row < len;
+      *reinterpret_cast<typename Raw8<T>::type*>(&t.dout[row * GB_LS + 8 * part]) = live ? pd[u] : z;
+      if constexpr (GRADS) {
+        *reinterpret_cast<typename Raw8<T>::type*>(&t.v[(part >> 2) * 2048 + row * 32 + 8 * (part & 3)]) = live ? pv[u] : z;
+        *reinterpret_cast<X8*>(t.s + 16 * p) = ps[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int off = t_off(t_piece(u, bt));
+      X4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { lo[e] = pt[u][e]; hi[e] = pt[u][4 + e]; }
+      *reinterpret_cast<X4*>(&t.t[off]) = lo;
+      *reinterpret_cast<X4*>(&t.t[off + 4]) = hi;
+    }
+  }
+};
+// per-token factors: one wave
+struct GbStageFactors {
+  float g, b, r;
+  __device__ __forceinline__ void issue(const unsigned char* rec, int lane) {
+    const float* fact = reinterpret_cast<const float*>(rec + T_BYTES);
+    g = fact[lane];
+    b = fact[64 + lane];
+    r = fact[128 + lane];
+  }
+  template <typename OT>
+  __device__ __forceinline__ void stage(const GbTiles<OT>& t, int lane) {
+    const float gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), 63));
+    t.gam[lane] = g;
+    t.beta[lane] = b;
+    t.rk[lane] = r;
+    t.eg[lane] = __builtin_amdgcn_exp2f(g);
+    t.dk[lane] = __builtin_amdgcn_exp2f(gl - g);
+  }
+};
+// the pieces of T that lie entirely above the diagonals, in both sets: zero once
+template <typename OT, bool GRADS>
+__device__ __forceinline__ void gb_zero_upper(unsigned char* smem, int tid) {
+  if (tid < 192) {
+    const int u = tid % 96;
+    int row, pc;
+    tri_upper_piece(u % 48, row, pc);
+    OT* at = &gb_tiles<OT, GRADS>(smem, tid / 96).t[((u < 48 ? 0 : 64) + row) * GB_TS + 8 * pc];
+    typename OpVec<OT>::x4 z;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z[e] = (OT)0.0f;
+    *reinterpret_cast<typename OpVec<OT>::x4*>(at) = z;
+    *reinterpret_cast<typename OpVec<OT>::x4*>(at + 4) = z;
+  }
+}
+
+// ---- source pass: every segment's N' (the walk from a zero gradient, no gradients written) --------------------------------
+// Grid segments x heads (long segments first), eight waves: 0, 1 the gradient of the state (32 value columns each), 4-6 the
+// tiles of P, 2 and 3 / 4-7 stage the next chunk into the other set of tiles. Two barriers per chunk, two workgroups per CU (80 KB
+// of LDS, 128 registers). 57 us at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the products).
+template <typename T>
+__global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
+    gdrb_source_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ dout,
+                       const unsigned char* __restrict__ recs, const GdrPlanView pv, const int32_t* __restrict__ chunk_tok0,
+                       const int32_t* __restrict__ chunk_len, unsigned char* __restrict__ Nr, int H, int HV, float scale,
+                       int l2norm) {
+  using OT = T;
   extern __shared__ __align__(16) unsigned char smem[];
-  OT* const b_k = reinterpret_cast<OT*>(smem + SM::OFF_K);
-  OT* const b_q = reinterpret_cast<OT*>(smem + SM::OFF_Q);
-  OT* const b_do = reinterpret_cast<OT*>(smem + SM::OFF_DO);
-  OT* const b_t = reinterpret_cast<OT*>(smem + SM::OFF_T);
-  unsigned char* const b_m = smem + SM::OFF_T;
-  unsigned char* const b_p = smem + SM::OFF_P;
-  unsigned char* const b_n = smem + SM::OFF_N;
-  unsigned char* const b_v = smem + SM::OFF_V;
-  unsigned char* const b_s = smem + SM::OFF_S;
-  unsigned char* const b_g = smem + SM::OFF_G;
-  unsigned char* const b_x = smem + SM::OFF_X;
-  float* const s_gam = reinterpret_cast<float*>(smem + SM::OFF_F);
-  float* const s_beta = s_gam + 64;
-  float* const s_eg = s_gam + 128;    // e^gamma
-  float* const s_dk = s_gam + 192;    // e^{gamma_L - gamma}
-  float* const s_rk = s_gam + 256;
-  float* const s_rq = s_gam + 320;
-  float* const s_sum = reinterpret_cast<float*>(b_p);  // GbSums (between barriers (2) and (6))
+  unsigned char* const b_p = smem + GbSourceSmem::OFF_P;
+  const int seg = pv.seg_order[blockIdx.x / HV], hv = blockIdx.x % HV, h = hv / (HV / H);
+  if (pv.seg_flags[seg] & SEG_FIRST) return;  // nothing precedes the first segment of a sequence
+  const int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg], cl = c0 + nc - 1;
+  const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63, hh = lane >> 5, ln = lane & 31;
+  // the chunks of a sequence follow one another, only its last one may be shorter: no table look-up in the loops
+  const int tok_first = nc > 0 ? chunk_tok0[c0] : 0, len_last = nc > 0 ? chunk_len[cl] : 0;
+  auto tok_of = [&](int c) { return tok_first + GDR_C * (c - c0); };
+  auto len_of = [&](int c) { return c == cl ? len_last : GDR_C; };
+  auto rec_of = [&](int c) { return recs + ((size_t)c * HV + hv) * REC_BYTES; };
+  // chunk c from the set (cl - c) % 2; a chunk's tiles are staged while the one behind it is worked on, its loads issued a
+  // chunk earlier still
+  auto set_of = [&](int c) { return gb_tiles<OT, false>(smem, (cl - c) & 1); };
+  gb_zero_upper<OT, false>(smem, tid);
+  if (wave < 2) {
+    GbChain<OT> ch;
+    ch.G[0] = zero16();
+    ch.G[1] = zero16();
+    if (nc > 0) lds_barrier();  // (0) the tiles of the first chunk are complete
+    for (int c = cl; c >= c0; --c) {
+      const GbTiles<OT> t = set_of(c);
+      ch.state_rows(t, nullptr, wave, lane, hh, ln);
+      lds_barrier();  // (1) P is complete
+      ch.chunk_rows(t, b_p, nullptr, wave, lane, hh);
+      ch.update(t, scale, wave, lane, hh);
+      lds_barrier();  // (2) the tiles of chunk c have been read, those of chunk c - 1 are complete
+    }
+    // N' in accumulator order, as the forward composites keep N
+    f32x4* out = reinterpret_cast<f32x4*>(Nr + (((size_t)seg * HV + hv) * 2 + wave) * GDR_STATE_BYTES);
+#pragma unroll
+    for (int km = 0; km < 2; ++km)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = ch.G[km][4 * q4 + e];
+        out[(km * 4 + q4) * 64 + lane] = x;
+      }
+  } else if (nc == 0) {
+    return;
+  } else if (wave < 4) {
+    GbStageRest<T, 128, false> st;
+    const int bt = tid - 128;
+    auto issue = [&](int c) {
+      c = uniform(max(c, c0));
+      st.issue(dout, nullptr, rec_of(c), nullptr, tok_of(c), len_of(c), HV, hv, bt);
+    };
+    issue(cl);
+    st.stage(set_of(cl), len_of(cl), bt);
+    issue(cl - 1);
+    lds_barrier();  // (0)
+    for (int c = cl; c >= c0; --c) {
+      if (c > c0) st.stage(set_of(c - 1), len_of(c - 1), bt);
+      issue(c - 2);
+      lds_barrier();  // (1)
+      lds_barrier();  // (2)
+    }
+  } else {
+    GbStageKQ<T> st;
+    GbStageFactors sf;
+    const int gt = tid - 256, tw = wave - 4, jt = tw == 2 ? 1 : 0, it = tw == 0 ? 0 : 1;
+    auto issue = [&](int c) {
+      c = uniform(max(c, c0));
+      st.issue(k, q, rec_of(c), tok_of(c), len_of(c), H, h, gt);
+      sf.issue(rec_of(c), lane);  // (wave 7 stages them)
+    };
+    auto stage = [&](int c) {
+      st.stage_k(set_of(c), len_of(c), l2norm, gt);
+      st.stage_q(set_of(c), len_of(c), l2norm, gt);
+      if (wave == 7) sf.stage(set_of(c), lane);
+    };
+    issue(cl);
+    stage(cl);
+    issue(cl - 1);
+    lds_barrier();  // (0)
+    for (int c = cl; c >= c0; --c) {
+      const GbTiles<OT> t = set_of(c);
+      if (wave < 7) {
+        f32x16 p = gb_pair<OT>(t.k, jt, t.q, it, ln, hh);
+        const f32x16 gm = gb_ratio(t.gam, jt, it, 0, ln, hh);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[r] *= scale * gm[r];
+        gb_store_tile<OT>(b_p + tw * GB_TRI, p, lane);
+      }
+      lds_barrier();  // (1)
+      if (c > c0) stage(c - 1);
+      issue(c - 2);
+      lds_barrier();  // (2)
+    }
+  }
+}
+
+// ---- the walk: every gradient of a segment's chunks, from the last to the first --------------------------------------------
+// Grid segments x heads (long segments first), twelve waves:
+//   0, 1   the gradient of the state, 32 value columns each (GbChain)
+//   2, 3   Vn = T B (V - E Kh S) for 32 value columns each, then dQh^T of 32 tokens each
+//   4-6    the three token x token tiles (j tile, i tile) = (0,0), (0,1), (1,1), rows j in the registers, the lane holds i: P,
+//          grad P and grad A with their gating and their sums over the rows and columns
+//   7      per-token factors, e^{gamma_L} <G', S>, and the sums for d g and d beta
+//   8-11   dKh^T, one 32 x 32 tile each (lane = token: per-token factors are one scalar, row sums mostly in-lane)
+// Waves 4-7 stage k, q of the next chunk into the other set of tiles, waves 8-11 dO, v, S, T; waves 0, 1 write dv, waves 2, 3
+// the rows of dq and dk of the chunk before. Barriers per chunk: (1) P, Vn, G' complete; (2) X, N complete; (3) M complete; (4)
+// the partial row sums are complete; (5) the next chunk's tiles and the rows of dq and dk are complete.
+// Bound by the latency of these five stages: 2.9 + 3.2 + 2.8 + 2.8 + 1.7 thousand cycles per chunk, of which a SIMD issues
+// vector instructions for about 7 000 (one workgroup per CU: 160 KB of LDS). 208 us at 60 000 tokens x 8 heads; all roles on
+// eight waves with one set of tiles and seven barriers took 256 us, two such workgroups per CU with 128 registers 395 us
+// (they spill, and every reload waits for the tiles being prefetched). Each role has its own loop for that reason too: a loop
+// shared by two roles copies the registers being loaded at its end and so waits for them (+7 us).
+template <typename T>
+__global__ void __launch_bounds__(GB_WALK_THREADS, 3)
+    gdrb_walk_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dout,
+                     const unsigned char* __restrict__ recs, const unsigned char* __restrict__ states, const GdrPlanView pv,
+                     const int32_t* __restrict__ chunk_tok0, const int32_t* __restrict__ chunk_len,
+                     const unsigned char* __restrict__ Mt, const float* __restrict__ Dc, const unsigned char* __restrict__ Nr,
+                     const unsigned char* __restrict__ Mgrp, const unsigned char* __restrict__ Ngrp,
+                     const float* __restrict__ Dgrp, int gmax, const float* __restrict__ dht, T* __restrict__ dq,
+                     T* __restrict__ dk, T* __restrict__ dv, float* __restrict__ dg, float* __restrict__ dbeta,
+                     float* __restrict__ dh0, int H, int HV, float scale, int l2norm) {
+  using OT = T;
+  using X8 = typename OpVec<OT>::x8;
+  using X4 = typename OpVec<OT>::x4;
+  using SM = GbWalkSmem;
+  extern __shared__ __align__(16) unsigned char smem[];
+  unsigned char *const b_p = smem + SM::OFF_P, *const b_n = smem + SM::OFF_N, *const b_m = smem + SM::OFF_M;
+  unsigned char *const b_g = smem + SM::OFF_G, *const b_x = smem + SM::OFF_X;
+  OT* const b_oq = reinterpret_cast<OT*>(smem + SM::OFF_OQ);
+  OT* const b_ok = reinterpret_cast<OT*>(smem + SM::OFF_OK);
+  float* const s_sum = reinterpret_cast<float*>(smem + SM::OFF_SUM);
 
   const int seg = pv.seg_order[blockIdx.x / HV], hv = blockIdx.x % HV, h = hv / (HV / H);
   const int flags = pv.seg_flags[seg];
-  if (!GRADS && (flags & SEG_FIRST)) return;  // nothing precedes the first segment of a sequence
-  const int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg], seq = pv.seg_seq[seg];
+  const int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg], seq = pv.seg_seq[seg], cl = c0 + nc - 1;
   const int wave = uniform(threadIdx.x >> 6);
-  const int kt = (wave >> 1) & 1, tt = wave & 1;  // this wave's tile of dQh^T / dKh^T: rows 32 kt, tokens 32 tt
-  // Everything below that depends on the lane is derived again for every chunk from a thread index the compiler cannot see
-  // through: left alone it computes some hundred LDS addresses before the loop and spills them.
-  int tid, lane, hh, ln, srow, part, tok, xtok, xpart;
+  // What depends on the lane is derived again for every chunk from a lane index the compiler cannot see through: left
+  // alone it computes some hundred LDS addresses before the loops and spills them (and a reload from scratch memory waits
+  // for every tile that is being prefetched).
+  int tid, lane, hh, ln;
   auto lanes = [&]() __attribute__((always_inline)) {
-    tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-    lane = tid & 63;
+    lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(lane));
+    tid = 64 * wave + lane;
     hh = lane >> 5;
     ln = lane & 31;
-    srow = tid >> 3;  // staging: thread = (row, 8-column piece) of every tile
-    part = tid & 7;
-    tok = 32 * tt + ln;
-    xtok = 16 * (wave & 3) + (lane & 15);  // this lane's piece of d v
-    xpart = 4 * (wave >> 2) + (lane >> 4);
   };
   lanes();
-  typename Raw8<T>::type pk, pq, pdo, pvv;
-  X8 pt, ps;
-  float pf0, pf1, pf2, prk;
-  int t_off = 0;  // where this thread's piece of T goes (elements)
-  {
-    int row, pc;
-    const int d = tid - 128;
-    tri_piece(d < T_DIAG_PIECES ? max(d, 0) : min(d - T_DIAG_PIECES, T_DIAG_PIECES - 1), row, pc);
-    t_off = tid < 128 ? (32 + (tid >> 2)) * GB_TS + 8 * (tid & 3)
-                      : ((d < T_DIAG_PIECES ? 0 : 64) + row) * GB_TS + 8 * pc;
-    if (tid >= 288) {  // the 96 pieces that lie entirely above the diagonals (written again for every chunk: M sits there)
-      const int u = min(tid - 288, 95);
-      tri_upper_piece(u % 48, row, pc);
-      t_off = ((u < 48 ? 0 : 64) + row) * GB_TS + 8 * pc;
-    }
-  }
-  auto issue = [&](int c) __attribute__((always_inline)) {
-    c = uniform(c);
-    const int tok0 = chunk_tok0[c], len = chunk_len[c];
-    const int r = min(srow, len - 1);
-    pk = *reinterpret_cast<const typename Raw8<T>::type*>(k + ((size_t)(tok0 + r) * H + h) * 64 + 8 * part);
-    pq = *reinterpret_cast<const typename Raw8<T>::type*>(q + ((size_t)(tok0 + r) * H + h) * 64 + 8 * part);
-    pdo = *reinterpret_cast<const typename Raw8<T>::type*>(dout + ((size_t)(tok0 + r) * HV + hv) * 64 + 8 * part);
-    if constexpr (GRADS) {
-      pvv = *reinterpret_cast<const typename Raw8<T>::type*>(v + ((size_t)(tok0 + r) * HV + hv) * 64 + 8 * part);
-      ps = reinterpret_cast<const X8*>(states + ((size_t)c * HV + hv) * GDR_STATE_BYTES)[tid];
-    }
-    const unsigned char* rec = recs + ((size_t)c * HV + hv) * REC_BYTES;
-    pt = reinterpret_cast<const X8*>(rec)[min(tid, 287)];
-    const float* fact = reinterpret_cast<const float*>(rec + T_BYTES);
-    if (wave >= 4) {  // (wave 7 stages them)
-      pf0 = fact[lane];
-      pf1 = fact[64 + lane];
-      pf2 = fact[128 + lane];
-    }
-    prk = fact[128 + srow];
-  };
-  auto stage = [&](int len) __attribute__((always_inline)) {
-    const bool live = srow < len;
-    float fk[8], fq[8], ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      fk[e] = live ? (float)pk[e] : 0.0f;
-      fq[e] = live ? (float)pq[e] : 0.0f;
-      ss = __builtin_fmaf(fq[e], fq[e], ss);
-    }
-    const float cq = l2_factor(gb_sum8(ss), l2norm);
-    X8 ok, oq, od;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      ok[e] = (OT)(fk[e] * prk);
-      oq[e] = (OT)(fq[e] * cq);
-      od[e] = live ? (OT)pdo[e] : (OT)0.0f;
-    }
-    *reinterpret_cast<X8*>(&b_k[srow * GB_LS + 8 * part]) = ok;
-    *reinterpret_cast<X8*>(&b_q[srow * GB_LS + 8 * part]) = oq;
-    *reinterpret_cast<X8*>(&b_do[srow * GB_LS + 8 * part]) = od;
-    if (part == 0) s_rq[srow] = cq;
-    if constexpr (GRADS) {
-      X8 ov;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ov[e] = live ? (OT)pvv[e] : (OT)0.0f;
-      *reinterpret_cast<X8*>(reinterpret_cast<OT*>(b_v) + (part >> 2) * 2048 + srow * 32 + 8 * (part & 3)) = ov;
-      *reinterpret_cast<X8*>(b_s + 16 * tid) = ps;
-    }
-    if (tid < 384) {
-      X4 lo, hi;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        lo[e] = tid < 288 ? pt[e] : (OT)0.0f;
-        hi[e] = tid < 288 ? pt[4 + e] : (OT)0.0f;
-      }
-      *reinterpret_cast<X4*>(&b_t[t_off]) = lo;
-      *reinterpret_cast<X4*>(&b_t[t_off + 4]) = hi;
-    }
-    if (wave == 7) {
-      const float gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pf0), 63));
-      s_gam[lane] = pf0;
-      s_beta[lane] = pf1;
-      s_rk[lane] = pf2;
-      s_eg[lane] = __builtin_amdgcn_exp2f(pf0);
-      s_dk[lane] = __builtin_amdgcn_exp2f(gl - pf0);
-    }
-  };
+  // the chunks of a sequence follow one another, only its last one may be shorter: no table look-up in the loops
+  const int tok_first = nc > 0 ? chunk_tok0[c0] : 0, len_last = nc > 0 ? chunk_len[cl] : 0;
+  auto tok_of = [&](int c) { return tok_first + GDR_C * (c - c0); };
+  auto len_of = [&](int c) { return c == cl ? len_last : GDR_C; };
+  auto rec_of = [&](int c) { return recs + ((size_t)c * HV + hv) * REC_BYTES; };
+  auto set_of = [&](int c) { return gb_tiles<OT, true>(smem, (cl - c) & 1); };  // (as in the source pass)
 
-  f32x16 G[2];  // (waves 0, 1) the gradient of the state behind the chunk, value columns 32 wave + ln
-  G[0] = zero16();
-  G[1] = zero16();
-  if (nc > 0) issue(c0 + nc - 1);
-  if constexpr (GRADS) {
+  // (the result goes to waves 0, 1 through LDS: in registers it would be live through the loops of every other role)
+  float* const xs = reinterpret_cast<float*>(b_g);
+  static_assert(SM::OFF_X == SM::OFF_G + 8192, "two column slabs of 64 rows of float");
+  {
     // The gradient behind the sequence pushed through the composites of the later segments: whole groups of
     // GDR_SCAN_GROUP first (gmax > 0), then the segments between them and this one; G <- d G + N' + M'^T G. Waves 0 .. 3:
     // wave w owns rows 32 (w / 2) .. of column slab w % 2 and takes the other rows as operand through LDS, so that the
@@ -303,43 +701,47 @@ __global__ void __launch_bounds__(GB_THREADS, GRADS ? 2 : 4)
     const int seg0 = pv.seq_seg0[seq], last = seg0 + pv.seq_nseg[seq] - 1, behind = last - seg;
     const int lead = gmax > 0 ? behind / GDR_SCAN_GROUP : 0, nst = lead + behind - lead * GDR_SCAN_GROUP;
     const int slab = wave & 1, km = (wave >> 1) & 1;
-    f32x16 S = zero16();
-    if (dht && wave < 4) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        S[r] = dht[(((size_t)seq * HV + hv) * 64 + 32 * km + acc_row(r, hh)) * 64 + 32 * slab + ln];
-    }
-    X8 rm[2][4];
-    f32x4 rn[2][4];
-    float rd[2];
-    auto walk_issue = [&](int p, X8* m, f32x4* n, float& d) __attribute__((always_inline)) {
-      p = uniform(max(0, min(p, nst - 1)));
-      const bool top = p < lead;
-      const size_t sh = (size_t)(top ? seq * gmax + p : last - lead * GDR_SCAN_GROUP - (p - lead)) * HV + hv;
-      const X8* M = reinterpret_cast<const X8*>((top ? Mgrp : Mt) + sh * GDR_STATE_BYTES);
-      const f32x4* N = reinterpret_cast<const f32x4*>((top ? Ngrp : Nr) + (sh * 2 + slab) * GDR_STATE_BYTES);
-#pragma unroll
-      for (int f = 0; f < 4; ++f) m[f] = M[(km * 4 + f) * 64 + lane];
-#pragma unroll
-      for (int f = 0; f < 4; ++f) n[f] = N[(km * 4 + f) * 64 + lane];
-      d = (top ? Dgrp : Dc)[sh];
-    };
-    auto walk_step = [&](int p, const X8* m, const f32x4* n, float d) __attribute__((always_inline)) {
-      unsigned char* xbuf = b_s + (p & 1) * 8192 + slab * 4096;
-      op_frag_store<OT>(xbuf, 2 * km + 0, lane, acc_to_op<OT>(S, 0));
-      op_frag_store<OT>(xbuf, 2 * km + 1, lane, acc_to_op<OT>(S, 8));
-      f32x16 acc;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * q4 + e] = __builtin_fmaf(d, S[4 * q4 + e], n[q4][e]);
+    if (wave >= 4) {
+      for (int p = 0; p < nst; ++p) lds_barrier();
       lds_barrier();
+      lds_barrier();
+    } else {
+      f32x16 S = zero16();
+      if (dht) {
 #pragma unroll
-      for (int f = 0; f < 4; ++f) acc = mfma32(m[f], op_frag_load<OT>(xbuf, f, lane), acc);
-      S = acc;
-    };
-    if (nst > 0) {
-      if (wave < 4) {
+        for (int r = 0; r < 16; ++r)
+          S[r] = dht[(((size_t)seq * HV + hv) * 64 + 32 * km + acc_row(r, hh)) * 64 + 32 * slab + ln];
+      }
+      X8 rm[2][4];
+      f32x4 rn[2][4];
+      float rd[2];
+      auto walk_issue = [&](int p, X8* m, f32x4* n, float& d) __attribute__((always_inline)) {
+        p = uniform(max(0, min(p, nst - 1)));
+        const bool top = p < lead;
+        const size_t sh = (size_t)(top ? seq * gmax + p : last - lead * GDR_SCAN_GROUP - (p - lead)) * HV + hv;
+        const X8* M = reinterpret_cast<const X8*>((top ? Mgrp : Mt) + sh * GDR_STATE_BYTES);
+        const f32x4* N = reinterpret_cast<const f32x4*>((top ? Ngrp : Nr) + (sh * 2 + slab) * GDR_STATE_BYTES);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) m[f] = M[(km * 4 + f) * 64 + lane];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) n[f] = N[(km * 4 + f) * 64 + lane];
+        d = (top ? Dgrp : Dc)[sh];
+      };
+      auto walk_step = [&](int p, const X8* m, const f32x4* n, float d) __attribute__((always_inline)) {
+        unsigned char* xbuf = (p & 1 ? b_x : b_g) + slab * 4096;
+        op_frag_store<OT>(xbuf, 2 * km + 0, lane, acc_to_op<OT>(S, 0));
+        op_frag_store<OT>(xbuf, 2 * km + 1, lane, acc_to_op<OT>(S, 8));
+        f32x16 acc;
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[4 * q4 + e] = __builtin_fmaf(d, S[4 * q4 + e], n[q4][e]);
+        lds_barrier();
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc = mfma32(m[f], op_frag_load<OT>(xbuf, f, lane), acc);
+        S = acc;
+      };
+      if (nst > 0) {
         walk_issue(0, rm[0], rn[0], rd[0]);
         walk_issue(1, rm[1], rn[1], rd[1]);
         for (int p = 0; p < nst; p += 2) {
@@ -348,137 +750,353 @@ __global__ void __launch_bounds__(GB_THREADS, GRADS ? 2 : 4)
           if (p + 1 < nst) walk_step(p + 1, rm[1], rn[1], rd[1]);
           walk_issue(p + 3, rm[1], rn[1], rd[1]);
         }
-      } else {
-        for (int p = 0; p < nst; ++p) lds_barrier();
       }
-    }
-    lds_barrier();  // (the last step's operands have been read)
-    float* xs = reinterpret_cast<float*>(b_s);  // rows 32 .. 63 go from waves 2, 3 to waves 0, 1
-    if (wave == 2 || wave == 3) {
+      lds_barrier();  // (the last step's operands have been read)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) xs[(slab * 16 + r) * 64 + lane] = S[r];
+      for (int r = 0; r < 16; ++r) xs[(32 * slab + 16 * km + r) * 64 + lane] = S[r];
+      lds_barrier();
     }
-    lds_barrier();
-    if (wave < 2) {
-      G[0] = S;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) G[1][r] = xs[(slab * 16 + r) * 64 + lane];
-    }
-    lds_barrier();
   }
+  gb_zero_upper<OT, true>(smem, tid);
 
-  // operand pieces of the row-major tiles
-  auto rows_k = [&](const OT* buf, int row, int c) __attribute__((always_inline)) {  // accumulator slot order
-    return op_ld_kappa<OT>(buf, GB_LS, row, c, hh);
-  };
-  auto cols = [&](const OT* buf, int col0, int row0) __attribute__((always_inline)) {
-    return op_ld_kappa_tr<OT, false>(buf, GB_LS, col0, row0, lane);
-  };
-
-  // steps k0 .. k1 - 1 (of 16) of a product: every operand fragment is requested before the first MFMA (left alone the
-  // compiler requests them one by one and pays the LDS latency for each)
-  auto mm = [&](f32x16 acc, int k0, int k1, auto fa, auto fb) __attribute__((always_inline)) {
-    X8 a[4], b[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      if (ks >= k0 && ks < k1) { a[ks] = fa(ks); b[ks] = fb(ks); }
-    // (an MFMA is no memory access: only passing its operands through an asm behind all the reads keeps it there)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      if (ks >= k0 && ks < k1) asm volatile("" : "+v"(a[ks]), "+v"(b[ks]));
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      if (ks >= k0 && ks < k1) acc = mfma32(a[ks], b[ks], acc);
-    return acc;
-  };
-  auto rows_n = [&](const OT* buf, int row, int c) __attribute__((always_inline)) {  // consecutive columns
-    return *reinterpret_cast<const X8*>(&buf[row * GB_LS + c + 8 * hh]);
-  };
-
-  // ---- what waves do alike at the end of a chunk: the rows of dq (waves 0-3) and dk (4-7) through the normalisation from
-  //      this wave's tile acc (rows 32 kt, tokens 32 tt), the rows of d v, and the stores
-  typename Raw8<T>::type vre;  // this lane's piece of v for d beta
+  // ---- d v = beta X and the products X . v (waves 0, 1): 32 tokens per wave, 16 at a time
+  typename Raw8<T>::type vre[2][2];
   auto load_v = [&](int tok0, int len) __attribute__((always_inline)) {
-    vre = *reinterpret_cast<const typename Raw8<T>::type*>(v + ((size_t)(tok0 + min(xtok, len - 1)) * HV + hv) * 64 +
-                                                           8 * xpart);
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const int xtok = 32 * wave + 16 * w + (lane & 15);
+      const T* at = v + ((size_t)tok0 * HV + hv) * 64 + (uint32_t)(min(xtok, len - 1) * HV * 64 + 8 * (lane >> 4));
+#pragma unroll
+      for (int u = 0; u < 2; ++u) vre[w][u] = *reinterpret_cast<const typename Raw8<T>::type*>(at + 32 * u);
+    }
   };
-  auto finish = [&](f32x16& acc, float rs_g, int tok0, int len) __attribute__((always_inline)) {
-    const OT* yin = wave < 4 ? b_q : b_k;
-    float dot = 0.0f;
-    X4 y4[4];
+  auto rows_dv = [&](const GbTiles<OT>& t, int tok0, int len) __attribute__((always_inline)) {
+    const int L = lane & 15, cc = 8 * (lane >> 4) + (L >> 2);
+    const unsigned char* p = b_x + wave * 2048 + (32 * (L & 1) + cc) * 16 + ((L >> 1) & 1) * 8;
+    X4 x4[2][4];
 #pragma unroll
-    for (int b4 = 0; b4 < 4; ++b4) {
-      y4[b4] = *reinterpret_cast<const X4*>(&yin[tok * GB_LS + 32 * kt + 8 * b4 + 4 * hh]);
+    for (int w = 0; w < 2; ++w)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dot += (float)y4[b4][e] * acc[4 * b4 + e];
-    }
-    float* const s_dot = s_sum + (wave < 4 ? GbSums::DOTQ : GbSums::DOTK);
-    dot = gb_both_halves(dot);
-    rs_g = gb_both_halves(rs_g);
-    if (hh == 0) {
-      s_dot[64 * kt + tok] = dot;
-      s_sum[GbSums::DGAM + 32 * wave + ln] = rs_g;
-    }
-    {  // d v = beta X and the product of X with v, 16 tokens x 4 pieces per wave
-      const int L = lane & 15, r0 = 16 * (wave & 3) + 4 * (L & 3), cc = 8 * xpart + (L >> 2);
-      const OT* p = reinterpret_cast<const OT*>(b_x + ((cc >> 5) * 4 + (r0 >> 4)) * 1024 +
-                                                (32 * ((r0 >> 2) & 1) + (cc & 31)) * 16 + ((r0 >> 3) & 1) * 8);
-      const X4 lo = op_lds_read_tr4<OT>(p), hi = op_lds_read_tr4<OT>(p + 4 * 8);
-      const float b = s_beta[xtok];
-      float t = 0.0f;
-      typename Raw8<T>::type out;
+      for (int u = 0; u < 4; ++u)
+        x4[w][u] = op_lds_read_tr4<OT>(reinterpret_cast<const OT*>(p + w * 1024 + (u >> 1) * 4096 + (u & 1) * 64));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        t += (float)lo[e] * (float)vre[e] + (float)hi[e] * (float)vre[4 + e];
-        out[e] = (T)(b * (float)lo[e]);
-        out[4 + e] = (T)(b * (float)hi[e]);
-      }
-      t += __shfl_xor(t, 16);
-      t = gb_both_halves(t);
-      if (lane < 16) s_sum[GbSums::XV + 64 * (wave >> 2) + xtok] = t;
-      if (xtok < len) {
-        *reinterpret_cast<typename Raw8<T>::type*>(dv + ((size_t)(tok0 + xtok) * HV + hv) * 64 + 8 * xpart) = out;
-      }
-    }
-    lds_barrier();  // (4) the row sums are complete, every tile has been read
-    {
-      dot = s_dot[tok] + s_dot[64 + tok];
-      const float cn = wave < 4 ? s_rq[tok] : s_rk[tok];
-      // c = 1 / (|x| + eps) in the recurrent form: |x| = 1 / c - eps
-      const float fy = l2norm == GDR_L2_CHUNK ? cn * dot
-                       : l2norm == GDR_L2_RECURRENT ? dot / fmaxf(1.0f / cn - 1e-6f, 1e-30f) : 0.0f;
-      OT* to = (wave < 4 ? b_q : b_k) + tok * GB_LS + 32 * kt;
+    for (int w = 0; w < 2; ++w) {
+      const int xtok = 32 * wave + 16 * w + L;
+      const float b = t.beta[xtok];
+      float x = 0.0f;
+      T* at = dv + ((size_t)tok0 * HV + hv) * 64 + (uint32_t)(xtok * HV * 64 + 8 * (lane >> 4));
 #pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) {
-        X4 o4;
+      for (int u = 0; u < 2; ++u) {
+        typename Raw8<T>::type out;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float gx = l2norm == GDR_L2_NONE ? acc[4 * b4 + e] : cn * acc[4 * b4 + e] - fy * (float)y4[b4][e];
-          o4[e] = (OT)gx;
+          const float lo = (float)x4[w][2 * u][e], hi = (float)x4[w][2 * u + 1][e];
+          x += lo * (float)vre[w][u][e] + hi * (float)vre[w][u][4 + e];
+          out[e] = (T)(b * lo);
+          out[4 + e] = (T)(b * hi);
         }
-        *reinterpret_cast<X4*>(&to[8 * b4 + 4 * hh]) = o4;
+        if (xtok < len) *reinterpret_cast<typename Raw8<T>::type*>(at + 32 * u) = out;
       }
+      x += __shfl_xor(x, 16);
+      x = gb_both_halves(x);
+      if (lane < 16) s_sum[GbSums::XV + xtok] = x;
     }
-    lds_barrier();  // (5) the rows of dq and dk are complete
-    const X8 o_k = *reinterpret_cast<const X8*>(&b_k[srow * GB_LS + 8 * part]);
-    const X8 o_q = *reinterpret_cast<const X8*>(&b_q[srow * GB_LS + 8 * part]);
-    if (srow < len) {
-      const size_t at = ((size_t)(tok0 + srow) * HV + hv) * 64 + 8 * part;
-      *reinterpret_cast<X8*>(dk + at) = o_k;
-      *reinterpret_cast<X8*>(dq + at) = o_q;
+  };
+  // rows of a gradient tile (rows 32 kt .., lane = token tok) through the l2 normalisation: y the normalised input row, dot
+  // the row's product with it, cn the normalisation factor (1 / (|x| + eps) in the recurrent form: |x| = 1 / c - eps)
+  auto rows_out = [&](OT* to, const OT* y, const f32x16& acc, int kt, int tok, float dot, float cn) __attribute__((always_inline)) {
+    float fy = 0.0f, fc = 1.0f;
+    if (l2norm != GDR_L2_NONE) {
+      fy = cn * dot;
+      fc = cn;
+      if (l2norm == GDR_L2_RECURRENT) fy = dot / fmaxf(1.0f / cn - 1e-6f, 1e-30f);
     }
-    if (wave == 2) {  // d g = the sum of d gamma over the later rows of the chunk (gamma_i = g_0 + ... + g_i); d beta
-      const float* w = s_sum + GbSums::DGAM + 32 * hh + ln;  // (lane = token: its waves are hh, hh + 2, hh + 4, hh + 6)
-      const float* t = s_sum + ln;                            // tiles (0,0), (0,1), (1,1)
-      float x = (w[0] + w[64]) + (w[128] + w[192]);
-      x += t[GbSums::TILE_G + 32 * hh] + (hh ? t[GbSums::TILE_G + 64] : 0.0f);
-      x -= t[GbSums::TILE_C + 64 * hh] + (hh ? 0.0f : t[GbSums::TILE_C + 32]);
-      const float db = (t[GbSums::TILE_B + 32 * hh] + (hh ? t[GbSums::TILE_B + 64] : 0.0f)) +
-                       (t[GbSums::DBETA + 32 * hh] + t[GbSums::DBETA + 64 + 32 * hh]) +
-                       (s_sum[GbSums::XV + lane] + s_sum[GbSums::XV + 64 + lane]);
+#pragma unroll
+    for (int b4 = 0; b4 < 4; ++b4) {
+      const int at = tok * GB_LS + 32 * kt + 8 * b4 + 4 * hh;
+      const X4 y4 = *reinterpret_cast<const X4*>(&y[at]);
+      X4 o4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o4[e] = (OT)(fc * acc[4 * b4 + e] - fy * (float)y4[e]);
+      *reinterpret_cast<X4*>(&to[at]) = o4;
+    }
+  };
+  auto row_dot = [&](const OT* y, const f32x16& acc, int kt, int tok) __attribute__((always_inline)) {
+    float dot = 0.0f;
+#pragma unroll
+    for (int b4 = 0; b4 < 4; ++b4) {
+      const X4 y4 = *reinterpret_cast<const X4*>(&y[tok * GB_LS + 32 * kt + 8 * b4 + 4 * hh]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dot += (float)y4[e] * acc[4 * b4 + e];
+    }
+    return dot;
+  };
+
+  if (wave < 2) {
+    // ======================================= the gradient of the state =======================================
+    GbChain<OT> ch;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      ch.G[0][r] = xs[(32 * wave + r) * 64 + lane];
+      ch.G[1][r] = xs[(32 * wave + 16 + r) * 64 + lane];
+    }
+    if (nc > 0) lds_barrier();  // (0) the tiles of the first chunk are complete
+    for (int c = cl; c >= c0; --c) {
+      lanes();
+      const int tok0 = tok_of(c), len = len_of(c);
+      const GbTiles<OT> t = set_of(c);
+      ch.state_rows(t, b_g, wave, lane, hh, ln);
+      lds_barrier();  // (1)
+      ch.chunk_rows(t, b_p, b_x, wave, lane, hh);
+      load_v(tok0, len);
+      lds_barrier();  // (2)
+      ch.update(t, scale, wave, lane, hh);
+      lds_barrier();  // (3)
+      rows_dv(t, tok0, len);
+      lds_barrier();  // (4)
+      lds_barrier();  // (5)
+    }
+    if (dh0 && (flags & SEG_FIRST)) {
+#pragma unroll
+      for (int km = 0; km < 2; ++km)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          dh0[(((size_t)seq * HV + hv) * 64 + 32 * km + acc_row(r, hh)) * 64 + 32 * wave + ln] = ch.G[km][r];
+    }
+  } else if (nc == 0) {
+    return;
+  } else if (wave < 4) {
+    // =============================================== Vn, dQh^T ===============================================
+    const int vn = wave - 2;
+    auto store_rows = [&](int c) __attribute__((always_inline)) {  // dq, dk of chunk c
+      const int tok0 = tok_of(c), len = len_of(c), row0 = 8 * vn + (lane >> 3), part = lane & 7;
+      const size_t first = ((size_t)tok0 * HV + hv) * 64;
+      X8 o[8];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        o[u] = *reinterpret_cast<const X8*>(&b_oq[(16 * u + row0) * GB_LS + 8 * part]);
+        o[4 + u] = *reinterpret_cast<const X8*>(&b_ok[(16 * u + row0) * GB_LS + 8 * part]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = 16 * u + row0;
+        if (row < len) {
+          const uint32_t at = (uint32_t)(row * HV * 64 + 8 * part);
+          *reinterpret_cast<X8*>(dq + first + at) = o[u];
+          *reinterpret_cast<X8*>(dk + first + at) = o[4 + u];
+        }
+      }
+    };
+    lds_barrier();  // (0)
+    for (int c = cl; c >= c0; --c) {
+      lanes();
+      const int tok = 32 * vn + ln;
+      const GbTiles<OT> t = set_of(c);
+      {
+        X8 Rb[4];
+        OT* const vt = t.v + vn * 2048;
+        {
+          X8 Sb[4], fk[8];
+#pragma unroll
+          for (int f = 0; f < 8; ++f) fk[f] = gb_rows_k<OT>(t.k, 32 * (f >> 2) + ln, 16 * (f & 3), hh);
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) Sb[ks] = op_frag_load<OT>(t.s, vn * 4 + ks, lane);
+          X4 vv[8];
+#pragma unroll
+          for (int b = 0; b < 8; ++b) vv[b] = op_ld_col4<OT>(vt, 32, 0, 8 * b, lane);
+          gb_pin(fk);
+          gb_pin(Sb);
+          f32x16 r[2];
+          r[0] = zero16();
+          r[1] = zero16();
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) {
+            r[0] = mfma32(fk[ks], Sb[ks], r[0]);
+            r[1] = mfma32(fk[4 + ks], Sb[ks], r[1]);
+          }
+#pragma unroll
+          for (int tm = 0; tm < 2; ++tm) {
+#pragma unroll
+            for (int b4 = 0; b4 < 4; ++b4) {  // R = beta (v - e^gamma Kh S)
+              const f32x4 fb = gb_rows4(t.beta, 32 * tm, b4, hh), fe = gb_rows4(t.eg, 32 * tm, b4, hh);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                r[tm][4 * b4 + e] = fb[e] * ((float)vv[4 * tm + b4][e] - fe[e] * r[tm][4 * b4 + e]);
+            }
+            Rb[2 * tm + 0] = acc_to_op<OT>(r[tm], 0);
+            Rb[2 * tm + 1] = acc_to_op<OT>(r[tm], 8);
+          }
+        }
+        X8 ft[6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) ft[f] = op_ld_kappa<OT>(t.t + (f >> 1) * 32 * GB_TS, GB_TS, ln, 16 * (f & 1), hh);
+        gb_pin(ft);
+        f32x16 r[2];
+        r[0] = zero16();
+        r[1] = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          if (ks < 2) r[0] = mfma32(ft[ks], Rb[ks], r[0]);
+          r[1] = mfma32(ft[2 + ks], Rb[ks], r[1]);
+        }
+        unsigned char* const vf = reinterpret_cast<unsigned char*>(t.v);  // (over this wave's own half of v, which it has read)
+#pragma unroll
+        for (int tm = 0; tm < 2; ++tm) {
+          op_frag_store<OT>(vf, vn * 4 + 2 * tm + 0, lane, acc_to_op<OT>(r[tm], 0));
+          op_frag_store<OT>(vf, vn * 4 + 2 * tm + 1, lane, acc_to_op<OT>(r[tm], 8));
+        }
+      }
+      lds_barrier();  // (1)
+      f32x16 acc[2];  // rows 0-31, 32-63 of dQh^T: scale e^gamma S dO^T + Kh^T N^T
+      float rs_g = 0.0f;
+      const float fs = scale * t.eg[tok];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        acc[kt] = gb_mm<OT>(zero16(), [&](int ks) { return fr_tr<OT, false>(t.s, 32 * kt, 16 * ks, lane); },
+                            [&](int ks) { return gb_rows_n<OT>(t.dout, tok, 16 * ks, hh); });
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[kt][r] *= fs;
+        rs_g += row_dot(t.q, acc[kt], kt, tok);
+      }
+      if (c < cl) store_rows(c + 1);
+      lds_barrier();  // (2)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        acc[kt] = gb_mm_tri<OT, true>(acc[kt], vn, [&](int ks) { return gb_cols<OT>(t.k, 32 * kt, 16 * ks, lane); },
+                                      [&](int ks) { return op_frag_load<OT>(b_n + (vn + ks / 2) * GB_TRI, ks & 1, lane); });
+      lds_barrier();  // (3)
+      rs_g = gb_both_halves(rs_g);
+      if (hh == 0) s_sum[GbSums::DGAM + 32 * vn + ln] = rs_g;
+      const float dot = gb_both_halves(row_dot(t.q, acc[0], 0, tok) + row_dot(t.q, acc[1], 1, tok));
+      const float cn = t.rq[tok];
+      rows_out(b_oq, t.q, acc[0], 0, tok, dot, cn);
+      rows_out(b_oq, t.q, acc[1], 1, tok, dot, cn);
+      lds_barrier();  // (4)
+      lds_barrier();  // (5)
+    }
+    store_rows(c0);
+  } else if (wave < 7) {
+    // ================================ the token x token tiles; staging of k, q ================================
+    GbStageKQ<T> st;
+    const int tw = wave - 4, jt = tw == 2 ? 1 : 0, it = tw == 0 ? 0 : 1;
+    auto issue = [&](int c) __attribute__((always_inline)) {
+      c = uniform(max(c, c0));
+      st.issue(k, q, rec_of(c), tok_of(c), len_of(c), H, h, tid - 256);
+    };
+    issue(cl);
+    st.stage_k(set_of(cl), len_of(cl), l2norm, tid - 256);
+    st.stage_q(set_of(cl), len_of(cl), l2norm, tid - 256);
+    issue(cl - 1);
+    lds_barrier();  // (0)
+    for (int c = cl; c >= c0; --c) {
+      lanes();
+      const GbTiles<OT> t = set_of(c);
+      const int i = 32 * it + ln;
+      f32x16 pm = gb_pair<OT>(t.k, jt, t.q, it, ln, hh), gm = gb_ratio(t.gam, jt, it, 0, ln, hh);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) pm[r] *= scale * gm[r];
+      gb_store_tile<OT>(b_p + tw * GB_TRI, pm, lane);
+      const f32x16 gk = gb_pair<OT>(t.k, jt, t.k, it, ln, hh);
+      lds_barrier();  // (1)
+      const unsigned char* vf = reinterpret_cast<const unsigned char*>(t.v);
+      float rs_g = 0.0f, rs_b = 0.0f, rs_c, cs[16];  // sums over the tile's rows (of column i) and columns (of a row)
+      {  // grad P = dO Vn^T
+        f32x16 n = gb_mm<OT>(zero16(), [&](int ks) { return fr_tr<OT, false>(vf, 32 * jt, 16 * ks, lane); },
+                             [&](int ks) { return gb_rows_n<OT>(t.dout, i, 16 * ks, hh); });
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          cs[r] = n[r] * pm[r];
+          rs_g += cs[r];
+          n[r] *= scale * gm[r];
+        }
+        gb_store_tile<OT>(b_n + tw * GB_TRI, n, lane);
+        rs_c = gb_half_sums16(cs, lane);
+      }
+      // (strictly below the diagonal for grad A)
+      if (jt == it) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) gm[r] = ln == acc_row(r, hh) ? 0.0f : gm[r];
+      }
+      const float bi = t.beta[i];
+      lds_barrier();  // (2)
+      f32x16 da = gb_mm<OT>(zero16(), [&](int ks) { return fr_tr<OT, false>(vf, 32 * jt, 16 * ks, lane); },
+                            [&](int ks) { return fr_tr<OT, false>(b_x, 32 * it, 16 * ks, lane); });
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {  // grad A = -X Vn^T
+        // grad A_ij Gamma_ij, and grad A_ij times A_ij / beta_i and times A_ij
+        const float ga = -da[r] * gm[r], b = ga * gk[r], a = b * bi;
+        rs_b += b;
+        rs_g += a;
+        cs[r] = a;
+        da[r] = ga * bi;
+      }
+      gb_store_tile<OT>(b_m + tw * GB_TRI, da, lane);
+      lds_barrier();  // (3)
+      rs_c += gb_half_sums16(cs, lane);
+      rs_g = gb_both_halves(rs_g);
+      rs_b = gb_both_halves(rs_b);
+      if (hh == 0) {
+        s_sum[GbSums::TILE_G + 32 * tw + ln] = rs_g;
+        s_sum[GbSums::TILE_B + 32 * tw + ln] = rs_b;
+      }
+      if (!(ln & 1)) s_sum[GbSums::TILE_C + 32 * tw + 8 * (ln >> 3) + 4 * hh + ((ln >> 1) & 3)] = rs_c;
+      if (c > c0) st.stage_k(set_of(c - 1), len_of(c - 1), l2norm, tid - 256);
+      lds_barrier();  // (4)
+      if (c > c0) st.stage_q(set_of(c - 1), len_of(c - 1), l2norm, tid - 256);
+      issue(c - 2);
+      lds_barrier();  // (5)
+    }
+  } else if (wave == 7) {
+    // ============================ per-token factors, d g, d beta; staging of k, q ============================
+    // (a loop of its own: joined with the one above, the registers being loaded are copied at its end, waiting for them)
+    GbStageKQ<T> st;
+    GbStageFactors sf;
+    auto issue = [&](int c) __attribute__((always_inline)) {
+      c = uniform(max(c, c0));
+      st.issue(k, q, rec_of(c), tok_of(c), len_of(c), H, h, tid - 256);
+      sf.issue(rec_of(c), lane);
+    };
+    issue(cl);
+    st.stage_k(set_of(cl), len_of(cl), l2norm, tid - 256);
+    st.stage_q(set_of(cl), len_of(cl), l2norm, tid - 256);
+    sf.stage(set_of(cl), lane);
+    issue(cl - 1);
+    lds_barrier();  // (0)
+    for (int c = cl; c >= c0; --c) {
+      lanes();
+      const int tok0 = tok_of(c), len = len_of(c);
+      const GbTiles<OT> t = set_of(c);
+      lds_barrier();  // (1)
+      float gs = 0.0f;  // e^{gamma_L} <G', S>
+#pragma unroll
+      for (int f = 0; f < 8; ++f) {
+        const X8 xa = op_frag_load<OT>(b_g, f, lane), xb = op_frag_load<OT>(t.s, f, lane);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gs = __builtin_fmaf((float)xa[e], (float)xb[e], gs);
+      }
+      gs = gb_half_sum(gs) * __builtin_amdgcn_exp2f(t.gam[63]);
+      if (ln == 0) s_sum[GbSums::GL + 8 + hh] = gs;
+      lds_barrier();  // (2)
+      lds_barrier();  // (3)
+      if (c > c0) {
+        st.stage_k(set_of(c - 1), len_of(c - 1), l2norm, tid - 256);
+        st.stage_q(set_of(c - 1), len_of(c - 1), l2norm, tid - 256);
+        sf.stage(set_of(c - 1), lane);
+      }
+      issue(c - 2);
+      lds_barrier();  // (4)
+      // d g = the sum of d gamma over the later rows of the chunk (gamma_i = g_0 + ... + g_i); d beta
+      const float* w = s_sum + GbSums::DGAM + 32 * hh + ln;  // (lane = token 32 hh + ln; tiles (0,0), (0,1), (1,1))
+      const float* s = s_sum + ln;
+      float x = w[0] + (w[64] + w[128]);
+      x += s[GbSums::TILE_G + 32 * hh] + (hh ? s[GbSums::TILE_G + 64] : 0.0f);
+      x -= s[GbSums::TILE_C + 64 * hh] + (hh ? 0.0f : s[GbSums::TILE_C + 32]);
+      const float db = (s[GbSums::TILE_B + 32 * hh] + (hh ? s[GbSums::TILE_B + 64] : 0.0f)) +
+                       (s[GbSums::DBETA + 32 * hh] + s[GbSums::DBETA + 64 + 32 * hh]) +
+                       s_sum[GbSums::XV + lane];
       if (lane == len - 1) {
-        const f32x4 ga = *reinterpret_cast<const f32x4*>(s_sum + GbSums::GL), gb = *reinterpret_cast<const f32x4*>(s_sum + GbSums::GL + 4);
-        x += ((ga[0] + ga[1]) + (ga[2] + ga[3])) + ((gb[0] + gb[1]) + (gb[2] + gb[3]));
+        const float* g = s_sum + GbSums::GL;
+        x += ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7])) + (g[8] + g[9]);
       }
       if (lane >= len) x = 0.0f;
       const float incl = wave_inclusive_scan(x);  // (inclusive scan from the last lane down: total - exclusive prefix)
@@ -487,379 +1105,79 @@ __global__ void __launch_bounds__(GB_THREADS, GRADS ? 2 : 4)
         dg[(size_t)(tok0 + lane) * HV + hv] = total - incl + x;
         dbeta[(size_t)(tok0 + lane) * HV + hv] = db;
       }
-    }
-    lds_barrier();  // (6) every tile has been read: the next chunk's may be staged
-  };
-  // scale e^gamma S dO^T of this wave's tile, and its share of d gamma
-  auto dq_state = [&](f32x16& acc, float& rs_g) __attribute__((always_inline)) {
-    acc = mm(zero16(), 0, 4, [&](int ks) { return fr_tr<OT, false>(b_s, 32 * kt, 16 * ks, lane); },
-             [&](int ks) { return rows_n(b_do, tok, 16 * ks); });
-    const float fs = scale * s_eg[tok];
-#pragma unroll
-    for (int b4 = 0; b4 < 4; ++b4) {
-      const X4 y = *reinterpret_cast<const X4*>(&b_q[tok * GB_LS + 32 * kt + 8 * b4 + 4 * hh]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[4 * b4 + e] *= fs;
-        rs_g += (float)y[e] * acc[4 * b4 + e];
-      }
-    }
-  };
-  // + Kh^T N^T
-  auto dq_chunk = [&](f32x16& acc) __attribute__((always_inline)) {
-    acc = mm(acc, 0, 2 * (tt + 1), [&](int ks) { return cols(b_k, 32 * kt, 16 * ks); },
-             [&](int ks) { return op_frag_load<OT>(b_n + (tt + ks / 2) * GB_TRI, ks & 1, lane); });
-  };
-
-  // (every role has a chunk loop of its own, so that what one role carries from chunk to chunk takes no registers in the
-  // others; the barriers pair up by their number)
-  const int cl = c0 + nc - 1;
-  if (wave < 2) {
-    // ======================================= the gradient of the state =======================================
-    for (int c = cl; c >= c0; --c) {
-      const int tok0 = chunk_tok0[uniform(c)], len = chunk_len[uniform(c)];
-      lanes();
-      stage(len);
-      if constexpr (GRADS) load_v(tok0, len);
-      else issue(max(c - 1, c0));
-      lds_barrier();  // (0) the tiles of chunk c are complete
-      f32x16 a[2];  // D Kh G', then dVn, then X
-      {
-        X8 Gb[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          Gb[ks] = acc_to_op<OT>(G[ks / 2], 8 * (ks % 2));
-          if constexpr (GRADS) op_frag_store<OT>(b_g, wave * 4 + ks, lane, Gb[ks]);
-        }
-#pragma unroll
-        for (int tm = 0; tm < 2; ++tm) {
-          a[tm] = mm(zero16(), 0, 4, [&](int ks) { return rows_k(b_k, 32 * tm + ln, 16 * ks); },
-                     [&](int ks) { return Gb[ks]; });
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {
-            const f32x4 f = gb_rows4(s_dk, 32 * tm, b4, hh);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a[tm][4 * b4 + e] *= f[e];
-          }
-        }
-      }
-      lds_barrier();  // (1) P, Vn and G' are complete
-      {
-        X8 dOb[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) dOb[ks] = cols(b_do, 32 * wave, 16 * ks);
-#pragma unroll
-        for (int tm = 0; tm < 2; ++tm)  // + P^T dO
-          a[tm] = mm(a[tm], 2 * tm, 4,
-                     [&](int ks) { return fr_tr<OT, true>(b_p + (tm == 0 ? ks / 2 : 2) * GB_TRI, 0, 16 * (ks & 1), lane); },
-                     [&](int ks) { return dOb[ks]; });
-      }
-      X8 Xb[4];
-      {
-        X8 Rb[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) Rb[ks] = acc_to_op<OT>(a[ks / 2], 8 * (ks % 2));
-#pragma unroll
-        for (int tm = 0; tm < 2; ++tm) {  // X = T^T dVn (blocks T11, T21 | T22)
-          a[tm] = mm(zero16(), 2 * tm, 4,
-                     [&](int ks) {
-                       return op_ld_kappa_tr<OT, false>(b_t + (tm == 0 ? ks / 2 : 2) * 32 * GB_TS, GB_TS, 0, 16 * (ks & 1), lane);
-                     },
-                     [&](int ks) { return Rb[ks]; });
-          if constexpr (GRADS) {
-            op_frag_store<OT>(b_x, wave * 4 + 2 * tm + 0, lane, acc_to_op<OT>(a[tm], 0));
-            op_frag_store<OT>(b_x, wave * 4 + 2 * tm + 1, lane, acc_to_op<OT>(a[tm], 8));
-          }
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {  // -beta e^gamma X, the operand of the update
-            const f32x4 fb = gb_rows4(s_beta, 32 * tm, b4, hh), fe = gb_rows4(s_eg, 32 * tm, b4, hh);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a[tm][4 * b4 + e] *= -fb[e] * fe[e];
-          }
-          Xb[2 * tm + 0] = acc_to_op<OT>(a[tm], 0);
-          Xb[2 * tm + 1] = acc_to_op<OT>(a[tm], 8);
-        }
-      }
-      if constexpr (GRADS) lds_barrier();  // (2) X and N are complete, T and P are dead
-      {
-        const float dec = __builtin_amdgcn_exp2f(s_gam[63]);
-#pragma unroll
-        for (int km = 0; km < 2; ++km)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) G[km][r] *= dec;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {  // + (scale e^gamma Qh)^T dO - (beta e^gamma Kh)^T X
-          X8 d = cols(b_do, 32 * wave, 16 * ks);
-          const f32x4 f0 = *reinterpret_cast<const f32x4*>(&s_eg[16 * ks + 4 * hh]);
-          const f32x4 f1 = *reinterpret_cast<const f32x4*>(&s_eg[16 * ks + 8 + 4 * hh]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            d[e] = (OT)((float)d[e] * (scale * f0[e]));
-            d[4 + e] = (OT)((float)d[4 + e] * (scale * f1[e]));
-          }
-          X8 q0 = cols(b_q, 0, 16 * ks), q1 = cols(b_q, 32, 16 * ks), k0 = cols(b_k, 0, 16 * ks), k1 = cols(b_k, 32, 16 * ks);
-          asm volatile("" : "+v"(q0), "+v"(q1), "+v"(k0), "+v"(k1));
-          G[0] = mfma32(q0, d, G[0]);
-          G[1] = mfma32(q1, d, G[1]);
-          G[0] = mfma32(k0, Xb[ks], G[0]);
-          G[1] = mfma32(k1, Xb[ks], G[1]);
-        }
-      }
-      if constexpr (GRADS) {
-        issue(max(c - 1, c0));
-        f32x16 acc;
-        float rs_g = 0.0f;
-        dq_state(acc, rs_g);
-        dq_chunk(acc);
-        lds_barrier();  // (3)
-        finish(acc, rs_g, tok0, len);
-      } else {
-        lds_barrier();  // every tile has been read: the next chunk's may be staged
-      }
-    }
-    if constexpr (!GRADS) {  // N' in accumulator order, as the forward composites keep N
-      f32x4* out = reinterpret_cast<f32x4*>(Nr + (((size_t)seg * HV + hv) * 2 + wave) * GDR_STATE_BYTES);
-#pragma unroll
-      for (int km = 0; km < 2; ++km)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          f32x4 t;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) t[e] = G[km][4 * q4 + e];
-          out[(km * 4 + q4) * 64 + lane] = t;
-        }
-    } else if (dh0 && (flags & SEG_FIRST)) {
-#pragma unroll
-      for (int km = 0; km < 2; ++km)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          dh0[(((size_t)seq * HV + hv) * 64 + 32 * km + acc_row(r, hh)) * 64 + 32 * wave + ln] = G[km][r];
-    }
-  } else if (GRADS && wave < 4) {
-    // =============================================== Vn, dQh ===============================================
-    const int vn = wave - 2;
-    for (int c = cl; c >= c0; --c) {
-      const int tok0 = chunk_tok0[uniform(c)], len = chunk_len[uniform(c)];
-      lanes();
-      stage(len);
-      load_v(tok0, len);
-      lds_barrier();  // (0)
-      issue(max(c - 1, c0));
-      X8 Rb[4];
-      {
-        X8 Sb[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) Sb[ks] = op_frag_load<OT>(b_s, vn * 4 + ks, lane);
-        const OT* vt = reinterpret_cast<const OT*>(b_v) + vn * 2048;
-#pragma unroll
-        for (int tm = 0; tm < 2; ++tm) {
-          f32x16 r = mm(zero16(), 0, 4, [&](int ks) { return rows_k(b_k, 32 * tm + ln, 16 * ks); },
-                        [&](int ks) { return Sb[ks]; });
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {  // R = beta (v - e^gamma Kh S)
-            const X4 vv = op_ld_col4<OT>(vt, 32, 0, 32 * tm + 8 * b4, lane);
-            const f32x4 fb = gb_rows4(s_beta, 32 * tm, b4, hh), fe = gb_rows4(s_eg, 32 * tm, b4, hh);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) r[4 * b4 + e] = fb[e] * ((float)vv[e] - fe[e] * r[4 * b4 + e]);
-          }
-          Rb[2 * tm + 0] = acc_to_op<OT>(r, 0);
-          Rb[2 * tm + 1] = acc_to_op<OT>(r, 8);
-        }
-      }
-      lds_fence();  // this wave's reads of its half of v are done: Vn goes over it
-#pragma unroll
-      for (int tm = 0; tm < 2; ++tm) {
-        const f32x16 r = mm(zero16(), 0, 2 * (tm + 1),
-                            [&](int ks) {
-                              return op_ld_kappa<OT>(b_t + (tm == 0 ? 0 : 1 + ks / 2) * 32 * GB_TS, GB_TS, ln, 16 * (ks & 1), hh);
-                            },
-                            [&](int ks) { return Rb[ks]; });
-        op_frag_store<OT>(b_v, vn * 4 + 2 * tm + 0, lane, acc_to_op<OT>(r, 0));
-        op_frag_store<OT>(b_v, vn * 4 + 2 * tm + 1, lane, acc_to_op<OT>(r, 8));
-      }
-      lds_barrier();  // (1)
-      f32x16 acc;
-      float rs_g = 0.0f;
-      dq_state(acc, rs_g);
-      lds_barrier();  // (2)
-      dq_chunk(acc);
-      lds_barrier();  // (3)
-      finish(acc, rs_g, tok0, len);
-    }
-  } else if (!GRADS && wave < 4) {
-    for (int c = cl; c >= c0; --c) {
-      lanes();
-      stage(chunk_len[uniform(c)]);
-      issue(max(c - 1, c0));
-      lds_barrier();  // (0)
-      lds_barrier();  // (1)
-      lds_barrier();
+      lds_barrier();  // (5)
     }
   } else {
-    // ================================ the token x token tiles, dKh (waves 4-7) ================================
-    const int tw = wave - 4, jt = tw == 2 ? 1 : 0, it = tw == 0 ? 0 : 1;
+    // ============================ dKh^T; staging of dO, v, S, T; the rows of dq and dk ============================
+    GbStageRest<T, 256, true> st;
+    const int tw = wave - 8, kt = tw >> 1, tt = tw & 1;
+    auto issue = [&](int c) {
+      c = uniform(max(c, c0));
+      st.issue(dout, v, rec_of(c), states + ((size_t)c * HV + hv) * GDR_STATE_BYTES, tok_of(c), len_of(c), HV, hv, tid - 512);
+    };
+    issue(cl);
+    st.stage(set_of(cl), len_of(cl), tid - 512);
+    issue(cl - 1);
+    lds_barrier();  // (0)
     for (int c = cl; c >= c0; --c) {
-      const int tok0 = chunk_tok0[uniform(c)], len = chunk_len[uniform(c)];
       lanes();
-      stage(len);
-      if constexpr (GRADS) load_v(tok0, len);
-      else issue(max(c - 1, c0));
-      lds_barrier();  // (0)
-      const int i = 32 * it + ln;
-      // P of this wave's tile (rows j, column i): the product here and once more for grad P (16 registers less to carry)
-      auto p_tile = [&]() __attribute__((always_inline)) {
-        return mm(zero16(), 0, 4, [&](int ks) { return rows_n(b_k, 32 * jt + ln, 16 * ks); },
-                  [&](int ks) { return rows_n(b_q, i, 16 * ks); });
-      };
-      // e^{gamma_i - gamma_j} for i >= j (strict: i > j), else 0, of accumulator registers 4 b4 .. + 3
-      auto ratio = [&](int b4, float gi, int e_min, float* out) __attribute__((always_inline)) {
-        const f32x4 gj = gb_rows4(s_gam, 32 * jt, b4, hh);
-        const int lx = ln - 4 * hh - e_min + (jt != it ? 64 : 0);  // (the tile below the diagonal is full)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) out[e] = __builtin_amdgcn_exp2f(lx >= 8 * b4 + e ? gi - gj[e] : -1e30f);
-      };
-      if (wave < 7) {
-        f32x16 pm = p_tile();
-        const float gi = s_gam[i];
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4) {
-          float gm[4];
-          ratio(b4, gi, 0, gm);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) pm[4 * b4 + e] *= scale * gm[e];
-        }
-        op_frag_store<OT>(b_p + tw * GB_TRI, 0, lane, acc_to_op<OT>(pm, 0));
-        op_frag_store<OT>(b_p + tw * GB_TRI, 1, lane, acc_to_op<OT>(pm, 8));
-      }
+      const int tok = 32 * tt + ln;
+      const GbTiles<OT> t = set_of(c);
+      if (c > c0) st.stage(set_of(c - 1), len_of(c - 1), tid - 512);
+      issue(c - 2);
       lds_barrier();  // (1)
-      if constexpr (GRADS) {
-        f32x16 acc;
-        float rs_g = 0.0f, rs_b = 0.0f;  // sums over the rows of the terms of d gamma / d beta: of token i, later of tok
-        float rs_c = 0.0f, tg = 0.0f;    // sum over the columns for the tile's row gb_half_sums16 leaves here; of tok
-        float gl = 0.0f;
-        if (wave < 7) {  // grad P = dO Vn^T
-          f32x16 n = mm(zero16(), 0, 4, [&](int ks) { return fr_tr<OT, false>(b_v, 32 * jt, 16 * ks, lane); },
-                        [&](int ks) { return rows_n(b_do, i, 16 * ks); });
-          const f32x16 pm = p_tile();
-          const float gi = s_gam[i];
-          float cs[16];  // the terms of d gamma, for their sums over the columns
+      const unsigned char* vf = reinterpret_cast<const unsigned char*>(t.v);
+      float rs_g, rs_b = 0.0f;  // the terms of d gamma / d beta of this lane's token
+      // D G' Vn^T
+      f32x16 acc = gb_mm<OT>(zero16(), [&](int ks) { return fr_tr<OT, false>(b_g, 32 * kt, 16 * ks, lane); },
+                             [&](int ks) { return fr_tr<OT, false>(vf, 32 * tt, 16 * ks, lane); });
+      {
+        const float fd = t.dk[tok];
 #pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {
-            float gm[4];
-            ratio(b4, gi, 0, gm);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int r = 4 * b4 + e;
-              n[r] *= scale * gm[e];
-              cs[r] = n[r] * pm[r];
-              rs_g += cs[r];
-            }
-          }
-          op_frag_store<OT>(b_n + tw * GB_TRI, 0, lane, acc_to_op<OT>(n, 0));
-          op_frag_store<OT>(b_n + tw * GB_TRI, 1, lane, acc_to_op<OT>(n, 8));
-          rs_c = gb_half_sums16(cs, lane);
-        } else {  // e^{gamma_L} <G', S>
-          float x = 0.0f;
-#pragma unroll
-          for (int f = 0; f < 8; ++f) {
-            const X8 xa = op_frag_load<OT>(b_g, f, lane), xb = op_frag_load<OT>(b_s, f, lane);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x = __builtin_fmaf((float)xa[e], (float)xb[e], x);
-          }
-          gl = x * __builtin_amdgcn_exp2f(s_gam[63]);
-        }
-        // dKh^T: D G' Vn^T first
-        acc = mm(zero16(), 0, 4, [&](int ks) { return fr_tr<OT, false>(b_g, 32 * kt, 16 * ks, lane); },
-                 [&](int ks) { return fr_tr<OT, false>(b_v, 32 * tt, 16 * ks, lane); });
-        {
-          const float fd = s_dk[tok];
-          float t = 0.0f;
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {
-            const X4 y = *reinterpret_cast<const X4*>(&b_k[tok * GB_LS + 32 * kt + 8 * b4 + 4 * hh]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              acc[4 * b4 + e] *= fd;
-              t += (float)y[e] * acc[4 * b4 + e];
-            }
-          }
-          gl += t;
-          tg = -t;
-        }
-        lds_barrier();  // (2)
-        if (wave < 7) {  // grad A = -X Vn^T
-          f32x16 da = mm(zero16(), 0, 4, [&](int ks) { return fr_tr<OT, false>(b_v, 32 * jt, 16 * ks, lane); },
-                         [&](int ks) { return fr_tr<OT, false>(b_x, 32 * it, 16 * ks, lane); });
-          const f32x16 kk = mm(zero16(), 0, 4, [&](int ks) { return rows_n(b_k, 32 * jt + ln, 16 * ks); },
-                               [&](int ks) { return rows_n(b_k, i, 16 * ks); });
-          const float bi = s_beta[i], gi = s_gam[i];
-          float cs[16];
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {
-            float gm[4];
-            ratio(b4, gi, 1, gm);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int r = 4 * b4 + e;
-              // grad A_ij Gamma_ij, and grad A_ij times A_ij / beta_i and times A_ij
-              const float ga = -da[r] * gm[e], b = ga * kk[r], a = b * bi;
-              rs_b += b;
-              rs_g += a;
-              cs[r] = a;
-              da[r] = ga * bi;
-            }
-          }
-          op_frag_store<OT>(b_m + tw * GB_TRI, 0, lane, acc_to_op<OT>(da, 0));
-          op_frag_store<OT>(b_m + tw * GB_TRI, 1, lane, acc_to_op<OT>(da, 8));
-          rs_c += gb_half_sums16(cs, lane);
-          rs_g = gb_both_halves(rs_g);
-          rs_b = gb_both_halves(rs_b);
-          if (hh == 0) {
-            s_sum[GbSums::TILE_G + 32 * tw + ln] = rs_g;
-            s_sum[GbSums::TILE_B + 32 * tw + ln] = rs_b;
-          }
-          if (!(ln & 1)) s_sum[GbSums::TILE_C + 32 * tw + 8 * (ln >> 3) + 4 * hh + ((ln >> 1) & 3)] = rs_c;
-          rs_b = 0.0f;
-        }
-        issue(max(c - 1, c0));
-        {  // -(S X^T), the gradient of beta e^gamma Kh
-          const f32x16 xw = mm(zero16(), 0, 4, [&](int ks) { return fr_tr<OT, false>(b_s, 32 * kt, 16 * ks, lane); },
-                               [&](int ks) { return fr_tr<OT, false>(b_x, 32 * tt, 16 * ks, lane); });
-          const float fe = -s_eg[tok], fb = s_beta[tok];
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4) {
-            const X4 y = *reinterpret_cast<const X4*>(&b_k[tok * GB_LS + 32 * kt + 8 * b4 + 4 * hh]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float t = fe * xw[4 * b4 + e];
-              rs_b += (float)y[e] * t;
-              acc[4 * b4 + e] = __builtin_fmaf(fb, t, acc[4 * b4 + e]);
-            }
-          }
-          rs_g = __builtin_fmaf(fb, rs_b, tg);
-          rs_b = gb_both_halves(rs_b);
-          if (hh == 0) s_sum[GbSums::DBETA + 32 * tw + ln] = rs_b;
-        }
-        // + (N^T Qh)^T
-        acc = mm(acc, 2 * tt, 4, [&](int ks) { return cols(b_q, 32 * kt, 16 * ks); },
-                 [&](int ks) { return fr_tr<OT, true>(b_n + (tt == 0 ? ks / 2 : 2) * GB_TRI, 0, 16 * (ks & 1), lane); });
-        {
-          const float t = gb_half_sum(gl);
-          if (ln == 0) s_sum[GbSums::GL + 2 * tw + hh] = t;
-        }
-        lds_barrier();  // (3) M is complete
-        // + (M Kh)^T + (M^T Kh)^T
-        acc = mm(acc, 0, 2 * (tt + 1), [&](int ks) { return cols(b_k, 32 * kt, 16 * ks); },
-                 [&](int ks) { return op_frag_load<OT>(b_m + (tt + ks / 2) * GB_TRI, ks & 1, lane); });
-        acc = mm(acc, 2 * tt, 4, [&](int ks) { return cols(b_k, 32 * kt, 16 * ks); },
-                 [&](int ks) { return fr_tr<OT, true>(b_m + (tt == 0 ? ks / 2 : 2) * GB_TRI, 0, 16 * (ks & 1), lane); });
-        finish(acc, rs_g, tok0, len);
-      } else {
-        lds_barrier();
+        for (int r = 0; r < 16; ++r) acc[r] *= fd;
+        const float x = row_dot(t.k, acc, kt, tok);
+        rs_g = -x;
+        const float gl = gb_half_sum(x);
+        if (ln == 0) s_sum[GbSums::GL + 2 * tw + hh] = gl;
       }
+      lds_barrier();  // (2)
+      {  // -(S X^T), the gradient of beta e^gamma Kh
+        f32x16 xw = gb_mm<OT>(zero16(), [&](int ks) { return fr_tr<OT, false>(t.s, 32 * kt, 16 * ks, lane); },
+                              [&](int ks) { return fr_tr<OT, false>(b_x, 32 * tt, 16 * ks, lane); });
+        const float fe = -t.eg[tok], fb = t.beta[tok];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          xw[r] *= fe;
+          acc[r] = __builtin_fmaf(fb, xw[r], acc[r]);
+        }
+        rs_b = row_dot(t.k, xw, kt, tok);
+        rs_g = gb_both_halves(__builtin_fmaf(fb, rs_b, rs_g));
+        rs_b = gb_both_halves(rs_b);
+        if (hh == 0) {
+          s_sum[GbSums::DBETA + 32 * tw + ln] = rs_b;
+          s_sum[GbSums::DGAM + 64 + 32 * tw + ln] = rs_g;
+        }
+      }
+      lds_barrier();  // (3)
+      // + (N^T Qh)^T
+      acc = gb_mm_tri<OT, false>(acc, tt, [&](int ks) { return gb_cols<OT>(t.q, 32 * kt, 16 * ks, lane); }, [&](int ks) {
+        return fr_tr<OT, true>(b_n + (tt == 0 ? ks / 2 : 2) * GB_TRI, 0, 16 * (ks & 1), lane);
+      });
+      // + (M Kh)^T + (M^T Kh)^T
+      acc = gb_mm_tri<OT, true>(acc, tt, [&](int ks) { return gb_cols<OT>(t.k, 32 * kt, 16 * ks, lane); }, [&](int ks) {
+        return op_frag_load<OT>(b_m + (tt + ks / 2) * GB_TRI, ks & 1, lane);
+      });
+      acc = gb_mm_tri<OT, false>(acc, tt, [&](int ks) { return gb_cols<OT>(t.k, 32 * kt, 16 * ks, lane); }, [&](int ks) {
+        return fr_tr<OT, true>(b_m + (tt == 0 ? ks / 2 : 2) * GB_TRI, 0, 16 * (ks & 1), lane);
+      });
+      float dot = gb_both_halves(row_dot(t.k, acc, kt, tok));
+      if (hh == 0) s_sum[GbSums::DOTK + 64 * kt + tok] = dot;
+      lds_barrier();  // (4)
+      dot = s_sum[GbSums::DOTK + tok] + s_sum[GbSums::DOTK + 64 + tok];
+      rows_out(b_ok, t.k, acc, kt, tok, dot, t.rk[tok]);
+      lds_barrier();  // (5)
     }
   }
-
 }
 
 // ---- host ----------------------------------------------------------------------------------------------------------
@@ -893,10 +1211,10 @@ static int gb_run(const void* q, const void* k, const void* v, const void* dout,
   {
     std::lock_guard<std::mutex> hold(attr_lock);
     if (!attr_set[dev]) {
-      if (hipFuncSetAttribute((const void*)gdrb_segment_kernel<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              GbSmem<false>::BYTES) != hipSuccess ||
-          hipFuncSetAttribute((const void*)gdrb_segment_kernel<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              GbSmem<true>::BYTES) != hipSuccess)
+      if (hipFuncSetAttribute((const void*)gdrb_source_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              GbSourceSmem::BYTES) != hipSuccess ||
+          hipFuncSetAttribute((const void*)gdrb_walk_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              GbWalkSmem::BYTES) != hipSuccess)
         return LAMPA_ERR_LAUNCH;
       attr_set[dev] = true;
     }
@@ -912,20 +1230,19 @@ static int gb_run(const void* q, const void* k, const void* v, const void* dout,
   const float* Dc = (const float*)(saved + sv.off_d);
   LAMPA_PROF(s, "start");
   if (segs > n_seq) {
-    hipLaunchKernelGGL((gdrb_segment_kernel<T, false>), dim3(segs * HV), dim3(GB_THREADS), GbSmem<false>::BYTES, s,
-                       (const T*)q, (const T*)k, (const T*)v, (const T*)dout, recs, states, pv, pv.chunk_tok0, pv.chunk_len,
-                       Mt, Dc, Nr, Gm, Gn, Gd, 0, dht, (T*)dq, (T*)dk, (T*)dv, dg, dbeta, dh0, H, HV, scale, l2norm);
-    LAMPA_PROF(s, "gdrb_segment_kernel<source>");
+    hipLaunchKernelGGL((gdrb_source_kernel<T>), dim3(segs * HV), dim3(GB_SOURCE_THREADS), GbSourceSmem::BYTES, s, (const T*)q,
+                       (const T*)k, (const T*)dout, recs, pv, pv.chunk_tok0, pv.chunk_len, Nr, H, HV, scale, l2norm);
+    LAMPA_PROF(s, "gdrb_source_kernel");
     if (gmax > 0) {
       hipLaunchKernelGGL((gdr_scan2_kernel<T, 64, 64, 4, SCAN_GROUP, true>), dim3(4 * gmax, n_seq, HV), dim3(128), 0, s, pv, Mt,
                          Nr, Dc, (const float*)nullptr, (float*)nullptr, Gm, Gn, Gd, HV, 0, gmax);
       LAMPA_PROF(s, "gdr_scan2_kernel<group, reversed>");
     }
   }
-  hipLaunchKernelGGL((gdrb_segment_kernel<T, true>), dim3(segs * HV), dim3(GB_THREADS), GbSmem<true>::BYTES, s, (const T*)q,
-                     (const T*)k, (const T*)v, (const T*)dout, recs, states, pv, pv.chunk_tok0, pv.chunk_len, Mt, Dc, Nr, Gm,
-                     Gn, Gd, gmax, dht, (T*)dq, (T*)dk, (T*)dv, dg, dbeta, dh0, H, HV, scale, l2norm);
-  LAMPA_PROF(s, "gdrb_segment_kernel<gradients>");
+  hipLaunchKernelGGL((gdrb_walk_kernel<T>), dim3(segs * HV), dim3(GB_WALK_THREADS), GbWalkSmem::BYTES, s, (const T*)q,
+                     (const T*)k, (const T*)v, (const T*)dout, recs, states, pv, pv.chunk_tok0, pv.chunk_len, Mt, Dc, Nr, Gm, Gn,
+                     Gd, gmax, dht, (T*)dq, (T*)dk, (T*)dv, dg, dbeta, dh0, H, HV, scale, l2norm);
+  LAMPA_PROF(s, "gdrb_walk_kernel");
   return lampa_launch_status();
 }
 

@@ -267,6 +267,21 @@ def test_chunked_gradients_one_chunk_per_segment(device, T, K, V, monkeypatch):
         _check(got, want, torch.bfloat16, chunked=True)
 
 
+@pytest.mark.parametrize("cps", [2, 3])
+@pytest.mark.parametrize("l2norm", [False, True])
+def test_chunked_gradients_tile_sets(device, cps, l2norm, monkeypatch):
+    """Segments of two and three chunks (the walks alternate between two sets of tiles and write a chunk's rows of dq and dk a
+    chunk later), a sequence ending in a partial chunk, an empty one and one of a single token, two value heads per head."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
+    cu = torch.tensor([0, 64 * 7 + 33, 64 * 7 + 33, 64 * 7 + 34])
+    (q, k, v, g, beta, do), gen = _inputs(1, int(cu[-1]), 1, 2, 64, 64, torch.bfloat16, 17 + cps, unit=not l2norm, g_scale=0.05)
+    h0 = 0.5 * torch.randn(3, 2, 64, 64, generator=gen)
+    dht = torch.randn(3, 2, 64, 64, generator=gen)
+    want = ob.backward_manual(q, k, v, g, beta, do, dht, None, h0, cu, og.L2_CHUNK if l2norm else og.L2_NONE)
+    got = _gpu_grads(device, q, k, v, g, beta, do, h0, dht, cu, l2norm)
+    _check(got, want, torch.bfloat16, chunked=True)
+
+
 def test_chunked_gradients_at_full_size_against_the_token_serial_form(device, monkeypatch):
     """Config-2 shape (60 000 tokens, 8 heads, K = V = 64, bf16), too long for the float64 loop: the chunked form on the
     MFMA against the fp32 token-serial form, two implementations that share no kernel of the backward pass."""
