@@ -90,6 +90,8 @@ _SIGNATURES = {
                                     _i32, _i32, _f32, _i32, _vp, _i64, _vp]),
     "lampa_hgdn_step": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32,
                                _i32, _i32, _f32, _i32, _vp]),
+    "lampa_hgdn_tail": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32,
+                               _i32, _i32, _i32, _f32, _i32, _vp]),
 }
 
 _lib = None

@@ -460,3 +460,208 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
   LAMPA_PROF(s, "hgdn_step_kernel");
   return lampa_launch_status();
 }
+
+// ---- the tokens behind the whole chunks, in one launch -----------------------------------------------------------------
+// A wavefront owns one value column of one (sequence, value head): lane = state row (two rows for K > 64), the row's LM level
+// values in registers from the first token to the last, so a token costs no barrier, no LDS and no pass over the states.
+// Sums over the rows (k^T S_l for the levels > 0, the output, the two norms) are exchanges between lanes: 16 levels at a time
+// are halved four times until a lane holds one level's sum over its group of 16 lanes (`wave_sums16`), and go back to all
+// lanes as scalars. What bounds it is that serial chain per token (B * HV * V wavefronts, two per compute unit at 8 heads of
+// 64 columns); the next token's values are loaded while this one is worked on.
+// A prefill of 15 000 tokens (24 behind its whole chunks, 8 heads of 64 x 64): 708 us with a launch of the single-token kernel
+// and its copies per token, 210 us with this kernel.
+#define HGS_TAIL_LEVELS 17  // levels of the narrow instantiation: sequences up to 65 536 tokens
+#define HGS_TAIL_WAVES 4
+#define HGS_DPP_ROR8 0x128
+#define HGS_DPP_HALF_MIRROR 0x141
+
+__device__ __forceinline__ float hgs_fold32(float a, float b) {  // lanes < 32: both halves of a, lanes >= 32: of b
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
+__device__ __forceinline__ float hgs_fold16(float a, float b) {  // even rows of 16 lanes: rows pairs of a, odd rows: of b
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
+__device__ __forceinline__ float wave_sum_all(float x) {
+  x = hgs_fold32(x, x);
+  x = hgs_fold16(x, x);
+  x += dpp_f32<HGS_DPP_ROR8, 0xF>(0.0f, x);
+  x += dpp_f32<HGS_DPP_HALF_MIRROR, 0xF>(0.0f, x);
+  x += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, x);
+  return x + dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, x);
+}
+
+// Sums of 16 values over the wave: lanes 4n .. 4n + 3 return the sum of p[n] over all 64 lanes.
+__device__ __forceinline__ float wave_sums16(float* p, int lane) {
+#pragma unroll
+  for (int n = 0; n < 8; ++n) p[n] = hgs_fold32(p[n], p[n + 8]);
+#pragma unroll
+  for (int n = 0; n < 4; ++n) p[n] = hgs_fold16(p[n], p[n + 4]);
+  const bool b3 = lane & 8, b2 = lane & 4;
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+    p[n] = (b3 ? p[n + 2] : p[n]) + dpp_f32<HGS_DPP_ROR8, 0xF>(0.0f, b3 ? p[n] : p[n + 2]);
+  float x = (b2 ? p[1] : p[0]) + dpp_f32<HGS_DPP_HALF_MIRROR, 0xF>(0.0f, b2 ? p[0] : p[1]);
+  x += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, x);
+  return x + dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, x);
+}
+
+__device__ __forceinline__ float hgs_lane(float x, int n) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), n));
+}
+
+template <typename T, int LM, int ROWS>
+__global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
+    hgdn_tail_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
+                     const float* __restrict__ g, const float* __restrict__ beta, const void* __restrict__ lam,
+                     int lam_dtype, float lam_div, float* __restrict__ states, T* __restrict__ o, int n_tok, int tok0, int H,
+                     int HV, int K, int V, int L, float scale, int l2norm) {
+  const int lane = threadIdx.x & 63;
+  const int j = blockIdx.y * HGS_TAIL_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (j >= V) return;
+  const int b = blockIdx.x / HV, hv = blockIdx.x % HV, h = hv / (HV / H);
+  float* col = states + (((size_t)b * HV + hv) * K * V + j) * L;  // row i: col + i * V * L
+  float S[ROWS][LM];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const int i = lane + 64 * r;
+#pragma unroll
+    for (int l = 0; l < LM; ++l) S[r][l] = (i < K && l < L) ? col[(size_t)i * V * L + l] : 0.0f;
+  }
+  struct Token {
+    float q[ROWS], k[ROWS], lam, v, g, beta;
+  };
+  auto load = [&](int t) {
+    Token x;
+    const size_t tok = (size_t)b * n_tok + t;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const int i = lane + 64 * r;
+      x.q[r] = i < K ? GdrElem<T>::to_float(q[(tok * H + h) * K + i]) : 0.0f;
+      x.k[r] = i < K ? GdrElem<T>::to_float(k[(tok * H + h) * K + i]) : 0.0f;
+    }
+    const size_t li = (tok * HV + hv) * L + lane;
+    x.lam = 0.0f;
+    if (lane < L)
+      x.lam = lam_dtype == GDR_FP32   ? reinterpret_cast<const float*>(lam)[li]
+              : lam_dtype == GDR_BF16 ? (float)reinterpret_cast<const __bf16*>(lam)[li]
+                                      : (float)reinterpret_cast<const _Float16*>(lam)[li];
+    x.v = GdrElem<T>::to_float(v[(tok * HV + hv) * V + j]);
+    x.g = g[tok * HV + hv];
+    x.beta = beta[tok * HV + hv];
+    return x;
+  };
+  Token next = load(tok0);
+  for (int t = tok0; t < n_tok; ++t) {
+    const Token x = next;
+    next = load(min(t + 1, n_tok - 1));
+    float lam_l = x.lam;
+    if (lam_div != 1.0f) {  // lambda / scale, rounded to lambda's own type as the element-wise division would
+      lam_l = __fdiv_rn(lam_l, lam_div);
+      lam_l = lam_dtype == GDR_FP32 ? lam_l : lam_dtype == GDR_BF16 ? (float)(__bf16)lam_l : (float)(_Float16)lam_l;
+    }
+    // cascade: after t tokens the levels below 1 + (trailing zero bits of t) are full
+    const int z = t == 0 ? 0 : 1 + __builtin_ctz(t);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      float acc = S[r][0];
+#pragma unroll
+      for (int l = 1; l < LM; ++l) {
+        const float s = S[r][l];
+        S[r][l] = l < z ? 0.0f : l == z ? s + acc : s;
+        acc = l < z ? acc + s : acc;
+      }
+      S[r][0] = 0.0f;  // (empty before the first token)
+    }
+    float qs = 0.0f, ks = 0.0f;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      qs = __builtin_fmaf(x.q[r], x.q[r], qs);
+      ks = __builtin_fmaf(x.k[r], x.k[r], ks);
+    }
+    float rq = scale, rk = 1.0f;
+    if (l2norm == GDR_L2_CHUNK) {
+      rq = scale / __fsqrt_rn(wave_sum_all(qs) + 1e-6f);
+      rk = 1.0f / __fsqrt_rn(wave_sum_all(ks) + 1e-6f);
+    } else if (l2norm == GDR_L2_RECURRENT) {
+      rq = scale / (__fsqrt_rn(wave_sum_all(qs)) + 1e-6f);
+      rk = 1.0f / (__fsqrt_rn(wave_sum_all(ks)) + 1e-6f);
+    }
+    const float a = __expf(x.g), bk = x.beta * rk;
+    float sl[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      S[r][0] = x.k[r] * (bk * x.v);
+      sl[r] = hgs_lane(lam_l, 0) * S[r][0];
+    }
+#pragma unroll
+    for (int l0 = 1; l0 < LM; l0 += 16) {
+      float p[16];
+#pragma unroll
+      for (int n = 0; n < 16; ++n) {
+        p[n] = 0.0f;
+        if (l0 + n < LM)
+#pragma unroll
+          for (int r = 0; r < ROWS; ++r) p[n] = __builtin_fmaf(x.k[r], S[r][l0 + n], p[n]);
+      }
+      const float d = wave_sums16(p, lane);
+#pragma unroll
+      for (int n = 0; n < 16; ++n) {
+        const int l = l0 + n;
+        if (l < LM) {
+          const float c = -bk * (rk * hgs_lane(d, 4 * n)), al = l < L ? a : 0.0f;
+#pragma unroll
+          for (int r = 0; r < ROWS; ++r) {
+            S[r][l] = al * __builtin_fmaf(x.k[r], c, S[r][l]);
+            sl[r] = __builtin_fmaf(hgs_lane(lam_l, l), S[r][l], sl[r]);
+          }
+        }
+      }
+    }
+    float acc_o = 0.0f;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) acc_o = __builtin_fmaf(x.q[r], sl[r], acc_o);
+    acc_o = rq * wave_sum_all(acc_o);
+    if (lane == 0) o[(((size_t)b * n_tok + t) * HV + hv) * V + j] = GdrElem<T>::from_float(acc_o);
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const int i = lane + 64 * r;
+#pragma unroll
+    for (int l = 0; l < LM; ++l)
+      if (i < K && l < L) col[(size_t)i * V * L + l] = S[r][l];
+  }
+}
+
+// Tokens tok0 .. n_tok - 1 of every sequence on the level states after its first tok0 tokens: q, k [B, n_tok, H, K],
+// v, o [B, n_tok, HV, V], g, beta [B, n_tok, HV], lam [B, n_tok, HV, L], states [B, HV, K, V, L] updated in place.
+extern "C" int lampa_hgdn_tail(const void* q, const void* k, const void* v, const float* g, const float* beta,
+                               const void* lam, int lam_dtype, float lam_div, float* states, void* o, int B, int n_tok,
+                               int tok0, int H, int HV, int K, int V, int L, int dtype, float scale, int l2norm,
+                               void* stream) {
+  if (!q || !k || !v || !g || !beta || !lam || !states || !o) return LAMPA_ERR_INVALID;
+  if (B < 0 || H < 1 || HV < H || HV % H != 0 || K < 1 || V < 1 || L < 1 || tok0 < 0 || n_tok < tok0)
+    return LAMPA_ERR_INVALID;
+  if (l2norm < 0 || l2norm > 2 || lam_dtype < 0 || lam_dtype > 2 || !(lam_div > 0.0f)) return LAMPA_ERR_INVALID;
+  if (V > 1024 || L > HGS_LMAX || K > 128 || dtype < 0 || dtype > 2) return LAMPA_ERR_UNSUPPORTED;
+  if (B == 0 || n_tok == tok0) return LAMPA_OK;
+  // the level that the fullest cascade of these tokens fills has to exist (token t fills level 1 + its trailing zero bits)
+  for (int t = tok0 > 1 ? tok0 : 1; t < n_tok; ++t)
+    if (1 + __builtin_ctz(t) >= L) return LAMPA_ERR_INVALID;
+  hipStream_t s = (hipStream_t)stream;
+  LAMPA_PROF(s, "start");
+#define HGS_TAIL(TT, LM, RR)                                                                                              hipLaunchKernelGGL((hgdn_tail_kernel<TT, LM, RR>), dim3(B * HV, (V + HGS_TAIL_WAVES - 1) / HGS_TAIL_WAVES),                                  dim3(64 * HGS_TAIL_WAVES), 0, s, (const TT*)q, (const TT*)k, (const TT*)v, g, beta, lam, lam_dtype,                      lam_div, states, (TT*)o, n_tok, tok0, H, HV, K, V, L, scale, l2norm)
+#define HGS_TAIL_ROWS(TT, LM)             do {                                      if (K <= 64) HGS_TAIL(TT, LM, 1);       else HGS_TAIL(TT, LM, 2);             } while (0)
+#define HGS_TAIL_CASE(TT)                                              do {                                                                   if (L <= HGS_TAIL_LEVELS) HGS_TAIL_ROWS(TT, HGS_TAIL_LEVELS);        else HGS_TAIL_ROWS(TT, HGS_LMAX);                                  } while (0)
+  if (dtype == GDR_BF16) HGS_TAIL_CASE(__bf16);
+  else if (dtype == GDR_FP16) HGS_TAIL_CASE(_Float16);
+  else HGS_TAIL_CASE(float);
+#undef HGS_TAIL_CASE
+#undef HGS_TAIL_ROWS
+#undef HGS_TAIL
+  LAMPA_PROF(s, "hgdn_tail_kernel");
+  return lampa_launch_status();
+}

@@ -96,6 +96,12 @@ class HState(object):
                 raise ValueError
         return z
 
+    def _set_counts(self, tokens: int) -> None:
+        """The counts after ``tokens`` > 0 tokens (``kernel.py:451-462``): the last token alone in level 0, level l > 0
+        holds 2^(l-1) tokens iff that bit of tokens - 1 is set."""
+        self._counts = [1] + [(1 << (level - 1)) if ((tokens - 1) >> (level - 1)) & 1 else 0
+                              for level in range(1, self.max_num_levels)]
+
     def reset_states(self) -> None:
         self.states = torch.zeros_like(self.states)
 
@@ -148,7 +154,8 @@ def _plan(B: int, T: int, device, n_value_heads: int, n_slabs: int):
 
 class _ForwardOnly(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, k, v, g, lam, beta, scale, lam_div, level_states=None):
+    def forward(ctx, q, k, v, g, lam, beta, scale, lam_div, level_states=None, n_out=None):
+        """``n_out``: tokens per sequence of the returned buffer (the caller fills those behind the whole chunks)."""
         require_cuda(q, k, v, g, lam, beta)
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
@@ -163,12 +170,19 @@ class _ForwardOnly(torch.autograd.Function):
         ws_bytes = check(lib.lampa_hgdn_chunk_workspace_bytes(chunks, segs, HV, K, V), "lampa_hgdn_chunk_workspace_bytes")
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         o = torch.empty_like(v)
+        if n_out is not None and n_out != T:
+            whole = v.new_empty((B, n_out, HV, V))
+            o = whole[:, :T] if B == 1 else o  # (one sequence: the chunks' rows are a piece of the buffer)
+        else:
+            whole = o
         check(lib.lampa_hgdn_chunk_fwd(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(lam), _gd._DTYPES[lam.dtype],
                                        float(lam_div), ptr(o), ptr(level_states),
                                        ctypes.c_void_p(plan_host.data_ptr()), ptr(plan_dev), H, HV, K, V, L,
                                        _gd._DTYPES[q.dtype], float(scale), _gd.L2_CHUNK, ptr(ws), ws_bytes, stream_of(q)),
               "lampa_hgdn_chunk_fwd")
-        return o
+        if whole is not o and B > 1:
+            whole[:, :T] = o
+        return whole
 
     @staticmethod
     def backward(ctx, *grads):
@@ -215,7 +229,10 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         require_cuda(q, k, v, g, l, beta)
         hstate = HState(2, HType.WEAK, HStruct.GDELTA, (B, HV, K, V, L), torch.float32, q.device)
         T0 = T - T % 64
-        o = torch.empty_like(v)
+        if T0 < T:  # (the tail kernel reads the whole tensors)
+            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+            g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
+            l = (l if l.dtype in _gd._DTYPES else l.to(torch.float32)).contiguous()
         if T0:
             _check_chunk_shapes(T0, K, V, L)
             cut = lambda x: x[:, :T0]
@@ -223,16 +240,17 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
             padded = pq.shape[-1] != K or pv.shape[-1] != V
             states = (torch.zeros(B, HV, pq.shape[-1], pv.shape[-1], L, dtype=torch.float32, device=q.device)
                       if padded else hstate.states)
-            o[:, :T0] = _ForwardOnly.apply(pq, pk, pv, cut(g), cut(l), cut(beta), scale, lam_div, states)[..., :V]
+            o = _ForwardOnly.apply(pq, pk, pv, cut(g), cut(l), cut(beta), scale, lam_div, states, T)[..., :V].contiguous()
             if padded:  # (the padded rows and columns of the states are zero)
                 hstate.states = states[:, :, :K, :V].contiguous()
-            # counts after T0 tokens (kernel.py:451-462): the last token alone in level 0, level l > 0 holds 2^(l-1)
-            # tokens iff that bit of T0 - 1 is set
-            hstate._counts[0] = 1
-            for level in range(1, L):
-                hstate._counts[level] = (1 << (level - 1)) if ((T0 - 1) >> (level - 1)) & 1 else 0
-        for t in range(T0, T):
-            o[:, t] = _step(hstate, q[:, t], k[:, t], v[:, t], g[:, t], l[:, t], beta[:, t], scale, lam_div)
+            hstate._set_counts(T0)
+        else:
+            o = torch.empty_like(v)
+        if T0 < T and K <= TAIL_MAX_K:
+            _tail(hstate, q, k, v, g, l, beta, o, T0, scale, lam_div)
+        else:
+            for t in range(T0, T):
+                o[:, t] = _step(hstate, q[:, t], k[:, t], v[:, t], g[:, t], l[:, t], beta[:, t], scale, lam_div)
         return o, hstate
     if not all([q.ndim == 4, q.shape[1] == 1, k.ndim == 4, k.shape[1] == 1, v.ndim == 4, v.shape[1] == 1,
                 beta.ndim == 3, beta.shape[1] == 1, g.ndim == 3, g.shape[1] == 1, l.ndim == 4, l.shape[1] == 1]):
@@ -259,6 +277,25 @@ def _check_chunk_shapes(T: int, K: int, V: int, L: int) -> None:
         raise ValueError
     if (T // 64) > 4096:
         raise NotImplementedError("hierarchical chunk kernels: at most 4096 chunks per sequence")
+
+
+TAIL_MAX_K = 128  # ``lampa_hgdn_tail`` holds a state column in two registers per lane and level at most
+
+
+def _tail(hstate: HState, q, k, v, g, l, beta, o, t0: int, scale, lam_div) -> None:
+    """Tokens ``t0 ..`` of contiguous ``[B, T, ...]`` tensors on the level states after the first ``t0`` tokens, in one
+    launch: what ``_step`` does token by token. Writes rows ``t0 ..`` of ``o`` and updates ``hstate`` in place."""
+    if not all([q.ndim == 4, k.ndim == 4, v.ndim == 4, beta.ndim == 3, g.ndim == 3, l.ndim == 4]):
+        raise TypeError
+    B, T, H, K = q.shape
+    HV, V, L = v.shape[2], v.shape[3], l.shape[-1]
+    # token t fills level 1 + the trailing zero bits of t: the largest power of two decides
+    if max((t & -t).bit_length() for t in range(t0, T)) >= L:
+        raise ValueError("the state has no level left for this many tokens")
+    check(_capi.lib().lampa_hgdn_tail(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(l), _gd._DTYPES[l.dtype], float(lam_div),
+                                      ptr(hstate.states), ptr(o), B, T, t0, H, HV, K, V, L, _gd._DTYPES[q.dtype],
+                                      float(scale), _gd.L2_CHUNK, stream_of(q)), "lampa_hgdn_tail")
+    hstate._set_counts(T)
 
 
 def _step(hstate: HState, q, k, v, g, l, beta, scale, lam_div, token_dim: bool = False) -> torch.Tensor:

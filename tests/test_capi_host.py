@@ -229,6 +229,13 @@ def test_hierarchical_forward_argument_checks(lib):
     assert lib.lampa_hgdn_step(d, d, d, d, d, d, 0, 0.125, d, d, 2, 2, 2, 64, 64, 13, 13, 0, 0.125, 1, None) == -1  # z < L
     assert lib.lampa_hgdn_step(d, d, d, d, d, d, 0, 0.125, d, d, 2, 2, 2, 64, 64, 40, 1, 0, 0.125, 1, None) == -4     # more than 32 levels
     assert lib.lampa_hgdn_step(d, d, d, d, d, d, 0, 0.125, d, d, 0, 2, 2, 64, 64, 13, 0, 0, 0.125, 1, None) == 0     # empty batch
+    # several tokens in one launch
+    tail = lambda B, n, t0, K, L: lib.lampa_hgdn_tail(d, d, d, d, d, d, 0, 0.125, d, d, B, n, t0, 2, 2, K, 64, L, 0, 0.125, 1,
+                                                      None)
+    assert tail(2, 70, 71, 64, 13) == -1  # starts behind its end
+    assert tail(2, 70, 64, 64, 7) == -1   # token 64 fills level 7
+    assert tail(2, 70, 64, 129, 13) == -4 and tail(2, 70, 64, 64, 33) == -4
+    assert tail(0, 70, 64, 64, 13) == 0 and tail(2, 64, 64, 64, 13) == 0
 
 
 def test_operators_refuse_cpu_tensors():

@@ -228,6 +228,45 @@ def test_step_entry_point_fp32_and_odd_sizes(device, B, T, H, HV, K, V, L):
     assert (states.cpu() - want_s).abs().max() <= 2e-5 * want_s.abs().max()
 
 
+@pytest.mark.parametrize("B,T,t0,H,HV,K,V,L,dtype", [
+    (2, 63, 0, 2, 4, 64, 64, 7, 2),    # from an empty state, exactly the levels needed
+    (2, 40, 1, 1, 1, 5, 3, 17, 2),     # most lanes idle, one workgroup with an idle wave, all levels of the narrow form
+    (1, 70, 33, 2, 2, 65, 6, 18, 2),   # second row of a lane holds one row; first size of the wide form
+    (3, 12, 5, 2, 2, 128, 33, 32, 0),  # both rows full, 32 levels, bf16 tokens
+])
+def test_tail_entry_point_odd_sizes(device, B, T, t0, H, HV, K, V, L, dtype):
+    # several tokens in one launch, continuing from the states the single-token kernel left after t0 tokens
+    import ctypes
+    from lampa_amd import _capi
+    from lampa_amd._capi import ptr
+    gen = torch.Generator().manual_seed(K + V)
+    tt = torch.float32 if dtype == 2 else torch.bfloat16
+    q, k = (torch.randn(B, T, H, K, generator=gen).to(tt) for _ in range(2))
+    v = torch.randn(B, T, HV, V, generator=gen).to(tt)
+    g, beta = -0.2 * torch.rand(B, T, HV, generator=gen), torch.rand(B, T, HV, generator=gen)
+    lam = torch.randn(B, T, HV, L, generator=gen)
+    want_o, want_s, want_c = oh.recurrent_c_state(q, k, v, g, beta, lam, scale=0.3)
+    args = [x.to(device) for x in (q, k, v, g, beta, lam)]
+    states = torch.zeros(B, HV, K, V, L, device=device)
+    st = hgdn.HState(2, hgdn.HType.WEAK, hgdn.HStruct.GDELTA, (B, HV, K, V, L), torch.float32, device)
+    lib, stream = _capi.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for t in range(t0):
+        a = [x[:, t].contiguous() for x in args]
+        assert lib.lampa_hgdn_step(*(ptr(x) for x in a), 2, 1.0, ptr(states), ptr(torch.empty_like(a[2])), B, H, HV, K, V, L,
+                                   st.cascade_weak(), dtype, 0.3, 1, stream) == 0
+        st._counts[0] += 1
+    o = torch.full_like(args[2], 7.0)
+    assert lib.lampa_hgdn_tail(*(ptr(x) for x in args), 2, 1.0, ptr(states), ptr(o), B, T, t0, H, HV, K, V, L, dtype, 0.3, 1,
+                               stream) == 0
+    st._set_counts(T)
+    assert st.counts.tolist() == want_c.tolist()
+    assert (o[:, :t0] == 7.0).all()  # rows before t0 are not touched
+    # fp32 arithmetic against fp64 (unit keys: no growth); bf16 outputs are rounded once, 2^-8 relative
+    assert (states.cpu() - want_s).abs().max() <= 2e-5 * want_s.abs().max()
+    bound = 2e-5 if dtype == 2 else 2 ** -8
+    assert (o[:, t0:].float().cpu() - want_o[:, t0:]).abs().max() <= bound * want_o.abs().max()
+
+
 @pytest.mark.parametrize("g_scale", [1.0, 0.003])
 def test_full_length_prefill_matches_oracle(device, g_scale):
     # the benchmark's sequence length (938 chunks, 17 levels, split into segments by the default rule), two heads:
