@@ -282,9 +282,9 @@ def _chunk_launch_any_head(q, k, v, g, beta, scale, initial_state, output_final_
         return _chunk_launch(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm)
     pad = torch.nn.functional.pad
     h0 = None if initial_state is None else pad(initial_state.to(torch.float32), (0, Vp - V, 0, Kp - K))
-    o, ht = _chunk_launch(pad(q, (0, Kp - K)), pad(k, (0, Kp - K)), pad(v, (0, Vp - V)), g, beta, scale, h0,
-                          output_final_state, cu_seqlens, l2norm)
-    return o[..., :V].contiguous(), None if ht is None else ht[..., :K, :V].contiguous()
+    o, ht = _chunk_launch(*_resize_heads((q, k, v), (Kp, Kp, Vp)), g, beta, scale, h0, output_final_state, cu_seqlens,
+                          l2norm)
+    return _resize_heads((o,), (V,))[0], None if ht is None else ht[..., :K, :V].contiguous()
 
 
 # Backward pass: about this many (segment, value head, 16-column slab) units, one wavefront each.
@@ -325,8 +325,24 @@ def _backward_chunk_supported(q, v) -> bool:
             and q.data_ptr() % 16 == 0)
 
 
-def _pad_last(x, n: int):
-    return x if x is None or x.shape[-1] == n else torch.nn.functional.pad(x, (0, n - x.shape[-1]))
+def _resize_heads(tensors, widths):
+    """Up to four tensors of 16-bit elements with their last dimension cut or zero-padded to the given widths, packed: in one
+    launch (``lampa_head_resize``), tensors that are already that wide as they are."""
+    out, todo = [], []
+    for x, n in zip(tensors, widths):
+        x = x.contiguous()
+        if x.shape[-1] != n:
+            src, x = x, (x.new_empty if x.numel() else x.new_zeros)((*x.shape[:-1], n))
+            if src.numel():
+                todo.append((src, x))
+        out.append(x)
+    if todo:
+        n = len(todo)
+        src, dst = ((ctypes.c_void_p * n)(*(pair[i].data_ptr() for pair in todo)) for i in (0, 1))
+        ws, wd = ((ctypes.c_int32 * n)(*(pair[i].shape[-1] for pair in todo)) for i in (0, 1))
+        rows = (ctypes.c_int64 * n)(*(a.numel() // a.shape[-1] for a, _ in todo))
+        check(_capi.lib().lampa_head_resize(n, src, ws, dst, wd, rows, stream_of(todo[0][0])), "lampa_head_resize")
+    return out
 
 
 def _pad_state(x):
@@ -407,15 +423,14 @@ def _cut_heads(grads, K: int, V: int):
     if (K, V) == (64, 64):
         return grads
     dq, dk, dv, dg, dbeta, dh0 = grads
-    return (dq[..., :K].contiguous(), dk[..., :K].contiguous(), dv[..., :V].contiguous(), dg, dbeta,
-            None if dh0 is None else dh0[..., :K, :V].contiguous())
+    return (*_resize_heads((dq, dk, dv), (K, K, V)), dg, dbeta, None if dh0 is None else dh0[..., :K, :V].contiguous())
 
 
 def _backward_chunk_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, do, dht):
     """Gradients in the chunked form from the inputs alone: the training form of the forward (its outputs dropped), then the
     backward pass over what it kept."""
     K, V = q.shape[-1], v.shape[-1]
-    q, k, v, do = (_pad_last(x, 64).contiguous() for x in (q, k, v, do))
+    q, k, v, do = _resize_heads((q, k, v, do), (64, 64, 64, 64))
     _, _, kept = _chunk_train_forward(q, k, v, g, beta, scale, initial_state, False, cu_seqlens, l2norm)
     return _cut_heads(_backward_kept_launch(q, k, v, kept, scale, l2norm, do, _pad_state(dht), initial_state is not None),
                       K, V)
@@ -481,13 +496,14 @@ class _GatedDelta(torch.autograd.Function):
             if (any(ctx.needs_input_grad) and launcher is _chunk_launch_any_head and _backward_chunk_supported(q, v)
                     and q.shape[0] * q.shape[1] > 0):
                 K, V = ctx.head
-                q, k, v = _pad_last(q, 64), _pad_last(k, 64), _pad_last(v, 64)
+                q, k, v = _resize_heads((q, k, v), (64, 64, 64))
                 o, ht, ctx.kept = _chunk_train_forward(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                                                        l2norm)
                 ctx.save_for_backward(q, k, v, initial_state, ctx.kept.buffer)
                 ctx.kept.buffer = None
                 if (K, V) != (64, 64):
-                    o, ht = o[..., :V].contiguous(), None if ht is None else ht[..., :K, :V].contiguous()
+                    o, = _resize_heads((o,), (V,))
+                    ht = None if ht is None else ht[..., :K, :V].contiguous()
                 return o, ht
             ctx.save_for_backward(q, k, v, g, beta, initial_state, cu_seqlens)
         return launcher(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm)
@@ -503,7 +519,7 @@ class _GatedDelta(torch.autograd.Function):
             q, k, v, initial_state, buffer = ctx.saved_tensors
             kept = _Kept()
             kept.plan, kept.buffer = ctx.kept.plan, buffer
-            do = torch.zeros_like(v) if do is None else _pad_last(do.to(v.dtype), 64).contiguous()
+            do = torch.zeros_like(v) if do is None else _resize_heads((do.to(v.dtype),), (64,))[0]
             grads = _cut_heads(_backward_kept_launch(q, k, v, kept, ctx.scale, ctx.l2norm, do, _pad_state(dht),
                                                      initial_state is not None), *ctx.head)
             # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them

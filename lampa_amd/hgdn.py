@@ -157,7 +157,11 @@ class _ForwardOnly(torch.autograd.Function):
     def forward(ctx, q, k, v, g, lam, beta, scale, lam_div, level_states=None, n_out=None):
         """``n_out``: tokens per sequence of the returned buffer (the caller fills those behind the whole chunks)."""
         require_cuda(q, k, v, g, lam, beta)
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        dtype, v_cols = _gd._DTYPES[q.dtype], v.shape[-1]
+        # the kernels are built for K = 64 and V in {64, 128}; smaller heads are zero-padded: zero columns of k and q add
+        # nothing to k k^T, q k^T, q S or the norms, zero columns of v give zero columns of every level state and of o, so
+        # the padded problem contains the original one exactly (`scale` is fixed from the original K by the caller)
+        q, k, v = _gd._resize_heads((q, k, v), (64, 64, 64 if v_cols <= 64 else 128))
         g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
         if lam.dtype not in _gd._DTYPES:
             lam = lam.to(torch.float32)
@@ -178,11 +182,11 @@ class _ForwardOnly(torch.autograd.Function):
         check(lib.lampa_hgdn_chunk_fwd(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(lam), _gd._DTYPES[lam.dtype],
                                        float(lam_div), ptr(o), ptr(level_states),
                                        ctypes.c_void_p(plan_host.data_ptr()), ptr(plan_dev), H, HV, K, V, L,
-                                       _gd._DTYPES[q.dtype], float(scale), _gd.L2_CHUNK, ptr(ws), ws_bytes, stream_of(q)),
+                                       dtype, float(scale), _gd.L2_CHUNK, ptr(ws), ws_bytes, stream_of(q)),
               "lampa_hgdn_chunk_fwd")
         if whole is not o and B > 1:
             whole[:, :T] = o
-        return whole
+        return _gd._resize_heads((whole,), (v_cols,))[0]
 
     @staticmethod
     def backward(ctx, *grads):
@@ -223,8 +227,7 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         _check_chunk_shapes(T, K, V, L)
         if T % 64 != 0:  # chunkwise_hgdn.py:598-601
             raise ValueError(f"T={T} and BT=64")
-        pq, pk, pv = _pad_heads(q, k, v)
-        return _ForwardOnly.apply(pq, pk, pv, g, l, beta, scale, lam_div)[..., :V].contiguous(), None
+        return _ForwardOnly.apply(q, k, v, g, l, beta, scale, lam_div), None
     if initial_state is None:  # hattention_prefill, kernel.py:467-575
         require_cuda(q, k, v, g, l, beta)
         hstate = HState(2, HType.WEAK, HStruct.GDELTA, (B, HV, K, V, L), torch.float32, q.device)
@@ -236,11 +239,10 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         if T0:
             _check_chunk_shapes(T0, K, V, L)
             cut = lambda x: x[:, :T0]
-            pq, pk, pv = _pad_heads(cut(q), cut(k), cut(v))
-            padded = pq.shape[-1] != K or pv.shape[-1] != V
-            states = (torch.zeros(B, HV, pq.shape[-1], pv.shape[-1], L, dtype=torch.float32, device=q.device)
-                      if padded else hstate.states)
-            o = _ForwardOnly.apply(pq, pk, pv, cut(g), cut(l), cut(beta), scale, lam_div, states, T)[..., :V].contiguous()
+            Vp = 64 if V <= 64 else 128
+            padded = (K, V) != (64, Vp)
+            states = torch.zeros(B, HV, 64, Vp, L, dtype=torch.float32, device=q.device) if padded else hstate.states
+            o = _ForwardOnly.apply(cut(q), cut(k), cut(v), cut(g), cut(l), cut(beta), scale, lam_div, states, T)
             if padded:  # (the padded rows and columns of the states are zero)
                 hstate.states = states[:, :, :K, :V].contiguous()
             hstate._set_counts(T0)
@@ -256,18 +258,6 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
                 beta.ndim == 3, beta.shape[1] == 1, g.ndim == 3, g.shape[1] == 1, l.ndim == 4, l.shape[1] == 1]):
         raise ValueError
     return _step(initial_state, q, k, v, g, l, beta, scale, lam_div, token_dim=True), initial_state
-
-
-def _pad_heads(q, k, v):
-    """The chunk kernels are built for K = 64 and V in {64, 128}; smaller heads are zero-padded along the head
-    dimension: zero columns of k and q add nothing to k k^T, q k^T, q S or the norms, zero columns of v give zero
-    columns of every level state and of o, so the padded problem contains the original one exactly (`scale` is fixed
-    from the original K by the caller)."""
-    K, V = q.shape[-1], v.shape[-1]
-    Kp, Vp = 64, (64 if V <= 64 else 128)
-    pad = torch.nn.functional.pad
-    return (q if K == Kp else pad(q, (0, Kp - K)), k if K == Kp else pad(k, (0, Kp - K)),
-            v if V == Vp else pad(v, (0, Vp - V)))
 
 
 def _check_chunk_shapes(T: int, K: int, V: int, L: int) -> None:

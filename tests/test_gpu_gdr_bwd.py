@@ -292,3 +292,16 @@ def test_chunked_gradients_at_full_size_against_the_token_serial_form(device, mo
     monkeypatch.setattr(gd, "CHUNKED_BACKWARD", False)
     b = _gpu_grads(device, q, k, v, g, beta, do, h0, dht, None, True)
     _check(a, [x.double().cpu() for x in b], torch.bfloat16, chunked=True)
+
+
+@pytest.mark.parametrize("rows,widths,offset", [(1, ((16, 64),), 0), (1023, ((16, 64), (64, 24), (32, 64)), 0),
+                                                (2049, ((10, 32), (6, 64), (128, 5), (64, 1)), 0),
+                                                (777, ((16, 64), (64, 16)), 1), (64, ((256, 8), (8, 256)), 0)])
+def test_resized_heads_are_padded_and_cut_copies(device, rows, widths, offset):
+    """Bit for bit what torch's pad and slice give: last blocks of rows, odd widths and odd addresses (one element per
+    thread), widths that do not divide a workgroup."""
+    src = [torch.arange(rows * w + offset, device=device).to(torch.int16).view(torch.bfloat16)[offset:].view(1, rows, w)
+           for w, _ in widths]
+    for x, y, (w, n) in zip(src, gd._resize_heads(src, [n for _, n in widths]), widths):
+        want = torch.nn.functional.pad(x.view(torch.int16), (0, n - w))  # (a negative pad cuts)
+        assert y.is_contiguous() and torch.equal(y.view(torch.int16), want)
