@@ -320,10 +320,15 @@ int lampa_gdr_bwd_saved(const void* q, const void* k, const void* v, const void*
                         void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, const int32_t* plan_host,
                         const int32_t* plan_dev, int H, int HV, int K, int V, int dtype, float scale, int l2norm,
                         void* workspace, int64_t workspace_bytes, void* stream);
-/* Heads to another width: n <= 4 packed tensors of 16-bit elements in one launch, src[i] [rows[i], src_width[i]] ->
- * dst[i] [rows[i], dst_width[i]], columns behind the source's last one zero. Widths 1 .. 256, no overlap. */
-int lampa_head_resize(int n, const void* const* src, const int32_t* src_width, void* const* dst, const int32_t* dst_width,
-                      const int64_t* rows, void* stream);
+/* Heads to another width: n <= 4 packed tensors of 16-bit elements in one launch, src [rows, src_width] ->
+ * dst [rows, dst_width], columns behind the source's last one zero. Widths 1 .. 256, no overlap. */
+typedef struct {
+  const void* src;
+  void* dst;
+  int64_t rows;
+  int32_t src_width, dst_width;
+} lampa_head_copy;
+int lampa_head_resize(int n, const lampa_head_copy* copies, void* stream);
 /* Both in one call, from the inputs alone (HV = H). plan: lampa_gdr_bwd_chunk_plan_fill's tables of the sequence boundaries
  * (cu_seqlens_host: int64 [n_seq+1]; any plan of lampa_gdr_plan_fill* will do), the same int32 array in host and in device
  * memory. workspace: lampa_gdr_bwd_chunk_workspace_bytes(plan_host, HV): about 25 KiB per (chunk, head). */

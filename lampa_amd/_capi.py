@@ -85,7 +85,7 @@ _SIGNATURES = {
     "lampa_gdr_chunk_fwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32,
                                    _f32, _i32, _vp, _i64, _vp]),
     "lampa_gdr_chunk_config": (_i32, [_i32]),
-    "lampa_head_resize": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "lampa_head_resize": (_i32, [_i32, _vp, _vp]),
     "lampa_hgdn_chunk_workspace_bytes": (_i64, [_i64, _i64, _i32, _i32, _i32]),
     "lampa_hgdn_chunk_fwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32,
                                     _i32, _i32, _f32, _i32, _vp, _i64, _vp]),
@@ -142,12 +142,17 @@ def check(code: int, what: str):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None -> NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (None -> NULL), for a c_void_p argument."""
+    return None if t is None else t.data_ptr()
+
+
+# The handle of the current stream without a ``torch.cuda.Stream`` around it, which costs 5 us (a whole call on a few tokens
+# takes 15).
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return _raw_stream(t.get_device())
 
 
 def require_cuda(*tensors):

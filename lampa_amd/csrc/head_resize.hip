@@ -43,31 +43,38 @@ __global__ void __launch_bounds__(256) head_resize_kernel(const HrArgs a) {
 
 typedef unsigned int hr_u32x4 __attribute__((ext_vector_type(4)));
 
-// n <= 4 tensors of 16-bit elements, packed: src[i] [rows[i], src_width[i]] -> dst[i] [rows[i], dst_width[i]], columns
-// beyond the source's width zero. Widths 1 .. 256; src and dst must not overlap.
-extern "C" int lampa_head_resize(int n, const void* const* src, const int32_t* src_width, void* const* dst,
-                                 const int32_t* dst_width, const int64_t* rows, void* stream) {
-  if (n < 1 || n > HR_MAX || !src || !dst || !src_width || !dst_width || !rows) return LAMPA_ERR_INVALID;
+struct lampa_head_copy {
+  const void* src;
+  void* dst;
+  int64_t rows;
+  int32_t src_width, dst_width;
+};
+
+// n <= 4 tensors of 16-bit elements, packed: src [rows, src_width] -> dst [rows, dst_width], columns beyond the source's
+// width zero. Widths 1 .. 256; src and dst must not overlap.
+extern "C" int lampa_head_resize(int n, const lampa_head_copy* copies, void* stream) {
+  if (n < 1 || n > HR_MAX || !copies) return LAMPA_ERR_INVALID;
   HrArgs a;
   int piece = 8;  // elements: 16 bytes where every row of every tensor starts on 16, else one element
   for (int i = 0; i < n; ++i) {
-    if (!src[i] || !dst[i] || rows[i] < 0) return LAMPA_ERR_INVALID;
-    if (src_width[i] < 1 || dst_width[i] < 1 || src_width[i] > 256 || dst_width[i] > 256) return LAMPA_ERR_UNSUPPORTED;
-    if (((uintptr_t)src[i] | (uintptr_t)dst[i]) & 1) return LAMPA_ERR_INVALID;
-    if ((src_width[i] | dst_width[i]) % 8 || (((uintptr_t)src[i] | (uintptr_t)dst[i]) & 15)) piece = 1;
+    const lampa_head_copy& c = copies[i];
+    if (!c.src || !c.dst || c.rows < 0) return LAMPA_ERR_INVALID;
+    if (c.src_width < 1 || c.dst_width < 1 || c.src_width > 256 || c.dst_width > 256) return LAMPA_ERR_UNSUPPORTED;
+    if (((uintptr_t)c.src | (uintptr_t)c.dst) & 1) return LAMPA_ERR_INVALID;
+    if ((c.src_width | c.dst_width) % 8 || (((uintptr_t)c.src | (uintptr_t)c.dst) & 15)) piece = 1;
   }
   int64_t blocks = 0;
   for (int i = 0; i < n; ++i) {
-    a.src[i] = src[i];
-    a.dst[i] = dst[i];
-    a.rows[i] = rows[i];
-    a.ws[i] = src_width[i] / piece;
-    a.wd[i] = dst_width[i] / piece;
-    const int64_t per_block = (int64_t)(256 / a.wd[i]) * HR_ROWS, b = (rows[i] + per_block - 1) / per_block;
+    a.src[i] = copies[i].src;
+    a.dst[i] = copies[i].dst;
+    a.rows[i] = copies[i].rows;
+    a.ws[i] = copies[i].src_width / piece;
+    a.wd[i] = copies[i].dst_width / piece;
+    const int64_t per_block = (int64_t)(256 / a.wd[i]) * HR_ROWS, b = (a.rows[i] + per_block - 1) / per_block;
     blocks = b > blocks ? b : blocks;
   }
   if (blocks == 0) return LAMPA_OK;
-  if (blocks > INT32_MAX / 256) return LAMPA_ERR_UNSUPPORTED;
+  if (blocks > INT32_MAX / 256) return LAMPA_ERR_UNSUPPORTED;  // (a grid holds fewer than 2^31 threads per dimension here)
   const dim3 grid((unsigned)blocks, n);
   if (piece == 8)
     hipLaunchKernelGGL(head_resize_kernel<hr_u32x4>, grid, dim3(256), 0, (hipStream_t)stream, a);

@@ -16,6 +16,7 @@ Differences that a caller can observe, all additive:
 """
 import ctypes
 import math
+import struct
 import warnings
 from typing import Optional
 
@@ -125,15 +126,16 @@ def _default_segmentation(chunks_per_seq, n_value_heads: int, slots: int, per_cu
 def _plan(cu_host, device, n_value_heads: int, head_dims):
     """Host + device copies of the chunk/segment tables for these sequence boundaries (cached)."""
     kind, arg = "cps", CHUNKS_PER_SEGMENT
-    if not arg:
-        cus = torch.cuda.get_device_properties(device).multi_processor_count
-        per_cu = 2 if max(head_dims) <= 64 else 1  # workgroups of the segment kernels a CU holds (LDS, registers)
-        chunks_per_seq = [(b - a + 63) // 64 for a, b in zip(cu_host[:-1], cu_host[1:])]
-        kind, arg = _default_segmentation(chunks_per_seq, n_value_heads, per_cu * cus, per_cu)
-    key = (tuple(cu_host), kind, tuple(arg) if kind == "lengths" else arg, str(device))
+    per_cu = 2 if max(head_dims) <= 64 else 1  # workgroups of the segment kernels a CU holds (LDS, registers)
+    # (everything the tables depend on: dealing out the segments of a packed call costs more than its launches)
+    key = (tuple(cu_host), device, n_value_heads, per_cu, arg, MAX_CHUNKS_PER_SEGMENT, LONG_SEGMENT_FACTOR)
     hit = _plan_cache.get(key)
     if hit is not None:
         return hit
+    if not arg:
+        cus = torch.cuda.get_device_properties(device).multi_processor_count
+        chunks_per_seq = [(b - a + 63) // 64 for a, b in zip(cu_host[:-1], cu_host[1:])]
+        kind, arg = _default_segmentation(chunks_per_seq, n_value_heads, per_cu * cus, per_cu)
     lib = _capi.lib()
     cu = (ctypes.c_int64 * len(cu_host))(*cu_host)
     n_seq = len(cu_host) - 1
@@ -325,6 +327,9 @@ def _backward_chunk_supported(q, v) -> bool:
             and q.data_ptr() % 16 == 0)
 
 
+_HEAD_COPY = struct.Struct("PPqii").pack  # lampa_head_copy
+
+
 def _resize_heads(tensors, widths):
     """Up to four tensors of 16-bit elements with their last dimension cut or zero-padded to the given widths, packed: in one
     launch (``lampa_head_resize``), tensors that are already that wide as they are."""
@@ -332,16 +337,15 @@ def _resize_heads(tensors, widths):
     for x, n in zip(tensors, widths):
         x = x.contiguous()
         if x.shape[-1] != n:
-            src, x = x, (x.new_empty if x.numel() else x.new_zeros)((*x.shape[:-1], n))
+            src, shape = x, (*x.shape[:-1], n)
             if src.numel():
-                todo.append((src, x))
+                x = torch.empty(shape, dtype=src.dtype, device=src.device)
+                todo.append(_HEAD_COPY(src.data_ptr(), x.data_ptr(), src.numel() // src.shape[-1], src.shape[-1], n))
+            else:
+                x = src.new_zeros(shape)
         out.append(x)
     if todo:
-        n = len(todo)
-        src, dst = ((ctypes.c_void_p * n)(*(pair[i].data_ptr() for pair in todo)) for i in (0, 1))
-        ws, wd = ((ctypes.c_int32 * n)(*(pair[i].shape[-1] for pair in todo)) for i in (0, 1))
-        rows = (ctypes.c_int64 * n)(*(a.numel() // a.shape[-1] for a, _ in todo))
-        check(_capi.lib().lampa_head_resize(n, src, ws, dst, wd, rows, stream_of(todo[0][0])), "lampa_head_resize")
+        check(_capi.lib().lampa_head_resize(len(todo), b"".join(todo), stream_of(out[0])), "lampa_head_resize")
     return out
 
 

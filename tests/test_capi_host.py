@@ -3,6 +3,7 @@ and its host-only planning logic is right. No kernel is launched here."""
 import ctypes
 import os
 import re
+import struct
 
 import pytest
 import torch
@@ -240,13 +241,10 @@ def test_hierarchical_forward_argument_checks(lib):
 
 def test_head_resize_refuses_what_it_cannot_copy(lib):
     def call(src_width, dst_width, rows=8, n=1, address=1 << 20):
-        arr = lambda t, x: (t * max(n, 1))(*([x] * max(n, 1)))
-        return lib.lampa_head_resize(n, arr(ctypes.c_void_p, address), arr(ctypes.c_int32, src_width),
-                                     arr(ctypes.c_void_p, 1 << 21), arr(ctypes.c_int32, dst_width),
-                                     arr(ctypes.c_int64, rows), None)
+        return lib.lampa_head_resize(n, 5 * struct.pack("PPqii", address, 1 << 21, rows, src_width, dst_width), None)
 
     assert call(16, 64, n=0) == -1 and call(16, 64, n=5) == -1 and call(16, 64, rows=-1) == -1
-    assert call(16, 64, address=None) == -1 and call(16, 64, address=(1 << 20) + 1) == -1
+    assert call(16, 64, address=0) == -1 and call(16, 64, address=(1 << 20) + 1) == -1
     assert call(0, 64) == -4 and call(16, 257) == -4 and call(257, 64) == -4
     assert call(16, 64, rows=0) == 0
     assert call(16, 256, rows=1 << 40) == -4  # more rows than a launch has workgroups for
