@@ -671,12 +671,21 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
 
   // long segments first (see the plan). Grid (segments, heads), or one row of segments x heads workgroups in which the
   // heads of a segment are neighbours, so that the order holds over all heads
-  const int seg = pv.seg_order[gridDim.y > 1 ? blockIdx.x : blockIdx.x / HV];
-  const int hv = gridDim.y > 1 ? blockIdx.y : blockIdx.x % HV;
+  // (hierarchical form, gmax > 0: grid (segments x gmax, heads), workgroup = one of the gmax equal pieces of a segment)
+  constexpr bool PIECES = !PASS_B && !SCALED_K;
+  const int bx = PIECES && gmax > 0 ? (int)blockIdx.x / gmax : (int)blockIdx.x;
+  const int seg = pv.seg_order[gridDim.y > 1 ? bx : bx / HV];
+  const int hv = gridDim.y > 1 ? blockIdx.y : bx % HV;
   const int h = hv / (HV / H);
   const int flags = pv.seg_flags[seg];
   if (!PASS_B && !KEEP && (flags & SEG_LAST)) return;  // nothing follows the last segment of a sequence
-  const int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg];
+  int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg], map = seg;  // map: where the composite goes
+  if (PIECES && gmax > 0) {
+    const int piece = (int)blockIdx.x % gmax;
+    nc /= gmax;
+    c0 += piece * nc;
+    map = seg * gmax + piece;
+  }
   const int c1 = c0 + nc;
   // (the per-chunk tables are separate restrict parameters: read through the view they could alias the kernel's
   // stores, would be fetched with vector loads and would sit in the same queue as the stagers' prefetches)
@@ -1774,7 +1783,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   } else if (is_m) {
     // M = dtot I + M': M' as bf16 A-operand fragments (rows = state rows, contraction over the columns in
     // accumulator slot order), element (row, col) -> fragment (row/32, col/16), lane 32*hh' + row%32, slot s
-    unsigned char* out = Mcomp + ((size_t)seg * HV + hv) * (KT * KT * 2) + late;
+    unsigned char* out = Mcomp + ((size_t)map * HV + hv) * (KT * KT * 2) + late;
     const int mcol = 32 * wave + ln, ks = mcol >> 4, c16 = mcol & 15;
     const int hs = (c16 >> 2) & 1, slot = 4 * (c16 >> 3) + (c16 & 3);
 #pragma unroll
@@ -1786,7 +1795,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         *reinterpret_cast<OT*>(out + ((size_t)((km * (KT / 16) + ks) * 64 + 32 * hs + (row & 31))) * 16 + 2 * slot) =
             (OT)val;
       }
-    if (wave == 0 && lane == 0) Dcomp[(size_t)seg * HV + hv] = dtot;
+    if (wave == 0 && lane == 0) Dcomp[(size_t)map * HV + hv] = dtot;
     if constexpr (KEEP) {  // accumulator tiles read as A operand are the transpose
       unsigned char* mt = keep + ((size_t)seg * HV + hv) * (KT * KT * 2);
 #pragma unroll
@@ -1800,7 +1809,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
     }
   } else {
     // N slab in accumulator order: tile (vslab, km), plane q (registers 4q..4q+3), lane -> 16 bytes
-    unsigned char* out = Ncomp + (((size_t)seg * HV + hv) * (VT / 32) + vslab) * (KT * 32 * 4) + late;
+    unsigned char* out = Ncomp + (((size_t)map * HV + hv) * (VT / 32) + vslab) * (KT * 32 * 4) + late;
 #pragma unroll
     for (int km = 0; km < KT / 32; ++km)
 #pragma unroll
@@ -1928,7 +1937,9 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan_kernel(const GdrPlanV
 //          cost a launch more), then its own segments, writing the state every segment starts from (what the
 //          single-level scan writes).
 // Same step code in both modes; loops are branch free with clamped operands and a spare store slot as above.
-enum { SCAN_GROUP = 1, SCAN_LEAF = 2 };
+//   PIECES as GROUP, the groups being the segments that the composite pass cut into G pieces: every segment but the last
+//          of a sequence gets its composite, at the segment's own index.
+enum { SCAN_GROUP = 1, SCAN_LEAF = 2, SCAN_PIECES = 3 };
 
 // REV (GROUP): the segments of a sequence are taken from the last to the first (the maps of the backward pass).
 template <typename OT, int KT, int VT, int DEPTH, int MODE, bool REV = false>
@@ -1942,30 +1953,31 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
                                                                   int HV, int spare_slot, int gmax) {
   using X8 = typename OpVec<OT>::x8;
   constexpr int G = GDR_SCAN_GROUP;
+  constexpr bool COMPOSE = MODE != SCAN_LEAF;
   static_assert(G % DEPTH == 0, "a group must be a whole number of ring rounds");
   constexpr int NKS = KT / 16;
   constexpr int M_BYTES = KT * KT * 2, N_BYTES = KT * 32 * 4;
-  constexpr int NCB = MODE == SCAN_GROUP ? (KT + VT) / 32 : VT / 32;  // 32-column blocks per item of the grid
+  constexpr int NCB = COMPOSE ? (KT + VT) / 32 : VT / 32;  // 32-column blocks per item of the grid
   __shared__ __align__(16) unsigned char s_x[2][NKS * 1024];
   const int vn = blockIdx.x % NCB, j = blockIdx.x / NCB, seq = blockIdx.y, hv = blockIdx.z;
   const int seg0 = pv.seq_seg0[seq], nseg = pv.seq_nseg[seq];
-  const int ngroups = (nseg + G - 1) / G;
+  const int ngroups = MODE == SCAN_PIECES ? nseg : (nseg + G - 1) / G;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
   // items = the maps this workgroup applies, slots = where it stores the running state before each of them
   int item0, nsteps, slot0, lead = 0;  // lead: group-level maps walked before the workgroup's own items (LEAF)
-  if (MODE == SCAN_GROUP) {
+  if (COMPOSE) {
     if (j >= ngroups - 1) return;  // the composite of a sequence's last group is never needed
-    item0 = REV ? seg0 + nseg - 1 - j * G : seg0 + j * G; nsteps = G - 1; slot0 = 0;
+    item0 = MODE == SCAN_PIECES ? (seg0 + j) * G : REV ? seg0 + nseg - 1 - j * G : seg0 + j * G; nsteps = G - 1; slot0 = 0;
   } else {
     if (j >= ngroups) return;
     item0 = seg0 + j * G; lead = j; nsteps = lead + min(G, nseg - j * G) - 1; slot0 = item0;
   }
-  const int last = MODE == SCAN_GROUP ? nsteps : nsteps - 1;   // last map that is really applied (prefetches are clamped to it)
-  const bool is_pm = MODE == SCAN_GROUP && vn < KT / 32;       // a block of P_M: no additive term, starts from I
-  const int nblk = MODE == SCAN_GROUP ? max(vn - KT / 32, 0) : vn;  // 32-column block of N / of the state
+  const int last = COMPOSE ? nsteps : nsteps - 1;   // last map that is really applied (prefetches are clamped to it)
+  const bool is_pm = COMPOSE && vn < KT / 32;       // a block of P_M: no additive term, starts from I
+  const int nblk = COMPOSE ? max(vn - KT / 32, 0) : vn;  // 32-column block of N / of the state
 
   f32x16 S = zero16();
-  if (MODE == SCAN_GROUP) {
+  if (COMPOSE) {
     if (is_pm) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) S[r] = (32 * wave + acc_row(r, hh) == 32 * vn + ln) ? 1.0f : 0.0f;
@@ -1995,7 +2007,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
 
   float dprod = 1.0f;
   auto step = [&](int p, X8* m, f32x4* n, float& dd) {
-    if (MODE != SCAN_GROUP) {
+    if (!COMPOSE) {
       const size_t slot = (p >= lead && p <= nsteps) ? (size_t)(slot0 + (p - lead)) : (size_t)spare_slot;
       f32x4* si = reinterpret_cast<f32x4*>(dst + ((slot * HV + hv) * (VT / 32) + vn) * (KT * 32));
 #pragma unroll
@@ -2027,7 +2039,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
   };
   constexpr int LONG = 4 * DEPTH;
   int p0 = 0;
-  if (MODE != SCAN_GROUP) {
+  if (!COMPOSE) {
     for (; p0 + LONG <= nsteps + 1; p0 += LONG) {
 #pragma unroll
       for (int u = 0; u < LONG; ++u) step(p0 + u, rm[u % DEPTH], rn[u % DEPTH], rd[u % DEPTH]);
@@ -2038,8 +2050,8 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
     for (int d = 0; d < DEPTH; ++d) step(p0 + d, rm[d], rn[d], rd[d]);
   }
 
-  if (MODE == SCAN_GROUP) {  // exactly G maps were applied (G is a multiple of DEPTH): store the composite
-    const size_t gh = (size_t)(seq * gmax + j) * HV + hv;
+  if (COMPOSE) {  // exactly G maps were applied (G is a multiple of DEPTH): store the composite
+    const size_t gh = (size_t)(MODE == SCAN_PIECES ? seg0 + j : seq * gmax + j) * HV + hv;
     if (is_pm) {
       unsigned char* out = Mout + gh * M_BYTES;
       const int mcol = 32 * vn + ln, ks = mcol >> 4, c16 = mcol & 15;

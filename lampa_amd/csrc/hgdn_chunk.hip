@@ -839,8 +839,20 @@ __global__ void __launch_bounds__(64 * HG_CW)
 
 // ---- host side ------------------------------------------------------------------------------------------------
 struct HgWorkspace {
-  int64_t off_t, off_m, off_n, off_d, off_rec, off_nc, off_oi, off_x, bytes;
+  int64_t off_t, off_m, off_n, off_d, off_rec, off_nc, off_oi, off_x, off_pm, off_pn, off_pd, bytes;
 };
+
+// Segment composites: one workgroup per (segment, head) walks its chunks one after the other, 3.4 us each, and the plan's
+// segments are as long as the walk needs them (one round of its workgroups), so with few long ones the composites take
+// longer than the prep kernel beside them: 220 + 17 us (scan) against 148 us at 60 032 tokens x 8 heads of 64 x 64 (15
+// segments of 64 chunks, 120 workgroups). While there are at most HG_PIECES_MAX_WGS workgroups (one per CU), segments of 64
+// and more chunks are cut into GDR_SCAN_GROUP pieces whose maps one more launch composes: the pieces take 59 us in front of
+// the prep kernel and the rest hides beside it. The call: 432 -> 411 us, with 128 value columns 792 -> 630 us, 40 000 x 6 x
+// 64 x 128 422 -> 347 us. Segments of 32 chunks take the same time either way (30 016 x 8: 240 / 240 us, 60 032 x 4: 259 /
+// 261 us), those of 16 are faster whole (15 000 x 8: 208 against 220 us).
+#define HG_PIECES_MAX_WGS 256
+#define HG_PIECES_MIN_LOG2 6
+static bool hg_pieces(int64_t segs, int HV, int p) { return p >= HG_PIECES_MIN_LOG2 && segs * HV <= HG_PIECES_MAX_WGS; }
 
 static HgWorkspace hg_workspace(int64_t chunks, int64_t segs, int HV, int K, int V) {
   HgWorkspace w;
@@ -854,6 +866,12 @@ static HgWorkspace hg_workspace(int64_t chunks, int64_t segs, int HV, int K, int
   w.off_nc = off;  off += lampa_align_up(chunks * HV * (int64_t)(V / 32) * 4096, 256);  // dk . U fragments
   w.off_oi = off;  off += lampa_align_up(chunks * HV * (int64_t)64 * V * 4, 256);
   w.off_x = off;   off += lampa_align_up(segs * HG_NLV * HV * (int64_t)K * V * 4, 256);
+  // the maps of the pieces (hg_pieces; fewer chunks make no two segments that long)
+  const int64_t pieces =
+      chunks > (1 << HG_PIECES_MIN_LOG2) && hg_pieces(segs, HV, HG_PIECES_MIN_LOG2) ? segs * GDR_SCAN_GROUP : 0;
+  w.off_pm = off;  off += lampa_align_up(pieces * HV * (int64_t)K * K * 2, 256);
+  w.off_pn = off;  off += lampa_align_up(pieces * HV * (int64_t)K * V * 4, 256);
+  w.off_pd = off;  off += lampa_align_up(pieces * HV * 4, 256);
   w.bytes = off > 0 ? off : 256;
   return w;
 }
@@ -868,7 +886,7 @@ extern "C" int64_t lampa_hgdn_chunk_workspace_bytes(int64_t total_chunks, int64_
 
 template <typename T, int KT, int VT>
 static int hg_launch(const void* q, const void* k, const void* v, const float* g, const float* beta, const void* lam,
-                     int lam_dtype, float lam_div, void* o, float* hstates, int chunks_per_seq, const GdrPlanView pv, int n_seq, int chunks, int segs, int p, int H, int HV, int L,
+                     int lam_dtype, float lam_div, void* o, float* hstates, int chunks_per_seq, const GdrPlanView pv, int n_seq, int chunks, int segs, int max_nseg, int p, int H, int HV, int L,
                      float scale, int l2norm, unsigned char* ws, hipStream_t s) {
   const HgWorkspace w = hg_workspace(chunks, segs, HV, KT, VT);
   unsigned char* tf = ws + w.off_t;
@@ -902,10 +920,11 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
                      beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, (int32_t*)nullptr);
   LAMPA_PROF(s, "gdr_local_kernel");
   const bool split = segs > n_seq;
-  // The segment composites and their scan depend on T only, like the prep kernel, and are latency bound on a few
-  // workgroups: they run on a second stream (default priority) beside the prep kernel (launched first, which
-  // measured slightly better than the other order) and join before the walk.
+  // The composites of pieces fill the chip and run in front of the prep kernel. What follows them, and the composites of
+  // whole segments, need T only, like the prep kernel, and are latency bound on a few workgroups: they run on a second
+  // stream (default priority) beside the prep kernel and join before the walk.
   // With a profile recording open everything stays on the caller's stream, so that the intervals mean one kernel each.
+  const int pieces = split && hg_pieces(segs, HV, p) ? GDR_SCAN_GROUP : 0;
   bool overlap = split && !lampa_prof_recording();
   std::unique_lock<std::mutex> hold(hg_side_lock, std::defer_lock);
   HgSide* sd = nullptr;
@@ -917,21 +936,36 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   hipStream_t side = sd ? sd->side : s;
   hipEvent_t ev_fork = sd ? sd->fork : nullptr, ev_join = sd ? sd->join : nullptr;
   hipStream_t cs = s;  // the stream of the composites
-  if (overlap) {
-    if (hipEventRecord(ev_fork, s) != hipSuccess || hipStreamWaitEvent(side, ev_fork, 0) != hipSuccess) return LAMPA_ERR_LAUNCH;
+  auto fork = [&]() {
+    if (!overlap) return true;
     cs = side;
-  }
+    return hipEventRecord(ev_fork, s) == hipSuccess && hipStreamWaitEvent(side, ev_fork, 0) == hipSuccess;
+  };
+  auto composites = [&]() {
+    // (only a sequence's last segment can be shorter than 2^p chunks, and its composite is not needed)
+    hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, false, __bf16>), dim3(pieces ? segs * pieces : segs, HV),
+                       dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, cs, (const T*)q, (const T*)k, (const T*)v, g,
+                       beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, pieces ? ws + w.off_pm : Mc,
+                       pieces ? ws + w.off_pn : Nm, pieces ? (float*)(ws + w.off_pd) : Dc, (T*)nullptr, (float*)nullptr, H, HV,
+                       scale, l2norm, (const unsigned char*)nullptr, (const unsigned char*)nullptr, (const float*)nullptr,
+                       (const float*)nullptr, pieces, (unsigned char*)nullptr);
+    LAMPA_PROF(s, "gdr_segment_kernel<composite>");
+  };
+  if (pieces) composites();
+  if (!fork()) return LAMPA_ERR_LAUNCH;
   hipLaunchKernelGGL((hgdn_prep_kernel<T, KT, VT>), dim3(chunks, HV), dim3(256), smem_p, s, (const T*)q, (const T*)k,
                      (const T*)v, lam, lam_dtype, lam_div, pv.chunk_tok0, pv.chunk_len, tf, rec, Ubw, Oi, hstates, chunks_per_seq, H, HV, L,
                      scale, l2norm);
   LAMPA_PROF(s, "hgdn_prep_kernel");
   if (split) {
-    hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, false, __bf16>), dim3(segs, HV),
-                       dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, cs, (const T*)q, (const T*)k, (const T*)v, g,
-                       beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, Mc, Nm, Dc, (T*)nullptr,
-                       (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
-                       (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, (unsigned char*)nullptr);
-    LAMPA_PROF(s, "gdr_segment_kernel<composite>");
+    if (pieces) {
+      hipLaunchKernelGGL((gdr_scan2_kernel<__bf16, KT, VT, 4, SCAN_PIECES>), dim3((KT + VT) / 32 * max_nseg, n_seq, HV),
+                         dim3(64 * (KT / 32)), 0, cs, pv, ws + w.off_pm, ws + w.off_pn, (const float*)(ws + w.off_pd),
+                         (const float*)nullptr, (float*)nullptr, Mc, Nm, Dc, HV, 0, 0);
+      LAMPA_PROF(s, "gdr_scan2_kernel<pieces>");
+    } else {
+      composites();
+    }
     hipLaunchKernelGGL((hgdn_scan_kernel<KT, VT>), dim3(VT / 32, n_seq, HV), dim3(64 * HG_CW), 0, cs, pv, Mc, Nm, Dc, Xi,
                        HV, p);
     LAMPA_PROF(s, "hgdn_scan_kernel");
@@ -975,12 +1009,13 @@ extern "C" int lampa_hgdn_chunk_fwd(const void* q, const void* k, const void* v,
     if (cps & (cps - 1)) return LAMPA_ERR_INVALID;
     while ((1 << p) < cps) ++p;
   }
-  int max_nc = 0;
+  int max_nc = 0, max_nseg = 0;
   for (int i = 0; i < n_seq; ++i) {
     const int s0 = plan_host[plan_host[PLAN_OFF_SEQ_SEG0] + i], ns = plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i];
     int nc = 0;
     for (int j = 0; j < ns; ++j) nc += plan_host[plan_host[PLAN_OFF_SEG_NCHUNKS] + s0 + j];
     max_nc = nc > max_nc ? nc : max_nc;
+    max_nseg = ns > max_nseg ? ns : max_nseg;
   }
   if (max_nc > (1 << HG_NLV)) return LAMPA_ERR_UNSUPPORTED;
   // whole chunks only, as the reference demands (chunkwise_hgdn.py:598-601)
@@ -996,7 +1031,7 @@ extern "C" int lampa_hgdn_chunk_fwd(const void* q, const void* k, const void* v,
   unsigned char* ws = (unsigned char*)workspace;
   const GdrPlanView pv = gdr_plan_view(plan_host, plan_dev);
 #define HG_CASE(TT, KK, VV) \
-  return hg_launch<TT, KK, VV>(q, k, v, g, beta, lam, lam_dtype, lam_div, o, level_states, max_nc, pv, n_seq, chunks, segs, p, H, HV, L, scale, l2norm, ws, s)
+  return hg_launch<TT, KK, VV>(q, k, v, g, beta, lam, lam_dtype, lam_div, o, level_states, max_nc, pv, n_seq, chunks, segs, max_nseg, p, H, HV, L, scale, l2norm, ws, s)
   if (dtype == GDR_BF16) {
     if (V == 64) HG_CASE(__bf16, 64, 64);
     if (V == 128) HG_CASE(__bf16, 64, 128);

@@ -60,6 +60,19 @@ def test_matches_oracle(device, T, cps):
     assert max_abs <= MAX_ABS and mean_rel <= MEAN_REL, f"T={T} cps={cps}: {max_abs:.3e} {mean_rel:.3e}"
 
 
+@pytest.mark.parametrize("B,chunks,HV,V,cps,dtype", [(3, 65, 2, 64, 64, torch.bfloat16), (1, 134, 4, 64, 64, torch.float16),
+                                                     (2, 129, 1, 128, 128, torch.bfloat16), (2, 65, 65, 64, 64, torch.bfloat16)])
+@pytest.mark.parametrize("g_scale", [1.0, 0.01])
+def test_segments_composed_from_pieces(device, B, chunks, HV, V, cps, dtype, g_scale):
+    """Segments of 64 and 128 chunks whose composites come from eight pieces each, behind short last segments (1, 6 and 1
+    chunks); 4 segments x 65 heads are more workgroups than CUs and keep the walk over the whole segment. The weak decay
+    carries the states over every segment."""
+    q, k, v, g, beta, lam = _inputs(B, 64 * chunks, 1, 64, V, dtype, seed=chunks, HV=HV, g_scale=g_scale)
+    o = _run(device, q, k, v, g, beta, lam, cps)
+    max_abs, mean_rel = _errors(o, _want(q, k, v, g, beta, lam))
+    assert max_abs <= MAX_ABS and mean_rel <= MEAN_REL, f"{max_abs:.3e} {mean_rel:.3e}"
+
+
 def test_batch_grouped_heads_wide_values_fp16(device):
     q, k, v, g, beta, lam = _inputs(2, 1536, 2, 64, 128, torch.float16, seed=5, HV=4, g_scale=0.3, L=14)
     for cps in (None, 8):
