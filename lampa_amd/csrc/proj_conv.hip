@@ -9,12 +9,21 @@
 //   plain columns: y[t, n] = pre[t, n]
 // The projection output never goes to HBM: x is read once (K = 128 columns), the outputs are written once.
 //
-// One workgroup = 4 waves = 256 output columns x a run of consecutive tokens. A wave keeps its 64 columns of W in
-// registers for the whole run (2 column tiles x K/16 B-operand fragments), walks the run in tiles of 32 tokens
-// (A operand = 32 rows of x straight from HBM, next tile prefetched), and turns each accumulator tile into outputs
-// through a private LDS tile that also holds the last 3 pre-activation rows of the previous tile, so the convolution
-// needs no recomputation except one extra tile at the start of a run that does not begin a sequence.
+// A workgroup is four waves of 64 output columns (256 of a job's columns x a run of consecutive tokens). A wave keeps its
+// columns of W in registers for the whole run (2 column tiles x K/16 operand fragments) and walks it in tiles of 32
+// tokens (32 rows of x straight from HBM, next tile prefetched). The product is computed transposed, W x^T: a lane then
+// holds one token and four neighbouring columns per quarter of its accumulators, so a tile goes to a private LDS tile as
+// 8-byte pieces (8 writes instead of 32 of 2 bytes, and packed conversions); below the last 3 pre-activation rows of the
+// previous tile it is turned into outputs, so the convolution needs no recomputation except one extra tile at the start of
+// a run that does not begin a sequence.
+//
+// Bound by VALU issue in the convolution's epilogue (4 fma and a SiLU with a quarter-rate exp2 and rcp per output), which the
+// plain columns do not have, at two workgroups per CU (256 registers). On a long input every workgroup therefore takes a
+// run of convolution columns, then a shorter run of plain columns and a tile of the few columns behind them: with workgroups
+// of one kind each the CUs that held two of the convolution worked on while the others were done.
+// 60 000 tokens, 2064 columns of which 1536 with the convolution: 107.5 -> 101.8 us.
 #include "gdr_common.h"
+#include <atomic>
 
 #define PC_K 128            // contraction length (hidden size) this kernel is built for
 #define PC_NKS (PC_K / 16)
@@ -30,100 +39,114 @@ struct PcBlock {   // one block of 256 consecutive rows of W
   __bf16* out;     // output tensor of the block's columns
   int out_stride;  // its row stride in elements
   int out_col0;    // column of `out` that the block's first column maps to
-  int n_valid;     // columns of the block that exist (the last block of W may be short)
-  int conv;        // 1: convolution + SiLU, 0: plain projection output
-  int conv_col0;   // row of the convolution weights of the block's first column
+};
+// The workgroups wg0 .. wg0 + n_wgs - 1 do the runs of a kind's blocks: workgroup wg0 + i block i % n_blocks, run i / n_blocks
+struct PcJobs {
+  int wg0, n_wgs, n_blocks, tokens;  // tokens per run
 };
 struct PcPlan {
-  PcBlock blocks[PC_MAX_BLOCKS];
+  PcBlock blocks[PC_MAX_BLOCKS];  // convolution blocks, then plain blocks
+  PcJobs conv, plain, tail;       // tail: the last columns of W (fewer than a wave's 64); a wave takes one tile at a time
+  __bf16* tail_out;
+  int tail_cols;
 };
 
 __device__ __forceinline__ float pc_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
-__global__ void __launch_bounds__(256) pc_proj_conv_kernel(const __bf16* __restrict__ x, int64_t x_stride, int64_t n_tokens,
-                                                          int64_t t_len, const __bf16* __restrict__ W,
-                                                          const float* __restrict__ conv_w, const float* __restrict__ conv_b,
-                                                          const PcPlan plan, int tokens_per_wg) {
-  __shared__ __align__(16) __bf16 s_y[4][(PC_ROWS + PC_W - 1) * PC_LD];
-  const PcBlock blk = plan.blocks[blockIdx.y];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, hh = lane >> 5, ln = lane & 31;
-  const int wcol = PC_COLS_WAVE * wave;  // first column of this wave inside the block
-  if (wcol >= blk.n_valid) return;       // no workgroup-wide barrier below: a wave may leave alone
-  const int64_t T0 = (int64_t)blockIdx.x * tokens_per_wg;
-  const int64_t T1 = T0 + tokens_per_wg < n_tokens ? T0 + tokens_per_wg : n_tokens;
-  __bf16* sy = s_y[wave];
-
-  // this wave's 64 rows of W as B-operand fragments (rows beyond the end of a short block read as zero)
-  bf16x8 bfrag[2][PC_NKS];
+// 64 rows of W, w0 .. (the first n_valid of them; zero beyond), as operand fragments
+__device__ __forceinline__ void pc_load_w(const __bf16* __restrict__ W, int64_t w0, int n_valid, int lane,
+                                          bf16x8 (*wf)[PC_NKS]) {
+  const int hh = lane >> 5, ln = lane & 31;
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct) {
-    const int c = wcol + 32 * ct + ln;
-    const bool ok = c < blk.n_valid;
-    const __bf16* wp = W + ((int64_t)blockIdx.y * PC_COLS_WG + (ok ? c : 0)) * PC_K + 8 * hh;
+    const int c = 32 * ct + ln;
+    const bool ok = c < n_valid;
+    const __bf16* wp = W + (w0 + (ok ? c : 0)) * PC_K + 8 * hh;
 #pragma unroll
     for (int ks = 0; ks < PC_NKS; ++ks) {
-      bfrag[ct][ks] = *reinterpret_cast<const bf16x8*>(wp + 16 * ks);
+      wf[ct][ks] = *reinterpret_cast<const bf16x8*>(wp + 16 * ks);
       if (!ok) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) bfrag[ct][ks][e] = (__bf16)0.0f;
+        for (int e = 0; e < 8; ++e) wf[ct][ks][e] = (__bf16)0.0f;
       }
     }
   }
-  // output role of the lane: 8 consecutive columns (cg) of the 4 consecutive token rows 4 tq .. 4 tq + 3 of a tile
-  const int cg = lane & 7, tq = lane >> 3;
-  float cw[PC_W][8], cb[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const int col = wcol + 8 * cg + c;
-    const bool ok = blk.conv && col < blk.n_valid;
-    cb[c] = (ok && conv_b) ? conv_b[blk.conv_col0 + col] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < PC_W; ++j)
-      cw[j][c] = ok ? conv_w[(int64_t)(blk.conv_col0 + col) * PC_W + j] : 0.0f;
-  }
+}
 
-  auto load_a = [&](int64_t t0, bf16x8* a) {
-    int64_t row = t0 + ln;
-    row = row < 0 ? 0 : (row >= n_tokens ? n_tokens - 1 : row);
-    const __bf16* xp = x + row * x_stride + 8 * hh;
+// 32 rows of x from t0 on (clamped to the tensor)
+__device__ __forceinline__ void pc_load_x(const __bf16* __restrict__ x, int64_t x_stride, int64_t n_tokens, int64_t t0, int lane,
+                                          bf16x8* a) {
+  int64_t row = t0 + (lane & 31);
+  row = row < 0 ? 0 : (row >= n_tokens ? n_tokens - 1 : row);
+  const __bf16* xp = x + row * x_stride + 8 * (lane >> 5);
 #pragma unroll
-    for (int ks = 0; ks < PC_NKS; ++ks) a[ks] = *reinterpret_cast<const bf16x8*>(xp + 16 * ks);
-  };
+  for (int ks = 0; ks < PC_NKS; ++ks) a[ks] = *reinterpret_cast<const bf16x8*>(xp + 16 * ks);
+}
 
-  // a run that starts inside a sequence first computes the tile before it, only for its last rows of history
-  const bool need_history = blk.conv && (T0 % t_len) != 0;
-  int64_t t0 = need_history ? T0 - PC_ROWS : T0;
-  if (!need_history) {
-    for (int i = lane; i < (PC_W - 1) * PC_LD; i += 64) sy[i] = (__bf16)0.0f;
-  }
-  // token position inside the sequence, kept per tile in 32 bits (a 64-bit modulo per output row would cost more than
-  // the convolution); sequences shorter than two tiles take the general modulo
-  const int tl32 = (int)(t_len < INT32_MAX ? t_len : INT32_MAX);
-  const bool small_seq = t_len < 2 * PC_ROWS;
-  int ts0 = (int)((t0 % t_len + t_len) % t_len);
-  bf16x8 afrag[PC_NKS], anext[PC_NKS];
-  load_a(t0, afrag);
-  for (; t0 < T1; t0 += PC_ROWS, ts0 = small_seq ? (ts0 + PC_ROWS) % tl32 : (ts0 + PC_ROWS >= tl32 ? ts0 + PC_ROWS - tl32 : ts0 + PC_ROWS)) {
-    load_a(t0 + PC_ROWS, anext);
-    f32x16 acc[2];
+// pre-activations of a tile, rounded to bf16, below the rows of history
+__device__ __forceinline__ void pc_tile(const bf16x8 (*wf)[PC_NKS], const bf16x8* xf, int lane, __bf16* sy) {
+  const int hh = lane >> 5, ln = lane & 31;
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
+  for (int ct = 0; ct < 2; ++ct) {
+    f32x16 acc;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[ct][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
 #pragma unroll
-      for (int ks = 0; ks < PC_NKS; ++ks) acc[ct] = mfma32(afrag[ks], bfrag[ct][ks], acc[ct]);
+    for (int ks = 0; ks < PC_NKS; ++ks) acc = mfma32(wf[ct][ks], xf[ks], acc);
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      bf16x4 p;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[e] = (__bf16)acc[4 * q4 + e];
+      *reinterpret_cast<bf16x4*>(&sy[(PC_W - 1 + ln) * PC_LD + 32 * ct + 8 * q4 + 4 * hh]) = p;
     }
-    // pre-activations of the tile, rounded to bf16, below the 3 rows of history
+  }
+}
+
+__global__ void __launch_bounds__(256, 2) pc_proj_conv_kernel(const __bf16* __restrict__ x, int64_t x_stride, int64_t n_tokens,
+                                                          int64_t t_len, const __bf16* __restrict__ W,
+                                                          const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+                                                          const PcPlan plan) {
+  __shared__ __align__(16) __bf16 s_y[4][(PC_ROWS + PC_W - 1) * PC_LD];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wcol = PC_COLS_WAVE * wave;  // first column of this wave inside a block
+  // (no workgroup-wide barrier below: a wave uses nothing but its own LDS tile)
+  __bf16* sy = s_y[wave];
+  // output role of the lane: 8 consecutive columns (cg) of the 4 consecutive token rows 4 tq .. 4 tq + 3 of a tile
+  const int cg = lane & 7, tq = lane >> 3, col = wcol + 8 * cg;
+  bf16x8 wf[2][PC_NKS], xf[PC_NKS], xnext[PC_NKS];
+
+  int job = (int)blockIdx.x - plan.conv.wg0;
+  if (job >= 0 && job < plan.conv.n_wgs) {
+    const int b = job % plan.conv.n_blocks;
+    const PcBlock blk = plan.blocks[b];
+    const int64_t T0 = (int64_t)(job / plan.conv.n_blocks) * plan.conv.tokens;
+    const int64_t T1 = T0 + plan.conv.tokens < n_tokens ? T0 + plan.conv.tokens : n_tokens;
+    pc_load_w(W, (int64_t)b * PC_COLS_WG + wcol, PC_COLS_WAVE, lane, wf);
+    float cw[PC_W][8], cb[8];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int c = 0; c < 8; ++c) {
+      cb[c] = conv_b ? conv_b[b * PC_COLS_WG + col + c] : 0.0f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        sy[(PC_W - 1 + 8 * (r / 4) + 4 * hh + (r % 4)) * PC_LD + 32 * ct + ln] = (__bf16)acc[ct][r];
-    lds_fence();
-    if (t0 >= T0) {
-      const int col = wcol + 8 * cg;
-      const bool store_cols = col < blk.n_valid;
-      if (blk.conv) {
+      for (int j = 0; j < PC_W; ++j) cw[j][c] = conv_w[(int64_t)(b * PC_COLS_WG + col + c) * PC_W + j];
+    }
+    // a run that starts inside a sequence first computes the tile before it, only for its last rows of history
+    const bool need_history = (T0 % t_len) != 0;
+    int64_t t0 = need_history ? T0 - PC_ROWS : T0;
+    if (!need_history) {
+      for (int i = lane; i < (PC_W - 1) * PC_LD; i += 64) sy[i] = (__bf16)0.0f;
+    }
+    // token position inside the sequence, kept per tile in 32 bits (a 64-bit modulo per output row would cost more than
+    // the convolution); sequences shorter than two tiles take the general modulo
+    const int tl32 = (int)(t_len < INT32_MAX ? t_len : INT32_MAX);
+    const bool small_seq = t_len < 2 * PC_ROWS;
+    int ts0 = (int)((t0 % t_len + t_len) % t_len);
+    pc_load_x(x, x_stride, n_tokens, t0, lane, xf);
+    for (; t0 < T1; t0 += PC_ROWS, ts0 = small_seq ? (ts0 + PC_ROWS) % tl32 : (ts0 + PC_ROWS >= tl32 ? ts0 + PC_ROWS - tl32 : ts0 + PC_ROWS)) {
+      pc_load_x(x, x_stride, n_tokens, t0 + PC_ROWS, lane, xnext);
+      pc_tile(wf, xf, lane, sy);
+      lds_fence();
+      if (t0 >= T0) {
         // the lane's 4 consecutive tokens share their taps: 7 rows of pre-activations for 4 outputs
         float pre[PC_ROWS_LANE + PC_W - 1][8];
 #pragma unroll
@@ -160,28 +183,67 @@ __global__ void __launch_bounds__(256) pc_proj_conv_kernel(const __bf16* __restr
 #pragma unroll
           for (int c = 0; c < 8; ++c) o[c] = (__bf16)(y[c] * pc_sigmoid(y[c]));
           const int64_t t = t0 + tr;
-          if (t < T1 && store_cols) *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
+          if (t < T1) *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
         }
-      } else {
+      }
+      lds_fence();
+      // the last 3 rows become the history of the next tile
+      for (int i = lane; i < (PC_W - 1) * (PC_COLS_WAVE / 8); i += 64) {
+        const int r = i / (PC_COLS_WAVE / 8), c8 = i % (PC_COLS_WAVE / 8);
+        *reinterpret_cast<bf16x8*>(&sy[r * PC_LD + 8 * c8]) =
+            *reinterpret_cast<const bf16x8*>(&sy[(PC_ROWS + r) * PC_LD + 8 * c8]);
+      }
+      lds_fence();
 #pragma unroll
-        for (int i = 0; i < PC_ROWS_LANE; ++i) {  // the projection output itself
+      for (int ks = 0; ks < PC_NKS; ++ks) xf[ks] = xnext[ks];
+    }
+  }
+
+  job = (int)blockIdx.x - plan.plain.wg0;
+  if (job >= 0 && job < plan.plain.n_wgs) {  // the projection output itself
+    const int b = plan.conv.n_blocks + job % plan.plain.n_blocks;
+    const PcBlock blk = plan.blocks[b];
+    const int64_t T0 = (int64_t)(job / plan.plain.n_blocks) * plan.plain.tokens;
+    const int64_t T1 = T0 + plan.plain.tokens < n_tokens ? T0 + plan.plain.tokens : n_tokens;
+    pc_load_w(W, (int64_t)b * PC_COLS_WG + wcol, PC_COLS_WAVE, lane, wf);
+    pc_load_x(x, x_stride, n_tokens, T0, lane, xf);
+    for (int64_t t0 = T0; t0 < T1; t0 += PC_ROWS) {
+      pc_load_x(x, x_stride, n_tokens, t0 + PC_ROWS, lane, xnext);
+      pc_tile(wf, xf, lane, sy);
+      lds_fence();
+#pragma unroll
+      for (int i = 0; i < PC_ROWS_LANE; ++i) {
+        const int tr = PC_ROWS_LANE * tq + i;
+        const bf16x8 o = *reinterpret_cast<const bf16x8*>(&sy[(tr + PC_W - 1) * PC_LD + 8 * cg]);
+        const int64_t t = t0 + tr;
+        if (t < T1) *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
+      }
+      lds_fence();
+#pragma unroll
+      for (int ks = 0; ks < PC_NKS; ++ks) xf[ks] = xnext[ks];
+    }
+  }
+
+  job = (int)blockIdx.x - plan.tail.wg0;
+  if (job >= 0 && job < plan.tail.n_wgs) {
+    const int64_t w0 = (int64_t)(plan.conv.n_blocks + plan.plain.n_blocks) * PC_COLS_WG;
+    for (int c0 = 0; c0 < plan.tail_cols; c0 += PC_COLS_WAVE) {
+      pc_load_w(W, w0 + c0, plan.tail_cols - c0, lane, wf);
+      for (int64_t t0 = (int64_t)(4 * job + wave) * PC_ROWS; t0 < n_tokens; t0 += (int64_t)4 * plan.tail.n_wgs * PC_ROWS) {
+        pc_load_x(x, x_stride, n_tokens, t0, lane, xf);
+        pc_tile(wf, xf, lane, sy);
+        lds_fence();
+        const int c = c0 + 8 * cg;
+#pragma unroll
+        for (int i = 0; i < PC_ROWS_LANE; ++i) {
           const int tr = PC_ROWS_LANE * tq + i;
           const bf16x8 o = *reinterpret_cast<const bf16x8*>(&sy[(tr + PC_W - 1) * PC_LD + 8 * cg]);
           const int64_t t = t0 + tr;
-          if (t < T1 && store_cols) *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
+          if (t < n_tokens && c < plan.tail_cols) *reinterpret_cast<bf16x8*>(plan.tail_out + t * plan.tail_cols + c) = o;
         }
+        lds_fence();
       }
     }
-    lds_fence();
-    // the last 3 rows become the history of the next tile
-    for (int i = lane; i < (PC_W - 1) * (PC_COLS_WAVE / 8); i += 64) {
-      const int r = i / (PC_COLS_WAVE / 8), c8 = i % (PC_COLS_WAVE / 8);
-      *reinterpret_cast<bf16x8*>(&sy[r * PC_LD + 8 * c8]) =
-          *reinterpret_cast<const bf16x8*>(&sy[(PC_ROWS + r) * PC_LD + 8 * c8]);
-    }
-    lds_fence();
-#pragma unroll
-    for (int ks = 0; ks < PC_NKS; ++ks) afrag[ks] = anext[ks];
   }
 }
 
@@ -208,42 +270,64 @@ extern "C" int lampa_proj_conv_fwd(const void* x, int64_t x_stride, int64_t n_to
   const int n_blocks = (n_cols + PC_COLS_WG - 1) / PC_COLS_WG;
   if (n_blocks > PC_MAX_BLOCKS) return LAMPA_ERR_UNSUPPORTED;
   if (n_tokens == 0) return LAMPA_OK;
-  if (tokens_per_wg <= 0) {
-    // as many runs of tokens as fill the chip once with two workgroups per CU (registers allow no more)
-    static int slots = 0;
-    if (!slots) {
-      int dev = 0, cus = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-        cus = 256;
-      slots = 2 * cus;
-    }
-    const int runs = slots / n_blocks > 0 ? slots / n_blocks : 1;
-    tokens_per_wg = (int)((n_tokens + runs - 1) / runs);
-    if (tokens_per_wg < 4 * PC_ROWS) tokens_per_wg = 4 * PC_ROWS;
+  const int n_conv_blocks = n_conv / PC_COLS_WG, n_plain_blocks = plain_cols / PC_COLS_WG;
+  static std::atomic<int> slots_of{0};  // workgroups the chip holds: two per CU (registers allow no more)
+  int slots = slots_of.load();
+  if (!slots) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+      cus = 256;
+    slots = 2 * cus;
+    slots_of.store(slots);
   }
-  tokens_per_wg = (tokens_per_wg + PC_ROWS - 1) / PC_ROWS * PC_ROWS;
+  // runs of `tokens` per block of a kind, at least min_tokens and whole tiles
+  auto runs_of = [&](PcJobs& j, int n_blocks, int64_t wgs, int64_t min_tokens) {
+    j.n_blocks = n_blocks;
+    if (n_blocks == 0) { j.wg0 = j.n_wgs = 0; j.tokens = PC_ROWS; return; }
+    const int64_t runs = wgs / n_blocks > 0 ? wgs / n_blocks : 1;
+    int64_t t = (n_tokens + runs - 1) / runs;
+    t = ((t < min_tokens ? min_tokens : t) + PC_ROWS - 1) / PC_ROWS * PC_ROWS;
+    j.tokens = (int)t;
+    j.n_wgs = (int)((n_tokens + t - 1) / t) * n_blocks;
+    j.wg0 = 0;
+  };
   PcPlan plan;
-  for (int b = 0; b < n_blocks; ++b) {
+  const int64_t tail_tiles = tail_cols ? (n_tokens + PC_ROWS - 1) / PC_ROWS : 0;
+  // A workgroup with a run of every kind, one round of them, pays once all slots would be taken by one-kind workgroups of
+  // more than the shortest run; below that the kinds side by side have fewer tiles in a row.
+  const bool mixed = tokens_per_wg <= 0 && n_conv_blocks && n_tokens > (int64_t)slots / n_blocks * (4 * PC_ROWS);
+  int64_t grid;
+  if (mixed) {
+    runs_of(plan.conv, n_conv_blocks, slots, 4 * PC_ROWS);
+    runs_of(plan.plain, n_plain_blocks, plan.conv.n_wgs, PC_ROWS);
+    plan.tail = {0, tail_cols ? plan.conv.n_wgs : 0, 1, PC_ROWS};
+    grid = plan.conv.n_wgs > plan.plain.n_wgs ? plan.conv.n_wgs : plan.plain.n_wgs;
+  } else {
+    const int64_t min_tokens = tokens_per_wg > 0 ? tokens_per_wg : 4 * PC_ROWS;
+    const int64_t wgs = tokens_per_wg > 0 ? INT32_MAX : slots / n_blocks;  // (per block)
+    runs_of(plan.conv, n_conv_blocks, wgs * n_conv_blocks, min_tokens);
+    runs_of(plan.plain, n_plain_blocks, wgs * n_plain_blocks, min_tokens);
+    plan.plain.wg0 = plan.conv.n_wgs;
+    plan.tail = {plan.conv.n_wgs + plan.plain.n_wgs, (int)((tail_tiles + 15) / 16), 1, PC_ROWS};
+    grid = plan.tail.wg0 + plan.tail.n_wgs;
+  }
+  plan.tail_out = (__bf16*)tail_out;
+  plan.tail_cols = tail_cols;
+  for (int b = 0; b < n_conv_blocks + n_plain_blocks; ++b) {
     PcBlock& k = plan.blocks[b];
     const int c0 = b * PC_COLS_WG;
     if (c0 < n_conv) {
       const int part = c0 / conv_split;
-      k.out = (__bf16*)conv_out + (int64_t)part * n_tokens * conv_split;
-      k.out_stride = conv_split; k.out_col0 = c0 - part * conv_split; k.n_valid = PC_COLS_WG; k.conv = 1; k.conv_col0 = c0;
-    } else if (c0 < n_conv + plain_cols) {
-      k.out = (__bf16*)plain_out;
-      k.out_stride = plain_cols; k.out_col0 = c0 - n_conv; k.n_valid = PC_COLS_WG; k.conv = 0; k.conv_col0 = 0;
+      k = {(__bf16*)conv_out + (int64_t)part * n_tokens * conv_split, conv_split, c0 - part * conv_split};
     } else {
-      k.out = (__bf16*)tail_out;
-      k.out_stride = tail_cols; k.out_col0 = 0; k.n_valid = tail_cols; k.conv = 0; k.conv_col0 = 0;
+      k = {(__bf16*)plain_out, plain_cols, c0 - n_conv};
     }
   }
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)((n_tokens + tokens_per_wg - 1) / tokens_per_wg), n_blocks);
   LAMPA_PROF(s, "start");
-  hipLaunchKernelGGL(pc_proj_conv_kernel, grid, dim3(256), 0, s, (const __bf16*)x, x_stride, n_tokens, t_len,
-                     (const __bf16*)W, conv_w, conv_b, plan, tokens_per_wg);
+  hipLaunchKernelGGL(pc_proj_conv_kernel, dim3((unsigned)grid), dim3(256), 0, s, (const __bf16*)x, x_stride, n_tokens, t_len,
+                     (const __bf16*)W, conv_w, conv_b, plan);
   LAMPA_PROF(s, "pc_proj_conv_kernel");
   return lampa_launch_status();
 }

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from lampa_amd import _capi
 from lampa_amd import layer_ops as lo
 from oracle import layer_ops as ol
 
@@ -110,6 +111,32 @@ def test_fused_projection_convolution(device, B, T, tokens_per_wg):
     for a, b2 in ((q, q2), (k, k2), (v, v2)):
         assert (a.float() - b2.float()).abs().max() < 0.1 and (a.float() - b2.float()).abs().mean() < 2e-3
     assert (g.float() - proj[..., 1536:2048].float()).abs().max() < 0.05
+
+
+@pytest.mark.parametrize("B,T,cols", [(1, 7169, (3, 512, 16)), (1, 20011, (3, 512, 16)), (3, 5003, (3, 512, 16)),
+                                      (700, 19, (3, 512, 16)), (1, 30001, (1, 0, 0)), (1, 30001, (2, 256, 200)),
+                                      (1, 30001, (0, 512, 8))])
+def test_projections_with_runs_of_every_kind_per_workgroup(device, B, T, cols):
+    """Inputs long enough for a workgroup to take a run of convolution columns, one of plain columns and tiles of the rest:
+    bit for bit the same as workgroups of one kind, which a given run length asks for; short and ragged sequences, and
+    projections that lack a kind or have more than a wave's columns left over."""
+    n_conv, plain, tail = cols
+    gen = torch.Generator(device=device).manual_seed(T)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=device)
+    x, W = rand(B, T, 128).bfloat16(), (rand(512 * n_conv + plain + tail, 128) * 0.1).bfloat16()
+    cws = [(rand(512, 1, 4) * 0.5).bfloat16() for _ in range(n_conv)]
+    cbs = [rand(512).bfloat16() for _ in range(n_conv)] or None
+    if not n_conv:  # (the wrapper always has convolutions)
+        got = [torch.empty(B * T, n, dtype=torch.bfloat16, device=device) for n in (plain, tail)]
+        _capi.check(_capi.lib().lampa_proj_conv_fwd(_capi.ptr(x), 128, B * T, T, 128, _capi.ptr(W), plain + tail, None, None, 0, 0,
+                                                    None, plain, _capi.ptr(got[0]), tail, _capi.ptr(got[1]), 0,
+                                                    _capi.stream_of(x)), "lampa_proj_conv_fwd")
+        want = torch.nn.functional.linear(x.float(), W.float()).view(B * T, -1)
+        for a, b in zip(got, want.split((plain, tail), dim=1)):
+            assert ((a.float() - b).abs() <= 2 ** -8 * b.abs() + 1e-4).all()
+        return
+    for a, b in zip(*(sum(((*y[0], *y[1:]) for y in [lo.proj_conv(x, W, cws, cbs, 512, plain, n)]), ()) for n in (0, 512))):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("B,T,tokens_per_wg", [(1, 1, 0), (2, 333, 64), (1, 6000, 0), (1, 100, 32)])
