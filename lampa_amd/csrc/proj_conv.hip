@@ -21,9 +21,11 @@
 // plain columns do not have, at two workgroups per CU (256 registers). On a long input every workgroup therefore takes a
 // run of convolution columns, then a shorter run of plain columns and a tile of the few columns behind them: with workgroups
 // of one kind each the CUs that held two of the convolution worked on while the others were done.
-// 60 000 tokens, 2064 columns of which 1536 with the convolution: 107.5 -> 101.8 us.
+// 60 000 tokens, 2064 columns of which 1536 with the convolution: 107.5 us with workgroups of one kind, 101.8 us this way,
+// 89.5 us since the rows of x requested ahead are not waited for together with the stores behind them (see `tile`).
 #include "gdr_common.h"
 #include <atomic>
+#include <type_traits>
 
 #define PC_K 128            // contraction length (hidden size) this kernel is built for
 #define PC_NKS (PC_K / 16)
@@ -130,70 +132,89 @@ __global__ void __launch_bounds__(256, 2) pc_proj_conv_kernel(const __bf16* __re
 #pragma unroll
       for (int j = 0; j < PC_W; ++j) cw[j][c] = conv_w[(int64_t)(b * PC_COLS_WG + col + c) * PC_W + j];
     }
-    // a run that starts inside a sequence first computes the tile before it, only for its last rows of history
-    const bool need_history = (T0 % t_len) != 0;
-    int64_t t0 = need_history ? T0 - PC_ROWS : T0;
-    if (!need_history) {
-      for (int i = lane; i < (PC_W - 1) * PC_LD; i += 64) sy[i] = (__bf16)0.0f;
-    }
-    // token position inside the sequence, kept per tile in 32 bits (a 64-bit modulo per output row would cost more than
-    // the convolution); sequences shorter than two tiles take the general modulo
-    const int tl32 = (int)(t_len < INT32_MAX ? t_len : INT32_MAX);
-    const bool small_seq = t_len < 2 * PC_ROWS;
-    int ts0 = (int)((t0 % t_len + t_len) % t_len);
-    pc_load_x(x, x_stride, n_tokens, t0, lane, xf);
-    for (; t0 < T1; t0 += PC_ROWS, ts0 = small_seq ? (ts0 + PC_ROWS) % tl32 : (ts0 + PC_ROWS >= tl32 ? ts0 + PC_ROWS - tl32 : ts0 + PC_ROWS)) {
-      pc_load_x(x, x_stride, n_tokens, t0 + PC_ROWS, lane, xnext);
-      pc_tile(wf, xf, lane, sy);
+    auto carry = [&]() __attribute__((always_inline)) {  // the last 3 rows become the history of the next tile
       lds_fence();
-      if (t0 >= T0) {
-        // the lane's 4 consecutive tokens share their taps: 7 rows of pre-activations for 4 outputs
-        float pre[PC_ROWS_LANE + PC_W - 1][8];
-#pragma unroll
-        for (int r = 0; r < PC_ROWS_LANE + PC_W - 1; ++r) {
-          const bf16x8 row = *reinterpret_cast<const bf16x8*>(&sy[(PC_ROWS_LANE * tq + r) * PC_LD + 8 * cg]);
-#pragma unroll
-          for (int c = 0; c < 8; ++c) pre[r][c] = (float)row[c];
-        }
-        // tokens closer than 3 to the start of their sequence lose the taps that reach across it; a tile that holds no
-        // such token (all but the first of a long sequence) skips the masks
-        const bool interior = ts0 >= PC_W - 1 && ts0 + PC_ROWS <= tl32;
-#pragma unroll
-        for (int i = 0; i < PC_ROWS_LANE; ++i) {
-          const int tr = PC_ROWS_LANE * tq + i;
-          float y[8];
-#pragma unroll
-          for (int c = 0; c < 8; ++c) y[c] = cb[c];
-          if (interior) {
-#pragma unroll
-            for (int j = 0; j < PC_W; ++j)
-#pragma unroll
-              for (int c = 0; c < 8; ++c) y[c] = __builtin_fmaf(pre[i + j][c], cw[j][c], y[c]);
-          } else {
-            int ts = ts0 + tr;
-            if (ts >= tl32) ts = small_seq ? ts % tl32 : ts - tl32;
-#pragma unroll
-            for (int j = 0; j < PC_W; ++j) {
-              const bool live = ts - (PC_W - 1) + j >= 0;
-#pragma unroll
-              for (int c = 0; c < 8; ++c) y[c] = __builtin_fmaf(live ? pre[i + j][c] : 0.0f, cw[j][c], y[c]);
-            }
-          }
-          bf16x8 o;
-#pragma unroll
-          for (int c = 0; c < 8; ++c) o[c] = (__bf16)(y[c] * pc_sigmoid(y[c]));
-          const int64_t t = t0 + tr;
-          if (t < T1) *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
-        }
-      }
-      lds_fence();
-      // the last 3 rows become the history of the next tile
       for (int i = lane; i < (PC_W - 1) * (PC_COLS_WAVE / 8); i += 64) {
         const int r = i / (PC_COLS_WAVE / 8), c8 = i % (PC_COLS_WAVE / 8);
         *reinterpret_cast<bf16x8*>(&sy[r * PC_LD + 8 * c8]) =
             *reinterpret_cast<const bf16x8*>(&sy[(PC_ROWS + r) * PC_LD + 8 * c8]);
       }
       lds_fence();
+    };
+    // token position inside the sequence, kept per tile in 32 bits (a 64-bit modulo per output row would cost more than
+    // the convolution); sequences shorter than two tiles take the general modulo
+    const int tl32 = (int)(t_len < INT32_MAX ? t_len : INT32_MAX);
+    const bool small_seq = t_len < 2 * PC_ROWS;
+    int ts0 = (int)(T0 % t_len);
+    if (ts0 != 0) {  // the run starts inside a sequence: the tile before it, for its last rows only
+      pc_load_x(x, x_stride, n_tokens, T0 - PC_ROWS, lane, xf);
+      pc_tile(wf, xf, lane, sy);
+      carry();
+    } else {
+      for (int i = lane; i < (PC_W - 1) * PC_LD; i += 64) sy[i] = (__bf16)0.0f;
+    }
+    // whole: all 32 rows exist. Stores without a condition: with one the compiler no longer knows how many are in flight
+    // and waits for all of them before it uses the rows of x that were requested ahead of them.
+    auto tile = [&](auto whole, int64_t t0, const bf16x8* xc, bf16x8* xn) __attribute__((always_inline)) {
+      pc_load_x(x, x_stride, n_tokens, t0 + PC_ROWS, lane, xn);
+      pc_tile(wf, xc, lane, sy);
+      lds_fence();
+      // the lane's 4 consecutive tokens share their taps: 7 rows of pre-activations for 4 outputs
+      float pre[PC_ROWS_LANE + PC_W - 1][8];
+#pragma unroll
+      for (int r = 0; r < PC_ROWS_LANE + PC_W - 1; ++r) {
+        const bf16x8 row = *reinterpret_cast<const bf16x8*>(&sy[(PC_ROWS_LANE * tq + r) * PC_LD + 8 * cg]);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) pre[r][c] = (float)row[c];
+      }
+      // tokens closer than 3 to the start of their sequence lose the taps that reach across it; a tile that holds no
+      // such token (all but the first of a long sequence) skips the masks
+      const bool interior = ts0 >= PC_W - 1 && ts0 + PC_ROWS <= tl32;
+      __bf16* out = blk.out + (t0 + PC_ROWS_LANE * tq) * blk.out_stride + blk.out_col0 + col;
+#pragma unroll
+      for (int i = 0; i < PC_ROWS_LANE; ++i) {
+        const int tr = PC_ROWS_LANE * tq + i;
+        float y[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) y[c] = cb[c];
+        if (interior) {
+#pragma unroll
+          for (int j = 0; j < PC_W; ++j)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) y[c] = __builtin_fmaf(pre[i + j][c], cw[j][c], y[c]);
+        } else {
+          int ts = ts0 + tr;
+          if (ts >= tl32) ts = small_seq ? ts % tl32 : ts - tl32;
+#pragma unroll
+          for (int j = 0; j < PC_W; ++j) {
+            const bool live = ts - (PC_W - 1) + j >= 0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) y[c] = __builtin_fmaf(live ? pre[i + j][c] : 0.0f, cw[j][c], y[c]);
+          }
+        }
+        bf16x8 o;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) o[c] = (__bf16)(y[c] * pc_sigmoid(y[c]));
+        if (decltype(whole)::value || t0 + tr < T1) *reinterpret_cast<bf16x8*>(out + i * (int64_t)blk.out_stride) = o;
+      }
+      carry();
+      ts0 = small_seq ? (ts0 + PC_ROWS) % tl32 : (ts0 + PC_ROWS >= tl32 ? ts0 + PC_ROWS - tl32 : ts0 + PC_ROWS);
+    };
+    int64_t t0 = T0;
+    pc_load_x(x, x_stride, n_tokens, t0, lane, xf);
+    if (t0 + 3 * PC_ROWS <= T1) {
+      // (the first tile on its own: then loads and stores are in flight in the same order at both ends of the loop)
+      tile(std::true_type{}, t0, xf, xnext);
+      t0 += PC_ROWS;
+      for (; t0 + 2 * PC_ROWS <= T1; t0 += 2 * PC_ROWS) {
+        tile(std::true_type{}, t0, xnext, xf);
+        tile(std::true_type{}, t0 + PC_ROWS, xf, xnext);
+      }
+#pragma unroll
+      for (int ks = 0; ks < PC_NKS; ++ks) xf[ks] = xnext[ks];
+    }
+    for (; t0 < T1; t0 += PC_ROWS) {  // at most two
+      tile(std::false_type{}, t0, xf, xnext);
 #pragma unroll
       for (int ks = 0; ks < PC_NKS; ++ks) xf[ks] = xnext[ks];
     }
@@ -207,18 +228,34 @@ __global__ void __launch_bounds__(256, 2) pc_proj_conv_kernel(const __bf16* __re
     const int64_t T1 = T0 + plan.plain.tokens < n_tokens ? T0 + plan.plain.tokens : n_tokens;
     pc_load_w(W, (int64_t)b * PC_COLS_WG + wcol, PC_COLS_WAVE, lane, wf);
     pc_load_x(x, x_stride, n_tokens, T0, lane, xf);
-    for (int64_t t0 = T0; t0 < T1; t0 += PC_ROWS) {
-      pc_load_x(x, x_stride, n_tokens, t0 + PC_ROWS, lane, xnext);
-      pc_tile(wf, xf, lane, sy);
+    auto tile = [&](auto whole, int64_t t0, const bf16x8* xc, bf16x8* xn) __attribute__((always_inline)) {
+      pc_load_x(x, x_stride, n_tokens, t0 + PC_ROWS, lane, xn);
+      pc_tile(wf, xc, lane, sy);
       lds_fence();
 #pragma unroll
       for (int i = 0; i < PC_ROWS_LANE; ++i) {
         const int tr = PC_ROWS_LANE * tq + i;
         const bf16x8 o = *reinterpret_cast<const bf16x8*>(&sy[(tr + PC_W - 1) * PC_LD + 8 * cg]);
         const int64_t t = t0 + tr;
-        if (t < T1) *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
+        if (decltype(whole)::value || t < T1)
+          *reinterpret_cast<bf16x8*>(blk.out + t * blk.out_stride + blk.out_col0 + col) = o;
       }
       lds_fence();
+    };
+    int64_t t0 = T0;
+    if (t0 + 3 * PC_ROWS <= T1) {
+      // (the first tile on its own: then loads and stores are in flight in the same order at both ends of the loop)
+      tile(std::true_type{}, t0, xf, xnext);
+      t0 += PC_ROWS;
+      for (; t0 + 2 * PC_ROWS <= T1; t0 += 2 * PC_ROWS) {
+        tile(std::true_type{}, t0, xnext, xf);
+        tile(std::true_type{}, t0 + PC_ROWS, xf, xnext);
+      }
+#pragma unroll
+      for (int ks = 0; ks < PC_NKS; ++ks) xf[ks] = xnext[ks];
+    }
+    for (; t0 < T1; t0 += PC_ROWS) {
+      tile(std::false_type{}, t0, xf, xnext);
 #pragma unroll
       for (int ks = 0; ks < PC_NKS; ++ks) xf[ks] = xnext[ks];
     }
