@@ -372,152 +372,166 @@ extern "C" int lampa_proj_conv_fwd(const void* x, int64_t x_stride, int64_t n_to
 // ------------------------------------------------------------------------------- gated RMS norm + output projection
 // y[t, :] = W_o * vec_h( rmsnorm(o[t, h, :]) * weight * swish(g[t, h, :]) ): the gated norm of every head
 // (models/hattention/fused_norm.py:40-111 with IS_RMS_NORM and the swish gate) feeding the bias-free output projection
-// (modeling_gated_deltaproduct.py:612-623) without writing the normalised tensor. One workgroup = 4 waves walks a run
-// of 32-token tiles: all threads normalise and gate the tile into LDS (bf16, the A operand; 8 lanes share a head's 64
-// channels), then every wave multiplies it with its 32 rows of W_o, which it keeps in registers as B-operand fragments.
+// (modeling_gated_deltaproduct.py:612-623) without writing the normalised tensor. One workgroup = 8 waves walks a run
+// of 32-token tiles: all threads normalise and gate a tile into LDS (bf16; 8 lanes share a head's 64 channels), every
+// wave multiplies it with its 16 rows of W_o, which it keeps in registers, and the result goes through LDS to whole rows,
+// 16 lanes each, for the residual add, the next norm's sum of squares and the stores.
+// Bound by latency: a tile is a chain of loads, norm, LDS, MFMA, LDS and stores on two waves per SIMD. The rows of o and g
+// are therefore requested a tile ahead (32 registers), for which 16 rows of W_o per wave (64 registers, 128 for 32 rows)
+// leave room; one workgroup per CU (with the 128 registers of two it spills 90). The sums over lanes are DPP moves. 60 000
+// tokens with residual and norm: 50.4 us (four waves of 32 rows, two workgroups per CU, loads waited for where they are
+// issued, two barriers that also drained them) -> 46 us.
 #define NP_D 64        // channels per head
-#define NP_KMAX 512    // heads * channels this kernel is built for (32 contraction steps of 16)
-#define NP_OUT 128     // output columns (4 waves x 32)
+#define NP_KMAX 512    // heads * channels this kernel is built for (16 contraction steps of 32)
+#define NP_OUT 128     // output columns (8 waves x 16)
 #define NP_LDA (NP_KMAX + 8)
+#define NP_LDO (NP_OUT + 8)
+#define NP_THREADS 512
+#define NP_PASSES 4    // rows of (token, head) a thread stages per tile: 64 per pass
+#define NP_DPP_ROR8 0x128
+#define NP_DPP_HALF_MIRROR 0x141
 
-__global__ void __launch_bounds__(256, 2) pc_norm_proj_kernel(const __bf16* __restrict__ o, const __bf16* __restrict__ g,
-                                                          int64_t g_stride, const float* __restrict__ norm_w,
-                                                          const __bf16* __restrict__ W, int64_t n_tokens, float eps,
-                                                          __bf16* __restrict__ y, const __bf16* __restrict__ residual,
-                                                          const float* __restrict__ next_w, float next_eps,
-                                                          __bf16* __restrict__ res_out, int tokens_per_wg) {
-  constexpr int NKS = NP_KMAX / 16;
+// RES: with a residual and the next layer's norm
+template <bool RES>
+__global__ void __launch_bounds__(NP_THREADS, 2) pc_norm_proj_kernel(
+    const __bf16* __restrict__ o, const __bf16* __restrict__ g, int64_t g_stride, const float* __restrict__ norm_w,
+    const __bf16* __restrict__ W, int64_t n_tokens, float eps, __bf16* __restrict__ y, const __bf16* __restrict__ residual,
+    const float* __restrict__ next_w, float next_eps, __bf16* __restrict__ res_out, int tokens_per_wg) {
+  constexpr int NKS = NP_KMAX / 32;
   __shared__ __align__(16) __bf16 s_a[2][PC_ROWS * NP_LDA];
-  __shared__ __align__(16) __bf16 s_out[4][PC_ROWS * (32 + 8)];
-  __shared__ float s_ss[4][PC_ROWS];  // with a residual: every wave's share of the rows' sums of squares
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
+  __shared__ __align__(16) __bf16 s_out[PC_ROWS * NP_LDO];
+  __shared__ __align__(16) float s_w[NP_D + NP_OUT];  // the weights of both norms (read where they are used, not held in registers)
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g4 = lane >> 4, ln = lane & 15;
   const int64_t T0 = (int64_t)blockIdx.x * tokens_per_wg;
   const int64_t T1 = T0 + tokens_per_wg < n_tokens ? T0 + tokens_per_wg : n_tokens;
 
-  bf16x8 bfrag[NKS];  // rows 32 wave + ln of W_o
+  bf16x8 wf[NKS];  // rows 16 wave + ln of W_o
   {
-    const __bf16* wp = W + (int64_t)(32 * wave + ln) * NP_KMAX + 8 * hh;
+    const __bf16* wp = W + (int64_t)(16 * wave + ln) * NP_KMAX + 8 * g4;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) bfrag[ks] = *reinterpret_cast<const bf16x8*>(wp + 16 * ks);
+    for (int ks = 0; ks < NKS; ++ks) wf[ks] = *reinterpret_cast<const bf16x8*>(wp + 32 * ks);
   }
-  // norm role: 8 lanes per (token, head) row, 8 channels each; 32 rows per pass, 8 passes per tile
-  const int sub = tid & 7, rrow = tid >> 3;
-  float nw[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) nw[c] = norm_w ? norm_w[8 * sub + c] : 1.0f;
+  // norm role: 8 lanes per (token, head) row, 8 channels each
+  const int sub = tid & 7, head = (tid >> 3) & 7, tok = wave;
+  const int orow = tid >> 4, ocol = 8 * (tid & 15);  // output role: 8 columns of a row
+  if (tid < NP_D) s_w[tid] = norm_w ? norm_w[tid] : 1.0f;
+  if (RES && tid < NP_OUT) s_w[NP_D + tid] = next_w ? next_w[tid] : 1.0f;
+  __syncthreads();
 
-  // (the loads of four passes are issued before the first is used: two memory round trips per tile, not one per pass;
-  // all eight at once would cost the second workgroup per CU its registers)
-  auto stage = [&](int64_t t0, int buf) {
+  bf16x8 ov[NP_PASSES], gv[NP_PASSES];
+  auto request = [&](int64_t t0) __attribute__((always_inline)) {
+    const int64_t first = t0 < n_tokens ? t0 : n_tokens - 1;
+    const int last = n_tokens - 1 - first < PC_ROWS ? (int)(n_tokens - 1 - first) : PC_ROWS - 1;
+    const __bf16 *ob = o + first * NP_KMAX, *gb = g + first * g_stride;
 #pragma unroll
-    for (int p0 = 0; p0 < 8; p0 += 4) {
-      bf16x8 ovs[4], gvs[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int r = 32 * (p0 + u) + rrow;       // (token, head) row of the tile: token r / 8, head r % 8
-        const int tok = r >> 3, head = r & 7;
-        int64_t t = t0 + tok;
-        t = t < n_tokens ? t : n_tokens - 1;
-        ovs[u] = *reinterpret_cast<const bf16x8*>(o + t * NP_KMAX + head * NP_D + 8 * sub);
-        gvs[u] = *reinterpret_cast<const bf16x8*>(g + t * g_stride + head * NP_D + 8 * sub);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int r = 32 * (p0 + u) + rrow;
-        const int tok = r >> 3, head = r & 7;
-        const bf16x8 ov = ovs[u], gv = gvs[u];
-        float x[8], ss = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) { x[c] = (float)ov[c]; ss = __builtin_fmaf(x[c], x[c], ss); }
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
-        const float rstd = 1.0f / sqrtf(ss * (1.0f / NP_D) + eps);
-        bf16x8 out;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const float gc = (float)gv[c];
-          out[c] = (__bf16)(x[c] * rstd * nw[c] * gc * pc_sigmoid(gc));
-        }
-        *reinterpret_cast<bf16x8*>(&s_a[buf][tok * NP_LDA + head * NP_D + 8 * sub]) = out;
-      }
+    for (int p = 0; p < NP_PASSES; ++p) {
+      const int t = min(8 * p + tok, last);
+      ov[p] = *reinterpret_cast<const bf16x8*>(ob + (uint32_t)(t * NP_KMAX + head * NP_D + 8 * sub));
+      gv[p] = *reinterpret_cast<const bf16x8*>(gb + t * g_stride + (uint32_t)(head * NP_D + 8 * sub));
     }
   };
-
-  const int cg = lane & 3, tq = lane >> 2;  // output role: row 2 tq + i (i < 2), columns 8 cg .. 8 cg + 7 of the wave's 32
-  float nxw[8];
+  auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-  for (int c = 0; c < 8; ++c) nxw[c] = (residual && next_w) ? next_w[32 * wave + 8 * cg + c] : 1.0f;
-  int buf = 0;
-  if (T0 < T1) stage(T0, 0);
-  __syncthreads();
-  for (int64_t t0 = T0; t0 < T1; t0 += PC_ROWS, buf ^= 1) {
-    // the residual rows of this tile are requested first: their latency hides behind the staging and the MFMAs
-    bf16x8 rv[2];
+    for (int p = 0; p < NP_PASSES; ++p) {
+      float x[8], ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+      for (int c = 0; c < 8; ++c) { x[c] = (float)ov[p][c]; ss = __builtin_fmaf(x[c], x[c], ss); }
+      ss += dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, ss);
+      ss += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, ss);
+      ss += dpp_f32<NP_DPP_HALF_MIRROR, 0xF>(0.0f, ss);
+      const float rstd = 1.0f / sqrtf(ss * (1.0f / NP_D) + eps);
+      bf16x8 out;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) rv[i][c] = (__bf16)0.0f;
-      const int64_t t = t0 + 2 * tq + i;
-      if (residual && t < T1) rv[i] = *reinterpret_cast<const bf16x8*>(residual + t * NP_OUT + 32 * wave + 8 * cg);
-    }
-    if (t0 + PC_ROWS < T1) stage(t0 + PC_ROWS, buf ^ 1);   // next tile while this one is multiplied
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    const __bf16* ap = &s_a[buf][ln * NP_LDA + 8 * hh];
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) acc = mfma32(*reinterpret_cast<const bf16x8*>(ap + 16 * ks), bfrag[ks], acc);
-    __bf16* so = s_out[wave];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) so[(8 * (r / 4) + 4 * hh + (r % 4)) * 40 + ln] = (__bf16)acc[r];
-    lds_fence();
-    if (!residual) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int tr = 2 * tq + i;
-        const int64_t t = t0 + tr;
-        if (t < T1)
-          *reinterpret_cast<bf16x8*>(y + t * NP_OUT + 32 * wave + 8 * cg) = *reinterpret_cast<const bf16x8*>(&so[tr * 40 + 8 * cg]);
+      for (int c = 0; c < 8; ++c) {
+        const float gc = (float)gv[p][c];
+        out[c] = (__bf16)(x[c] * rstd * s_w[8 * sub + c] * gc * pc_sigmoid(gc));
       }
+      *reinterpret_cast<bf16x8*>(&s_a[buf][(8 * p + tok) * NP_LDA + head * NP_D + 8 * sub]) = out;
+    }
+  };
+  auto request_residual = [&](int64_t t0) __attribute__((always_inline)) {
+    bf16x8 r = {};
+    if constexpr (RES) {
+      int64_t t = t0 + orow;
+      t = t < n_tokens ? t : n_tokens - 1;
+      r = *reinterpret_cast<const bf16x8*>(residual + t * NP_OUT + ocol);
+    }
+    return r;
+  };
+  // One tile: buf holds it, the registers the rows of the next one; whole: all 32 rows exist (no condition on the stores, so
+  // that the compiler can count them and does not wait for them with the rows requested ahead of them).
+  auto tile = [&](auto whole, int64_t t0, int buf, const bf16x8& res, bf16x8& res_next) __attribute__((always_inline)) {
+    stage(buf ^ 1);
+    res_next = request_residual(t0 + PC_ROWS);
+    request(t0 + 2 * PC_ROWS);
+    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    const __bf16* ap = &s_a[buf][ln * NP_LDA + 8 * g4];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            wf[ks], *reinterpret_cast<const bf16x8*>(ap + 16 * m * NP_LDA + 32 * ks), acc[m], 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {  // lane = token, registers = neighbouring columns
+      bf16x4 p;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[e] = (__bf16)acc[m][e];
+      *reinterpret_cast<bf16x4*>(&s_out[(16 * m + ln) * NP_LDO + 16 * wave + 4 * g4]) = p;
+    }
+    lds_barrier();  // the output tile is complete, the next A tile is staged
+    const bf16x8 yv = *reinterpret_cast<const bf16x8*>(&s_out[orow * NP_LDO + ocol]);
+    lds_barrier();  // the output tile has been read
+    const int64_t t = t0 + orow;
+    const bool live = decltype(whole)::value || t < T1;
+    if constexpr (!RES) {
+      if (live) *reinterpret_cast<bf16x8*>(y + t * NP_OUT + ocol) = yv;
     } else {
       // residual add and the next layer's RMS norm over the 128 output columns (fused_norm.py:1436-1506 with a
       // residual): res_out = residual + y, y = rmsnorm(res_out) * next_w, the sum of squares taken before rounding
-      float sres[2][8];
+      float sres[8], ss = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int tr = 2 * tq + i;
-        const bf16x8 yv = *reinterpret_cast<const bf16x8*>(&so[tr * 40 + 8 * cg]);
-        float ss = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          sres[i][c] = (float)yv[c] + (float)rv[i][c];
-          ss = __builtin_fmaf(sres[i][c], sres[i][c], ss);
-        }
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        if (cg == 0) s_ss[wave][tr] = ss;
+      for (int c = 0; c < 8; ++c) {
+        sres[c] = (float)yv[c] + (float)res[c];
+        ss = __builtin_fmaf(sres[c], sres[c], ss);
       }
-      __syncthreads();
+      ss += dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, ss);
+      ss += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, ss);
+      ss += dpp_f32<NP_DPP_HALF_MIRROR, 0xF>(0.0f, ss);
+      ss += dpp_f32<NP_DPP_ROR8, 0xF>(0.0f, ss);
+      const float rstd = 1.0f / sqrtf(ss * (1.0f / NP_OUT) + next_eps);
+      bf16x8 ro, ho;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int tr = 2 * tq + i;
-        const int64_t t = t0 + tr;
-        const float tot = s_ss[0][tr] + s_ss[1][tr] + s_ss[2][tr] + s_ss[3][tr];
-        const float rstd = 1.0f / sqrtf(tot * (1.0f / NP_OUT) + next_eps);
-        bf16x8 ro, ho;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          ro[c] = (__bf16)sres[i][c];
-          ho[c] = (__bf16)(sres[i][c] * rstd * nxw[c]);
-        }
-        if (t < T1) {
-          *reinterpret_cast<bf16x8*>(res_out + t * NP_OUT + 32 * wave + 8 * cg) = ro;
-          *reinterpret_cast<bf16x8*>(y + t * NP_OUT + 32 * wave + 8 * cg) = ho;
-        }
+      for (int c = 0; c < 8; ++c) {
+        ro[c] = (__bf16)sres[c];
+        ho[c] = (__bf16)(sres[c] * rstd * s_w[NP_D + ocol + c]);
+      }
+      if (live) {
+        *reinterpret_cast<bf16x8*>(res_out + t * NP_OUT + ocol) = ro;
+        *reinterpret_cast<bf16x8*>(y + t * NP_OUT + ocol) = ho;
       }
     }
-    __syncthreads();  // the next tile is staged, this tile's A operand and the row sums are free again
+  };
+  if (T0 >= T1) return;
+  bf16x8 rA = request_residual(T0), rB;
+  request(T0);
+  stage(0);
+  request(T0 + PC_ROWS);
+  lds_barrier();
+  int64_t t0 = T0;
+  if (t0 + 3 * PC_ROWS <= T1) {
+    // (the first tile on its own: then loads and stores are in flight in the same order at both ends of the loop)
+    tile(std::true_type{}, t0, 0, rA, rB);
+    t0 += PC_ROWS;
+    for (; t0 + 2 * PC_ROWS <= T1; t0 += 2 * PC_ROWS) {
+      tile(std::true_type{}, t0, 1, rB, rA);
+      tile(std::true_type{}, t0 + PC_ROWS, 0, rA, rB);
+    }
+    rA = rB;
+  }
+  for (int buf = (int)((t0 - T0) / PC_ROWS) & 1; t0 < T1; t0 += PC_ROWS, buf ^= 1) {  // at most two
+    tile(std::false_type{}, t0, buf, rA, rB);
+    rA = rB;
   }
 }
 
@@ -540,15 +554,20 @@ extern "C" int lampa_norm_proj_fwd(const void* o, const void* g, int64_t g_strid
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
       cus = 256;
-    tokens_per_wg = (int)((n_tokens + 2 * cus - 1) / (2 * cus));
+    tokens_per_wg = (int)((n_tokens + cus - 1) / cus);
     if (tokens_per_wg < 2 * PC_ROWS) tokens_per_wg = 2 * PC_ROWS;
   }
   tokens_per_wg = (tokens_per_wg + PC_ROWS - 1) / PC_ROWS * PC_ROWS;
   hipStream_t s = (hipStream_t)stream;
   LAMPA_PROF(s, "start");
-  hipLaunchKernelGGL(pc_norm_proj_kernel, dim3((unsigned)((n_tokens + tokens_per_wg - 1) / tokens_per_wg)), dim3(256), 0, s,
-                     (const __bf16*)o, (const __bf16*)g, g_stride, norm_w, (const __bf16*)W, n_tokens, eps, (__bf16*)y,
-                     (const __bf16*)residual, next_w, next_eps, (__bf16*)res_out, tokens_per_wg);
+  const dim3 grid((unsigned)((n_tokens + tokens_per_wg - 1) / tokens_per_wg));
+#define NP_LAUNCH(RES)                                                                                                        \
+  hipLaunchKernelGGL(pc_norm_proj_kernel<RES>, grid, dim3(NP_THREADS), 0, s, (const __bf16*)o, (const __bf16*)g, g_stride,    \
+                     norm_w, (const __bf16*)W, n_tokens, eps, (__bf16*)y, (const __bf16*)residual, next_w, next_eps,          \
+                     (__bf16*)res_out, tokens_per_wg)
+  if (residual) NP_LAUNCH(true);
+  else NP_LAUNCH(false);
+#undef NP_LAUNCH
   LAMPA_PROF(s, "pc_norm_proj_kernel");
   return lampa_launch_status();
 }

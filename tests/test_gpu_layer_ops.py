@@ -249,3 +249,18 @@ def test_norm_modules_and_errors(device):
 def _capi_error():
     from lampa_amd._capi import LampaError
     return LampaError
+
+
+@pytest.mark.parametrize("T", [1, 33, 3007])
+def test_norm_projection_runs_of_any_length_agree(device, T):
+    """Runs of one tile, of two, of three and more (whose loop takes tiles in pairs behind the first) and a ragged last tile give
+    the same bits, with and without the residual; a strided gate whose last row ends the allocation."""
+    gen = torch.Generator(device=device).manual_seed(T)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=device).bfloat16()
+    o, W, nw, nxt, res = rand(1, T, 8, 64), rand(128, 512) * 0.05, rand(64).abs(), rand(128).abs(), rand(1, T, 128)
+    g = rand(1, T, 520)[..., 8:].unflatten(-1, (8, 64))
+    want = lo.norm_proj(o, g, nw, W, 1e-6, 32), lo.norm_proj(o, g, nw, W, 1e-6, 32, residual=res, next_norm_weight=nxt)
+    for n in (64, 96, 128, 160, 4096, 0):
+        assert torch.equal(lo.norm_proj(o, g, nw, W, 1e-6, n), want[0])
+        for a, b in zip(lo.norm_proj(o, g, nw, W, 1e-6, n, residual=res, next_norm_weight=nxt), want[1]):
+            assert torch.equal(a, b)
