@@ -655,7 +655,7 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
                      const unsigned char* __restrict__ Mgrp, const unsigned char* __restrict__ Ngrp,
                      const float* __restrict__ Dgrp, int gmax, const float* __restrict__ dht, T* __restrict__ dq,
                      T* __restrict__ dk, T* __restrict__ dv, float* __restrict__ dg, float* __restrict__ dbeta,
-                     float* __restrict__ dh0, int H, int HV, float scale, int l2norm) {
+                     float* __restrict__ dh0, int H, int HV, float scale, int l2norm, int Kw, int Vw) {
   using OT = T;
   using X8 = typename OpVec<OT>::x8;
   using X4 = typename OpVec<OT>::x4;
@@ -784,7 +784,7 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
       const int xtok = 32 * wave + 16 * w + L;
       const float b = t.beta[xtok];
       float x = 0.0f;
-      T* at = dv + ((size_t)tok0 * HV + hv) * 64 + (uint32_t)(xtok * HV * 64 + 8 * (lane >> 4));
+      T* at = dv + ((size_t)tok0 * HV + hv) * Vw + (uint32_t)(xtok * HV * Vw + 8 * (lane >> 4));
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         typename Raw8<T>::type out;
@@ -795,7 +795,7 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
           out[e] = (T)(b * lo);
           out[4 + e] = (T)(b * hi);
         }
-        if (xtok < len) *reinterpret_cast<typename Raw8<T>::type*>(at + 32 * u) = out;
+        if (xtok < len && 32 * u + 8 * (lane >> 4) < Vw) *reinterpret_cast<typename Raw8<T>::type*>(at + 32 * u) = out;
       }
       x += __shfl_xor(x, 16);
       x = gb_both_halves(x);
@@ -870,7 +870,7 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
     const int vn = wave - 2;
     auto store_rows = [&](int c) __attribute__((always_inline)) {  // dq, dk of chunk c
       const int tok0 = tok_of(c), len = len_of(c), row0 = 8 * vn + (lane >> 3), part = lane & 7;
-      const size_t first = ((size_t)tok0 * HV + hv) * 64;
+      const size_t first = ((size_t)tok0 * HV + hv) * Kw;
       X8 o[8];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -880,8 +880,8 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int row = 16 * u + row0;
-        if (row < len) {
-          const uint32_t at = (uint32_t)(row * HV * 64 + 8 * part);
+        if (row < len && 8 * part < Kw) {
+          const uint32_t at = (uint32_t)(row * HV * Kw + 8 * part);
           *reinterpret_cast<X8*>(dq + first + at) = o[u];
           *reinterpret_cast<X8*>(dk + first + at) = o[4 + u];
         }
@@ -1200,7 +1200,8 @@ static GbWorkspace gb_workspace(int64_t segs, int HV) {
 template <typename T>
 static int gb_run(const void* q, const void* k, const void* v, const void* dout, const float* dht, void* dq, void* dk,
                   void* dv, float* dg, float* dbeta, float* dh0, const int32_t* ph, const int32_t* pd,
-                  const unsigned char* saved, int H, int HV, float scale, int l2norm, unsigned char* ws, hipStream_t s) {
+                  const unsigned char* saved, int H, int HV, int Kw, int Vw, float scale, int l2norm, unsigned char* ws,
+                  hipStream_t s) {
   const int n_seq = ph[PLAN_N_SEQ], chunks = ph[PLAN_TOTAL_CHUNKS], segs = ph[PLAN_N_SEGMENTS];
   const GdrSaved sv = gdr_saved_layout(chunks, segs, HV);
   const GbWorkspace w = gb_workspace(segs, HV);
@@ -1241,7 +1242,7 @@ static int gb_run(const void* q, const void* k, const void* v, const void* dout,
   }
   hipLaunchKernelGGL((gdrb_walk_kernel<T>), dim3(segs * HV), dim3(GB_WALK_THREADS), GbWalkSmem::BYTES, s, (const T*)q,
                      (const T*)k, (const T*)v, (const T*)dout, recs, states, pv, pv.chunk_tok0, pv.chunk_len, Mt, Dc, Nr, Gm, Gn,
-                     Gd, gmax, dht, (T*)dq, (T*)dk, (T*)dv, dg, dbeta, dh0, H, HV, scale, l2norm);
+                     Gd, gmax, dht, (T*)dq, (T*)dk, (T*)dv, dg, dbeta, dh0, H, HV, scale, l2norm, Kw, Vw);
   LAMPA_PROF(s, "gdrb_walk_kernel");
   return lampa_launch_status();
 }
@@ -1255,8 +1256,8 @@ extern "C" int64_t lampa_gdr_bwd_saved_workspace_bytes(const int32_t* plan_host,
   return gb_workspace(plan_host[PLAN_N_SEGMENTS], HV).bytes;
 }
 
-// Gradients from what lampa_gdr_chunk_fwd_train kept. q, k [tokens, H, 64]; v, dout, dv and dq, dk (one row per VALUE head)
-// [tokens, HV, 64]; dg, dbeta fp32 [tokens, HV]; dht, dh0 fp32 [n_seq, HV, 64, 64] (nullable).
+// Gradients from what lampa_gdr_chunk_fwd_train kept. q, k [tokens, H, 64]; v, dout [tokens, HV, 64]; dq, dk (one row per
+// VALUE head) [tokens, HV, K], dv [tokens, HV, V] with K, V <= 64, multiples of 8 (the heads before they were padded); dg, dbeta fp32 [tokens, HV]; dht, dh0 fp32 [n_seq, HV, 64, 64] (nullable).
 extern "C" int lampa_gdr_bwd_saved(const void* q, const void* k, const void* v, const void* saved, const void* dout,
                                    const float* dht, void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
                                    const int32_t* plan_host, const int32_t* plan_dev, int H, int HV, int K, int V, int dtype,
@@ -1264,7 +1265,7 @@ extern "C" int lampa_gdr_bwd_saved(const void* q, const void* k, const void* v, 
   if (!q || !k || !v || !saved || !dout || !dq || !dk || !dv || !dg || !dbeta || !plan_host || !plan_dev)
     return LAMPA_ERR_INVALID;
   if (H < 1 || HV < H || HV % H != 0 || l2norm < 0 || l2norm > 2) return LAMPA_ERR_INVALID;
-  if (K != 64 || V != 64 || (dtype != GDR_BF16 && dtype != GDR_FP16)) return LAMPA_ERR_UNSUPPORTED;
+  if (!gdr_train_width(K) || !gdr_train_width(V) || (dtype != GDR_BF16 && dtype != GDR_FP16)) return LAMPA_ERR_UNSUPPORTED;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) & 15)
     return LAMPA_ERR_INVALID;
   if (!gb_plan_ok(plan_host)) return LAMPA_ERR_INVALID;
@@ -1273,8 +1274,8 @@ extern "C" int lampa_gdr_bwd_saved(const void* q, const void* k, const void* v, 
   unsigned char* ws = (unsigned char*)workspace;
   const unsigned char* sv = (const unsigned char*)saved;
   if (dtype == GDR_BF16)
-    return gb_run<__bf16>(q, k, v, dout, dht, dq, dk, dv, dg, dbeta, dh0, plan_host, plan_dev, sv, H, HV, scale, l2norm, ws, s);
-  return gb_run<_Float16>(q, k, v, dout, dht, dq, dk, dv, dg, dbeta, dh0, plan_host, plan_dev, sv, H, HV, scale, l2norm, ws, s);
+    return gb_run<__bf16>(q, k, v, dout, dht, dq, dk, dv, dg, dbeta, dh0, plan_host, plan_dev, sv, H, HV, K, V, scale, l2norm, ws, s);
+  return gb_run<_Float16>(q, k, v, dout, dht, dq, dk, dv, dg, dbeta, dh0, plan_host, plan_dev, sv, H, HV, K, V, scale, l2norm, ws, s);
 }
 
 // ---- the same from the inputs alone: the training form of the forward, then the pass above ------------------------------

@@ -50,6 +50,7 @@ struct GdrKeep {
   unsigned char *rec, *states, *mt;
   float* d;
   int32_t* positive_g;
+  int o_width;
 };
 
 template <typename T, int KT, int VT, bool KEEP = false>
@@ -92,7 +93,7 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
       hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
                          (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, Mc, Nc, Dc,
                          (T*)nullptr, (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
-                         (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, kp.mt);
+                         (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, kp.mt, VT);
       LAMPA_PROF(s, "gdr_segment_kernel<composite>");
     }
   }
@@ -125,11 +126,11 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
     hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true, false, T, CWN>), dim3(segs * HV),
                        dim3(64 * GdrSegShape<KT, VT, true, CWN>::WAVES), smem_n, s, (const T*)q, (const T*)k, (const T*)v, g, beta,
                        pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, Nc, Dc, (T*)o, ht, H, HV, scale, l2norm,
-                       (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states);
+                       (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states, KEEP ? kp.o_width : VT);
   else
   hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true, false, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, true>::WAVES), smem_b, s, (const T*)q,
                      (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, Nc, Dc, (T*)o, ht, H, HV, scale,
-                     l2norm, (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states);
+                     l2norm, (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states, KEEP ? kp.o_width : VT);
   LAMPA_PROF(s, "gdr_segment_kernel<output>");
   return lampa_launch_status();
 }
@@ -194,7 +195,8 @@ extern "C" int64_t lampa_gdr_train_workspace_bytes(const int32_t* plan_host, int
   return gdr_workspace(0, plan_host[PLAN_N_SEGMENTS], HV, 64, 64).bytes;
 }
 
-// As lampa_gdr_chunk_fwd for K = V = 64. saved: lampa_gdr_train_saved_bytes bytes for lampa_gdr_bwd_saved. positive_g_host
+// As lampa_gdr_chunk_fwd for q, k, v of 64 columns; the rows of o are V <= 64 columns, a multiple of 8 (K, V: the heads before
+// they were padded to 64). saved: lampa_gdr_train_saved_bytes bytes for lampa_gdr_bwd_saved. positive_g_host
 // (nullable): pinned host memory, zeroed by the caller; becomes 1 when an entry of g is positive.
 extern "C" int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const void* v, const float* g, const float* beta,
                                          void* o, const float* h0, float* ht, const int32_t* plan_host,
@@ -203,7 +205,7 @@ extern "C" int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const voi
                                          int64_t workspace_bytes, void* stream) {
   if (!q || !k || !v || !g || !beta || !o || !plan_host || !plan_dev || !saved) return LAMPA_ERR_INVALID;
   if (H < 1 || HV < H || HV % H != 0 || l2norm < 0 || l2norm > 2) return LAMPA_ERR_INVALID;
-  if (K != 64 || V != 64 || (dtype != GDR_BF16 && dtype != GDR_FP16)) return LAMPA_ERR_UNSUPPORTED;
+  if (!gdr_train_width(K) || !gdr_train_width(V) || (dtype != GDR_BF16 && dtype != GDR_FP16)) return LAMPA_ERR_UNSUPPORTED;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o | (uintptr_t)saved) & 15) return LAMPA_ERR_INVALID;
   const int n_seq = plan_host[PLAN_N_SEQ], chunks = plan_host[PLAN_TOTAL_CHUNKS], segs = plan_host[PLAN_N_SEGMENTS];
   if (n_seq < 1 || segs < n_seq) return LAMPA_ERR_INVALID;
@@ -213,7 +215,7 @@ extern "C" int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const voi
   for (int i = 0; i < n_seq; ++i) max_nseg = plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] > max_nseg ? plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] : max_nseg;
   const GdrSaved sv = gdr_saved_layout(chunks, segs, HV);
   unsigned char* sp = (unsigned char*)saved;
-  GdrKeep kp{sp + sv.off_rec, sp + sv.off_states, sp + sv.off_mt, (float*)(sp + sv.off_d), nullptr};
+  GdrKeep kp{sp + sv.off_rec, sp + sv.off_states, sp + sv.off_mt, (float*)(sp + sv.off_d), nullptr, V};
   if (positive_g_host && hipHostGetDevicePointer((void**)&kp.positive_g, positive_g_host, 0) != hipSuccess) {
     (void)hipGetLastError();
     return LAMPA_ERR_INVALID;

@@ -602,7 +602,8 @@ __device__ __forceinline__ bf16x8 ld_kappa_tr(const __bf16* arr, int stride, int
 
 // KEEP (training form, K = V = 64, see gdr_train.h): PASS_A also maps the last segment of a sequence and stores M' once
 // more in the fragment order of its transpose; PASS_B stores the state in front of every chunk -- the operand fragments
-// the chain waves hold anyway, 8 KiB per chunk and head in 1 KiB runs.
+// the chain waves hold anyway, 8 KiB per chunk and head in 1 KiB runs. o's rows are then o_width <= VT elements (a multiple
+// of 8): of heads that were padded to VT columns only the caller's own leave the chip.
 template <typename T, int KT, int VT, bool PASS_B, bool SCALED_K = !PASS_B, typename OT = T, int CW = 32, bool KEEP = false>
 __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
                                   ((SCALED_K || CW == 16) ? GdrSegShape<KT, VT, PASS_B, CW>::WAVES_PER_SIMD : 2))
@@ -615,7 +616,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
                        float* __restrict__ ht, int H, int HV, float scale, int l2norm,
                        const unsigned char* __restrict__ Mgrp, const unsigned char* __restrict__ Ngrp,
                        const float* __restrict__ Dgrp, const float* __restrict__ h0, int gmax,
-                       unsigned char* __restrict__ keep) {
+                       unsigned char* __restrict__ keep, int o_width) {
   // OT: the 16-bit type of every MFMA operand (tiles in LDS, T, R, v_new, P, the state as operand, M' of the
   // composites): the input type, so that fp16 inputs run on the fp16 MFMA without losing mantissa bits
   using X8 = typename OpVec<OT>::x8;
@@ -631,6 +632,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   // 32-column output pass: the o tile of a chunk is written to HBM by the STAGER waves (after the next chunk's barrier
   // B, whole rows), so the read-back and the stores are off the recurrence waves' chain.
   constexpr bool STAGER_FLUSH = PASS_B && CW == 32 && KT + VT <= 128;  // (the wider heads have no registers for it)
+  static_assert(STAGER_FLUSH || !PASS_B || !KEEP, "o_width is applied where the stagers write o");
   // Output pass at K <= 64: a stager builds the P tiles of the q rows it staged itself (stager 0 the tile (0,0),
   // stager 1 the tiles (1,0) and (1,1)), so no barrier separates staging q from building P. At K = 128 a P tile is
   // twice the work, the two stagers share the middle tile, and the barrier Qb(c) (q(c) is staged) comes back.
@@ -1159,7 +1161,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       // the o tile (rows of chunk `tok0`) -> HBM, 16-byte pieces, whole rows (non-temporal: o is not read again here)
       auto stager_flush = [&](int tok0, int len) __attribute__((always_inline)) {
         constexpr int PPR = VT / 8, NP = 64 * PPR / 128;
-        T* ob = o + ((size_t)tok0 * HV + hv) * VT;
+        const int ow = KEEP ? o_width : VT;
+        T* ob = o + ((size_t)tok0 * HV + hv) * ow;
         uint4 val[NP];
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
@@ -1172,8 +1175,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
           typedef unsigned int nt_u32x4 __attribute__((ext_vector_type(4)));
           nt_u32x4 nv;
           nv[0] = val[j].x; nv[1] = val[j].y; nv[2] = val[j].z; nv[3] = val[j].w;
-          if (row < len)
-            __builtin_nontemporal_store(nv, reinterpret_cast<nt_u32x4*>(ob + (unsigned)(row * (HV * VT) + 8 * part)));
+          if (row < len && (!KEEP || 8 * part < ow))
+            __builtin_nontemporal_store(nv, reinterpret_cast<nt_u32x4*>(ob + (unsigned)(row * (HV * ow) + 8 * part)));
         }
       };
       issue_tiles(c0, tk0, ln0, rkA);

@@ -7,6 +7,9 @@
 
 #define GDR_STATE_BYTES 8192  // 64 x 64 elements of 2 bytes (and one 64 x 32 slab in fp32)
 
+// widths of the rows that o and the gradients of padded heads can have
+static inline bool gdr_train_width(int n) { return n >= 8 && n <= 64 && n % 8 == 0; }
+
 struct GdrSaved {
   int64_t off_rec, off_states, off_mt, off_d, bytes;
 };

@@ -948,7 +948,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
                        beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, pieces ? ws + w.off_pm : Mc,
                        pieces ? ws + w.off_pn : Nm, pieces ? (float*)(ws + w.off_pd) : Dc, (T*)nullptr, (float*)nullptr, H, HV,
                        scale, l2norm, (const unsigned char*)nullptr, (const unsigned char*)nullptr, (const float*)nullptr,
-                       (const float*)nullptr, pieces, (unsigned char*)nullptr);
+                       (const float*)nullptr, pieces, (unsigned char*)nullptr, VT);
     LAMPA_PROF(s, "gdr_segment_kernel<composite>");
   };
   if (pieces) composites();

@@ -365,8 +365,14 @@ class _Kept:
     __slots__ = ("plan", "buffer", "flag", "done")
 
 
-def _chunk_train_forward(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm):
-    """The forward for inputs that require gradients: q, k, v padded to 64 x 64 heads -> (o, final state, kept)."""
+def _written_heads(head):
+    """The head sizes the training kernels write: the caller's own where they are multiples of 8, else the padded ones."""
+    return tuple(n if n % 8 == 0 else 64 for n in head)
+
+
+def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm):
+    """The forward for inputs that require gradients: q, k, v padded from ``head`` = (K, V) to 64 x 64 heads -> (o with rows
+    of V elements, final state [N, HV, 64, 64], kept)."""
     B, T, H, _ = q.shape
     HV = v.shape[2]
     cu_host = _sequence_bounds(cu_seqlens, B, T)
@@ -380,16 +386,17 @@ def _chunk_train_forward(q, k, v, g, beta, scale, initial_state, output_final_st
     kept.buffer = torch.empty(n_saved, dtype=torch.uint8, device=q.device)
     kept.flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    o = torch.empty_like(v)
+    K, V = _written_heads(head)
+    o = torch.empty((B, T, HV, V), dtype=v.dtype, device=v.device)
     ht = torch.empty((n_seq, HV, 64, 64), dtype=torch.float32, device=q.device) if output_final_state else None
     h0 = _pad_state(initial_state)
     check(lib.lampa_gdr_chunk_fwd_train(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(o), ptr(h0), ptr(ht), host_ptr,
-                                        ptr(plan_dev), H, HV, 64, 64, _DTYPES[q.dtype], float(scale), l2norm,
+                                        ptr(plan_dev), H, HV, K, V, _DTYPES[q.dtype], float(scale), l2norm,
                                         ptr(kept.buffer), ctypes.c_void_p(kept.flag.data_ptr()), ptr(ws), ws_bytes,
                                         stream_of(q)), "lampa_gdr_chunk_fwd_train")
     kept.done = torch.cuda.Event()
     kept.done.record(torch.cuda.current_stream(q.device))
-    return o, ht, kept
+    return _resize_heads((o,), (head[1],))[0], ht, kept
 
 
 def _raise_positive_g():
@@ -400,44 +407,41 @@ def _raise_positive_g():
                      "the unmasked recurrence)")
 
 
-def _backward_kept_launch(q, k, v, kept, scale, l2norm, do, dht, want_dh0):
-    """Gradients (dq, dk, dv, dg, dbeta, dh0) through ``lampa_gdr_bwd_saved``; q, k, v, do with 64 x 64 heads. dq and dk come
-    back with one row per value head when value heads share q / k heads: summed over each group here."""
+def _backward_kept_launch(q, k, v, head, kept, scale, l2norm, do, dht, want_dh0):
+    """Gradients (dq, dk, dv, dg, dbeta, dh0) of heads of ``head`` = (K, V) through ``lampa_gdr_bwd_saved``; q, k, v, do, dht
+    padded to 64 x 64 heads. dq and dk come from the kernel with one row per value head when value heads share q / k heads:
+    summed over each group here."""
     B, T, H, _ = q.shape
     HV = v.shape[2]
     plan_host, plan_dev = kept.plan
     lib, host_ptr = _capi.lib(), ctypes.c_void_p(plan_host.data_ptr())
     ws_bytes = check(lib.lampa_gdr_bwd_saved_workspace_bytes(host_ptr, HV), "lampa_gdr_bwd_saved_workspace_bytes")
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    dq, dk, dv = (torch.empty((B, T, HV, 64), dtype=q.dtype, device=q.device) for _ in range(3))
+    K, V = _written_heads(head)
+    dq, dk, dv = (torch.empty((B, T, HV, n), dtype=q.dtype, device=q.device) for n in (K, K, V))
     dg, dbeta = (torch.empty((B, T, HV), dtype=torch.float32, device=q.device) for _ in range(2))
     n_seq = int(plan_host[0])
     dh0 = torch.empty((n_seq, HV, 64, 64), dtype=torch.float32, device=q.device) if want_dh0 else None
     check(lib.lampa_gdr_bwd_saved(ptr(q), ptr(k), ptr(v), ptr(kept.buffer), ptr(do), ptr(dht), ptr(dq), ptr(dk), ptr(dv),
-                                  ptr(dg), ptr(dbeta), ptr(dh0), host_ptr, ptr(plan_dev), H, HV, 64, 64, _DTYPES[q.dtype],
+                                  ptr(dg), ptr(dbeta), ptr(dh0), host_ptr, ptr(plan_dev), H, HV, K, V, _DTYPES[q.dtype],
                                   float(scale), l2norm, ptr(ws), ws_bytes, stream_of(q)), "lampa_gdr_bwd_saved")
     if HV > H:
-        dq = dq.view(B, T, H, HV // H, 64).float().sum(3).to(q.dtype)
-        dk = dk.view(B, T, H, HV // H, 64).float().sum(3).to(k.dtype)
+        dq = dq.view(B, T, H, HV // H, K).float().sum(3).to(q.dtype)
+        dk = dk.view(B, T, H, HV // H, K).float().sum(3).to(k.dtype)
+    if head != (64, 64):
+        K, V = head
+        dq, dk, dv = _resize_heads((dq, dk, dv), (K, K, V))
+        dh0 = None if dh0 is None else dh0[..., :K, :V].contiguous()
     return dq, dk, dv, dg, dbeta, dh0
-
-
-def _cut_heads(grads, K: int, V: int):
-    """The gradients of padded heads -> the caller's head sizes."""
-    if (K, V) == (64, 64):
-        return grads
-    dq, dk, dv, dg, dbeta, dh0 = grads
-    return (*_resize_heads((dq, dk, dv), (K, K, V)), dg, dbeta, None if dh0 is None else dh0[..., :K, :V].contiguous())
 
 
 def _backward_chunk_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, do, dht):
     """Gradients in the chunked form from the inputs alone: the training form of the forward (its outputs dropped), then the
     backward pass over what it kept."""
-    K, V = q.shape[-1], v.shape[-1]
+    head = q.shape[-1], v.shape[-1]
     q, k, v, do = _resize_heads((q, k, v, do), (64, 64, 64, 64))
-    _, _, kept = _chunk_train_forward(q, k, v, g, beta, scale, initial_state, False, cu_seqlens, l2norm)
-    return _cut_heads(_backward_kept_launch(q, k, v, kept, scale, l2norm, do, _pad_state(dht), initial_state is not None),
-                      K, V)
+    _, _, kept = _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, False, cu_seqlens, l2norm)
+    return _backward_kept_launch(q, k, v, head, kept, scale, l2norm, do, _pad_state(dht), initial_state is not None)
 
 
 def _backward_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, do, dht):
@@ -501,13 +505,12 @@ class _GatedDelta(torch.autograd.Function):
                     and q.shape[0] * q.shape[1] > 0):
                 K, V = ctx.head
                 q, k, v = _resize_heads((q, k, v), (64, 64, 64))
-                o, ht, ctx.kept = _chunk_train_forward(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
-                                                       l2norm)
+                o, ht, ctx.kept = _chunk_train_forward(q, k, v, ctx.head, g, beta, scale, initial_state, output_final_state,
+                                                       cu_seqlens, l2norm)
                 ctx.save_for_backward(q, k, v, initial_state, ctx.kept.buffer)
                 ctx.kept.buffer = None
-                if (K, V) != (64, 64):
-                    o, = _resize_heads((o,), (V,))
-                    ht = None if ht is None else ht[..., :K, :V].contiguous()
+                if (K, V) != (64, 64) and ht is not None:
+                    ht = ht[..., :K, :V].contiguous()
                 return o, ht
             ctx.save_for_backward(q, k, v, g, beta, initial_state, cu_seqlens)
         return launcher(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm)
@@ -524,8 +527,8 @@ class _GatedDelta(torch.autograd.Function):
             kept = _Kept()
             kept.plan, kept.buffer = ctx.kept.plan, buffer
             do = torch.zeros_like(v) if do is None else _resize_heads((do.to(v.dtype),), (64,))[0]
-            grads = _cut_heads(_backward_kept_launch(q, k, v, kept, ctx.scale, ctx.l2norm, do, _pad_state(dht),
-                                                     initial_state is not None), *ctx.head)
+            grads = _backward_kept_launch(q, k, v, ctx.head, kept, ctx.scale, ctx.l2norm, do, _pad_state(dht),
+                                          initial_state is not None)
             # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them
             ctx.kept.done.synchronize()
             if int(ctx.kept.flag[0]):

@@ -305,3 +305,25 @@ def test_resized_heads_are_padded_and_cut_copies(device, rows, widths, offset):
     for x, y, (w, n) in zip(src, gd._resize_heads(src, [n for _, n in widths]), widths):
         want = torch.nn.functional.pad(x.view(torch.int16), (0, n - w))  # (a negative pad cuts)
         assert y.is_contiguous() and torch.equal(y.view(torch.int16), want)
+
+
+@pytest.mark.parametrize("K,V,H,HV", [(8, 8, 2, 2), (16, 32, 3, 3), (48, 56, 1, 2), (64, 24, 2, 2), (20, 64, 2, 2), (40, 30, 1, 1)])
+def test_small_heads_are_written_in_their_own_width(device, K, V, H, HV):
+    """Output, final state and gradients of heads below 64 x 64 (in sizes the kernels write themselves and in sizes that are
+    cut afterwards) against the same call with the heads zero-padded by hand: the same bits. Ragged last chunk, several
+    segments, packed sequences."""
+    cu = torch.tensor([0, 700, 700, 1501], device=device)
+    (q, k, v, g, beta, do), gen = _inputs(1, 1501, H, HV, K, V, torch.float16, K + V, unit=False)
+    pad = torch.nn.functional.pad
+    wide = [pad(q, (0, 64 - K)), pad(k, (0, 64 - K)), pad(v, (0, 64 - V)), g, beta]
+
+    def run(args, do):
+        leaves = [x.to(device).requires_grad_(True) for x in args]
+        o, ht = gd.chunk_gated_delta_rule(*leaves, scale=0.25, output_final_state=True, cu_seqlens=cu,
+                                          use_qk_l2norm_in_kernel=True)
+        return o, ht, *torch.autograd.grad(o, leaves, do.to(device))
+
+    got, want = run((q, k, v, g, beta), do), run(wide, pad(do, (0, 64 - V)))
+    cut = (want[0][..., :V], want[1][..., :K, :V], want[2][..., :K], want[3][..., :K], want[4][..., :V], *want[5:])
+    for a, b in zip(got, cut):
+        assert a.is_contiguous() and torch.equal(a, b)
