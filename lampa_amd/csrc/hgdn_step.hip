@@ -469,7 +469,8 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
 // lanes as scalars. What bounds it is that serial chain per token (B * HV * V wavefronts, two per compute unit at 8 heads of
 // 64 columns); the next token's values are loaded while this one is worked on.
 // A prefill of 15 000 tokens (24 behind its whole chunks, 8 heads of 64 x 64): 708 us with a launch of the single-token kernel
-// and its copies per token, 210 us with this kernel.
+// and its copies per token, 210 us with this kernel (54 us of them its own), 188 us (37) since no load is converted on the
+// spot under a condition.
 #define HGS_TAIL_LEVELS 17  // levels of the narrow instantiation: sequences up to 65 536 tokens
 #define HGS_TAIL_WAVES 4
 #define HGS_DPP_ROR8 0x128
@@ -524,41 +525,69 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
   if (j >= V) return;
   const int b = blockIdx.x / HV, hv = blockIdx.x % HV, h = hv / (HV / H);
   float* col = states + (((size_t)b * HV + hv) * K * V + j) * L;  // row i: col + i * V * L
+  // Loads come from clamped addresses without conditions on the lane, and are converted and masked where they are used: a
+  // conditional load that is converted on the spot is a branch with a wait for memory inside (one per value: four round
+  // trips per token, and one per level at either end).
   float S[ROWS][LM];
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) {
-    const int i = lane + 64 * r;
+  for (int r = 0; r < ROWS; ++r)
 #pragma unroll
-    for (int l = 0; l < LM; ++l) S[r][l] = (i < K && l < L) ? col[(size_t)i * V * L + l] : 0.0f;
-  }
+    for (int l = 0; l < LM; ++l) S[r][l] = col[(size_t)min(lane + 64 * r, K - 1) * V * L + min(l, L - 1)];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int l = 0; l < LM; ++l) S[r][l] = (lane + 64 * r < K && l < L) ? S[r][l] : 0.0f;
   struct Token {
-    float q[ROWS], k[ROWS], lam, v, g, beta;
+    T q[ROWS], k[ROWS], v;
+    uint32_t lam;
+    float g, beta;
   };
+  const int lam_at = min(lane, L - 1);
   auto load = [&](int t) {
     Token x;
     const size_t tok = (size_t)b * n_tok + t;
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-      const int i = lane + 64 * r;
-      x.q[r] = i < K ? GdrElem<T>::to_float(q[(tok * H + h) * K + i]) : 0.0f;
-      x.k[r] = i < K ? GdrElem<T>::to_float(k[(tok * H + h) * K + i]) : 0.0f;
+      const int i = min(lane + 64 * r, K - 1);
+      x.q[r] = q[(tok * H + h) * K + i];
+      x.k[r] = k[(tok * H + h) * K + i];
     }
-    const size_t li = (tok * HV + hv) * L + lane;
-    x.lam = 0.0f;
-    if (lane < L)
-      x.lam = lam_dtype == GDR_FP32   ? reinterpret_cast<const float*>(lam)[li]
-              : lam_dtype == GDR_BF16 ? (float)reinterpret_cast<const __bf16*>(lam)[li]
-                                      : (float)reinterpret_cast<const _Float16*>(lam)[li];
-    x.v = GdrElem<T>::to_float(v[(tok * HV + hv) * V + j]);
+    const size_t li = (tok * HV + hv) * L + lam_at;
+    if (lam_dtype == GDR_FP32) x.lam = reinterpret_cast<const uint32_t*>(lam)[li];
+    else x.lam = reinterpret_cast<const uint16_t*>(lam)[li];
+    x.v = v[(tok * HV + hv) * V + j];
     x.g = g[tok * HV + hv];
     x.beta = beta[tok * HV + hv];
     return x;
   };
+  auto lam_value = [&](uint32_t raw) {
+    if (lane >= L) return 0.0f;
+    return lam_dtype == GDR_FP32   ? __uint_as_float(raw)
+           : lam_dtype == GDR_BF16 ? __uint_as_float(raw << 16)
+                                   : (float)__builtin_bit_cast(_Float16, (uint16_t)raw);
+  };
+  // A token's output is stored at the start of the next token, ahead of the loads that are requested there: behind them the
+  // wait for those loads would also be one for the store.
+  float acc_o = 0.0f;
+  auto store = [&](int t) {
+    if (lane == 0) o[(((size_t)b * n_tok + t) * HV + hv) * V + j] = GdrElem<T>::from_float(acc_o);
+  };
   Token next = load(tok0);
   for (int t = tok0; t < n_tok; ++t) {
-    const Token x = next;
+    struct {
+      float q[ROWS], k[ROWS], v, g, beta;
+    } x;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      x.q[r] = lane + 64 * r < K ? GdrElem<T>::to_float(next.q[r]) : 0.0f;
+      x.k[r] = lane + 64 * r < K ? GdrElem<T>::to_float(next.k[r]) : 0.0f;
+    }
+    x.v = GdrElem<T>::to_float(next.v);
+    x.g = next.g;
+    x.beta = next.beta;
+    float lam_l = lam_value(next.lam);
+    if (t > tok0) store(t - 1);
     next = load(min(t + 1, n_tok - 1));
-    float lam_l = x.lam;
     if (lam_div != 1.0f) {  // lambda / scale, rounded to lambda's own type as the element-wise division would
       lam_l = __fdiv_rn(lam_l, lam_div);
       lam_l = lam_dtype == GDR_FP32 ? lam_l : lam_dtype == GDR_BF16 ? (float)(__bf16)lam_l : (float)(_Float16)lam_l;
@@ -570,9 +599,10 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
       float acc = S[r][0];
 #pragma unroll
       for (int l = 1; l < LM; ++l) {
+        if (l > z) break;  // (uniform; every other token touches one level)
         const float s = S[r][l];
-        S[r][l] = l < z ? 0.0f : l == z ? s + acc : s;
-        acc = l < z ? acc + s : acc;
+        S[r][l] = l < z ? 0.0f : s + acc;
+        acc += s;
       }
       S[r][0] = 0.0f;  // (empty before the first token)
     }
@@ -621,12 +651,12 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
         }
       }
     }
-    float acc_o = 0.0f;
+    acc_o = 0.0f;
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) acc_o = __builtin_fmaf(x.q[r], sl[r], acc_o);
     acc_o = rq * wave_sum_all(acc_o);
-    if (lane == 0) o[(((size_t)b * n_tok + t) * HV + hv) * V + j] = GdrElem<T>::from_float(acc_o);
   }
+  store(n_tok - 1);
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
     const int i = lane + 64 * r;
