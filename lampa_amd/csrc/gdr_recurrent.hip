@@ -180,7 +180,9 @@ __global__ void __launch_bounds__(64)
   // round instead of two: 1.11 -> 0.73 ms; with fewer waves the longer groups are faster, 207 against 230 us)
   constexpr int G = (SHORT_GROUPS ? 512 : 1024) / KT < 64 ? (SHORT_GROUPS ? 512 : 1024) / KT : 64;
   constexpr int ROW4 = (2 * KT + 4) / 4;              // 16-byte pieces per token in LDS: k | q, padded against conflicts
-  constexpr int PPT = 2 * KT / 4;                     // 4-element pieces of k | q per token
+  // 4-element pieces of k | q per token; the maps need no q (left out under a condition on the lane instead, its loads made
+  // every load a branch, with a wait for memory inside for 16-bit inputs: 8 192 x 4 x 32 x 32 fp32 18.0 against 16.1 us)
+  constexpr int PPT = (COMPOSITE ? KT : 2 * KT) / 4;
   constexpr int PIECES = G * PPT / 64;                // pieces per lane and group
   constexpr int VALS = G * 32 / 64;                   // v elements per lane and group
   static_assert((G * PPT) % 64 == 0, "group shape");
@@ -219,8 +221,7 @@ __global__ void __launch_bounds__(64)
         const int pi = lane + 64 * n, j = pi / PPT, c = 4 * (pi % PPT);
         const int64_t t = t0 + j < eos ? t0 + j : eos - 1;
         const int e = c < KT ? c : c - KT;
-        if (COMPOSITE && c >= KT) piece[n] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // (q is not used)
-        else piece[n] = rec_load4<T>((c < KT ? k : q) + (t * H + h) * K + (e < K ? e : K - 4));
+        piece[n] = rec_load4<T>((c < KT ? k : q) + (t * H + h) * K + (e < K ? e : K - 4));
       }
 #pragma unroll
       for (int n = 0; n < VALS; ++n) {
@@ -259,9 +260,12 @@ __global__ void __launch_bounds__(64)
         float kss = 0.0f, qss = 0.0f;
 #pragma unroll
         for (int c4 = 0; c4 < KT / 4; ++c4) {
-          const float4 a = s_kq[buf][lane * ROW4 + c4], b = s_kq[buf][lane * ROW4 + KT / 4 + c4];
+          const float4 a = s_kq[buf][lane * ROW4 + c4];
           kss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
-          qss += b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
+          if constexpr (!COMPOSITE) {
+            const float4 b = s_kq[buf][lane * ROW4 + KT / 4 + c4];
+            qss += b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
+          }
         }
         float kinv = 1.0f, qinv = 1.0f;
         if (l2norm == GDR_L2_CHUNK) {

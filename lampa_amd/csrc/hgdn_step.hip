@@ -469,8 +469,8 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
 // lanes as scalars. What bounds it is that serial chain per token (B * HV * V wavefronts, two per compute unit at 8 heads of
 // 64 columns); the next token's values are loaded while this one is worked on.
 // A prefill of 15 000 tokens (24 behind its whole chunks, 8 heads of 64 x 64): 708 us with a launch of the single-token kernel
-// and its copies per token, 210 us with this kernel (54 us of them its own), 188 us (37) since no load is converted on the
-// spot under a condition.
+// and its copies per token, 210 us with this kernel (54 us of them its own), 188 us (37) since no load is converted on
+// the spot under a condition.
 #define HGS_TAIL_LEVELS 17  // levels of the narrow instantiation: sequences up to 65 536 tokens
 #define HGS_TAIL_WAVES 4
 #define HGS_DPP_ROR8 0x128
@@ -599,10 +599,9 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
       float acc = S[r][0];
 #pragma unroll
       for (int l = 1; l < LM; ++l) {
-        if (l > z) break;  // (uniform; every other token touches one level)
         const float s = S[r][l];
-        S[r][l] = l < z ? 0.0f : s + acc;
-        acc += s;
+        S[r][l] = l < z ? 0.0f : l == z ? s + acc : s;
+        acc = l < z ? acc + s : acc;
       }
       S[r][0] = 0.0f;  // (empty before the first token)
     }
