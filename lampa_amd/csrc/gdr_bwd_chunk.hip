@@ -779,27 +779,35 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         x4[w][u] = op_lds_read_tr4<OT>(reinterpret_cast<const OT*>(p + w * 1024 + (u >> 1) * 4096 + (u & 1) * 64));
+    // (X . v of both before the first store: the compiler cannot count conditional stores, and a wait for v behind them was
+    // also one for them)
+    float x[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          x[w] += (float)x4[w][2 * u][e] * (float)vre[w][u][e] + (float)x4[w][2 * u + 1][e] * (float)vre[w][u][4 + e];
+    asm volatile("" : "+v"(x[0]), "+v"(x[1]));
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
       const int xtok = 32 * wave + 16 * w + L;
       const float b = t.beta[xtok];
-      float x = 0.0f;
       T* at = dv + ((size_t)tok0 * HV + hv) * Vw + (uint32_t)(xtok * HV * Vw + 8 * (lane >> 4));
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         typename Raw8<T>::type out;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float lo = (float)x4[w][2 * u][e], hi = (float)x4[w][2 * u + 1][e];
-          x += lo * (float)vre[w][u][e] + hi * (float)vre[w][u][4 + e];
-          out[e] = (T)(b * lo);
-          out[4 + e] = (T)(b * hi);
+          out[e] = (T)(b * (float)x4[w][2 * u][e]);
+          out[4 + e] = (T)(b * (float)x4[w][2 * u + 1][e]);
         }
         if (xtok < len && 32 * u + 8 * (lane >> 4) < Vw) *reinterpret_cast<typename Raw8<T>::type*>(at + 32 * u) = out;
       }
-      x += __shfl_xor(x, 16);
-      x = gb_both_halves(x);
-      if (lane < 16) s_sum[GbSums::XV + xtok] = x;
+      x[w] += __shfl_xor(x[w], 16);
+      x[w] = gb_both_halves(x[w]);
+      if (lane < 16) s_sum[GbSums::XV + xtok] = x[w];
     }
   };
   // rows of a gradient tile (rows 32 kt .., lane = token tok) through the l2 normalisation: y the normalised input row, dot
