@@ -16,7 +16,7 @@ hierarchy, base 2.
 
 All three branches of the operator are here: outputs only (``hattention_kernel``), prefill returning the level
 states (``hattention_prefill``, ``kernel.py:467-575``: the whole chunks through the chunk kernels, the remaining
-tokens one by one) and the single-token step on an ``HState`` (``hattention_step``, ``kernel.py:577-633``).
+tokens in one launch) and the single-token step on an ``HState`` (``hattention_step``, ``kernel.py:577-633``).
 
 Differences a caller can observe: forward only; the chunk kernels are built for K = 64 and V in {64, 128}, smaller
 heads are zero-padded to those, larger ones are refused (the single-token step takes any K and V, up to 32 levels); ``HState.counts`` lives on the host (the reference keeps it on the device and synchronises
