@@ -556,9 +556,8 @@ def main():
 
     backward = {"config2_shape": backward_leg(T, H, K, V, torch.bfloat16),
                 "reference_model_heads": backward_leg(30016, 6, 16, 32, torch.float16),
-                "note": "chunked: per-chunk affine maps of the state (forwards) and of its gradient (backwards) on the "
-                        "MFMA, a three-level scan over the maps, then every gradient of a chunk from its tiles and the "
-                        "two states; operands in the input type (heads below 64 x 64 zero-padded). token_serial: fp32, "
+                "note": "chunked: the forward again, keeping records, states and segment maps, then one walk per "
+                        "segment from the last chunk to the first on the MFMA; operands in the input type (heads below 64 x 64 zero-padded). token_serial: fp32, "
                         "parallel segments, a state kept every 8 tokens. Both: dq, dk, dv, dg, dbeta out, q/k "
                         "normalisation included"}
 
