@@ -388,8 +388,8 @@ extern "C" int lampa_proj_conv_fwd(const void* x, int64_t x_stride, int64_t n_to
 #define NP_LDO (NP_OUT + 8)
 #define NP_THREADS 512
 #define NP_PASSES 4    // rows of (token, head) a thread stages per tile: 64 per pass
-#define NP_DPP_ROR8 0x128
 #define NP_DPP_HALF_MIRROR 0x141
+#define NP_DPP_ROW_LANE(n) (0x150 + (n))  /* lane n of each row of 16 -> the whole row */
 
 // RES: with a residual and the next layer's norm
 template <bool RES>
@@ -497,8 +497,10 @@ __global__ void __launch_bounds__(NP_THREADS, 2) pc_norm_proj_kernel(
       }
       ss += dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, ss);
       ss += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, ss);
-      ss += dpp_f32<NP_DPP_HALF_MIRROR, 0xF>(0.0f, ss);
-      ss += dpp_f32<NP_DPP_ROR8, 0xF>(0.0f, ss);
+      // every quad of lanes holds the sum over its 32 columns: added from the first to the last (another order changes the
+      // bits of the norm now and then, and a stack of layers in bf16 spreads that over its whole output)
+      ss = ((dpp_f32<NP_DPP_ROW_LANE(0), 0xF>(0.0f, ss) + dpp_f32<NP_DPP_ROW_LANE(4), 0xF>(0.0f, ss)) +
+            dpp_f32<NP_DPP_ROW_LANE(8), 0xF>(0.0f, ss)) + dpp_f32<NP_DPP_ROW_LANE(12), 0xF>(0.0f, ss);
       const float rstd = 1.0f / sqrtf(ss * (1.0f / NP_OUT) + next_eps);
       bf16x8 ro, ho;
 #pragma unroll

@@ -264,3 +264,34 @@ def test_norm_projection_runs_of_any_length_agree(device, T):
         assert torch.equal(lo.norm_proj(o, g, nw, W, 1e-6, n), want[0])
         for a, b in zip(lo.norm_proj(o, g, nw, W, 1e-6, n, residual=res, next_norm_weight=nxt), want[1]):
             assert torch.equal(a, b)
+
+
+def test_residual_norm_adds_its_columns_in_order(device):
+    """The sum of squares behind the fused residual norm: eight columns one after the other, four such sums in pairs, the four
+    sums over 32 columns from the first to the last -- checked bit for bit on a row whose sum rounds differently in pairs,
+    with weights that put every product next to a rounding boundary of bf16. (W = 0, so that the row is the residual.)"""
+    f32 = np.float32
+    rows = torch.randn(4096, 128, generator=torch.Generator().manual_seed(0)).bfloat16()
+    x = rows.float().numpy()
+    part = np.zeros((4096, 16), f32)
+    for c in range(8):
+        part = part + x[:, c::8] * x[:, c::8]          # (products of bf16 are exact in fp32: the fma of the kernel)
+    quad = (part[:, 0::4] + part[:, 1::4]) + (part[:, 2::4] + part[:, 3::4])
+    in_order = ((quad[:, 0] + quad[:, 1]) + quad[:, 2]) + quad[:, 3]
+    in_pairs = (quad[:, 0] + quad[:, 1]) + (quad[:, 2] + quad[:, 3])
+    rstd = lambda ss: f32(1) / np.sqrt(ss * f32(1 / 128) + f32(1e-6))
+    row = int(np.nonzero(rstd(in_order) != rstd(in_pairs))[0][0])
+    a, b = x[row] * rstd(in_order)[row], x[row] * rstd(in_pairs)[row]
+    bf16 = lambda y: torch.from_numpy(y).bfloat16()
+    w = np.ones(128, f32)
+    for c in range(128):                               # weights near the one that makes the product 1 + 2^-8 (a tie)
+        near = f32((1 + 2.0 ** -8) / abs(a[c])) if a[c] else f32(1)
+        tries = near + np.arange(-8, 9, dtype=f32) * np.spacing(near)
+        split = np.nonzero((bf16(a[c] * tries) != bf16(b[c] * tries)).numpy())[0]
+        w[c] = tries[split[0]] if len(split) else near
+    want = bf16(x * rstd(in_order)[:, None] * w)
+    assert not torch.equal(want[row], bf16(b * w))
+    zero = torch.zeros(1, 4096, 8, 64, device=device).bfloat16()
+    h, r = lo.norm_proj(zero, zero, None, torch.zeros(128, 512, device=device).bfloat16(), 1e-6,
+                        residual=rows[None].to(device), next_norm_weight=torch.from_numpy(w).to(device), next_eps=1e-6)
+    assert torch.equal(r[0].cpu(), rows) and torch.equal(h[0].cpu(), want)
