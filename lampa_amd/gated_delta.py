@@ -361,7 +361,7 @@ def _pad_state(x):
 class _Kept:
     """What the training form of the chunk forward (``lampa_gdr_chunk_fwd_train``) leaves for the backward pass: the plan,
     the kept buffer (chunk records, states in front of the chunks, transposed segment maps) and the flag for positive
-    entries of g in pinned host memory, valid once ``done`` has passed."""
+    entries of g in pinned host memory, valid once ``done`` has passed (None: nothing watches g)."""
     __slots__ = ("plan", "buffer", "flag", "done")
 
 
@@ -372,7 +372,8 @@ def _written_heads(head):
 
 def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm):
     """The forward for inputs that require gradients: q, k, v padded from ``head`` = (K, V) to 64 x 64 heads -> (o with rows
-    of V elements, final state [N, HV, 64, 64], kept)."""
+    of V elements, final state [N, HV, 64, 64], kept). The kernels note positive entries of g, but not while the stream is being
+    captured (a replay would write to a word of pinned memory, and waits for an event, that belong to the captured call)."""
     B, T, H, _ = q.shape
     HV = v.shape[2]
     cu_host = _sequence_bounds(cu_seqlens, B, T)
@@ -384,7 +385,8 @@ def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_fi
     n_saved = check(lib.lampa_gdr_train_saved_bytes(host_ptr, HV), "lampa_gdr_train_saved_bytes")
     ws_bytes = check(lib.lampa_gdr_train_workspace_bytes(host_ptr, HV), "lampa_gdr_train_workspace_bytes")
     kept.buffer = torch.empty(n_saved, dtype=torch.uint8, device=q.device)
-    kept.flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    watch_g = not torch.cuda.is_current_stream_capturing()
+    kept.flag = torch.zeros(1, dtype=torch.int32, pin_memory=True) if watch_g else None
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     K, V = _written_heads(head)
     o = torch.empty((B, T, HV, V), dtype=v.dtype, device=v.device)
@@ -392,10 +394,11 @@ def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_fi
     h0 = _pad_state(initial_state)
     check(lib.lampa_gdr_chunk_fwd_train(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(o), ptr(h0), ptr(ht), host_ptr,
                                         ptr(plan_dev), H, HV, K, V, _DTYPES[q.dtype], float(scale), l2norm,
-                                        ptr(kept.buffer), ctypes.c_void_p(kept.flag.data_ptr()), ptr(ws), ws_bytes,
-                                        stream_of(q)), "lampa_gdr_chunk_fwd_train")
-    kept.done = torch.cuda.Event()
-    kept.done.record(torch.cuda.current_stream(q.device))
+                                        ptr(kept.buffer), ptr(kept.flag), ptr(ws), ws_bytes, stream_of(q)),
+          "lampa_gdr_chunk_fwd_train")
+    if watch_g:
+        kept.done = torch.cuda.Event()
+        kept.done.record(torch.cuda.current_stream(q.device))
     return _resize_heads((o,), (head[1],))[0], ht, kept
 
 
@@ -507,7 +510,7 @@ class _GatedDelta(torch.autograd.Function):
                 q, k, v = _resize_heads((q, k, v), (64, 64, 64))
                 o, ht, ctx.kept = _chunk_train_forward(q, k, v, ctx.head, g, beta, scale, initial_state, output_final_state,
                                                        cu_seqlens, l2norm)
-                ctx.save_for_backward(q, k, v, initial_state, ctx.kept.buffer)
+                ctx.save_for_backward(q, k, v, initial_state, ctx.kept.buffer, None if ctx.kept.flag is not None else g)
                 ctx.kept.buffer = None
                 if (K, V) != (64, 64) and ht is not None:
                     ht = ht[..., :K, :V].contiguous()
@@ -523,16 +526,19 @@ class _GatedDelta(torch.autograd.Function):
                 "because we haven't figured out how to compute dg without materializing the full "
                 "hidden states for all time steps.")
         if ctx.kept is not None:
-            q, k, v, initial_state, buffer = ctx.saved_tensors
+            q, k, v, initial_state, buffer, g = ctx.saved_tensors
+            if g is not None and bool((g > 0).any()):
+                _raise_positive_g()
             kept = _Kept()
             kept.plan, kept.buffer = ctx.kept.plan, buffer
             do = torch.zeros_like(v) if do is None else _resize_heads((do.to(v.dtype),), (64,))[0]
             grads = _backward_kept_launch(q, k, v, ctx.head, kept, ctx.scale, ctx.l2norm, do, _pad_state(dht),
                                           initial_state is not None)
-            # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them
-            ctx.kept.done.synchronize()
-            if int(ctx.kept.flag[0]):
-                _raise_positive_g()
+            if ctx.kept.flag is not None:
+                # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them
+                ctx.kept.done.synchronize()
+                if int(ctx.kept.flag[0]):
+                    _raise_positive_g()
         else:
             q, k, v, g, beta, initial_state, cu_seqlens = ctx.saved_tensors
             if bool((g > 0).any()):

@@ -327,3 +327,37 @@ def test_small_heads_are_written_in_their_own_width(device, K, V, H, HV):
     cut = (want[0][..., :V], want[1][..., :K, :V], want[2][..., :K], want[3][..., :K], want[4][..., :V], *want[5:])
     for a, b in zip(got, cut):
         assert a.is_contiguous() and torch.equal(a, b)
+
+
+def test_forward_of_a_training_call_in_a_captured_graph(device):
+    """A forward captured into a graph, replayed on other inputs and with eager work in between, then differentiated: the bits
+    of the eager call; the check of g looks at the values of the last replay, and a positive entry of an earlier one is
+    forgotten."""
+    make = lambda seed: [x.to(device) for x in _inputs(1, 1000, 2, 2, 64, 64, torch.bfloat16, seed, unit=False)[0]]
+    static = [x.requires_grad_(True) for x in make(1)[:5]]
+    call = lambda args: gd.chunk_gated_delta_rule(*args, use_qk_l2norm_in_kernel=True)[0]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        o = call(static)
+    for seed in (2, 3):
+        *new, do = make(seed)
+        for x, y in zip(static, new):
+            x.data.copy_(y)
+        graph.replay()
+        leaves = [x.requires_grad_(True) for x in new]
+        want = call(leaves)
+        assert torch.equal(o, want)
+        for a, b in zip(torch.autograd.grad(o, static, do, retain_graph=True), torch.autograd.grad(want, leaves, do)):
+            assert torch.equal(a, b)
+    static[3].data[0, 5, 1] = 0.25
+    graph.replay()
+    with pytest.raises(ValueError, match="g <= 0"):
+        torch.autograd.grad(o, static, do, retain_graph=True)
+    static[3].data[0, 5, 1] = -0.25
+    graph.replay()
+    torch.autograd.grad(o, static, do)
