@@ -14,9 +14,11 @@ Differences that a caller can observe, all additive:
 * head sizes up to 128 other than the built ones (K, V in {64, 128} and 32 x 32) are zero-padded along the head
   dimension to the next built shape and run on the same chunk kernels; larger heads take the token-serial kernel.
 """
+import collections
 import ctypes
 import math
 import struct
+import threading
 import warnings
 from typing import Optional
 
@@ -365,15 +367,46 @@ class _Kept:
     __slots__ = ("plan", "buffer", "flag", "done")
 
 
+class _InFlight:
+    """Pinned memory that queued kernels still write to, held until the event behind them has passed: torch's allocator does
+    not know of a kernel that was given the address of a block, and hands the block out again as soon as its tensor dies. One
+    queue per stream, oldest first; what has passed is let go at the next call, whichever thread makes it."""
+
+    def __init__(self):
+        self._lock, self._streams = threading.Lock(), {}
+
+    def hold(self, stream, memory, done):
+        with self._lock:
+            self._release()
+            self._streams.setdefault(stream, collections.deque()).append((memory, done))
+
+    def release(self):
+        with self._lock:
+            self._release()
+
+    def _release(self):
+        for stream in list(self._streams):
+            queue = self._streams[stream]
+            while queue and queue[0][1].query():
+                queue.popleft()
+            if not queue:
+                del self._streams[stream]
+
+
+_in_flight = _InFlight()
+
+
 def _written_heads(head):
     """The head sizes the training kernels write: the caller's own where they are multiples of 8, else the padded ones."""
     return tuple(n if n % 8 == 0 else 64 for n in head)
 
 
-def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm):
+def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm,
+                         watch_g=True):
     """The forward for inputs that require gradients: q, k, v padded from ``head`` = (K, V) to 64 x 64 heads -> (o with rows
-    of V elements, final state [N, HV, 64, 64], kept). The kernels note positive entries of g, but not while the stream is being
-    captured (a replay would write to a word of pinned memory, and waits for an event, that belong to the captured call)."""
+    of V elements, final state [N, HV, 64, 64], kept). ``watch_g``: have the kernels note positive entries of g; not while
+    the stream is being captured (a replay would write to a word of pinned memory, and waits for events, that belong to the
+    call that was captured)."""
     B, T, H, _ = q.shape
     HV = v.shape[2]
     cu_host = _sequence_bounds(cu_seqlens, B, T)
@@ -385,20 +418,23 @@ def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_fi
     n_saved = check(lib.lampa_gdr_train_saved_bytes(host_ptr, HV), "lampa_gdr_train_saved_bytes")
     ws_bytes = check(lib.lampa_gdr_train_workspace_bytes(host_ptr, HV), "lampa_gdr_train_workspace_bytes")
     kept.buffer = torch.empty(n_saved, dtype=torch.uint8, device=q.device)
-    watch_g = not torch.cuda.is_current_stream_capturing()
+    watch_g = watch_g and not torch.cuda.is_current_stream_capturing()
     kept.flag = torch.zeros(1, dtype=torch.int32, pin_memory=True) if watch_g else None
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     K, V = _written_heads(head)
     o = torch.empty((B, T, HV, V), dtype=v.dtype, device=v.device)
     ht = torch.empty((n_seq, HV, 64, 64), dtype=torch.float32, device=q.device) if output_final_state else None
     h0 = _pad_state(initial_state)
-    check(lib.lampa_gdr_chunk_fwd_train(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(o), ptr(h0), ptr(ht), host_ptr,
-                                        ptr(plan_dev), H, HV, K, V, _DTYPES[q.dtype], float(scale), l2norm,
-                                        ptr(kept.buffer), ptr(kept.flag), ptr(ws), ws_bytes, stream_of(q)),
-          "lampa_gdr_chunk_fwd_train")
-    if watch_g:
-        kept.done = torch.cuda.Event()
-        kept.done.record(torch.cuda.current_stream(q.device))
+    try:
+        check(lib.lampa_gdr_chunk_fwd_train(ptr(q), ptr(k), ptr(v), ptr(g), ptr(beta), ptr(o), ptr(h0), ptr(ht), host_ptr,
+                                            ptr(plan_dev), H, HV, K, V, _DTYPES[q.dtype], float(scale), l2norm,
+                                            ptr(kept.buffer), ptr(kept.flag), ptr(ws), ws_bytes, stream_of(q)),
+              "lampa_gdr_chunk_fwd_train")
+    finally:
+        if watch_g:
+            stream, kept.done = torch.cuda.current_stream(q.device), torch.cuda.Event()
+            kept.done.record(stream)
+            _in_flight.hold((q.device, stream.cuda_stream), kept.flag, kept.done)
     return _resize_heads((o,), (head[1],))[0], ht, kept
 
 
@@ -443,7 +479,7 @@ def _backward_chunk_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l
     backward pass over what it kept."""
     head = q.shape[-1], v.shape[-1]
     q, k, v, do = _resize_heads((q, k, v, do), (64, 64, 64, 64))
-    _, _, kept = _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, False, cu_seqlens, l2norm)
+    _, _, kept = _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, False, cu_seqlens, l2norm, watch_g=False)
     return _backward_kept_launch(q, k, v, head, kept, scale, l2norm, do, _pad_state(dht), initial_state is not None)
 
 
@@ -537,6 +573,7 @@ class _GatedDelta(torch.autograd.Function):
             if ctx.kept.flag is not None:
                 # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them
                 ctx.kept.done.synchronize()
+                _in_flight.release()
                 if int(ctx.kept.flag[0]):
                     _raise_positive_g()
         else:

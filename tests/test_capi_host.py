@@ -287,6 +287,70 @@ def test_gated_delta_shape_checks_come_before_any_gpu_work():
         gd.chunk_gated_delta_rule(q, q[:, :32], v, g, g)
 
 
+@pytest.fixture
+def training_calls(monkeypatch):
+    """The operator on CPU tensors without a GPU: launches return at once, events pass when the test says so, pinned memory is
+    ordinary memory. Returns the module and the list of events made."""
+    from lampa_amd import gated_delta as gd
+
+    class Event:
+        def __init__(self):
+            self.passed = False
+            events.append(self)
+
+        def record(self, stream):
+            pass
+
+        def query(self):
+            return self.passed
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *args: 64 if name.endswith("_bytes") else 0
+
+    events, zeros = [], torch.zeros
+    plan = torch.ones(8, dtype=torch.int32)
+    monkeypatch.setattr(gd, "_in_flight", gd._InFlight())
+    monkeypatch.setattr(gd, "require_cuda", lambda *tensors: None)
+    monkeypatch.setattr(gd, "stream_of", lambda t: 0)
+    monkeypatch.setattr(gd, "_plan", lambda *args: (plan, plan))
+    monkeypatch.setattr(gd._capi, "lib", Lib)
+    monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **kw: zeros(*a, **kw))
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: type("Stream", (), {"cuda_stream": 0}))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    return gd, events
+
+
+def _training_inputs():
+    return [torch.randn(1, 70, 2, 64).bfloat16().requires_grad_(True) for _ in range(3)] + [-torch.rand(1, 70, 2) for _ in "gb"]
+
+
+def test_flag_of_a_training_call_outlives_its_kernels(training_calls, monkeypatch):
+    """The word that the forward's kernel may write is not given back before that kernel has run, also when the graph is
+    dropped without a backward pass or the launch reports an error; afterwards it is."""
+    import weakref
+
+    gd, events = training_calls
+    flags, make = [], torch.zeros
+    monkeypatch.setattr(torch, "zeros", lambda *a, **kw: flags.append(make(*a, **kw)) or flags[-1])
+    gd.chunk_gated_delta_rule(*_training_inputs())
+    monkeypatch.setattr(gd, "check", lambda code, what: 64 if what.endswith("_bytes") else 1 / 0)
+    with pytest.raises(ZeroDivisionError):
+        gd.chunk_gated_delta_rule(*_training_inputs())
+    alive = [weakref.ref(f) for f in flags]
+    flags.clear()
+    assert len(alive) == len(events) == 2
+    gd._in_flight.release()
+    assert all(f() is not None for f in alive)
+    events[0].passed = True
+    gd._in_flight.release()
+    assert alive[0]() is None and alive[1]() is not None
+    events[1].passed = True
+    gd._in_flight.release()
+    assert alive[1]() is None and not gd._in_flight._streams
+
+
 def test_static_sort_symbols_and_limit():
     lib = _capi.lib()
     assert lib.lampa_sort_pairs_static_max_bytes() == 8 << 20

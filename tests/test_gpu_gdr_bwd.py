@@ -361,3 +361,22 @@ def test_forward_of_a_training_call_in_a_captured_graph(device):
     static[3].data[0, 5, 1] = -0.25
     graph.replay()
     torch.autograd.grad(o, static, do)
+
+
+def test_positive_g_of_a_dropped_graph_does_not_reach_the_next_call(device):
+    """Forwards that accept a positive g and are never differentiated, each followed at once by a training step on valid values,
+    with small pinned buffers made in between: the steps are not refused and the buffers stay as they are."""
+    make = lambda seed: [x.to(device) for x in _inputs(1, 20000, 2, 2, 64, 64, torch.bfloat16, seed, unit=False)[0]]
+    *bad, do = make(1)
+    bad[3] = bad[3].clone()
+    bad[3][0, -1, 1] = 0.25
+    bad = [x.requires_grad_(True) for x in bad]
+    good = [x.requires_grad_(True) for x in make(2)[:5]]
+    buffers = []
+    for _ in range(20):
+        gd.chunk_gated_delta_rule(*bad)
+        buffers.append(torch.zeros(1, dtype=torch.int32, pin_memory=True))
+        o, _ = gd.chunk_gated_delta_rule(*good)
+        torch.autograd.grad(o, good, do)
+    torch.cuda.synchronize()
+    assert not any(int(b) for b in buffers)
