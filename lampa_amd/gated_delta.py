@@ -526,11 +526,12 @@ def _backward_launch(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm,
 class _GatedDelta(torch.autograd.Function):
     """Forward through ``launcher``; backward through ``lampa_gdr_bwd`` (``ChunkGatedDeltaRuleFunction``,
     ``gated_delta_rule_ori.py:163-233``). ``differentiable=False`` keeps the reference's behaviour for the fused
-    recurrent operator, whose backward raises (``gated_delta_rule_ori.py:555-562``)."""
+    recurrent operator, whose backward raises (``gated_delta_rule_ori.py:555-562``). ``grad_mode``: whether the caller has
+    gradients enabled (inside ``forward`` they never are)."""
 
     @staticmethod
     def forward(ctx, launcher, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm,
-                differentiable):
+                differentiable, grad_mode):
         require_cuda(q, k, v, g, beta, initial_state)
         ctx.g_dtype, ctx.beta_dtype = g.dtype, beta.dtype
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
@@ -540,7 +541,9 @@ class _GatedDelta(torch.autograd.Function):
         ctx.set_materialize_grads(False)
         if differentiable:
             ctx.scale, ctx.l2norm, ctx.head = scale, l2norm, (q.shape[-1], v.shape[-1])
-            if (any(ctx.needs_input_grad) and launcher is _chunk_launch_any_head and _backward_chunk_supported(q, v)
+            # (`needs_input_grad` looks at the inputs alone: it is set for leaves under `no_grad` too)
+            if (grad_mode and any(ctx.needs_input_grad) and launcher is _chunk_launch_any_head
+                    and _backward_chunk_supported(q, v)
                     and q.shape[0] * q.shape[1] > 0):
                 K, V = ctx.head
                 q, k, v = _resize_heads((q, k, v), (64, 64, 64))
@@ -585,7 +588,7 @@ class _GatedDelta(torch.autograd.Function):
         dq, dk, dv, dg, dbeta, dh0 = grads
         if dh0 is not None:
             dh0 = dh0.to(initial_state.dtype)
-        return (None, dq, dk, dv, dg.to(ctx.g_dtype), dbeta.to(ctx.beta_dtype), None, dh0, None, None, None, None)
+        return (None, dq, dk, dv, dg.to(ctx.g_dtype), dbeta.to(ctx.beta_dtype), None, dh0, None, None, None, None, None)
 
 
 def _check_shapes(q, k, v, g, beta, what, headwise_beta_ok=False):
@@ -647,7 +650,7 @@ def chunk_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g:
     l2norm = L2_CHUNK if use_qk_l2norm_in_kernel else L2_NONE
     launcher = _chunk_launch_any_head if _chunk_path_supported(q, v) else _recurrent_launch
     o, final_state = _GatedDelta.apply(launcher, q, k, v, g, beta, scale, initial_state, output_final_state,
-                                       cu_seqlens, l2norm, True)
+                                       cu_seqlens, l2norm, True, torch.is_grad_enabled())
     return o.to(q.dtype), final_state
 
 
@@ -669,4 +672,4 @@ def fused_recurrent_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.
     _check_shapes(q, k, v, g, beta, "fused_recurrent_gated_delta_rule", headwise_beta_ok=True)
     l2norm = L2_RECURRENT if use_qk_l2norm_in_kernel else L2_NONE
     return _GatedDelta.apply(_recurrent_launch, q, k, v, g, beta, scale, initial_state, output_final_state,
-                             cu_seqlens, l2norm, False)
+                             cu_seqlens, l2norm, False, torch.is_grad_enabled())

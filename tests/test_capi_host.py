@@ -351,6 +351,23 @@ def test_flag_of_a_training_call_outlives_its_kernels(training_calls, monkeypatc
     assert alive[1]() is None and not gd._in_flight._streams
 
 
+@pytest.mark.parametrize("mode", [torch.no_grad, torch.inference_mode])
+def test_training_form_runs_only_where_gradients_can_be_asked_for(training_calls, monkeypatch, mode):
+    """Inputs that require gradients take the plain forward while gradients are disabled, and the training form otherwise."""
+    gd, _ = training_calls
+    taken = []
+    plain = lambda q, k, v, *rest: taken.append("plain") or (torch.zeros_like(v), None)
+    train = gd._chunk_train_forward
+    monkeypatch.setattr(gd, "_chunk_launch_any_head", plain)
+    monkeypatch.setattr(gd, "_chunk_train_forward", lambda *args: taken.append("train") or train(*args))
+    args = _training_inputs()
+    with mode():
+        o, _ = gd.chunk_gated_delta_rule(*args)
+        assert not o.requires_grad
+    o, _ = gd.chunk_gated_delta_rule(*args)
+    assert o.requires_grad and taken == ["plain", "train"]
+
+
 def test_static_sort_symbols_and_limit():
     lib = _capi.lib()
     assert lib.lampa_sort_pairs_static_max_bytes() == 8 << 20
