@@ -230,6 +230,7 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         return _ForwardOnly.apply(q, k, v, g, l, beta, scale, lam_div), None
     if initial_state is None:  # hattention_prefill, kernel.py:467-575
         require_cuda(q, k, v, g, l, beta)
+        k, v, g, l, beta = _rows_of(B, T, k=(k, H, K), v=(v, HV, V), g=(g, HV), l=(l, HV, L), beta=(beta, HV))
         hstate = HState(2, HType.WEAK, HStruct.GDELTA, (B, HV, K, V, L), torch.float32, q.device)
         T0 = T - T % 64
         if T0 < T:  # (the tail kernel reads the whole tensors)
@@ -269,14 +270,25 @@ def _check_chunk_shapes(T: int, K: int, V: int, L: int) -> None:
         raise NotImplementedError("hierarchical chunk kernels: at most 4096 chunks per sequence")
 
 
+def _rows_of(B: int, T: int, **tensors):
+    """The first B sequences and T tokens of tensors given as (tensor, sizes behind the tokens); a tensor that does not hold
+    them is refused here, since the kernels index it by these sizes."""
+    out = []
+    for name, (x, *rest) in tensors.items():
+        if tuple(x.shape) != (B, T, *rest):
+            x = x[:B, :T]
+            if tuple(x.shape) != (B, T, *rest):
+                raise ValueError(f"{name} must have shape {(B, T, *rest)}, got {tuple(x.shape)}")
+        out.append(x)
+    return out
+
+
 TAIL_MAX_K = 128  # ``lampa_hgdn_tail`` holds a state column in two registers per lane and level at most
 
 
 def _tail(hstate: HState, q, k, v, g, l, beta, o, t0: int, scale, lam_div) -> None:
     """Tokens ``t0 ..`` of contiguous ``[B, T, ...]`` tensors on the level states after the first ``t0`` tokens, in one
     launch: what ``_step`` does token by token. Writes rows ``t0 ..`` of ``o`` and updates ``hstate`` in place."""
-    if not all([q.ndim == 4, k.ndim == 4, v.ndim == 4, beta.ndim == 3, g.ndim == 3, l.ndim == 4]):
-        raise TypeError
     B, T, H, K = q.shape
     HV, V, L = v.shape[2], v.shape[3], l.shape[-1]
     # token t fills level 1 + the trailing zero bits of t: the largest power of two decides

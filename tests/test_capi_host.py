@@ -368,6 +368,35 @@ def test_training_form_runs_only_where_gradients_can_be_asked_for(training_calls
     assert o.requires_grad and taken == ["plain", "train"]
 
 
+@pytest.mark.parametrize("T", [10, 70])
+def test_prefill_refuses_tensors_that_do_not_hold_its_tokens(monkeypatch, T):
+    """The kernels index every operand by the sizes of q, v and l: a tensor with a token, a sequence or a head too few is
+    refused before any launch; of longer ones the first tokens count."""
+    from lampa_amd import hgdn
+
+    def launch(*args):
+        raise AssertionError("launched")
+
+    monkeypatch.setattr(hgdn, "require_cuda", lambda *tensors: None)
+    monkeypatch.setattr(hgdn._capi, "lib", launch)
+    q = torch.randn(2, T, 2, 64).bfloat16()
+    make = {"k": lambda B, T, H: torch.randn(B, T, H, 64).bfloat16(), "v": lambda B, T, H: torch.randn(B, T, H, 64).bfloat16(),
+            "g": torch.zeros, "beta": torch.zeros, "l": lambda B, T, H: torch.ones(B, T, H, 8)}
+    whole = {name: f(2, T, 2) for name, f in make.items()}
+    call = lambda **kw: hgdn.chunk_h_gated_delta_rule(q, **{**whole, **kw}, output_final_state=True,
+                                                      use_qk_l2norm_in_kernel=True)
+    for name, f in make.items():
+        sizes = [(2, T - 1, 2), (1, T, 2)] + ([] if name == "v" else [(2, T, 1)])  # (the heads of v are those of the rest)
+        for size in sizes:
+            with pytest.raises(ValueError, match=name):
+                call(**{name: f(*size)})
+    if T < 64:
+        seen = []
+        monkeypatch.setattr(hgdn, "_tail", lambda state, q, k, v, g, l, beta, o, *rest: seen.extend((k, v, g, l, beta, o)))
+        call(**{name: f(3, T + 5, 2) for name, f in make.items()})
+        assert all(x.shape[:3] == (2, T, 2) and x.is_contiguous() for x in seen)
+
+
 def test_static_sort_symbols_and_limit():
     lib = _capi.lib()
     assert lib.lampa_sort_pairs_static_max_bytes() == 8 << 20
