@@ -1786,7 +1786,10 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   } else if (is_m) {
     // M = dtot I + M': M' as bf16 A-operand fragments (rows = state rows, contraction over the columns in
     // accumulator slot order), element (row, col) -> fragment (row/32, col/16), lane 32*hh' + row%32, slot s
-    unsigned char* out = Mcomp + ((size_t)map * HV + hv) * (KT * KT * 2) + late;
+    // (a piece's M' is kept as value and remainder: gdr_scan2_kernel<PIECES>)
+    const bool parts = PIECES && gmax > 0;
+    using OT2 = typename OpVec<OT>::x2;
+    unsigned char* out = Mcomp + ((size_t)map * HV + hv) * ((parts ? 2 : 1) * KT * KT * 2) + late;
     const int mcol = 32 * wave + ln, ks = mcol >> 4, c16 = mcol & 15;
     const int hs = (c16 >> 2) & 1, slot = 4 * (c16 >> 3) + (c16 & 3);
 #pragma unroll
@@ -1795,8 +1798,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       for (int r = 0; r < 16; ++r) {
         const int row = 32 * km + acc_row(r, hh);
         const float val = S[km][r] - (row == mcol ? dtot : 0.0f);
-        *reinterpret_cast<OT*>(out + ((size_t)((km * (KT / 16) + ks) * 64 + 32 * hs + (row & 31))) * 16 + 2 * slot) =
-            (OT)val;
+        const size_t at = (size_t)((km * (KT / 16) + ks) * 64 + 32 * hs + (row & 31)) * 8 + slot;
+        if (parts) reinterpret_cast<OT2*>(out)[at] = OT2{(OT)val, (OT)(val - (float)(OT)val)};
+        else reinterpret_cast<OT*>(out)[at] = (OT)val;
       }
     if (wave == 0 && lane == 0) Dcomp[(size_t)map * HV + hv] = dtot;
     if constexpr (KEEP) {  // accumulator tiles read as A operand are the transpose
@@ -1941,7 +1945,11 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan_kernel(const GdrPlanV
 //          single-level scan writes).
 // Same step code in both modes; loops are branch free with clamped operands and a spare store slot as above.
 //   PIECES as GROUP, the groups being the segments that the composite pass cut into G pieces: every segment but the last
-//          of a sequence gets its composite, at the segment's own index.
+//          of a sequence gets its composite, at the segment's own index. Where a segment's chunks are walked in one go its
+//          M stays in fp32 accumulators and is rounded once, at the end; so that it is no different here, the pieces' M'
+//          come as two 16-bit parts (value and remainder), and so does the running composite as operand: three products
+//          per step. Rounding the pieces to 16 bits raised the error against float64 (16 448 tokens, bf16: 4.401e-3 ->
+//          4.406e-3 at a mean log-decay of 4e-4, now 4.400e-3); twice the bytes of M' cost 4 to 7 us of a call of 408 us.
 enum { SCAN_GROUP = 1, SCAN_LEAF = 2, SCAN_PIECES = 3 };
 
 // REV (GROUP): the segments of a sequence are taken from the last to the first (the maps of the backward pass).
@@ -1961,7 +1969,9 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
   constexpr int NKS = KT / 16;
   constexpr int M_BYTES = KT * KT * 2, N_BYTES = KT * 32 * 4;
   constexpr int NCB = COMPOSE ? (KT + VT) / 32 : VT / 32;  // 32-column blocks per item of the grid
-  __shared__ __align__(16) unsigned char s_x[2][NKS * 1024];
+  constexpr bool PARTS = MODE == SCAN_PIECES;
+  constexpr int NM = PARTS ? 2 * NKS : NKS;  // fragments of M' per step
+  __shared__ __align__(16) unsigned char s_x[2][NM * 1024];
   const int vn = blockIdx.x % NCB, j = blockIdx.x / NCB, seq = blockIdx.y, hv = blockIdx.z;
   const int seg0 = pv.seq_seg0[seq], nseg = pv.seq_nseg[seq];
   const int ngroups = MODE == SCAN_PIECES ? nseg : (nseg + G - 1) / G;
@@ -1991,16 +2001,24 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
       S[r] = h0[(((size_t)seq * HV + hv) * KT + 32 * wave + acc_row(r, hh)) * VT + 32 * vn + ln];
   }
 
-  X8 rm[DEPTH][NKS];
+  X8 rm[DEPTH][NM];
   f32x4 rn[DEPTH][4];
   float rd[DEPTH];
   auto issue = [&](int p, X8* m, f32x4* n, float& d) {
     const bool top = MODE == SCAN_LEAF && p < lead;  // a group composite (read through the *out pointers)
     const size_t sh = (size_t)(top ? seq * gmax + p : REV ? item0 - p : item0 + (p - lead)) * HV + hv;
-    const X8* M = reinterpret_cast<const X8*>((top ? Mout : Msrc) + sh * M_BYTES);
+    const X8* M = reinterpret_cast<const X8*>((top ? Mout : Msrc) + sh * (PARTS ? 2 * M_BYTES : M_BYTES));
     const f32x4* N = reinterpret_cast<const f32x4*>((top ? Nout : Nsrc) + (sh * (VT / 32) + nblk) * N_BYTES);
 #pragma unroll
-    for (int f = 0; f < NKS; ++f) m[f] = M[(wave * NKS + (2 * wave + f) % NKS) * 64 + lane];  // own fragments first
+    for (int f = 0; f < NKS; ++f) {  // own fragments first
+      const int at = (wave * NKS + (2 * wave + f) % NKS) * 64 + lane;
+      if constexpr (PARTS) {  // pairs of value and remainder: elements 0 - 3 and 4 - 7 until they are used
+        m[f] = M[2 * at];
+        m[NKS + f] = M[2 * at + 1];
+      } else {
+        m[f] = M[at];
+      }
+    }
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) n[q4] = N[(wave * 4 + q4) * 64 + lane];
     d = (top ? Dout : Dsrc)[sh];
@@ -2032,11 +2050,42 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
     for (int q4 = 0; q4 < 4; ++q4)
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[4 * q4 + e] = __builtin_fmaf(dec, S[4 * q4 + e], is_pm ? 0.0f : n[q4][e]);
+    X8 rest0, rest1;  // what own0 and own1 leave of S
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        rest0[e] = (OT)(S[e] - (float)own0[e]);
+        rest1[e] = (OT)(S[8 + e] - (float)own1[e]);
+      }
+      op_frag_store<OT>(xbuf, NKS + 2 * wave + 0, lane, rest0);
+      op_frag_store<OT>(xbuf, NKS + 2 * wave + 1, lane, rest1);
+    }
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int f = 0; f < NKS; ++f) {
+        const X8 lo = m[f], hi = m[NKS + f];
+        m[f] = __builtin_shufflevector(lo, hi, 0, 2, 4, 6, 8, 10, 12, 14);
+        m[NKS + f] = __builtin_shufflevector(lo, hi, 1, 3, 5, 7, 9, 11, 13, 15);
+      }
+    }
     acc = mfma32(m[0], own0, acc);
     acc = mfma32(m[1], own1, acc);
+    if constexpr (PARTS) {
+      acc = mfma32(m[0], rest0, acc);
+      acc = mfma32(m[1], rest1, acc);
+      acc = mfma32(m[NKS], own0, acc);
+      acc = mfma32(m[NKS + 1], own1, acc);
+    }
     lds_barrier();
 #pragma unroll
-    for (int f = 2; f < NKS; ++f) acc = mfma32(m[f], op_frag_load<OT>(xbuf, (2 * wave + f) % NKS, lane), acc);
+    for (int f = 2; f < NKS; ++f) {
+      const X8 x = op_frag_load<OT>(xbuf, (2 * wave + f) % NKS, lane);
+      acc = mfma32(m[f], x, acc);
+      if constexpr (PARTS) {
+        acc = mfma32(m[f], op_frag_load<OT>(xbuf, NKS + (2 * wave + f) % NKS, lane), acc);
+        acc = mfma32(m[NKS + f], x, acc);
+      }
+    }
     S = acc;
     issue(max(0, min(p + DEPTH, last)), m, n, dd);
   };

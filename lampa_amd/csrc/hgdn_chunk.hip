@@ -847,8 +847,8 @@ struct HgWorkspace {
 // longer than the prep kernel beside them: 220 + 17 us (scan) against 148 us at 60 032 tokens x 8 heads of 64 x 64 (15
 // segments of 64 chunks, 120 workgroups). While there are at most HG_PIECES_MAX_WGS workgroups (one per CU), segments of 64
 // and more chunks are cut into GDR_SCAN_GROUP pieces whose maps one more launch composes: the pieces take 59 us in front of
-// the prep kernel and the rest hides beside it. The call: 432 -> 411 us, with 128 value columns 792 -> 630 us, 40 000 x 6 x
-// 64 x 128 422 -> 347 us. Segments of 32 chunks take the same time either way (30 016 x 8: 240 / 240 us, 60 032 x 4: 259 /
+// the prep kernel and the rest hides beside it. The call: 430 -> 415 us, with 128 value columns 790 -> 629 us, 40 000 x 6 x
+// 64 x 128 422 -> 350 us. Segments of 32 chunks take the same time either way (30 016 x 8: 240 / 240 us, 60 032 x 4: 259 /
 // 261 us), those of 16 are faster whole (15 000 x 8: 208 against 220 us).
 #define HG_PIECES_MAX_WGS 256
 #define HG_PIECES_MIN_LOG2 6
@@ -869,7 +869,7 @@ static HgWorkspace hg_workspace(int64_t chunks, int64_t segs, int HV, int K, int
   // the maps of the pieces (hg_pieces; fewer chunks make no two segments that long)
   const int64_t pieces =
       chunks > (1 << HG_PIECES_MIN_LOG2) && hg_pieces(segs, HV, HG_PIECES_MIN_LOG2) ? segs * GDR_SCAN_GROUP : 0;
-  w.off_pm = off;  off += lampa_align_up(pieces * HV * (int64_t)K * K * 2, 256);
+  w.off_pm = off;  off += lampa_align_up(pieces * HV * (int64_t)K * K * 4, 256);  // M' in two 16-bit parts
   w.off_pn = off;  off += lampa_align_up(pieces * HV * (int64_t)K * V * 4, 256);
   w.off_pd = off;  off += lampa_align_up(pieces * HV * 4, 256);
   w.bytes = off > 0 ? off : 256;
