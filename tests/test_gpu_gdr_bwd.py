@@ -380,3 +380,43 @@ def test_positive_g_of_a_dropped_graph_does_not_reach_the_next_call(device):
         torch.autograd.grad(o, good, do)
     torch.cuda.synchronize()
     assert not any(int(b) for b in buffers)
+
+
+@pytest.mark.parametrize("lens", [[64 * 40 + 7, 0, 1, 64 * 16, 700], [33]])
+def test_c_entry_from_the_inputs_alone(device, lens, monkeypatch):
+    """``lampa_gdr_bwd_chunk`` with its own plan (segments of 16 chunks) and exactly the workspace it asks for: the bits of the
+    operator's gradients on the same segments, nothing written behind the workspace; with and without states."""
+    import ctypes
+
+    from lampa_amd import _capi
+
+    lib, ptr = _capi.lib(), _capi.ptr
+    T, n = sum(lens), len(lens)
+    (q, k, v, g, beta, do), gen = _inputs(1, T, 3, 3, 64, 64, torch.bfloat16, n, unit=False, g_scale=0.05)
+    q, k, v, g, beta, do, h0, dht = (x.to(device) for x in (q, k, v, g, beta, do, 0.5 * torch.randn(n, 3, 64, 64, generator=gen),
+                                                            torch.randn(n, 3, 64, 64, generator=gen)))
+    bounds = [0] + torch.tensor(lens).cumsum(0).tolist()
+    cu = (ctypes.c_int64 * (n + 1))(*bounds)
+    plan = torch.zeros(_capi.check(lib.lampa_gdr_bwd_chunk_plan_size(cu, n), "plan_size"), dtype=torch.int32)
+    host = ctypes.c_void_p(plan.data_ptr())
+    _capi.check(lib.lampa_gdr_bwd_chunk_plan_fill(cu, n, host), "plan_fill")
+    plan_dev = plan.to(device)
+    n_bytes = _capi.check(lib.lampa_gdr_bwd_chunk_workspace_bytes(host, 3), "workspace_bytes")
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 16)
+    for states in (True, False):
+        ws = torch.full((n_bytes + 65536,), 0xA5, dtype=torch.uint8, device=device)
+        s0, ds = (h0, dht) if states else (None, None)
+        got = [torch.empty_like(x) for x in (q, k, v, g, beta)] + [torch.empty_like(h0) if states else None]
+        _capi.check(lib.lampa_gdr_bwd_chunk(*(ptr(x) for x in (q, k, v, g, beta, s0, do, ds, *got)), host, ptr(plan_dev), 3, 3,
+                                            64, 64, 0, 0.2, gd.L2_CHUNK, ptr(ws), n_bytes, _capi.stream_of(q)), "bwd_chunk")
+        assert bool((ws[n_bytes:] == 0xA5).all())
+        leaves = [x.detach().clone().requires_grad_(True) for x in (q, k, v, g, beta)] + ([h0.clone().requires_grad_(True)] * states)
+        o, ht = gd.chunk_gated_delta_rule(*leaves[:5], scale=0.2, initial_state=leaves[5] if states else None,
+                                          output_final_state=states, cu_seqlens=torch.tensor(bounds, device=device),
+                                          use_qk_l2norm_in_kernel=True)
+        want = torch.autograd.grad((o, ht), leaves, (do, dht)) if states else torch.autograd.grad(o, leaves, do)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    short = ptr(ws), n_bytes - 1
+    assert lib.lampa_gdr_bwd_chunk(*(ptr(x) for x in (q, k, v, g, beta, None, do, None, *got)), host, ptr(plan_dev), 3, 3, 64,
+                                   64, 0, 0.2, gd.L2_CHUNK, *short, _capi.stream_of(q)) == -2
