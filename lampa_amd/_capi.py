@@ -147,8 +147,8 @@ def ptr(t):
 
 
 # The handle of the current stream without a ``torch.cuda.Stream`` around it, which costs 5 us (a whole call on a few tokens
-# takes 15).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# takes 15). A torch built without GPU support does not have it; the package imports there all the same.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_of(t: torch.Tensor):

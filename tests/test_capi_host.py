@@ -250,6 +250,15 @@ def test_head_resize_refuses_what_it_cannot_copy(lib):
     assert call(16, 256, rows=1 << 40) == -4  # more rows than a launch has workgroups for
 
 
+def test_package_imports_on_a_torch_without_gpu_support():
+    import subprocess
+    import sys
+
+    code = ("import torch\nif hasattr(torch._C, '_cuda_getCurrentRawStream'): del torch._C._cuda_getCurrentRawStream\n"
+            "from lampa_amd import block, gated_delta, hept, hgdn, layer_ops, lsh, synth")
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True)
+
+
 def test_operators_refuse_cpu_tensors():
     from lampa_amd import gated_delta as gd
     from lampa_amd import lsh
