@@ -26,18 +26,22 @@ __global__ void __launch_bounds__(256) head_resize_kernel(const HrArgs a) {
   if (r >= per_pass) return;
   const P* src = reinterpret_cast<const P*>(a.src[t]);
   P* dst = reinterpret_cast<P*>(a.dst[t]);
-  const int64_t rows = a.rows[t], first = (int64_t)blockIdx.x * (per_pass * HR_ROWS) + r;
-  P x[HR_ROWS];
+  const int64_t rows = a.rows[t];
+  // (one round, but for tensors of more rows than a grid holds)
+  for (int64_t first = (int64_t)blockIdx.x * (per_pass * HR_ROWS) + r; first < rows;
+       first += (int64_t)gridDim.x * (per_pass * HR_ROWS)) {
+    P x[HR_ROWS];
 #pragma unroll
-  for (int i = 0; i < HR_ROWS; ++i) {
-    const int64_t row = first + (int64_t)i * per_pass;
-    x[i] = P{};
-    if (c < ws && row < rows) x[i] = src[row * ws + c];
-  }
+    for (int i = 0; i < HR_ROWS; ++i) {
+      const int64_t row = first + (int64_t)i * per_pass;
+      x[i] = P{};
+      if (c < ws && row < rows) x[i] = src[row * ws + c];
+    }
 #pragma unroll
-  for (int i = 0; i < HR_ROWS; ++i) {
-    const int64_t row = first + (int64_t)i * per_pass;
-    if (row < rows) dst[row * wd + c] = x[i];
+    for (int i = 0; i < HR_ROWS; ++i) {
+      const int64_t row = first + (int64_t)i * per_pass;
+      if (row < rows) dst[row * wd + c] = x[i];
+    }
   }
 }
 
@@ -74,7 +78,7 @@ extern "C" int lampa_head_resize(int n, const lampa_head_copy* copies, void* str
     blocks = b > blocks ? b : blocks;
   }
   if (blocks == 0) return LAMPA_OK;
-  if (blocks > INT32_MAX / 256) return LAMPA_ERR_UNSUPPORTED;  // (a grid holds fewer than 2^31 threads per dimension here)
+  if (blocks > INT32_MAX / 256) blocks = INT32_MAX / 256;  // (a grid holds fewer than 2^31 threads per dimension here)
   const dim3 grid((unsigned)blocks, n);
   if (piece == 8)
     hipLaunchKernelGGL(head_resize_kernel<hr_u32x4>, grid, dim3(256), 0, (hipStream_t)stream, a);

@@ -307,6 +307,16 @@ def test_resized_heads_are_padded_and_cut_copies(device, rows, widths, offset):
         assert y.is_contiguous() and torch.equal(y.view(torch.int16), want)
 
 
+def test_resized_heads_of_more_rows_than_a_grid_holds(device):
+    """Rows of 129 elements, one at a time: four rows to a workgroup, and 4 (2^23 - 1) rows to a grid."""
+    rows = 4 * (2 ** 23 - 1) + 9
+    src = torch.arange(rows, device=device).to(torch.int16).view(torch.bfloat16).view(1, rows, 1)
+    dst = gd._resize_heads((src,), (129,))[0].view(torch.int16)
+    assert torch.equal(dst[..., :1], src.view(torch.int16))
+    for a in range(0, rows, 2 ** 22):
+        assert not bool(dst[:, a:a + 2 ** 22, 1:].any())
+
+
 @pytest.mark.parametrize("K,V,H,HV", [(8, 8, 2, 2), (16, 32, 3, 3), (48, 56, 1, 2), (64, 24, 2, 2), (20, 64, 2, 2), (40, 30, 1, 1)])
 def test_small_heads_are_written_in_their_own_width(device, K, V, H, HV):
     """Output, final state and gradients of heads below 64 x 64 (in sizes the kernels write themselves and in sizes that are
