@@ -682,9 +682,20 @@ extern "C" int lampa_hgdn_tail(const void* q, const void* k, const void* v, cons
     if (1 + __builtin_ctz(t) >= L) return LAMPA_ERR_INVALID;
   hipStream_t s = (hipStream_t)stream;
   LAMPA_PROF(s, "start");
-#define HGS_TAIL(TT, LM, RR)                                                                                              hipLaunchKernelGGL((hgdn_tail_kernel<TT, LM, RR>), dim3(B * HV, (V + HGS_TAIL_WAVES - 1) / HGS_TAIL_WAVES),                                  dim3(64 * HGS_TAIL_WAVES), 0, s, (const TT*)q, (const TT*)k, (const TT*)v, g, beta, lam, lam_dtype,                      lam_div, states, (TT*)o, n_tok, tok0, H, HV, K, V, L, scale, l2norm)
-#define HGS_TAIL_ROWS(TT, LM)             do {                                      if (K <= 64) HGS_TAIL(TT, LM, 1);       else HGS_TAIL(TT, LM, 2);             } while (0)
-#define HGS_TAIL_CASE(TT)                                              do {                                                                   if (L <= HGS_TAIL_LEVELS) HGS_TAIL_ROWS(TT, HGS_TAIL_LEVELS);        else HGS_TAIL_ROWS(TT, HGS_LMAX);                                  } while (0)
+#define HGS_TAIL(TT, LM, RR)                                                                                               \
+  hipLaunchKernelGGL((hgdn_tail_kernel<TT, LM, RR>), dim3(B * HV, (V + HGS_TAIL_WAVES - 1) / HGS_TAIL_WAVES),              \
+                     dim3(64 * HGS_TAIL_WAVES), 0, s, (const TT*)q, (const TT*)k, (const TT*)v, g, beta, lam, lam_dtype,   \
+                     lam_div, states, (TT*)o, n_tok, tok0, H, HV, K, V, L, scale, l2norm)
+#define HGS_TAIL_ROWS(TT, LM)         \
+  do {                                \
+    if (K <= 64) HGS_TAIL(TT, LM, 1); \
+    else HGS_TAIL(TT, LM, 2);         \
+  } while (0)
+#define HGS_TAIL_CASE(TT)                                          \
+  do {                                                             \
+    if (L <= HGS_TAIL_LEVELS) HGS_TAIL_ROWS(TT, HGS_TAIL_LEVELS);  \
+    else HGS_TAIL_ROWS(TT, HGS_LMAX);                              \
+  } while (0)
   if (dtype == GDR_BF16) HGS_TAIL_CASE(__bf16);
   else if (dtype == GDR_FP16) HGS_TAIL_CASE(_Float16);
   else HGS_TAIL_CASE(float);
