@@ -9,6 +9,7 @@
 #include "common.h"
 
 #define HR_MAX 4
+#define HR_MAX_ELEMENTS (INT64_C(1) << 40)  // far more than any memory holds: no tensor
 #define HR_ROWS 4  // rows per thread: their loads are in flight together
 
 struct HrArgs {
@@ -64,6 +65,7 @@ extern "C" int lampa_head_resize(int n, const lampa_head_copy* copies, void* str
     const lampa_head_copy& c = copies[i];
     if (!c.src || !c.dst || c.rows < 0) return LAMPA_ERR_INVALID;
     if (c.src_width < 1 || c.dst_width < 1 || c.src_width > 256 || c.dst_width > 256) return LAMPA_ERR_UNSUPPORTED;
+    if (c.rows > HR_MAX_ELEMENTS / 256) return LAMPA_ERR_UNSUPPORTED;
     if (((uintptr_t)c.src | (uintptr_t)c.dst) & 1) return LAMPA_ERR_INVALID;
     if ((c.src_width | c.dst_width) % 8 || (((uintptr_t)c.src | (uintptr_t)c.dst) & 15)) piece = 1;
   }

@@ -247,7 +247,7 @@ def test_head_resize_refuses_what_it_cannot_copy(lib):
     assert call(16, 64, address=0) == -1 and call(16, 64, address=(1 << 20) + 1) == -1
     assert call(0, 64) == -4 and call(16, 257) == -4 and call(257, 64) == -4
     assert call(16, 64, rows=0) == 0
-    assert call(16, 256, rows=1 << 40) == -4  # more rows than a launch has workgroups for
+    assert call(16, 256, rows=1 << 40) == -4  # more elements than any memory holds
 
 
 def test_package_imports_on_a_torch_without_gpu_support():
