@@ -65,7 +65,7 @@ extern "C" int lampa_head_resize(int n, const lampa_head_copy* copies, void* str
     const lampa_head_copy& c = copies[i];
     if (!c.src || !c.dst || c.rows < 0) return LAMPA_ERR_INVALID;
     if (c.src_width < 1 || c.dst_width < 1 || c.src_width > 256 || c.dst_width > 256) return LAMPA_ERR_UNSUPPORTED;
-    if (c.rows > HR_MAX_ELEMENTS / 256) return LAMPA_ERR_UNSUPPORTED;
+    if (c.rows > HR_MAX_ELEMENTS / (c.src_width > c.dst_width ? c.src_width : c.dst_width)) return LAMPA_ERR_UNSUPPORTED;
     if (((uintptr_t)c.src | (uintptr_t)c.dst) & 1) return LAMPA_ERR_INVALID;
     if ((c.src_width | c.dst_width) % 8 || (((uintptr_t)c.src | (uintptr_t)c.dst) & 15)) piece = 1;
   }
