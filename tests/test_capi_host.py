@@ -406,6 +406,27 @@ def test_prefill_refuses_tensors_that_do_not_hold_its_tokens(monkeypatch, T):
         assert all(x.shape[:3] == (2, T, 2) and x.is_contiguous() for x in seen)
 
 
+def test_single_tokens_of_large_states_take_the_step(monkeypatch):
+    """The tail kernel takes more than twice the step's time for one token on a large state, and less from two tokens on."""
+    from lampa_amd import hgdn
+
+    taken = []
+    monkeypatch.setattr(hgdn, "require_cuda", lambda *tensors: None)
+    monkeypatch.setattr(hgdn, "_step", lambda state, q, k, v, *rest, **kw: taken.append("step") or torch.zeros_like(v))
+    monkeypatch.setattr(hgdn, "_tail", lambda *args: taken.append("tail"))
+    monkeypatch.setattr(hgdn._ForwardOnly, "apply", lambda q, k, v, *rest: torch.zeros(v.shape[0], rest[-1], *v.shape[2:]))
+
+    def route(B, T, L=8):
+        q, v = torch.zeros(B, T, 8, 64, dtype=torch.bfloat16), torch.zeros(B, T, 8, 64, dtype=torch.bfloat16)
+        gate, lam = torch.zeros(B, T, 8), torch.zeros(B, T, 8, L)
+        o, _ = hgdn.chunk_h_gated_delta_rule(q, q, v, gate, lam, gate, output_final_state=True, use_qk_l2norm_in_kernel=True)
+        assert o.shape == v.shape
+        return taken.pop()
+
+    assert [route(7, 1), route(8, 1), route(31, 65), route(32, 65), route(32, 2), route(64, 66)] == [
+        "tail", "step", "tail", "step", "tail", "tail"]
+
+
 def test_static_sort_symbols_and_limit():
     lib = _capi.lib()
     assert lib.lampa_sort_pairs_static_max_bytes() == 8 << 20

@@ -359,3 +359,17 @@ def test_interleaved_calls_on_two_streams(device):
             assert torch.equal(o, ref[i])  # same kernels, same data: bit-identical whatever runs beside them
         max_abs, mean_rel = _errors(ref[i], alone[i].cpu())
         assert max_abs <= MAX_ABS and mean_rel <= MEAN_REL
+
+
+@pytest.mark.parametrize("T,K,V", [(1, 64, 64), (65, 64, 64), (65, 32, 96), (1, 160, 32)])
+def test_single_token_by_the_step_and_by_the_tail_kernel(device, T, K, V, monkeypatch):
+    """One token alone or behind a chunk: both routes give the same output, states (fp32 sums in another order) and counts."""
+    q, k, v, g, beta, lam = (x.to(device) for x in _inputs(2, T, 2, K, V, torch.bfloat16, T + K, L=9))
+    out = []
+    for limits in ((0, 0), (2 ** 60, 2 ** 60)):
+        monkeypatch.setattr(hgdn, "ONE_TOKEN_STEP", limits)
+        out.append(hgdn.chunk_h_gated_delta_rule(q, k, v, g, lam, beta, output_final_state=True, use_qk_l2norm_in_kernel=True))
+    (o, s), (o2, s2) = out
+    assert o.shape == v.shape and torch.equal(s.counts, s2.counts)
+    assert torch.allclose(s.states, s2.states, rtol=1e-5, atol=1e-6)
+    assert torch.allclose(o.float(), o2.float(), rtol=2 ** -7, atol=1e-5)          # one rounding to bf16 of sums that differ
