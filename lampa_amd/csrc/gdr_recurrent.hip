@@ -261,11 +261,10 @@ __global__ void __launch_bounds__(64)
 #pragma unroll
         for (int c4 = 0; c4 < KT / 4; ++c4) {
           const float4 a = s_kq[buf][lane * ROW4 + c4];
+          float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // (read in front of the sums: 85 us, behind kss 89 us at
+          if constexpr (!COMPOSITE) b = s_kq[buf][lane * ROW4 + KT / 4 + c4];  // 128 x 64 tokens x 8 heads of 64 x 64, bf16)
           kss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
-          if constexpr (!COMPOSITE) {
-            const float4 b = s_kq[buf][lane * ROW4 + KT / 4 + c4];
-            qss += b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
-          }
+          qss += b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
         }
         float kinv = 1.0f, qinv = 1.0f;
         if (l2norm == GDR_L2_CHUNK) {
