@@ -296,7 +296,9 @@ def test_chunked_gradients_at_full_size_against_the_token_serial_form(device, mo
 
 @pytest.mark.parametrize("rows,widths,offset", [(1, ((16, 64),), 0), (1023, ((16, 64), (64, 24), (32, 64)), 0),
                                                 (2049, ((10, 32), (6, 64), (128, 5), (64, 1)), 0),
-                                                (777, ((16, 64), (64, 16)), 1), (64, ((256, 8), (8, 256)), 0)])
+                                                (777, ((16, 64), (64, 16)), 1), (64, ((256, 8), (8, 256)), 0),
+                                                (1000, ((100, 128), (20, 64)), 0), (515, ((66, 128), (128, 30)), 0),
+                                                (4097, ((127, 128), (65, 256), (256, 255), (3, 1)), 0), (999, ((2, 3), (64, 2)), 2)])
 def test_resized_heads_are_padded_and_cut_copies(device, rows, widths, offset):
     """Bit for bit what torch's pad and slice give: last blocks of rows, odd widths and odd addresses (one element per
     thread), widths that do not divide a workgroup."""
@@ -307,9 +309,9 @@ def test_resized_heads_are_padded_and_cut_copies(device, rows, widths, offset):
         assert y.is_contiguous() and torch.equal(y.view(torch.int16), want)
 
 
-def test_resized_heads_of_more_rows_than_a_grid_holds(device):
-    """Rows of 129 elements, one at a time: four rows to a workgroup, and 4 (2^23 - 1) rows to a grid."""
-    rows = 4 * (2 ** 23 - 1) + 9
+def test_resized_heads_of_more_rows_than_one_turn_of_the_grid(device):
+    """Rows of 129 elements, one at a time: 31 rows to a workgroup, and 2^20 workgroups."""
+    rows = 31 * 2 ** 20 + 9
     src = torch.arange(rows, device=device).to(torch.int16).view(torch.bfloat16).view(1, rows, 1)
     dst = gd._resize_heads((src,), (129,))[0].view(torch.int16)
     assert torch.equal(dst[..., :1], src.view(torch.int16))
