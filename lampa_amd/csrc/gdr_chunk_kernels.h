@@ -1949,7 +1949,9 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan_kernel(const GdrPlanV
 //          M stays in fp32 accumulators and is rounded once, at the end; so that it is no different here, the pieces' M'
 //          come as two 16-bit parts (value and remainder), and so does the running composite as operand: three products
 //          per step. Rounding the pieces to 16 bits raised the error against float64 (16 448 tokens, bf16: 4.401e-3 ->
-//          4.406e-3 at a mean log-decay of 4e-4, now 4.400e-3); twice the bytes of M' cost 4 to 7 us of a call of 408 us.
+//          4.406e-3 at a mean log-decay of 4e-4, now 4.400e-3); twice the bytes of M' cost 2 to 3 us of a call of 409 us. Two
+//          maps are loaded ahead, not four, and one exchange buffer does: with the registers of four (136 against 56) the
+//          workgroups found no room beside the kernel they run next to until its end (415 us).
 enum { SCAN_GROUP = 1, SCAN_LEAF = 2, SCAN_PIECES = 3 };
 
 // REV (GROUP): the segments of a sequence are taken from the last to the first (the maps of the backward pass).
@@ -1971,7 +1973,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
   constexpr int NCB = COMPOSE ? (KT + VT) / 32 : VT / 32;  // 32-column blocks per item of the grid
   constexpr bool PARTS = MODE == SCAN_PIECES;
   constexpr int NM = PARTS ? 2 * NKS : NKS;  // fragments of M' per step
-  __shared__ __align__(16) unsigned char s_x[2][NM * 1024];
+  __shared__ __align__(16) unsigned char s_x[PARTS ? 1 : 2][NM * 1024];
   const int vn = blockIdx.x % NCB, j = blockIdx.x / NCB, seq = blockIdx.y, hv = blockIdx.z;
   const int seg0 = pv.seq_seg0[seq], nseg = pv.seq_nseg[seq];
   const int ngroups = MODE == SCAN_PIECES ? nseg : (nseg + G - 1) / G;
@@ -2041,7 +2043,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
     }
     const float dec = dd;
     dprod *= dec;
-    unsigned char* xbuf = s_x[p & 1];
+    unsigned char* xbuf = s_x[PARTS ? 0 : p & 1];
     const X8 own0 = acc_to_op<OT>(S, 0), own1 = acc_to_op<OT>(S, 8);
     op_frag_store<OT>(xbuf, 2 * wave + 0, lane, own0);
     op_frag_store<OT>(xbuf, 2 * wave + 1, lane, own1);
@@ -2086,6 +2088,7 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
         acc = mfma32(m[NKS + f], x, acc);
       }
     }
+    if constexpr (PARTS) lds_barrier();  // (one buffer: it has been read)
     S = acc;
     issue(max(0, min(p + DEPTH, last)), m, n, dd);
   };

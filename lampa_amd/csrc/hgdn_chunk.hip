@@ -847,7 +847,7 @@ struct HgWorkspace {
 // longer than the prep kernel beside them: 220 + 17 us (scan) against 148 us at 60 032 tokens x 8 heads of 64 x 64 (15
 // segments of 64 chunks, 120 workgroups). While there are at most HG_PIECES_MAX_WGS workgroups (one per CU), segments of 64
 // and more chunks are cut into GDR_SCAN_GROUP pieces whose maps one more launch composes: the pieces take 59 us in front of
-// the prep kernel and the rest hides beside it. The call: 430 -> 415 us, with 128 value columns 790 -> 629 us, 40 000 x 6 x
+// the prep kernel and the rest hides beside it. The call: 430 -> 412 us, with 128 value columns 790 -> 629 us, 40 000 x 6 x
 // 64 x 128 422 -> 350 us. Segments of 32 chunks take the same time either way (30 016 x 8: 240 / 240 us, 60 032 x 4: 259 /
 // 261 us), those of 16 are faster whole (15 000 x 8: 208 against 220 us).
 #define HG_PIECES_MAX_WGS 256
@@ -959,7 +959,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   LAMPA_PROF(s, "hgdn_prep_kernel");
   if (split) {
     if (pieces) {
-      hipLaunchKernelGGL((gdr_scan2_kernel<__bf16, KT, VT, 4, SCAN_PIECES>), dim3((KT + VT) / 32 * max_nseg, n_seq, HV),
+      hipLaunchKernelGGL((gdr_scan2_kernel<__bf16, KT, VT, 2, SCAN_PIECES>), dim3((KT + VT) / 32 * max_nseg, n_seq, HV),
                          dim3(64 * (KT / 32)), 0, cs, pv, ws + w.off_pm, ws + w.off_pn, (const float*)(ws + w.off_pd),
                          (const float*)nullptr, (float*)nullptr, Mc, Nm, Dc, HV, 0, 0);
       LAMPA_PROF(s, "gdr_scan2_kernel<pieces>");
