@@ -530,7 +530,8 @@ def main():
     del d4
 
     # ---- backward pass of the layer at the headline shape and at the reference model's head sizes: the chunked form on
-    #      the MFMA (lampa_gdr_bwd_chunk) and, beside it, the fp32 token-serial form (lampa_gdr_bwd) ----
+    #      the MFMA (lampa_gdr_chunk_fwd_train, then lampa_gdr_bwd_saved) and, beside it, the fp32 token-serial form
+    #      (lampa_gdr_bwd) ----
     def backward_leg(T_, H_, K_, V_, dtype_):
         qb, kb, vb, gb_, bb = (x.to(dev) for x in synth.gdr_inputs(1, T_, H_, K_, V_, dtype_, seed=0))
         dob = torch.randn_like(vb)

@@ -304,11 +304,12 @@ int lampa_gdr_bwd(const void* q, const void* k, const void* v, const float* g, c
  * lampa_gdr_chunk_fwd_train is lampa_gdr_chunk_fwd (the same plan, the same o and ht) and also fills `saved`
  * (lampa_gdr_train_saved_bytes: about 13.6 KB per chunk and head -- its record and the state in front of it in the 16-bit
  * input type -- and 8 KB per segment and head). positive_g_host (nullable): an int32 in pinned host memory, zeroed by the
- * caller, becomes 1 when an entry of g is positive (to be read once the call's kernels have run).
+ * caller, becomes 1 when an entry of g is positive (to be read, and not to be freed or used otherwise, before the call's
+ * kernels have run; NULL in a captured graph, whose replays would go on writing to it).
  * lampa_gdr_bwd_saved computes the gradients from q, k, v and `saved`: the gradient of the state is walked from the last
  * chunk of every segment to its first, segments in parallel, as the forward pass walks the state. dq and dk have one row
  * per VALUE head, [tokens, HV, 64]: with grouped value heads the caller sums them over each group. dht, dh0 nullable.
- * `saved` is only read; workspace: about 24 KB per segment and head.
+ * `saved` is only read; workspace: about 19 KB per segment and head.
  * Smaller heads are padded to 64 x 64 by the caller (zero columns of q, k, v, dout; lampa_head_resize), K and V (multiples of
  * 8, at most 64) are their sizes: o and dv then have rows of V, dq and dk rows of K elements. */
 int64_t lampa_gdr_train_saved_bytes(const int32_t* plan_host, int HV);

@@ -4,8 +4,8 @@ the gradient oracle (``oracle.gated_delta_bwd.backward_manual``, float64 on the 
 Tolerances: the token-serial kernels (``lampa_gdr_bwd``) compute in fp32 from the inputs as given, so fp32 inputs must
 agree to 1e-4 (max-abs relative to the largest entry of the gradient; 1e-5 mean-relative); with bf16 / fp16 inputs dq,
 dk and dv are rounded to that type on output (mean-relative 5e-3, the forward's bound), dg, dbeta and d(initial state)
-stay fp32 (1e-4). The chunked form (``lampa_gdr_bwd_chunk``: 16-bit inputs, K = V = 64, one value head per q/k head)
-rounds every MFMA operand to the input type, as the reference's backward kernels do: all six gradients then carry that
+stay fp32 (1e-4). The chunked form (``lampa_gdr_chunk_fwd_train`` and ``lampa_gdr_bwd_saved``: 16-bit inputs, heads up to
+64 x 64) rounds every MFMA operand to the input type, as the reference's backward kernels do: all six gradients then carry that
 type's rounding through a chain of five to six rounded intermediates (max-abs 2e-2 of the largest entry; mean-relative
 8e-3; measured 3e-3 to 5.2e-3 for bf16, 5e-4 for fp16).
 """
@@ -203,8 +203,8 @@ def test_backward_refuses_positive_log_decay(device):
 @pytest.mark.parametrize("l2", [False, True])
 @pytest.mark.parametrize("T", [1, 64, 75, 1000])
 def test_chunked_gradients_match_oracle(device, dtype, l2, T):
-    """K = V = 64, H = HV, 16-bit inputs take ``lampa_gdr_bwd_chunk``: batches with an initial state and a gradient into
-    the final state; one token, one chunk, a partial second chunk, 16 chunks (two levels of the scan)."""
+    """K = V = 64, 16-bit inputs take the chunked form: batches with an initial state and a gradient into the final state; one
+    token, one chunk, a partial second chunk, 16 chunks in four segments."""
     assert gd._backward_chunk_supported(torch.empty(1, 1, 2, 64, dtype=dtype), torch.empty(1, 1, 2, 64, dtype=dtype))
     (q, k, v, g, beta, do), gen = _inputs(2, T, 2, 2, 64, 64, dtype, T, unit=not l2)
     h0 = 0.5 * torch.randn(2, 2, 64, 64, generator=gen)
@@ -214,8 +214,8 @@ def test_chunked_gradients_match_oracle(device, dtype, l2, T):
 
 
 def test_chunked_gradients_varlen_and_without_states(device):
-    """Packed sequences (an empty one, one token, lengths off the chunk size, one of 80 chunks: three levels of the
-    scan) with states; then no initial state and no gradient into the final state; then a loss on the final state only."""
+    """Packed sequences (an empty one, one token, lengths off the chunk size, one of 80 chunks in 20
+    segments) with states; then no initial state and no gradient into the final state; then a loss on the final state only."""
     lens = [0, 5, 333, 64, 1, 5100, 97]
     T = sum(lens)
     (q, k, v, g, beta, do), gen = _inputs(1, T, 3, 3, 64, 64, torch.bfloat16, 7, unit=False, g_scale=0.3)
@@ -235,7 +235,7 @@ def test_chunked_gradients_varlen_and_without_states(device):
 
 
 def test_chunked_gradients_long_sequence_weak_decay_against_oracle(device):
-    """16 448 tokens (257 chunks + the extra item: three levels of the scan, a ragged last group) with g of the order of
+    """16 448 tokens (257 chunks in 65 segments: groups of 8 and a remainder of one) with g of the order of
     -0.003 per token, so that states and their gradients carry over thousands of tokens, against the float64 loop."""
     (q, k, v, g, beta, do), gen = _inputs(1, 16448, 2, 2, 64, 64, torch.bfloat16, 11, unit=True, g_scale=0.003)
     h0 = 0.5 * torch.randn(1, 2, 64, 64, generator=gen)
@@ -265,6 +265,17 @@ def test_chunked_gradients_one_chunk_per_segment(device, T, K, V, monkeypatch):
     for _ in range(2):
         got = torch.autograd.grad((o, ht), leaves, (do.to(device), dht.to(device)), retain_graph=True)
         _check(got, want, torch.bfloat16, chunked=True)
+
+
+def test_chunked_gradients_of_a_long_sequence_beside_a_short_one(device, monkeypatch):
+    """40 segments beside 3: more groups of 8 than the workspace has slots for when every sequence gets as many as the longest,
+    so that the walk passes all 39 segments behind the first one by one."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 1)
+    cu = torch.tensor([0, 64 * 40, 64 * 43])
+    (q, k, v, g, beta, do), gen = _inputs(1, 64 * 43, 2, 2, 64, 64, torch.bfloat16, 43, unit=False, g_scale=0.02)
+    h0, dht = (torch.randn(2, 2, 64, 64, generator=gen) for _ in range(2))
+    want = ob.backward_manual(q, k, v, g, beta, do, dht, None, h0, cu, og.L2_CHUNK)
+    _check(_gpu_grads(device, q, k, v, g, beta, do, h0, dht, cu, True), want, torch.bfloat16, chunked=True)
 
 
 @pytest.mark.parametrize("cps", [2, 3])
