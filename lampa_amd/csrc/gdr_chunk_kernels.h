@@ -1786,10 +1786,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   } else if (is_m) {
     // M = dtot I + M': M' as bf16 A-operand fragments (rows = state rows, contraction over the columns in
     // accumulator slot order), element (row, col) -> fragment (row/32, col/16), lane 32*hh' + row%32, slot s
-    // (a piece's M' is kept as value and remainder: gdr_scan2_kernel<PIECES>)
-    const bool parts = PIECES && gmax > 0;
-    using OT2 = typename OpVec<OT>::x2;
-    unsigned char* out = Mcomp + ((size_t)map * HV + hv) * ((parts ? 2 : 1) * KT * KT * 2) + late;
+    // (a piece's M' is kept as pairs of value and remainder: gdr_scan2_kernel<PIECES>)
+    unsigned char* out = Mcomp + ((size_t)map * HV + hv) * (KT * KT * 2) + late;
+    if constexpr (PIECES) out += gmax > 0 ? ((size_t)map * HV + hv) * (KT * KT * 2) : 0;
     const int mcol = 32 * wave + ln, ks = mcol >> 4, c16 = mcol & 15;
     const int hs = (c16 >> 2) & 1, slot = 4 * (c16 >> 3) + (c16 & 3);
 #pragma unroll
@@ -1798,9 +1797,20 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       for (int r = 0; r < 16; ++r) {
         const int row = 32 * km + acc_row(r, hh);
         const float val = S[km][r] - (row == mcol ? dtot : 0.0f);
-        const size_t at = (size_t)((km * (KT / 16) + ks) * 64 + 32 * hs + (row & 31)) * 8 + slot;
-        if (parts) reinterpret_cast<OT2*>(out)[at] = OT2{(OT)val, (OT)(val - (float)(OT)val)};
-        else reinterpret_cast<OT*>(out)[at] = (OT)val;
+        if constexpr (PIECES) {
+          const size_t at = (size_t)((km * (KT / 16) + ks) * 64 + 32 * hs + (row & 31)) * 8 + slot;
+          if (gmax > 0) {
+            typename OpVec<OT>::x2 pair;
+            pair[0] = (OT)val;
+            pair[1] = (OT)(val - (float)pair[0]);
+            reinterpret_cast<typename OpVec<OT>::x2*>(out)[at] = pair;
+          } else {
+            reinterpret_cast<OT*>(out)[at] = (OT)val;
+          }
+        } else {
+          *reinterpret_cast<OT*>(out + ((size_t)((km * (KT / 16) + ks) * 64 + 32 * hs + (row & 31))) * 16 + 2 * slot) =
+              (OT)val;
+        }
       }
     if (wave == 0 && lane == 0) Dcomp[(size_t)map * HV + hv] = dtot;
     if constexpr (KEEP) {  // accumulator tiles read as A operand are the transpose
