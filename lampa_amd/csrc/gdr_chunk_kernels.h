@@ -1648,7 +1648,10 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float ks_ = SCALED ? acc[4 * b4 + e] : ek[4 * tm + b4][e] * acc[4 * b4 + e];
-          acc[4 * b4 + e] = be[4 * tm + b4][e] * (vmask * (float)vv[4 * tm + b4][e] - ks_);
+          // (training form: selected, not multiplied away, so that a v that is not finite stays out of M' and with it out
+          // of the gradients of the tokens before it)
+          const float v_ = KEEP ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e]) : vmask * (float)vv[4 * tm + b4][e];
+          acc[4 * b4 + e] = be[4 * tm + b4][e] * (v_ - ks_);
         }
       Rb[2 * tm + 0] = acc_to_op<OT>(acc, 0);
       Rb[2 * tm + 1] = acc_to_op<OT>(acc, 8);

@@ -443,3 +443,20 @@ def test_c_entry_from_the_inputs_alone(device, lens, monkeypatch):
     short = ptr(ws), n_bytes - 1
     assert lib.lampa_gdr_bwd_chunk(*(ptr(x) for x in (q, k, v, g, beta, None, do, None, *got)), host, ptr(plan_dev), 3, 3, 64,
                                    64, 0, 0.2, gd.L2_CHUNK, *short, _capi.stream_of(q)) == -2
+
+
+@pytest.mark.parametrize("token,value", [(700, float("inf")), (400, float("nan")), (767, float("-inf"))])
+def test_values_that_are_not_finite_stay_out_of_earlier_gradients(device, token, value, monkeypatch):
+    """A token whose v is not finite, with no loss on its chunk and the later ones: the gradients of the chunks before it are
+    those of finite values, bit for bit (no v enters the gradient of a state), across the segments' boundaries."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 4)
+    (q, k, v, g, beta, do), gen = _inputs(1, 768, 2, 2, 64, 64, torch.bfloat16, 5, unit=False, g_scale=0.02)
+    h0 = torch.randn(1, 2, 64, 64, generator=gen)
+    end = token // 64 * 64
+    do[:, end:] = 0
+    broken = v.clone()
+    broken[0, token, 0, 3] = value
+    want, got = (_gpu_grads(device, q, k, x, g, beta, do, h0, None, None, True) for x in (v, broken))
+    for a, b in zip(got[:5], want[:5]):
+        assert torch.equal(a[:, :end], b[:, :end])
+    assert torch.equal(got[5], want[5])
