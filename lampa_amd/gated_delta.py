@@ -370,7 +370,8 @@ class _Kept:
 class _InFlight:
     """Pinned memory that queued kernels still write to, held until the event behind them has passed: torch's allocator does
     not know of a kernel that was given the address of a block, and hands the block out again as soon as its tensor dies. One
-    queue per stream, oldest first; what has passed is let go at the next call, whichever thread makes it."""
+    queue per stream, oldest first; what has passed is let go at the next call, whichever thread makes it. (Not by the backward
+    pass as well: an event looked at there left a training step of a few tokens at 198 us instead of 113, most of the time.)"""
 
     def __init__(self):
         self._lock, self._streams = threading.Lock(), {}
@@ -379,10 +380,6 @@ class _InFlight:
         with self._lock:
             self._release()
             self._streams.setdefault(stream, collections.deque()).append((memory, done))
-
-    def release(self):
-        with self._lock:
-            self._release()
 
     def _release(self):
         for stream in list(self._streams):
@@ -576,7 +573,6 @@ class _GatedDelta(torch.autograd.Function):
             if ctx.kept.flag is not None:
                 # every launch is queued: the flag of the forward's first kernel is read while the GPU works on them
                 ctx.kept.done.synchronize()
-                _in_flight.release()
                 if int(ctx.kept.flag[0]):
                     _raise_positive_g()
         else:

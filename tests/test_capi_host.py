@@ -350,13 +350,13 @@ def test_flag_of_a_training_call_outlives_its_kernels(training_calls, monkeypatc
     alive = [weakref.ref(f) for f in flags]
     flags.clear()
     assert len(alive) == len(events) == 2
-    gd._in_flight.release()
+    gd._in_flight._release()
     assert all(f() is not None for f in alive)
     events[0].passed = True
-    gd._in_flight.release()
+    gd._in_flight._release()
     assert alive[0]() is None and alive[1]() is not None
     events[1].passed = True
-    gd._in_flight.release()
+    gd._in_flight._release()
     assert alive[1]() is None and not gd._in_flight._streams
 
 
