@@ -370,8 +370,8 @@ class _Kept:
 class _InFlight:
     """Pinned memory that queued kernels still write to, held until the event behind them has passed: torch's allocator does
     not know of a kernel that was given the address of a block, and hands the block out again as soon as its tensor dies. One
-    queue per stream, oldest first; what has passed is let go at the next call, whichever thread makes it. (Not by the backward
-    pass as well: an event looked at there left a training step of a few tokens at 198 us instead of 113, most of the time.)"""
+    queue per stream, oldest first; what has passed is let go at the next call, whichever thread makes it. Costs a forward
+    3 us of host time; once more in the backward pass would cost as much again."""
 
     def __init__(self):
         self._lock, self._streams = threading.Lock(), {}
