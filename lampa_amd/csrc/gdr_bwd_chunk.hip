@@ -529,7 +529,7 @@ __device__ __forceinline__ void gb_zero_upper(unsigned char* smem, int tid) {
 // ---- source pass: every segment's N' (the walk from a zero gradient, no gradients written) --------------------------------
 // Grid segments x heads (long segments first), eight waves: 0, 1 the gradient of the state (32 value columns each), 4-6 the
 // tiles of P, 2 and 3 / 4-7 stage the next chunk into the other set of tiles. Two barriers per chunk, two workgroups per CU (80 KB
-// of LDS, 128 registers). 52 - 57 us by box at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the products).
+// of LDS, 128 registers). 52 - 57 us, by card, at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the products).
 template <typename T>
 __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
     gdrb_source_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ dout,
@@ -642,7 +642,7 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
 // the rows of dq and dk of the chunk before. Barriers per chunk: (1) P, Vn, G' complete; (2) X, N complete; (3) M complete; (4)
 // the partial row sums are complete; (5) the next chunk's tiles and the rows of dq and dk are complete.
 // Bound by the latency of these five stages: 2.9 + 3.2 + 2.8 + 2.8 + 1.7 thousand cycles per chunk, of which a SIMD issues
-// vector instructions for about 7 000 (one workgroup per CU: 160 KB of LDS). 184 - 205 us by box at 60 000 tokens x 8 heads; all roles on
+// vector instructions for about 7 000 (one workgroup per CU: 160 KB of LDS). 184 - 205 us, by card, at 60 000 tokens x 8 heads; all roles on
 // eight waves with one set of tiles and seven barriers took 256 us, two such workgroups per CU with 128 registers 395 us
 // (they spill, and every reload waits for the tiles being prefetched). Each role has its own loop for that reason too: a loop
 // shared by two roles copies the registers being loaded at its end and so waits for them (+7 us).
