@@ -82,6 +82,16 @@ __device__ __forceinline__ void tri_upper_piece(int u, int& row, int& part) {
 #define REC_BYTES (T_BYTES + 3 * 64 * 4)  // (third row: the l2-norm factors of the k rows, written by gdr_local_kernel)
 #define GDR_SCAN_GROUP 8  // segments per group of the two-level scan; a multiple of its ring depth
 
+// Decay of a composite (d, M', N) with d = 0, M' = 0 and a finite N: minus zero (the decay itself never is).
+__device__ __forceinline__ bool gdr_d_cut(float d) { return __float_as_uint(d) == 0x80000000u; }
+// How many of the first maps of a walk of n cut off all that lies before them, one after the other from the first (lane p
+// holds the decay of map p; of a longer walk the first 64 are looked at): a walk from a finite state may start at the last
+// of them.
+__device__ __forceinline__ int gdr_leading_cuts(float d, int n, int lane) {
+  const unsigned long long open = __ballot(!(lane < n && gdr_d_cut(d)));
+  return open ? __builtin_ctzll(open) : 64;
+}
+
 __device__ __forceinline__ bf16x8 frag_load(const unsigned char* base, int frag, int lane) {
   return *reinterpret_cast<const bf16x8*>(base + (size_t)frag * 1024 + lane * 16);
 }
@@ -692,6 +702,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   // (the per-chunk tables are separate restrict parameters: read through the view they could alias the kernel's
   // stores, would be fetched with vector loads and would sit in the same queue as the stagers' prefetches)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
+  // Segments that cut off what lies before them are found (see the end of the kernel), in the composite pass of the plain rule.
+  constexpr bool CUTS = !PASS_B && SCALED_K;
+  constexpr bool SKIP_M = CUTS && KT + VT > 128;
 
   if (wave >= NSLAB) {
     // ================================================ stager ================================================
@@ -1223,6 +1236,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         lds_barrier();  // the o tile of the last chunk is complete
         stager_flush(tk_p, ln_p);
       }
+      if constexpr (CUTS) lds_barrier();  // (the chain waves' notes on their columns, below)
     }
     return;
   }
@@ -1551,9 +1565,26 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       }
     };
     if (nst > 0) {
+      // (strong decays: the walk starts at the last map of a run of maps that cut off what lies before them; 60 000 tokens x
+      // 8 heads at e^-0.8 a token: pass 60.1 -> 57.2 us, call 130 -> 124, and 39.7 -> 39.3 for 6 007 tokens where none does)
+      const int pl = min(lane, nst - 1);
+      const float dl = (pl < lead ? Dgrp : Dcomp)[(size_t)(pl < lead ? seq * gmax + pl : item0 + (pl - lead)) * HV + hv];
       issue(0, rm[0], rn[0], rd[0]);
       issue(1, rm[1], rn[1], rd[1]);
-      for (int p = 0; p < nst; p += 2) {
+      int from = max(0, uniform(gdr_leading_cuts(dl, nst, lane)) - 1);
+      if (from > 0 && h0) {
+        float probe = 0.0f;
+#pragma unroll
+        for (int km = 0; km < NKM; ++km)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(S[km][r], 0.0f, probe);
+        if (__ballot(!(probe == 0.0f))) from = 0;
+      }
+      if (from > 0) {
+        issue(from, rm[0], rn[0], rd[0]);
+        issue(from + 1, rm[1], rn[1], rd[1]);
+      }
+      for (int p = from; p < nst; p += 2) {
         step(rm[0], rn[0], rd[0]);
         issue(p + 2, rm[0], rn[0], rd[0]);
         if (p + 1 < nst) step(rm[1], rn[1], rd[1]);
@@ -1600,6 +1631,15 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
 #pragma unroll
       for (int ks = 0; ks < KT / 16; ++ks) fk[tm * (KT / 16) + ks] = SWZ ? op_ld_kappa_swz<OT>(tx.k, SK, 32 * tm + ln, 16 * ks, hh)
                                         : op_ld_kappa<OT>(tx.k, SK, 32 * tm + ln, 16 * ks, hh);
+  };
+  bool gone = false;  // (M) this wave's columns are zero
+  auto m_is_zero = [&]() __attribute__((always_inline)) {
+    unsigned any = 0;
+#pragma unroll
+    for (int km = 0; km < KT / 32; ++km)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) any |= __float_as_uint(S[km][r]) << 1;
+    return __ballot(any != 0) == 0;
   };
   if (nc > 0) lds_barrier();  // tiles (c0) are ready
   if constexpr (EARLY_K) load_k_rows(tiles(0));
@@ -1710,6 +1750,23 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) S[km] = mfma32(fk[km * 4 + ks], Vsb[ks], S[km]);
     }
+    if constexpr (SKIP_M) {
+      // Columns of M that have become zero stay zero, whatever chunks follow: a wave whose columns all have only takes part
+      // in the barriers from there on and leaves the LDS and the matrix cores, which bound this pass at the wide heads, to
+      // the columns of N. The result is the same to the bit (a k, g or beta of a later chunk that is not finite reaches
+      // every column of N, and through N what comes after the segment). With decays of e^-0.8 a token a segment's M has
+      // left the fp32 range after three chunks, with e^-0.24 after eight, with e^-0.04 after 47; looked at only once the
+      // decays' own product has. 16 packed events of 520 000 tokens, 8 x 128 x 128, e^-0.8: pass 890 -> 691 us,
+      // call 2 166 -> 2 000; no change where M lives on. Heads up to
+      // 64 x 64 are bound by the chain of a chunk and gain nothing (the loop's second exit cost them registers: 127 -> 144 us).
+      if (is_m && uniform(__float_as_int(dtot)) == 0) {
+        gone = m_is_zero();
+        if (gone) {
+          for (int left = c1 - c - 1; left > 0; --left) lds_barrier();  // B(c + 1) ..
+          break;
+        }
+      }
+    }
     if constexpr (PASS_B) {
       if constexpr (!EARLY_Q) {  // batch: Q rows, P fragments, output factors
 #pragma unroll
@@ -1777,6 +1834,31 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   // epilogue; the opaque zero keeps the compiler from computing all these addresses before the loop
   int late = 0;
   asm volatile("" : "+v"(late));
+  if constexpr (CUTS) {
+    // A segment whose M is zero and whose N is finite hands N on whatever finite state it starts from: its decay is
+    // stored as -0 (gdr_d_cut), which those who walk the composites look for. Every wave notes what it knows of its own
+    // columns, wave 0 stores the decay.
+    if (nc > 0) {
+      bool fine = false;
+      if (uniform(__float_as_int(dtot)) == 0) {
+        float probe = 0.0f;  // 0 x every entry: NaN unless all are finite
+#pragma unroll
+        for (int km = 0; km < KT / 32; ++km)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(S[km][r], 0.0f, probe);
+        fine = is_m ? gone || m_is_zero() : __ballot(!(probe == 0.0f)) == 0;
+      }
+      float* note = tiles(0).misc + 8;
+      if (lane == 0) note[wave] = fine ? 0.0f : 1.0f;
+      lds_barrier();
+      if (wave == 0) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NSLAB; ++w) sum += note[w];
+        if (sum == 0.0f) dtot = -0.0f;
+      }
+    }
+  }
   if constexpr (PASS_B) {
     if (ht && (flags & SEG_LAST)) {
       const int seq = pv.seg_seq[seg];
@@ -2041,6 +2123,22 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) issue(max(0, min(d, last)), rm[d], rn[d], rd[d]);
 
+  // Strong decays: a group whose maps all cut off what lies before them is its last map (60 000 tokens x 8 heads:
+  // 7.9 -> 5.5 us).
+  bool cut = false;
+  if constexpr (MODE == SCAN_GROUP && !REV) {
+    cut = gdr_leading_cuts(Dsrc[(size_t)(item0 + min(lane, nsteps)) * HV + hv], G, lane) >= G;
+    if (cut) {
+      const f32x4* N = reinterpret_cast<const f32x4*>(Nsrc + (((size_t)(item0 + nsteps) * HV + hv) * (VT / 32) + nblk) * N_BYTES);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 t = N[(wave * 4 + q4) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[4 * q4 + e] = is_pm ? 0.0f : t[e];
+      }
+    }
+  }
+
   float dprod = 1.0f;
   auto step = [&](int p, X8* m, f32x4* n, float& dd) {
     if (!COMPOSE) {
@@ -2113,10 +2211,11 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
       for (int u = 0; u < LONG; ++u) step(p0 + u, rm[u % DEPTH], rn[u % DEPTH], rd[u % DEPTH]);
     }
   }
-  for (; p0 <= nsteps; p0 += DEPTH) {
+  for (; !cut && p0 <= nsteps; p0 += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) step(p0 + d, rm[d], rn[d], rd[d]);
   }
+  if constexpr (COMPOSE) dprod = cut ? -0.0f : __builtin_fabsf(dprod);
 
   if (COMPOSE) {  // exactly G maps were applied (G is a multiple of DEPTH): store the composite
     const size_t gh = (size_t)(MODE == SCAN_PIECES ? seg0 + j : seq * gmax + j) * HV + hv;

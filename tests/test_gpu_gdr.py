@@ -572,3 +572,34 @@ def test_traffic_probe_writes_every_output_row(device):
     assert torch.equal(words2[..., 0], torch.arange(n2).view(-1, 1, 1, 1).expand(n2, 64, H, 8).int())
     assert _capi.lib().lampa_gdr_traffic_probe_walk(q2.data_ptr(), k2.data_ptr(), v2.data_ptr(), rec2.data_ptr(), None,
                                                     o2.data_ptr(), n2, H, 1, None) == -1
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (64, 64, torch.float16), (64, 128, torch.bfloat16),
+                                       (128, 128, torch.bfloat16), (32, 32, torch.bfloat16)])
+def test_segments_that_cut_off_what_lies_before_them(device, K, V, dtype, monkeypatch):
+    # 33 segments of four chunks. Decays whose product leaves the fp32 range inside a segment (the segment's M is zero, the
+    # walk over the composites starts behind it) in every segment, in none, in the first half only and in the second half
+    # only; with an initial state. Then the same call with a v, or an initial state, that is not finite: its column must not
+    # be finite anywhere behind it, however strong the decays, and the other heads keep their bits.
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 4)
+    T = 64 * 4 * 33 - 9
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 4, K, V, dtype, seed=K + V, g_scale=0.02)
+    g[:, :, 0] *= 80
+    g[:, : T // 2, 2] *= 80
+    g[:, T // 2:, 3] *= 80
+    h0 = torch.randn(1, 4, K, V, generator=torch.Generator().manual_seed(3)) * 0.3
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta, initial_state=h0)
+    args = _to(device, q, k, v, g, beta)
+    o, s = gd.chunk_gated_delta_rule(*args, initial_state=h0.to(device), output_final_state=True)
+    _assert_bf16_close(o, want_o, "o")
+    _assert_bf16_close(s, want_s, "state")
+    bad = args[2].clone()
+    bad[0, 70, 0, 5] = float("inf")
+    o1, s1 = gd.chunk_gated_delta_rule(args[0], args[1], bad, *args[3:], initial_state=h0.to(device), output_final_state=True)
+    assert not torch.isfinite(o1[0, 71:, 0, 5]).any() and not torch.isfinite(s1[0, 0, :, 5]).any()
+    assert torch.equal(o1[:, :, 1:], o[:, :, 1:]) and torch.equal(s1[:, 1:], s[:, 1:])
+    bad_h0 = h0.clone()
+    bad_h0[0, 0, 3, 7] = float("nan")
+    o2, s2 = gd.chunk_gated_delta_rule(*args, initial_state=bad_h0.to(device), output_final_state=True)
+    assert not torch.isfinite(o2[0, :, 0, 7]).any() and not torch.isfinite(s2[0, 0, :, 7]).any()
+    assert torch.equal(o2[:, :, 1:], o[:, :, 1:]) and torch.equal(s2[:, 1:], s[:, 1:])
