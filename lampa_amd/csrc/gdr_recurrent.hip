@@ -130,20 +130,34 @@ __global__ void __launch_bounds__(64) gdr_recurrent_kernel(const T* __restrict__
   }
 }
 
-// ---- the same recurrence with the state rows of a column split over the two halves of the wave ----------------------
-// One wave owns 32 value columns of one (sequence, value head): lane = (half, column), and a lane keeps KT / 2 state
-// rows of its column, so a step is half as many instructions per wave as above and V <= 32 fills the wave; the two
-// partial sums of S^T k and of S^T q meet through one cross-half exchange each. The wave is bound by instruction issue
-// (one wave per SIMD: four cycles per instruction), so everything that is not the recurrence leaves the step: k and q
-// of a group of tokens are loaded 4 elements at a time one group ahead, widened and parked in LDS (a lane reads its
-// KT / 2 values of a token with 16-byte broadcast reads instead of one cross-lane read per element), and the per-token
-// scalars (1 / |k|, scale / |q|, e^g, beta) are computed for the whole group at once, lane = token. The l2 norms are
-// applied as factors on the sums, not on the vectors. K a multiple of 4, q and k 16-byte aligned.
-// x of the lower half of the wave plus x of the upper half, in every lane (one cross-half swap, no LDS)
-__device__ __forceinline__ float rec_half_sum(float x) {
-  const unsigned u = __float_as_uint(x);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // r[0] = lower half's, r[1] = upper half's
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+// ---- the same recurrence with the state rows of a column split over eight lanes ---------------------------------------
+// For launches of few waves. A wave owns 16 value columns of one (sequence, value head): lane = (column pair, row group), a
+// lane keeps KT / 8 state rows of two columns, and the partial sums of S^T k and of S^T q meet over eight neighbouring lanes
+// (three DPP additions each, no LDS). One wave per SIMD is bound by the instructions of a step, four cycles each, and by the
+// dependent chain S^T k -> d -> S; the four waves of a CU, by the LDS reads of the token's k and q: with two columns to a lane
+// those are KT / 8 values of each where a lane with one column reads twice as many. What is not the recurrence leaves the
+// step: the waves of a workgroup, which own neighbouring columns of the same head, load a group of tokens ahead, widen q, k
+// and v and park them in LDS together, and the per-token scalars (1 / |k|, scale / |q|, e^g, beta) are made with them: the
+// squares are summed where the pieces of a row sit in neighbouring lanes, the decays scanned with lane = token. The l2 norms
+// are applied as factors on the sums, not on the vectors. K a multiple of 4, q and k 16-byte aligned.
+// Against two row groups, 32 columns and a workgroup per wave (us, 64 tokens, states in and out): 16 x 8 x 64 x 64 bf16
+// 32.8 -> 20.7 (one token 8.0 -> 5.8), 32 x 4 x 128 x 128 110 -> 32, 128 x 8 x 64 x 64 82 -> 54, 40 x 6 x 32 x 64 fp32
+// 20.8 -> 16.3, 128 x 6 x 16 x 64 22.5 -> 16.6, but 128 x 8 x 16 x 32 17.9 -> 19.4; against a lane per column, where that was
+// taken before: 512 x 8 x 32 x 32 187 -> 73, 128 x 8 x 128 x 128 355 -> 159, 1 024 x 8 x 64 x 64 608 -> 357. (Groups of 16 or
+// 64 tokens at K = 16, four row groups of 32 columns a wave: slower.)
+// x summed over aligned runs of N lanes, in every lane
+template <int N>
+__device__ __forceinline__ float rec_run_sum(float x) {
+  x += dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, x);
+  x += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, x);
+  if constexpr (N >= 8) x += dpp_f32<0x141, 0xF>(0.0f, x);   // row_half_mirror: the other quad of the 8
+  if constexpr (N >= 16) x += dpp_f32<0x140, 0xF>(0.0f, x);  // row_mirror: the other 8 of the 16
+  if constexpr (N >= 32) {
+    const unsigned u = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return x;
 }
 
 template <bool B>
@@ -151,121 +165,147 @@ struct RecLazy {
   static constexpr bool value = B;
 };
 
+// four elements as they come from memory, and widened
 template <typename T>
-__device__ __forceinline__ float4 rec_load4(const T* p) {
-  if constexpr (sizeof(T) == 4) {
-    return *reinterpret_cast<const float4*>(p);
-  } else {
-    typedef T vec4 __attribute__((ext_vector_type(4)));
-    const vec4 x = *reinterpret_cast<const vec4*>(p);
-    return make_float4(GdrElem<T>::to_float(x[0]), GdrElem<T>::to_float(x[1]), GdrElem<T>::to_float(x[2]),
-                       GdrElem<T>::to_float(x[3]));
-  }
+struct RecRaw4 {
+  typedef T type __attribute__((ext_vector_type(4)));
+};
+template <typename T>
+__device__ __forceinline__ float4 rec_widen4(typename RecRaw4<T>::type x) {
+  return make_float4(GdrElem<T>::to_float(x[0]), GdrElem<T>::to_float(x[1]), GdrElem<T>::to_float(x[2]),
+                     GdrElem<T>::to_float(x[3]));
 }
 
 // COMPOSITE: the affine map of the sequence instead of its outputs. The state of a gated delta sequence is affine in
 // the state it starts from, S_end = M S_0 + N: the wave's columns are columns of [M | N] (V = K + the value width),
 // started from [I | 0], the M columns see v = 0; nothing is written but ht (fp32 [n_seq, HV, K, V]). ht_map (nullable)
 // gives the row of ht that a sequence's final state goes to (negative: not stored).
-template <typename T, int KT, bool COMPOSITE, bool SHORT_GROUPS = false>
-__global__ void __launch_bounds__(64)
+template <typename T, int KT, int WAVES, bool COMPOSITE>
+__global__ void __launch_bounds__(64 * WAVES, 2)
     gdr_recurrent_split_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                const float* __restrict__ g, const float* __restrict__ beta, T* __restrict__ o,
                                const float* __restrict__ h0, float* __restrict__ ht,
                                const int64_t* __restrict__ cu_seqlens, int64_t t_len, int H, int HV, int K, int V,
                                float scale, int l2norm, const int32_t* __restrict__ ht_map) {
-  constexpr int RP = KT / 2;                          // state rows per lane
-  // tokens per group: 24 KB of LDS per wave at K >= 64 (six waves per CU); SHORT_GROUPS halves that for launches of
-  // more waves than that holds at once (built for KT = 64, where eight then fit and a launch of 2016 waves needs one
-  // round instead of two: 1.11 -> 0.73 ms; with fewer waves the longer groups are faster, 207 against 230 us)
-  constexpr int G = (SHORT_GROUPS ? 512 : 1024) / KT < 64 ? (SHORT_GROUPS ? 512 : 1024) / KT : 64;
-  constexpr int ROW4 = (2 * KT + 4) / 4;              // 16-byte pieces per token in LDS: k | q, padded against conflicts
-  // 4-element pieces of k | q per token; the maps need no q (left out under a condition on the lane instead, its loads made
-  // every load a branch, with a wait for memory inside for 16-bit inputs: 8 192 x 4 x 32 x 32 fp32 18.0 against 16.1 us)
-  constexpr int PPT = (COMPOSITE ? KT : 2 * KT) / 4;
-  constexpr int PIECES = G * PPT / 64;                // pieces per lane and group
-  constexpr int VALS = G * 32 / 64;                   // v elements per lane and group
-  static_assert((G * PPT) % 64 == 0, "group shape");
+  constexpr int RG = 8, WCOLS = 128 / RG;       // row groups and columns of a wave
+  constexpr int NT = 64 * WAVES, COLS = WCOLS * WAVES;
+  constexpr int RP = KT / RG;                   // state rows per lane
+  constexpr int G = KT <= 64 ? 32 : 16;         // tokens per group
+  constexpr int P = KT / 4;                     // 4-element pieces of a row of k
+  constexpr int ROW4 = (2 * KT + 4) / 4;        // 16-byte pieces per token in LDS: k | q, padded against conflicts
+  constexpr int PIECES = (G * P + NT - 1) / NT; // pieces of k (and of q) per thread and group
+  constexpr int VALS = G * COLS / NT;           // v elements per thread and group
+  static_assert((G * P) % NT == 0 || G * P < NT, "group shape");
   // two buffers of a group each; two more tokens' room behind each group, so that the reads ahead need no bound
   // (what they return for tokens after the group is never used)
   __shared__ float4 s_kq[2][(G + 2) * ROW4];
   __shared__ float4 s_sc[2][G + 2];
-  __shared__ float s_v[2][(G + 2) * 32];
-  __shared__ float s_fold[2];  // per group: the decay over the whole group if it runs in the lazy form, else 0
-  const int lane = threadIdx.x, half = lane >> 5, cl = lane & 31;
-  const int col = blockIdx.x * 32 + cl;
-  const bool active = col < V;
+  __shared__ float s_v[2][(G + 2) * COLS];
+  __shared__ T s_o[COMPOSITE ? 1 : G * COLS];  // o of a group, stored behind its last step
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rg = lane % RG, cl = WCOLS * wave + 2 * (lane / RG);
+  const int wcol = (int)blockIdx.x * COLS, col = wcol + cl;  // the first of this lane's two columns
   const int seq = blockIdx.y / HV, hv = blockIdx.y % HV;
   const int h = hv / (HV / H);
   const int64_t bos = cu_seqlens ? cu_seqlens[seq] : seq * t_len;
   const int64_t eos = cu_seqlens ? cu_seqlens[seq + 1] : bos + t_len;
 
-  const int v_dim = COMPOSITE ? V - K : V;   // width of a row of v
-  const int v_col = COMPOSITE ? col - K : col;  // this lane's column of v (negative: an M column, v = 0)
-  float S[RP];  // rows half * RP + r
+  const int v_dim = COMPOSITE ? V - K : V;  // width of a row of v
+  const bool even = V % 2 == 0 && ((reinterpret_cast<uintptr_t>(h0) | reinterpret_cast<uintptr_t>(ht)) & 7) == 0;  // columns in pairs
+  float S[2][RP];  // rows rg * RP + r
 #pragma unroll
   for (int r = 0; r < RP; ++r) {
-    const int i = half * RP + r;
-    if constexpr (COMPOSITE) S[r] = (i == col && col < K) ? 1.0f : 0.0f;
-    else S[r] = (h0 && active && i < K) ? h0[(((int64_t)seq * HV + hv) * K + i) * V + col] : 0.0f;
+    const int i = rg * RP + r;
+    if constexpr (COMPOSITE) {
+      S[0][r] = (i == col && i < K) ? 1.0f : 0.0f;
+      S[1][r] = (i == col + 1 && i < K) ? 1.0f : 0.0f;
+    } else {
+      const float* at = h0 + (((int64_t)seq * HV + hv) * K + i) * V + col;
+      float2 x = make_float2(0.0f, 0.0f);
+      if (h0 && i < K && col < V) {
+        if (even) x = *reinterpret_cast<const float2*>(at);
+        else x = make_float2(at[0], col + 1 < V ? at[1] : 0.0f);
+      }
+      S[0][r] = x.x;
+      S[1][r] = x.y;
+    }
   }
   if (bos < eos) {
-    float4 piece[PIECES];
-    float vals[VALS];
+    using Raw = typename RecRaw4<T>::type;
+    Raw kp[PIECES], qp[COMPOSITE ? 1 : PIECES];  // (as they come: a conversion here would wait for the loads)
+    T vals[VALS];
     float g_tok = 0.0f, b_tok = 0.0f;
     // loads of the group that starts at token t0: every address is inside the tensors (tokens past the end re-read the
-    // last one, elements past K or V the last element) and what is out of range is replaced when it is parked
-    auto fetch = [&](int64_t t0) __attribute__((always_inline)) {
+    // last one, elements past K or V the last element) and what is out of range is replaced when it is parked. Uniform
+    // base pointers and 32-bit offsets, the same for every whole group.
+    int k_off[PIECES], v_off[VALS], g_off;
+    auto offsets = [&](int last) __attribute__((always_inline)) {  // last: the group's last token that exists
 #pragma unroll
       for (int n = 0; n < PIECES; ++n) {
-        const int pi = lane + 64 * n, j = pi / PPT, c = 4 * (pi % PPT);
-        const int64_t t = t0 + j < eos ? t0 + j : eos - 1;
-        const int e = c < KT ? c : c - KT;
-        piece[n] = rec_load4<T>((c < KT ? k : q) + (t * H + h) * K + (e < K ? e : K - 4));
+        const int pi = tid + NT * n, c = 4 * (pi % P);
+        k_off[n] = min(pi / P, last) * (H * K) + (c < K ? c : K - 4);
       }
 #pragma unroll
       for (int n = 0; n < VALS; ++n) {
-        const int vi = lane + 64 * n, j = vi / 32;
-        const int cc = (int)blockIdx.x * 32 + vi % 32 - (COMPOSITE ? K : 0);
-        const int64_t t = t0 + j < eos ? t0 + j : eos - 1;
-        vals[n] = GdrElem<T>::to_float(v[(t * HV + hv) * v_dim + max(0, min(cc, v_dim - 1))]);
+        const int vi = tid + NT * n, cc = wcol + vi % COLS - (COMPOSITE ? K : 0);
+        v_off[n] = min(vi / COLS, last) * (HV * v_dim) + max(0, min(cc, v_dim - 1));
       }
-      const int64_t t = t0 + lane < eos ? t0 + lane : eos - 1;
-      g_tok = g[t * HV + hv];
-      b_tok = beta[t * HV + hv];
+      g_off = min(lane, last) * HV;
     };
-    // the fetched group into LDS buffer `buf`, then its per-token scalars (lane = token)
-    auto commit = [&](int buf, bool live) __attribute__((always_inline)) {
+    auto fetch = [&](int64_t t0) __attribute__((always_inline)) {
+      const int64_t left = eos - t0;
+      if (left < G) offsets((int)left - 1);
+      const T* kb = k + (t0 * H + h) * K;
+      const T* qb = q + (t0 * H + h) * K;
+      const T* vb = v + (t0 * HV + hv) * v_dim;
 #pragma unroll
       for (int n = 0; n < PIECES; ++n) {
-        const int pi = lane + 64 * n, j = pi / PPT, c4 = pi % PPT;
-        const int c = 4 * c4, e = c < KT ? c : c - KT;
-        s_kq[buf][j * ROW4 + c4] = e < K ? piece[n] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (n > 0 && n * NT / P >= left) break;  // (a few tokens in all: nothing there)
+        kp[n] = *reinterpret_cast<const Raw*>(kb + (unsigned)k_off[n]);
+        if constexpr (!COMPOSITE) qp[n] = *reinterpret_cast<const Raw*>(qb + (unsigned)k_off[n]);
       }
 #pragma unroll
       for (int n = 0; n < VALS; ++n) {
-        const int cc = (int)blockIdx.x * 32 + (lane + 64 * n) % 32 - (COMPOSITE ? K : 0);
-        s_v[buf][lane + 64 * n] = (COMPOSITE && cc < 0) ? 0.0f : vals[n];
+        if (n > 0 && n * NT / COLS >= left) break;
+        vals[n] = vb[(unsigned)v_off[n]];
       }
-      // The decay is not applied to the state token by token: within a group the registers hold S / c_j, c_j = the
-      // decay from the group's start up to token j, and c_j goes into the token's scalars instead (a multiply per
-      // state element and token less); the state is brought back to scale once per group. With more than e^60 of
-      // decay (or growth) inside one group 1 / c_j would leave the fp32 range: such a group runs in the direct form.
-      const float g_use = (lane < G && live) ? g_tok : 0.0f;
-      const float cum = wave_inclusive_scan(g_use);
-      const float span = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wave_inclusive_scan(fabsf(g_use))), 63));
-      const bool lazy = span <= 60.0f;  // (false for a NaN as well)
-      if (lane == G - 1) s_fold[buf] = lazy ? expf(cum) : 0.0f;
-      if (lane < G) {
-        float kss = 0.0f, qss = 0.0f;
+      g_tok = g[t0 * HV + hv + (unsigned)g_off];
+      b_tok = beta[t0 * HV + hv + (unsigned)g_off];
+    };
+    offsets(G - 1);
+    // the fetched group, which starts at t0, into LDS buffer `buf`, with its per-token scalars.
+    // The decay is not applied to the state token by token: within a run of eight tokens the registers hold S / c_j, c_j =
+    // the decay from the run's start up to token j, and c_j goes into the token's scalars instead (a multiply per state
+    // element and token less); the state is brought back to scale after the run. (Runs as long as the group, 16 to 64 tokens,
+    // cost nothing less and up to 2.5 times the error against 64 bits, from the rounding of the longer sums in e^.) A group
+    // with more than e^60 of decay (or growth) in one of its runs, where 1 / c_j would leave the fp32 range, takes the direct
+    // form. c_run: of lane 8 r + 7, the decay over run r.
+    float c_run = 1.0f;
+    bool lazy = false;
+    auto commit = [&](int64_t t0, int buf) __attribute__((always_inline)) {
+      const float g_use = (lane < G && t0 + lane < eos) ? g_tok : 0.0f;  // (lane = token; every wave for itself)
+      float cum = g_use;
+      const float up1 = dpp_f32<GDR_DPP_ROW_SHR(1), 0xF>(0.0f, cum);  // (every lane enabled)
+      cum += (lane & 7) >= 1 ? up1 : 0.0f;
+      const float up2 = dpp_f32<GDR_DPP_ROW_SHR(2), 0xF>(0.0f, cum);
+      cum += (lane & 7) >= 2 ? up2 : 0.0f;
+      const float up4 = dpp_f32<GDR_DPP_ROW_SHR(4), 0xF>(0.0f, cum);
+      cum += (lane & 7) >= 4 ? up4 : 0.0f;
+      lazy = __ballot(!(rec_run_sum<8>(fabsf(g_use)) <= 60.0f)) == 0;  // (false for a NaN as well)
+      const float c_tok = expf(lazy ? cum : g_tok), rc_tok = lazy ? expf(-cum) : 1.0f;
+      c_run = c_tok;
 #pragma unroll
-        for (int c4 = 0; c4 < KT / 4; ++c4) {
-          const float4 a = s_kq[buf][lane * ROW4 + c4];
-          float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // (read in front of the sums: 85 us, behind kss 89 us at
-          if constexpr (!COMPOSITE) b = s_kq[buf][lane * ROW4 + KT / 4 + c4];  // 128 x 64 tokens x 8 heads of 64 x 64, bf16)
-          kss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
-          qss += b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
-        }
+      for (int n = 0; n < PIECES; ++n) {
+        if (n > 0 && n * NT / P > eos - t0) break;  // (one token past an odd count is read as a step)
+        const int pi = tid + NT * n, j = min(pi / P, G - 1), c4 = pi % P;
+        const bool live = t0 + j < eos;
+        // a token past the end is a step that changes nothing (d = 0, decay 1), so the steps need no branch
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const float4 a = live && 4 * c4 < K ? rec_widen4<T>(kp[n]) : zero;
+        float4 b = zero;
+        if constexpr (!COMPOSITE) b = live && 4 * c4 < K ? rec_widen4<T>(qp[n]) : zero;
+        const float kss = rec_run_sum<P>(a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w);
+        const float qss = COMPOSITE ? 0.0f : rec_run_sum<P>(b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w);
+        const float c = __shfl(c_tok, j), rc = __shfl(rc_tok, j), bt = __shfl(b_tok, j);
         float kinv = 1.0f, qinv = 1.0f;
         if (l2norm == GDR_L2_CHUNK) {
           kinv = 1.0f / __fsqrt_rn(kss + 1e-6f);
@@ -274,33 +314,68 @@ __global__ void __launch_bounds__(64)
           kinv = 1.0f / (__fsqrt_rn(kss) + 1e-6f);
           qinv = 1.0f / (__fsqrt_rn(qss) + 1e-6f);
         }
-        // a token past the end is a step that changes nothing (d = 0, decay 1), so the steps need no branch
-        // direct: 1 / |k|, scale / |q|, e^g, beta; lazy: c / |k|, c scale / |q|, 1 / (c |k|), beta
-        float4 sc = live ? make_float4(kinv, qinv * scale, expf(g_tok), b_tok) : make_float4(0.0f, 0.0f, 1.0f, 0.0f);
-        if (lazy) {
-          const float c = expf(cum), rc = expf(-cum);
-          sc = live ? make_float4(kinv * c, qinv * scale * c, kinv * rc, b_tok) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (G * P >= NT || pi < G * P) {
+          s_kq[buf][j * ROW4 + c4] = a;
+          if constexpr (!COMPOSITE) s_kq[buf][j * ROW4 + P + c4] = b;
+          // direct: 1 / |k|, scale / |q|, e^g, beta; lazy: c / |k|, c scale / |q|, 1 / (c |k|), beta
+          float4 sc = lazy ? make_float4(kinv * c, qinv * scale * c, kinv * rc, bt) : make_float4(kinv, qinv * scale, c, bt);
+          if (!live) sc = make_float4(0.0f, 0.0f, lazy ? 0.0f : 1.0f, 0.0f);
+          if (c4 == 0) s_sc[buf][j] = sc;
         }
-        s_sc[buf][lane] = sc;
+      }
+#pragma unroll
+      for (int n = 0; n < VALS; ++n) {
+        if (n > 0 && n * NT / COLS > eos - t0) break;
+        const int vi = tid + NT * n, cc = wcol + vi % COLS - (COMPOSITE ? K : 0);
+        s_v[buf][vi] = (t0 + vi / COLS >= eos || (COMPOSITE && cc < 0)) ? 0.0f : GdrElem<T>::to_float(vals[n]);
       }
     };
-    // a token's operands: its scalars, this lane's RP elements of k and of q, its v
+    // a token's operands: its scalars, this lane's RP elements of k and of q, the v of its columns
     struct Operands {
-      float4 sc, kk[RP / 4], qq[RP / 4];
-      float v;
+      float4 sc;
+      float kk[RP], qq[COMPOSITE ? 1 : RP];
+      float2 v;
+    };
+    auto read_row = [&](const float* p, float* to) __attribute__((always_inline)) {
+      if constexpr (RP == 2) {
+        const float2 x = *reinterpret_cast<const float2*>(p);
+        to[0] = x.x; to[1] = x.y;
+      } else {
+#pragma unroll
+        for (int r = 0; r < RP; r += 4) {
+          const float4 x = *reinterpret_cast<const float4*>(p + r);
+          to[r] = x.x; to[r + 1] = x.y; to[r + 2] = x.z; to[r + 3] = x.w;
+        }
+      }
     };
     auto read_token = [&](int buf, int j, Operands& x) __attribute__((always_inline)) {
       x.sc = s_sc[buf][j];  // the token's four scalars (direct or lazy form, see commit)
-      const float4* kr = &s_kq[buf][j * ROW4 + half * (RP / 4)];
-#pragma unroll
-      for (int r4 = 0; r4 < RP / 4; ++r4) {
-        x.kk[r4] = kr[r4];
-        x.qq[r4] = kr[KT / 4 + r4];
-      }
-      x.v = s_v[buf][j * 32 + cl];
+      const float* kr = reinterpret_cast<const float*>(&s_kq[buf][j * ROW4]) + rg * RP;
+      read_row(kr, x.kk);
+      if constexpr (!COMPOSITE) read_row(kr + KT, x.qq);
+      x.v = *reinterpret_cast<const float2*>(&s_v[buf][j * COLS + cl]);
     };
     fetch(bos);
-    commit(0, bos + lane < eos);
+    commit(bos, 0);
+    lds_barrier();
+    // o of a group goes through LDS (row groups 0 and 1 write the first of two tokens, 2 and 3 the second) and leaves behind
+    // the commit of the next group: stored token by token, the wait for that group's loads would be one for the stores too,
+    // 2 us a group.
+    const int o_tok = (rg >> 1) & 1;
+    T* const so = s_o + o_tok * COLS + cl + (rg & 1);
+    auto flush = [&](int64_t t0, int n_tok) __attribute__((always_inline)) {
+      if constexpr (!COMPOSITE) {
+        const int c = WCOLS * wave + lane % WCOLS, j0 = lane / WCOLS;  // this wave's columns, four tokens at a time
+        T* ob = o + (t0 * HV + hv) * V + wcol;
+        const unsigned at = (unsigned)(j0 * (HV * V) + c), step = (unsigned)(64 / WCOLS * HV * V);
+#pragma unroll
+        for (int n = 0; n < G * WCOLS / 64; ++n) {
+          if (n * (64 / WCOLS) >= n_tok) break;
+          const T x = s_o[(n * (64 / WCOLS) + j0) * COLS + c];
+          if (n * (64 / WCOLS) + j0 < n_tok && wcol + c < V) ob[at + n * step] = x;
+        }
+      }
+    };
     int buf = 0;
     for (int64_t t0 = bos; t0 < eos; t0 += G, buf ^= 1) {
       const bool more = t0 + G < eos;
@@ -311,95 +386,129 @@ __global__ void __launch_bounds__(64)
       // that changes nothing.
       auto run_group = [&](auto lazy_tag) __attribute__((always_inline)) {
         constexpr bool LAZY = decltype(lazy_tag)::value;
-        auto step = [&](const Operands& x, int64_t t) __attribute__((always_inline)) {
-          float kk[RP], qq[RP];
+        auto step = [&](const Operands& x) __attribute__((always_inline)) {
+          float d[2], dk[2], out[2];
+          const float4 sc = x.sc;
 #pragma unroll
-          for (int r4 = 0; r4 < RP / 4; ++r4) {
-            kk[4 * r4] = x.kk[r4].x; kk[4 * r4 + 1] = x.kk[r4].y; kk[4 * r4 + 2] = x.kk[r4].z; kk[4 * r4 + 3] = x.kk[r4].w;
-            qq[4 * r4] = x.qq[r4].x; qq[4 * r4 + 1] = x.qq[r4].y; qq[4 * r4 + 2] = x.qq[r4].z; qq[4 * r4 + 3] = x.qq[r4].w;
+          for (int c = 0; c < 2; ++c) {
+            d[c] = S[c][0] * x.kk[0];
+#pragma unroll
+            for (int r = 1; r < RP; ++r) d[c] = __builtin_fmaf(S[c][r], x.kk[r], d[c]);
           }
-          float dot4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-          for (int r = 0; r < RP; ++r) dot4[r & 3] = __builtin_fmaf(S[r], kk[r], dot4[r & 3]);
-          const float dot = rec_half_sum((dot4[0] + dot4[1]) + (dot4[2] + dot4[3]));
+          for (int c = 0; c < 2; ++c) d[c] = rec_run_sum<RG>(d[c]);
           // S <- e^g S, then d = beta (v - S^T k), S <- S + k d^T, o = S^T q, with k = k_raw / |k|; in the lazy form on
           // S / c_j, where the decay is part of the scalars
-          const float4 sc = x.sc;
-          const float d = LAZY ? sc.w * (x.v - sc.x * dot) : sc.w * (x.v - sc.z * sc.x * dot);
-          const float dk = LAZY ? d * sc.z : d * sc.x;
-          if constexpr (COMPOSITE) {
 #pragma unroll
-            for (int r = 0; r < RP; ++r) S[r] = __builtin_fmaf(kk[r], dk, LAZY ? S[r] : sc.z * S[r]);
-          } else {
-            float out4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+          for (int c = 0; c < 2; ++c) {
+            const float vc = c ? x.v.y : x.v.x;
+            const float dc = LAZY ? sc.w * (vc - sc.x * d[c]) : sc.w * (vc - sc.z * sc.x * d[c]);
+            dk[c] = LAZY ? dc * sc.z : dc * sc.x;
+          }
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
 #pragma unroll
             for (int r = 0; r < RP; ++r) {
-              S[r] = __builtin_fmaf(kk[r], dk, LAZY ? S[r] : sc.z * S[r]);
-              out4[r & 3] = __builtin_fmaf(S[r], qq[r], out4[r & 3]);
+              S[c][r] = __builtin_fmaf(x.kk[r], dk[c], LAZY ? S[c][r] : sc.z * S[c][r]);
+              if constexpr (!COMPOSITE) out[c] = r == 0 ? S[c][0] * x.qq[0] : __builtin_fmaf(S[c][r], x.qq[r], out[c]);
             }
-            const float out = rec_half_sum((out4[0] + out4[1]) + (out4[2] + out4[3]));
-            if (active && half == 0 && t < eos) o[(t * HV + hv) * V + col] = GdrElem<T>::from_float(out * sc.y);
+          }
+          if constexpr (COMPOSITE) return 0.0f;
+          else {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) out[c] = rec_run_sum<RG>(out[c]);
+            return (rg & 1 ? out[1] : out[0]) * sc.y;
           }
         };
         Operands xa, xb;
         read_token(buf, 0, xa);
-        for (int j = 0; j < n_tok; j += 2) {
-          read_token(buf, j + 1, xb);
-          __builtin_amdgcn_sched_barrier(0);
-          step(xa, t0 + j);
-          read_token(buf, j + 2, xa);
-          __builtin_amdgcn_sched_barrier(0);
-          step(xb, t0 + j + 1);
+#pragma unroll 1
+        for (int run = 0; run < n_tok; run += 8) {
+          const int end = min(n_tok, run + 8);
+#pragma unroll 1
+          for (int j = run; j < end; j += 2) {
+            read_token(buf, j + 1, xb);
+            __builtin_amdgcn_sched_barrier(0);
+            const float oa = step(xa);
+            read_token(buf, j + 2, xa);
+            __builtin_amdgcn_sched_barrier(0);
+            const float ob = step(xb);
+            if constexpr (!COMPOSITE) {
+              if (rg < 4) so[j * COLS] = GdrElem<T>::from_float(o_tok ? ob : oa);
+            }
+          }
+          if constexpr (LAZY) {
+            const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c_run), run + 7));
+#pragma unroll
+            for (int r = 0; r < RP; ++r) {  // back to scale: S = c_last (S / c_last)
+              S[0][r] *= c;
+              S[1][r] *= c;
+            }
+          }
         }
       };
-      const float fold = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s_fold[buf])));
-      if (fold != 0.0f) {
-        run_group(RecLazy<true>{});
-#pragma unroll
-        for (int r = 0; r < RP; ++r) S[r] *= fold;  // back to scale: S = c_last (S / c_last)
+      if (lazy) run_group(RecLazy<true>{});
+      else run_group(RecLazy<false>{});
+      if (more) {
+        commit(t0 + G, buf ^ 1);  // (that buffer was last read before the barrier in front of this group)
+        lds_barrier();
       } else {
-        run_group(RecLazy<false>{});
+        lds_fence();
       }
-      if (more) commit(buf ^ 1, t0 + G + lane < eos);
+      flush(t0, n_tok);
     }
   }
   const int out_row = ht_map ? ht_map[seq] : seq;
-  if (ht && active && out_row >= 0) {
+  if (ht && out_row >= 0) {
 #pragma unroll
     for (int r = 0; r < RP; ++r) {
-      const int i = half * RP + r;
-      if (i < K) ht[(((int64_t)out_row * HV + hv) * K + i) * V + col] = S[r];
+      const int i = rg * RP + r;
+      float* at = ht + (((int64_t)out_row * HV + hv) * K + i) * V + col;
+      if (i < K && col < V) {
+        if (even) *reinterpret_cast<float2*>(at) = make_float2(S[0][r], S[1][r]);
+        else {
+          at[0] = S[0][r];
+          if (col + 1 < V) at[1] = S[1][r];
+        }
+      }
     }
   }
 }
 
-// more waves than six per CU of the 256 (what the long groups' LDS holds at once)
-static inline bool gdr_rec_short_groups(const dim3& grid) { return (int64_t)grid.x * grid.y > 6 * 256; }
+// Launch of the split kernel over `n_seq` runs of tokens; V: all the wave's columns (COMPOSITE: K + the value width).
+template <typename T, bool COMPOSITE>
+static void gdr_split_launch(const void* q, const void* k, const void* v, const float* g, const float* beta, void* o,
+                             const float* h0, float* ht, const int64_t* cu, int n_seq, int64_t t_len, int H, int HV, int K,
+                             int V, float scale, int l2norm, const int32_t* ht_map, hipStream_t s) {
+#define GDR_REC_SPLIT(KT, WAVES)                                                                                         \
+  hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, KT, WAVES, COMPOSITE>),                                              \
+                     dim3((V + 16 * WAVES - 1) / (16 * WAVES), n_seq * HV), dim3(64 * WAVES), 0, s, (const T*)q,         \
+                     (const T*)k, (const T*)v, g, beta, (T*)o, h0, ht, cu, t_len, H, HV, K, V, scale, l2norm, ht_map)
+#define GDR_REC_SPLIT_K(WAVES)                  \
+  do {                                          \
+    if (K <= 16) GDR_REC_SPLIT(16, WAVES);      \
+    else if (K <= 32) GDR_REC_SPLIT(32, WAVES); \
+    else if (K <= 64) GDR_REC_SPLIT(64, WAVES); \
+    else GDR_REC_SPLIT(128, WAVES);             \
+  } while (0)
+  if (V <= 32) GDR_REC_SPLIT_K(2);
+  else GDR_REC_SPLIT_K(4);
+#undef GDR_REC_SPLIT_K
+#undef GDR_REC_SPLIT
+}
 
 template <typename T>
 static int gdr_recurrent_launch(const void* q, const void* k, const void* v, const float* g, const float* beta,
                                 void* o, const float* h0, float* ht, const int64_t* cu, int n_seq, int64_t t_len,
-                                int H, int HV, int K, int V, float scale, int l2norm, hipStream_t s,
-                                const int32_t* ht_map = nullptr) {
+                                int H, int HV, int K, int V, float scale, int l2norm, hipStream_t s) {
   LAMPA_PROF(s, "start");
-  // the split form while its waves (twice as many) still find a SIMD each or nearly so
-  const int64_t split_waves = (int64_t)((V + 31) / 32) * n_seq * HV;
-  if (K % 4 == 0 && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) & 15) == 0 &&
-      split_waves <= 2048) {
-    const dim3 grid2((V + 31) / 32, n_seq * HV);
-#define GDR_REC_SPLIT(KT)                                                                                          \
-  hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, KT, false>), grid2, dim3(64), 0, s, (const T*)q, (const T*)k,  \
-                     (const T*)v, g, beta, (T*)o, h0, ht, cu, t_len, H, HV, K, V, scale, l2norm, ht_map)
-    if (K <= 16) GDR_REC_SPLIT(16);
-    else if (K <= 32) GDR_REC_SPLIT(32);
-    else if (K <= 64) {
-      if (gdr_rec_short_groups(grid2))
-        hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, 64, false, true>), grid2, dim3(64), 0, s, (const T*)q,
-                           (const T*)k, (const T*)v, g, beta, (T*)o, h0, ht, cu, t_len, H, HV, K, V, scale, l2norm,
-                           ht_map);
-      else GDR_REC_SPLIT(64);
-    } else GDR_REC_SPLIT(128);
-#undef GDR_REC_SPLIT
+  // The split form, but for one or two tokens each of very many sequences at K = 64 (a third of the registers, so more loads
+  // of the states in flight: 1 024 x 8 x 64 x 64, one token 73 against 86 us, two 82 against 89, four 100 against 98; at half
+  // as many sequences 37 against 44, a quarter 26 against 24; at K = 16, 32 and 128 the split form is faster throughout).
+  const int64_t waves = (int64_t)((V + 31) / 32) * n_seq * HV, tokens = cu ? t_len / n_seq : t_len;
+  const bool few_of_many = K > 32 && K <= 64 && tokens <= 2 && waves > 4096;
+  if (K % 4 == 0 && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) & 15) == 0 && !few_of_many) {
+    gdr_split_launch<T, false>(q, k, v, g, beta, o, h0, ht, cu, n_seq, t_len, H, HV, K, V, scale, l2norm, nullptr, s);
     LAMPA_PROF(s, "gdr_recurrent_split_kernel");
     return lampa_launch_status();
   }
@@ -423,185 +532,125 @@ static int gdr_recurrent_launch(const void* q, const void* k, const void* v, con
 //   B  every segment again from the state it really starts with, writing o (the plain kernel, segments as sequences)
 // all in fp32: the same function as the token loop up to fp32 rounding.
 
-// 32 columns of the state per workgroup; mn [n_seg, HV, K, K + V], sinit [n_seg, HV, K, V]. A step is short, so what
-// counts is that nothing serial is left in it but the product itself:
-//  - M_p is loaded with 16-byte accesses into registers DEPTH segments ahead (its 1 - 2 us of memory latency would
-//    otherwise be paid once per segment) and parked in LDS; the register sets are fixed per step of an unrolled group
-//    (moving a set would wait for its load), and every memory operation of a step is unconditional (under a condition
-//    it becomes a branch, after which the compiler no longer counts the operations in flight and drains them);
-//  - M_p S runs on the fp32 MFMA (v_mfma_f32_32x32x2f32: 4 bytes per lane and operand from LDS). As multiply-adds with
-//    M read as broadcasts it was bound by LDS bandwidth (512 KB per step at K = 64: 4.8 us). The four waves split the
-//    product into row tiles of 32 and, where there are fewer than four of those, into parts of the contraction whose
-//    partial tiles are added afterwards;
-//  - LDS-only barriers.
-// LDS: M [max(KT, 32)][KT + 4] | S [KT][33] | partial tiles [KS][max(KT, 32)][33], floats.
-typedef float rs_f32x16 __attribute__((ext_vector_type(16)));
+// 16 columns of the state per workgroup; mn [n_seg, HV, K, K + V], sinit [n_seg, HV, K, V]. A step is a chain, so nothing
+// else may be on it:
+//  - M_p S runs on the fp32 MFMA (v_mfma_f32_16x16x4f32), with S in the accumulators it comes out in: register r of row
+//    tile t of lane 16 g + j is row 16 t + 4 g + r of column j, which is what the next product wants as its B operand if it
+//    takes the contraction index 16 t + 4 g + r in its step (t, r); the A operand of the four steps r is then one 16-byte
+//    piece of a row of M_p, from memory straight to registers. A wave owns a row tile, and the tiles are exchanged through
+//    LDS (double-buffered, one barrier per step) behind the wave's own four products;
+//  - the maps are loaded DEPTH steps ahead into register sets that are fixed per step of an unrolled group (moving a set
+//    would wait for its load), and every memory operation of a step is unconditional (under a condition it becomes a branch,
+//    after which the compiler no longer counts the operations in flight and drains them).
+// Before, with M through LDS, 32 columns per workgroup of four waves and three launches, 32 us of a call of 8 192 x 4 x 32 x 32
+// tokens; now 5 + 10. (All rows on one wave up to K = 32: 7 + 15; eight steps of maps ahead instead of four: 8 + 16.)
+typedef float rs_f32x4 __attribute__((ext_vector_type(4)));
 template <int KT>
 struct RsScanShape {
-  static constexpr int RT = KT >= 32 ? KT / 32 : 1;  // row tiles of 32
-  static constexpr int KS = 4 / RT;                  // parts of the contraction (one wave each)
-  static constexpr int ROWS = RT * 32;
-  static constexpr int MS = KT + 4;                  // row stride of M in LDS (floats)
-  static constexpr size_t LDS_BYTES = ((size_t)ROWS * MS + (size_t)KT * 33 + (size_t)KS * ROWS * 33) * sizeof(float);
+  static constexpr int NT = KT / 16;  // row tiles, a wave each
+  static constexpr int DEPTH = 4;
 };
 
-// What a workgroup's range of maps is (blockIdx.y) and what it writes:
-//   RS_PLAIN    a sequence's segments; the state each segment starts from (the last map is not applied)
-//   RS_COMPOSE  group `grp` (gs consecutive segments) of sequence `seq`, blockIdx.y = seq * maxg + grp, on the K + V
-//               columns of [I | 0]: every map of the group is applied and only the result, the group's own map
-//               [M | N], is stored (template COMPOSE; V counts all K + V columns there)
-//   RS_GROUPS   a sequence's groups, the maps being the groups' maps: the state each group starts from
-//   RS_WITHIN   a group's segments from the state the group starts with (h0 row = blockIdx.y)
-// A long sequence is scanned as RS_COMPOSE -> RS_GROUPS -> RS_WITHIN: three launches of about sqrt(n) dependent steps
-// each instead of one of n.
-enum { RS_PLAIN = 0, RS_COMPOSE = 1, RS_GROUPS = 2, RS_WITHIN = 3 };
+// COMPOSE: workgroup (blockIdx.y = seq * maxg + grp) = group `grp` (gs consecutive segments) of sequence `seq`, on the K + V
+// columns of [I | 0]: every map of the group is applied and the result, the group's own map [M | N], stored (V counts all
+// K + V columns). Otherwise: the state every segment of the group starts from; a group in front of which there are others
+// walks their maps (gmaps) first. A long sequence is scanned in groups of about sqrt(n / 2) segments, two launches of at
+// most sqrt(2 n) dependent steps, any other as one group (gs >= its segments, maxg = 1) in one.
+template <int KT, bool COMPOSE>
+__global__ void __launch_bounds__(64 * RsScanShape<KT>::NT)
+    gdr_segment_scan_kernel(const float* __restrict__ mn, const float* __restrict__ gmaps, const float* __restrict__ h0,
+                            const int32_t* __restrict__ seq_seg0, int HV, int K, int V, float* __restrict__ out, int gs,
+                            int maxg, int W) {
+  constexpr int NT = RsScanShape<KT>::NT, DEPTH = RsScanShape<KT>::DEPTH;
+  __shared__ rs_f32x4 s_x[2][NT][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g4 = lane >> 4, j16 = lane & 15;
+  const int hv = blockIdx.z, seq = blockIdx.y / maxg, grp = blockIdx.y - seq * maxg;
+  const int seg0 = seq_seg0[seq], seg1 = seq_seg0[seq + 1];
+  const int p0 = seg0 + grp * gs, cnt = min(gs, seg1 - p0);  // this group's segments
+  if (cnt <= 0 || (COMPOSE && p0 + gs >= seg1)) return;       // (no one asks for the map of a sequence's last group)
+  const int lead = COMPOSE ? 0 : grp, n_apply = lead + (COMPOSE ? cnt : cnt - 1);
+  // Lanes past V shadow the last column, rows past K the last rows of the same place in their run of four: they load, compute
+  // and store the same as those. What they feed into a product is met by a zero of M.
+  const int col = min((int)blockIdx.x * 16 + j16, V - 1);
+  const bool is_m = COMPOSE && col < K;  // (a column of M: no additive term, starts from I)
+  const int ncol = COMPOSE ? max(col - K, 0) : col;
+  auto row_of = [&](int i) { return i < K ? i : K - 4 + (i & 3); };
+  // offsets of this lane's 16-byte pieces of M (its tile's row j16; own tile's columns first) and of its four rows
+  unsigned m_at[NT], row[4];
+  bool inside[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int c = 16 * ((wave + t) % NT) + 4 * g4;
+    inside[t] = c < K;
+    m_at[t] = (unsigned)(row_of(16 * wave + j16) * W + min(c, K - 4));
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) row[r] = (unsigned)row_of(16 * wave + 4 * g4 + r);
 
-template <int KT, int DEPTH, bool COMPOSE = false>
-__global__ void __launch_bounds__(256) gdr_segment_scan_kernel(const float* __restrict__ mn, const float* __restrict__ h0,
-                                                              const int32_t* __restrict__ seq_seg0, int HV, int K, int V,
-                                                              float* __restrict__ sinit, int mode, int gs, int maxg,
-                                                              int W) {
-  using SH = RsScanShape<KT>;
-  constexpr int MS = SH::MS, RT = SH::RT, KS = SH::KS, ROWS = SH::ROWS;
-  constexpr int K4 = KT / 4;                          // 16-byte pieces per row of M
-  constexpr int RPB = 256 / K4 < ROWS ? 256 / K4 : ROWS;  // rows of M that the workgroup stores to LDS at once
-  constexpr int MREGS = (ROWS + RPB - 1) / RPB;       // such batches = pieces per thread
-  constexpr int NR = KT / 8;                          // rows of the new column per thread in the combine step
-  constexpr int KL = KT / KS;                         // contraction length of a wave
-  static_assert(KT % 8 == 0 && KL % 2 == 0, "shape");
-  extern __shared__ float4 s_scan4[];
-  float* s_M = reinterpret_cast<float*>(s_scan4);
-  float* s_S = s_M + ROWS * MS;
-  float* s_P = s_S + KT * 33;
-  const int tid = threadIdx.x, c = tid & 31, rg = tid >> 5;
-  const int wave = tid >> 6, ln = tid & 31, hh = (tid >> 5) & 1;
-  const int rt = wave % RT, ks = wave / RT;
-  const int hv = blockIdx.z;
-  const int col = blockIdx.x * 32 + c;
-  const int colc = col < V ? col : V - 1;  // (lanes past V shadow the last column: same loads, same stores)
-  // the range of maps [p0, p1) and the row of h0
-  int p0, p1, row0 = blockIdx.y;
-  if (mode == RS_PLAIN) {
-    p0 = seq_seg0[blockIdx.y];
-    p1 = seq_seg0[blockIdx.y + 1];
-  } else if (mode == RS_GROUPS) {
-    const int n = seq_seg0[blockIdx.y + 1] - seq_seg0[blockIdx.y];
-    p0 = blockIdx.y * maxg;
-    p1 = p0 + (n + gs - 1) / gs;
-  } else {  // a group of a sequence
-    const int seq = blockIdx.y / maxg, grp = blockIdx.y - seq * maxg;
-    const int s1 = seq_seg0[seq + 1];
-    p0 = seq_seg0[seq] + grp * gs;
-    p1 = min(p0 + gs, s1);
-  }
-  if (p0 >= p1) return;
-  const int p_last = p1 - 1;      // the last map that exists in the range
-  if (COMPOSE) p1 += 1;           // one more (virtual) segment, so that the loop below applies all of them
-#pragma unroll
-  for (int n = 0; n < NR; ++n) {
-    const int i = rg + 8 * n;
-    if (COMPOSE) s_S[i * 33 + c] = (i == col && col < K) ? 1.0f : 0.0f;
-    else s_S[i * 33 + c] = (h0 && i < K) ? h0[(((int64_t)row0 * HV + hv) * K + i) * V + colc] : 0.0f;
-  }
-  // the column of the maps' N part that goes with this column of the state (COMPOSE: none for the first K columns)
-  const int ncol = COMPOSE ? min(max(col - K, 0), W - K - 1) : colc;
-  const bool has_n = !COMPOSE || col >= K;
-  const int my_row = tid / K4, my_c4 = tid % K4;
-  const bool loader = my_row < RPB;
-  float4 mreg[DEPTH][MREGS];
-  float nreg[DEPTH][NR];
-  // M_p and this thread's entries of N_p into register set `slot`: unconditional loads from clamped addresses (a
-  // segment index past the end, a row or column past K); what lies past K is replaced by zero when it is used
-  auto fetch = [&](int p, int slot) __attribute__((always_inline)) {
-    p = min(p, p_last);
-    const float* M = mn + ((int64_t)p * HV + hv) * K * W;
-#pragma unroll
-    for (int u = 0; u < MREGS; ++u)
-      mreg[slot][u] = *reinterpret_cast<const float4*>(M + (int64_t)min(u * RPB + my_row, K - 1) * W + min(4 * my_c4, K - 4));
-#pragma unroll
-    for (int n = 0; n < NR; ++n) nreg[slot][n] = M[(int64_t)min(rg + 8 * n, K - 1) * W + K + ncol];
+  struct Set {
+    rs_f32x4 m[NT];
+    float n[4];
   };
-  // the state segment p starts from (every lane stores every time: rows past K repeat the last row's store)
-  auto store_start = [&](int p) __attribute__((always_inline)) {
-    if (COMPOSE) return;
-    float* out = sinit + ((int64_t)p * HV + hv) * K * V;
+  Set set[DEPTH];
+  auto fetch = [&](int p, Set& x) __attribute__((always_inline)) {
+    p = min(p, n_apply - 1);
+    const float* M = p < lead ? gmaps + ((int64_t)(seq * maxg + p) * HV + hv) * K * W
+                              : mn + ((int64_t)(p0 + p - lead) * HV + hv) * K * W;
 #pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      const int i = min(rg + 8 * n, K - 1);
-      out[(int64_t)i * V + colc] = s_S[i * 33 + c];
-    }
+    for (int t = 0; t < NT; ++t) x.m[t] = *reinterpret_cast<const rs_f32x4*>(M + m_at[t]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x.n[r] = M[row[r] * W + K + ncol];
   };
-  // one step: the state segment p starts from is stored, then S <- M_p S + N_p from register set `slot`, which is then
-  // loaded again for segment p + DEPTH
-  auto advance = [&](int p, int slot) __attribute__((always_inline)) {
-    store_start(p);
+  rs_f32x4 S;
 #pragma unroll
-    for (int u = 0; u < MREGS; ++u) {
-      const int i = u * RPB + my_row;
-      const bool inside = i < K && 4 * my_c4 < K;
-      if (loader && i < ROWS)
-        *reinterpret_cast<float4*>(s_M + i * MS + 4 * my_c4) = inside ? mreg[slot][u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    float acc[NR];
+  for (int r = 0; r < 4; ++r) {
+    if (COMPOSE) S[r] = (is_m && (int)row[r] == col) ? 1.0f : 0.0f;
+    else S[r] = h0 ? h0[(((int64_t)seq * HV + hv) * K + row[r]) * V + col] : 0.0f;
+  }
+  auto store = [&](int64_t at, int width) __attribute__((always_inline)) {
+    float* to = out + (at * HV + hv) * K * width + col;
 #pragma unroll
-    for (int n = 0; n < NR; ++n) acc[n] = (has_n && rg + 8 * n < K) ? nreg[slot][n] : 0.0f;
-    lds_barrier();  // M_p is in LDS (an LDS-only barrier: the loads issued ahead stay in flight)
-    fetch(p + DEPTH, slot);
-    {
-      // this wave's tile: rows 32 rt .., contraction indices ks KL .. ; step s takes the indices s (lanes 0-31) and
-      // KL / 2 + s (lanes 32-63) of that range, so that a lane walks consecutive addresses
-      const float* ap = s_M + (32 * rt + ln) * MS + ks * KL + hh * (KL / 2);
-      const float* bp = s_S + (ks * KL + hh * (KL / 2)) * 33 + ln;
-      rs_f32x16 t;
+    for (int r = 0; r < 4; ++r) to[row[r] * width] = S[r];
+  };
+  auto advance = [&](int p, Set& x) __attribute__((always_inline)) {
+    // (in front of the group's own segments: to the place of the first of them, which is written again)
+    if (!COMPOSE) store(p0 + max(p - lead, 0), V);
+    s_x[p & 1][wave][lane] = S;
+    // two sums, so that a product does not wait for the one in front of it; N joins last (the smaller roundings)
+    rs_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, more = acc, n;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) t[r] = 0.0f;
+    for (int r = 0; r < 4; ++r) n[r] = is_m ? 0.0f : x.n[r];
+    auto products = [&](int t, const rs_f32x4& b) __attribute__((always_inline)) {
 #pragma unroll
-      for (int s0 = 0; s0 < KL / 2; s0 += 8) {  // operands of eight steps, then their MFMAs
-        float av[8], bv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (s0 + u < KL / 2) {
-            av[u] = ap[s0 + u];
-            bv[u] = bp[(s0 + u) * 33];
-          }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (s0 + u < KL / 2) t = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u], t, 0, 0, 0);
+      for (int r = 0; r < 4; ++r) {
+        rs_f32x4& to = r & 1 ? more : acc;
+        to = __builtin_amdgcn_mfma_f32_16x16x4f32(inside[t] ? x.m[t][r] : 0.0f, b[r], to, 0, 0, 0);
       }
-      float* pp = s_P + (ks * ROWS + 32 * rt + 4 * hh) * 33 + ln;  // accumulator register r: row 8 (r / 4) + 4 hh + r % 4
-#pragma unroll
-      for (int r = 0; r < 16; ++r) pp[(8 * (r / 4) + (r % 4)) * 33] = t[r];
-    }
-    lds_barrier();  // the partial tiles are in LDS; every wave has read the old S and M_p
-#pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      const int i = rg + 8 * n;
-#pragma unroll
-      for (int part = 0; part < KS; ++part) acc[n] += s_P[(part * ROWS + i) * 33 + c];
-      s_S[i * 33 + c] = acc[n];
-    }
+    };
+    products(0, S);
     lds_barrier();
+    rs_f32x4 b[NT];
+#pragma unroll
+    for (int t = 1; t < NT; ++t) b[t] = s_x[p & 1][(wave + t) % NT][lane];
+#pragma unroll
+    for (int t = 1; t < NT; ++t) products(t, b[t]);
+    S = (acc + more) + n;
+    fetch(p + DEPTH, x);
   };
+  if (n_apply > 0) {
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) fetch(p0 + d, d);
-  __syncthreads();
-  int p = p0;
-  for (; p + DEPTH < p1; p += DEPTH) {  // DEPTH steps on fixed register sets
+    for (int d = 0; d < DEPTH; ++d) fetch(d, set[d]);
+    int p = 0;
+    for (; p + DEPTH <= n_apply; p += DEPTH) {  // DEPTH steps on fixed register sets
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) advance(p + d, d);
-  }
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d)
-    if (p + d + 1 < p1) advance(p + d, d);
-  store_start(p1 - 1);
-  if (COMPOSE) {  // the group's map, in the layout of the segments' maps
-    float* out = sinit + ((int64_t)blockIdx.y * HV + hv) * K * W;
-#pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      const int i = min(rg + 8 * n, K - 1);
-      out[(int64_t)i * W + colc] = s_S[i * 33 + c];
+      for (int d = 0; d < DEPTH; ++d) advance(p + d, set[d]);
     }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (p + d < n_apply) advance(p + d, set[d]);
   }
+  if (COMPOSE) store(blockIdx.y, W);
+  else store(p0 + cnt - 1, V);
 }
 
 template <typename T>
@@ -611,109 +660,52 @@ static int gdr_recurrent_segmented(const void* q, const void* k, const void* v, 
                                    int K, int V, float scale, int l2norm, float* mn, float* sinit, float* groups,
                                    hipStream_t s) {
   LAMPA_PROF(s, "start");
-  const dim3 grid_a((K + V + 31) / 32, n_seg * HV), grid_b((V + 31) / 32, n_seg * HV);
-#define GDR_REC_SEG(KT) GDR_REC_SEG2(KT, false, false)
-#define GDR_REC_SEG2(KT, SHORT_A, SHORT_B)                                                                           \
-  do {                                                                                                               \
-    hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, KT, true, SHORT_A>), grid_a, dim3(64), 0, s, (const T*)k, (const T*)k,  \
-                       (const T*)v, g, beta, (T*)nullptr, (const float*)nullptr, mn, cu_seg, (int64_t)0, H, HV, K,   \
-                       K + V, scale, l2norm, (const int32_t*)nullptr);                                               \
-    LAMPA_PROF(s, "gdr_recurrent_split_kernel<composite>");                                                          \
-    if (gdr_segment_scan(mn, h0, seq_seg0, n_seq, n_seg, HV, K, V, sinit, groups, s) != LAMPA_OK)                    \
-      return LAMPA_ERR_LAUNCH;                                                                                       \
-    LAMPA_PROF(s, "start");                                                                                          \
-    hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, KT, false, SHORT_B>), grid_b, dim3(64), 0, s, (const T*)q, (const T*)k, \
-                       (const T*)v, g, beta, (T*)o, sinit, ht, cu_seg, (int64_t)0, H, HV, K, V, scale, l2norm,       \
-                       seg_out);                                                                                     \
-    LAMPA_PROF(s, "gdr_recurrent_split_kernel");                                                                     \
-  } while (0)
-  const bool short_a = gdr_rec_short_groups(grid_a), short_b = gdr_rec_short_groups(grid_b);
-  if (K <= 16) GDR_REC_SEG(16);
-  else if (K <= 32) GDR_REC_SEG(32);
-  else if (K <= 64) {
-    if (short_a && short_b) GDR_REC_SEG2(64, true, true);
-    else if (short_a) GDR_REC_SEG2(64, true, false);
-    else if (short_b) GDR_REC_SEG2(64, false, true);
-    else GDR_REC_SEG(64);
-  } else GDR_REC_SEG(128);
-#undef GDR_REC_SEG
-#undef GDR_REC_SEG2
+  gdr_split_launch<T, true>(k, k, v, g, beta, nullptr, nullptr, mn, cu_seg, n_seg, 0, H, HV, K, K + V, scale, l2norm, nullptr, s);
+  LAMPA_PROF(s, "gdr_recurrent_split_kernel<composite>");
+  if (gdr_segment_scan(mn, h0, seq_seg0, n_seq, n_seg, HV, K, V, sinit, groups, s) != LAMPA_OK) return LAMPA_ERR_LAUNCH;
+  LAMPA_PROF(s, "start");
+  gdr_split_launch<T, false>(q, k, v, g, beta, o, sinit, ht, cu_seg, n_seg, 0, H, HV, K, V, scale, l2norm, seg_out, s);
+  LAMPA_PROF(s, "gdr_recurrent_split_kernel");
   return lampa_launch_status();
 }
 
 // The first two launches above on their own, for the backward pass (gdr_backward.hip), which needs the maps and the
 // states the segments start from but not the outputs; the scan is also run a second time there, over the transposed
 // maps in reverse segment order.
-static int gdr_scan_attr() {
-  static bool attr_set[64] = {};  // per device: the widest scans' dynamic LDS limit (a repeated set is harmless)
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return LAMPA_ERR_LAUNCH;
-  if (!attr_set[dev]) {
-    if (hipFuncSetAttribute((const void*)gdr_segment_scan_kernel<128, 1, false>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)RsScanShape<128>::LDS_BYTES) != hipSuccess ||
-        hipFuncSetAttribute((const void*)gdr_segment_scan_kernel<128, 1, true>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)RsScanShape<128>::LDS_BYTES) != hipSuccess)
-      return LAMPA_ERR_LAUNCH;
-    attr_set[dev] = true;
-  }
-  return LAMPA_OK;
-}
-
-template <typename T>
-static void gdr_segment_maps_typed(const void* k, const void* v, const float* g, const float* beta,
-                                   const int64_t* cu_seg, int n_seg, int H, int HV, int K, int V, int l2norm, float* mn,
-                                   hipStream_t s) {
-  const dim3 grid_a((K + V + 31) / 32, n_seg * HV);
-#define GDR_REC_MAPS(KT)                                                                                            \
-  hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, KT, true>), grid_a, dim3(64), 0, s, (const T*)k, (const T*)k,   \
-                     (const T*)v, g, beta, (T*)nullptr, (const float*)nullptr, mn, cu_seg, (int64_t)0, H, HV, K,    \
-                     K + V, 1.0f, l2norm, (const int32_t*)nullptr)
-  if (K <= 16) GDR_REC_MAPS(16);
-  else if (K <= 32) GDR_REC_MAPS(32);
-  else if (K <= 64) {
-    if (gdr_rec_short_groups(grid_a))
-      hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, 64, true, true>), grid_a, dim3(64), 0, s, (const T*)k,
-                         (const T*)k, (const T*)v, g, beta, (T*)nullptr, (const float*)nullptr, mn, cu_seg, (int64_t)0,
-                         H, HV, K, K + V, 1.0f, l2norm, (const int32_t*)nullptr);
-    else GDR_REC_MAPS(64);
-  } else GDR_REC_MAPS(128);
-#undef GDR_REC_MAPS
-}
-
 int gdr_segment_maps(const void* k, const void* v, const float* g, const float* beta, const int64_t* cu_seg, int n_seg,
                      int H, int HV, int K, int V, int dtype, int l2norm, float* mn, hipStream_t s) {
   LAMPA_PROF(s, "start");
+#define GDR_MAPS(T)                                                                                                      \
+  gdr_split_launch<T, true>(k, k, v, g, beta, nullptr, nullptr, mn, cu_seg, n_seg, 0, H, HV, K, K + V, 1.0f, l2norm, nullptr, s)
   switch (dtype) {
-    case GDR_BF16: gdr_segment_maps_typed<__bf16>(k, v, g, beta, cu_seg, n_seg, H, HV, K, V, l2norm, mn, s); break;
-    case GDR_FP16: gdr_segment_maps_typed<_Float16>(k, v, g, beta, cu_seg, n_seg, H, HV, K, V, l2norm, mn, s); break;
-    case GDR_FP32: gdr_segment_maps_typed<float>(k, v, g, beta, cu_seg, n_seg, H, HV, K, V, l2norm, mn, s); break;
+    case GDR_BF16: GDR_MAPS(__bf16); break;
+    case GDR_FP16: GDR_MAPS(_Float16); break;
+    case GDR_FP32: GDR_MAPS(float); break;
     default: return LAMPA_ERR_INVALID;
   }
+#undef GDR_MAPS
   LAMPA_PROF(s, "gdr_recurrent_split_kernel<composite>");
   return lampa_launch_status();
 }
 
-// Group slots of the three-launch scan: at most GDR_SCAN_GROUP_SEQS sequences of together at most
-// GDR_SCAN_GROUP_SEGS segments take it; groups of gs = ceil(sqrt(n_seg / n_seq)) segments, at most
-// maxg = ceil(n_seg / gs) of them in a sequence however the segments are spread, so n_seq * maxg <=
-// n_seq^1.5 sqrt(n_seg) + n_seq slots of a map [K, K + V] and a state [K, V] each.
+// Group slots of the two-launch scan: at most GDR_SCAN_GROUP_SEQS sequences of together at most GDR_SCAN_GROUP_SEGS
+// segments take it; groups of gs = ceil(sqrt(n_seg / (2 n_seq))) segments, at most maxg = ceil(n_seg / gs) of them in a
+// sequence however the segments are spread, so n_seq * maxg <= n_seq^1.5 sqrt(2 n_seg) + n_seq slots of a map [K, K + V].
 #define GDR_SCAN_GROUP_SEQS 4
 #define GDR_SCAN_GROUP_SEGS 4096
 int64_t gdr_scan_group_floats(int n_seg, int HV, int K, int V) {
   if (n_seg > GDR_SCAN_GROUP_SEGS) return 0;
   int64_t root = 1;
   while (root * root < n_seg) ++root;
-  return (8 * root + GDR_SCAN_GROUP_SEQS) * HV * K * (int64_t)(K + 2 * V);
+  return (12 * root + GDR_SCAN_GROUP_SEQS) * HV * K * (int64_t)(K + V);
 }
 
 int gdr_segment_scan(const float* mn, const float* h0, const int32_t* seq_seg0, int n_seq, int n_seg, int HV, int K,
                      int V, float* sinit, float* groups, hipStream_t s) {
-  const int rc = gdr_scan_attr();
-  if (rc != LAMPA_OK) return rc;
   const int W = K + V;
-#define GDR_REC_SCAN(KT, COMPOSE, GRID, MAPS, H0, COLS, OUT, MODE, GS, MAXG)                                      \
-  hipLaunchKernelGGL((gdr_segment_scan_kernel<KT, (KT <= 32 ? 4 : KT == 64 ? 2 : 1), COMPOSE>), GRID, dim3(256),   \
-                     RsScanShape<KT>::LDS_BYTES, s, MAPS, H0, seq_seg0, HV, K, COLS, OUT, MODE, GS, MAXG, W)
+#define GDR_REC_SCAN(KT, COMPOSE, GROUPS, COLS, OUT, GS, MAXG)                                                          \
+  hipLaunchKernelGGL((gdr_segment_scan_kernel<KT, COMPOSE>), dim3((COLS + 15) / 16, n_seq * (MAXG), HV),                \
+                     dim3(64 * RsScanShape<KT>::NT), 0, s, mn, GROUPS, h0, seq_seg0, HV, K, COLS, OUT, GS, MAXG, W)
 #define GDR_REC_SCAN_ANY(...)                        \
   do {                                               \
     if (K <= 16) GDR_REC_SCAN(16, __VA_ARGS__);      \
@@ -721,27 +713,16 @@ int gdr_segment_scan(const float* mn, const float* h0, const int32_t* seq_seg0, 
     else if (K <= 64) GDR_REC_SCAN(64, __VA_ARGS__); \
     else GDR_REC_SCAN(128, __VA_ARGS__);             \
   } while (0)
-  // a few long sequences: groups of about sqrt(segments per sequence) segments, three launches of that many steps
-  if (groups && n_seq <= GDR_SCAN_GROUP_SEQS && n_seg <= GDR_SCAN_GROUP_SEGS && n_seg >= 24 * n_seq) {
-    int gs = 1;
-    while (gs * gs * n_seq < n_seg) ++gs;
-    const int maxg = (n_seg + gs - 1) / gs;
-    float* gmaps = groups;                                                  // [n_seq * maxg, HV, K, K + V]
-    float* gstart = groups + (int64_t)n_seq * maxg * HV * K * W;            // [n_seq * maxg, HV, K, V]
-    LAMPA_PROF(s, "start");
-    const dim3 grid_a((W + 31) / 32, n_seq * maxg, HV), grid_b((V + 31) / 32, n_seq, HV),
-        grid_c((V + 31) / 32, n_seq * maxg, HV);
-    GDR_REC_SCAN_ANY(true, grid_a, mn, (const float*)nullptr, W, gmaps, RS_COMPOSE, gs, maxg);
-    LAMPA_PROF(s, "gdr_segment_scan_kernel<compose>");
-    GDR_REC_SCAN_ANY(false, grid_b, (const float*)gmaps, h0, V, gstart, RS_GROUPS, gs, maxg);
-    LAMPA_PROF(s, "gdr_segment_scan_kernel<groups>");
-    GDR_REC_SCAN_ANY(false, grid_c, mn, (const float*)gstart, V, sinit, RS_WITHIN, gs, maxg);
-    LAMPA_PROF(s, "gdr_segment_scan_kernel<within>");
-    return lampa_launch_status();
-  }
   LAMPA_PROF(s, "start");
-  const dim3 grid((V + 31) / 32, n_seq, HV);
-  GDR_REC_SCAN_ANY(false, grid, mn, h0, V, sinit, RS_PLAIN, 0, 1);
+  int gs = n_seg, maxg = 1;
+  if (groups && n_seq <= GDR_SCAN_GROUP_SEQS && n_seg <= GDR_SCAN_GROUP_SEGS && n_seg >= 24 * n_seq) {
+    gs = 1;
+    while (2 * gs * gs * n_seq < n_seg) ++gs;
+    maxg = (n_seg + gs - 1) / gs;
+    GDR_REC_SCAN_ANY(true, (const float*)nullptr, W, groups, gs, maxg);
+    LAMPA_PROF(s, "gdr_segment_scan_kernel<compose>");
+  }
+  GDR_REC_SCAN_ANY(false, (const float*)groups, V, sinit, gs, maxg);
 #undef GDR_REC_SCAN_ANY
 #undef GDR_REC_SCAN
   LAMPA_PROF(s, "gdr_segment_scan_kernel");

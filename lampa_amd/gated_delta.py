@@ -171,6 +171,19 @@ def output_pass_config(narrow: int = 1) -> None:
 # would otherwise occupy less than a quarter of the chip (None: never).
 SEGMENT_MIN_TOKENS: Optional[int] = 512
 
+def _segment_tokens(tokens: int, n_value_heads: int, K: int, V: int) -> int:
+    """Segment length of the segmented token-serial operator, a multiple of 32 (the kernel's groups of tokens): two waves
+    of 16 value columns per SIMD in the output pass; one per SIMD where that leaves heads wider than 32 fewer than 128 tokens
+    a segment (their maps are the larger part then). Measured against all lengths from 16 to 1 024, fp32, us with this rule
+    / best: 8 192 x 4 x 32 x 32 53 / 51, 1 000 x 4 x 32 x 32 27 / 27, 30 000 x 8 x 32 x 32 148 / 148, 3 000 x 8 x 64 x 64
+    76 / 76, 8 192 x 4 x 64 x 64 93 / 93, 30 000 x 8 x 64 x 64 410 / 410, 2 x 8 192 x 4 x 128 x 128 499 / 447."""
+    work = tokens * n_value_heads * -(-V // 16)
+    seg_len = -(-work // 2048 // 32) * 32
+    if K > 32 and seg_len < 128:
+        seg_len = -(-work // 1024 // 32) * 32
+    return max(32, seg_len)
+
+
 _segment_cache = {}
 
 
@@ -227,9 +240,7 @@ def _recurrent_launch(q, k, v, g, beta, scale, initial_state, output_final_state
         # a few long sequences: one or two waves each would leave most of the chip idle
         cu_host = _sequence_bounds(cu_seqlens, B, T)
         if max(b - a for a, b in zip(cu_host[:-1], cu_host[1:])) >= SEGMENT_MIN_TOKENS:
-            want = max(1, 1024 // (HV * slabs))  # segments for about one wave per SIMD in the output pass (the scan
-            # between the passes is serial in the groups of segments: no more of them than fill the chip)
-            seg_len = max(64, -(-(cu_host[-1] // want) // 64) * 64)
+            seg_len = _segment_tokens(cu_host[-1], HV, K, V)
             return _recurrent_segmented_launch(q, k, v, g, beta, scale, initial_state, output_final_state, cu_host,
                                                seg_len, l2norm)
     if cu_seqlens is not None:

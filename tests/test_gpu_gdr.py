@@ -603,3 +603,39 @@ def test_segments_that_cut_off_what_lies_before_them(device, K, V, dtype, monkey
     o2, s2 = gd.chunk_gated_delta_rule(*args, initial_state=bad_h0.to(device), output_final_state=True)
     assert not torch.isfinite(o2[0, :, 0, 7]).any() and not torch.isfinite(s2[0, 0, :, 7]).any()
     assert torch.equal(o2[:, :, 1:], o[:, :, 1:]) and torch.equal(s2[:, 1:], s[:, 1:])
+
+
+@pytest.mark.parametrize("K,V", [(4, 1), (16, 33), (32, 15), (36, 64), (64, 17), (68, 130), (128, 16)])
+def test_recurrent_groups_of_tokens_and_odd_columns(device, K, V):
+    # the split kernel at the edges of its groups of 16 and 32 tokens, of its 16 columns a wave and of its row tiles, with
+    # states that do not lie in pairs of columns; more sequences of it than the chip has room for at once
+    cu = torch.tensor([0, 1, 1, 3, 34, 66, 99, 114, 130, 147, 212], dtype=torch.long)
+    T, H, HV = int(cu[-1]), 2, 4
+    q, k, _, _, _ = synth.gdr_inputs(1, T, H, K, V, torch.float32, seed=K, g_scale=0.2)
+    _, _, v, g, beta = synth.gdr_inputs(1, T, HV, K, V, torch.float32, seed=V, g_scale=0.2)
+    h0 = torch.randn(len(cu) - 1, HV, K, V, generator=torch.Generator().manual_seed(2))
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta, initial_state=h0, cu_seqlens=cu, l2=og.L2_RECURRENT)
+    o, s = gd.fused_recurrent_gated_delta_rule(*_to(device, q, k, v, g, beta), initial_state=h0.to(device),
+                                               output_final_state=True, cu_seqlens=cu.to(device), use_qk_l2norm_in_kernel=True)
+    assert _errors(o, want_o)[0] <= FP32_TOL and _errors(s, want_s)[0] <= FP32_TOL
+    B = 600
+    many = [x[:, :33].expand(B, *x[:, :33].shape[1:]).contiguous().to(device) for x in (q, k, v, g, beta)]
+    hb = h0[:1].expand(B, HV, K, V).contiguous().to(device)
+    want_o, want_s = og.recurrent_c(*[x[:, :33].contiguous() for x in (q, k, v, g, beta)], initial_state=h0[:1])
+    o, s = gd.fused_recurrent_gated_delta_rule(*many, initial_state=hb, output_final_state=True)
+    assert torch.equal(o, o[:1].expand_as(o)) and torch.equal(s, s[:1].expand_as(s))
+    assert _errors(o[:1], want_o)[0] <= FP32_TOL and _errors(s[:1], want_s)[0] <= FP32_TOL
+
+
+@pytest.mark.parametrize("K,V,lens", [(16, 8, [1500]), (32, 32, [513, 0, 1700]), (48, 20, [900, 800]), (64, 64, [2300]),
+                                      (68, 12, [1100]), (128, 36, [700, 640, 520, 40])])
+def test_recurrent_scan_in_groups_of_segments(device, K, V, lens):
+    # 32-token segments scanned in groups, in two launches: ragged last groups and segments, row tiles that are not full,
+    # columns that are not a multiple of 16, an empty and a short sequence among the long ones; weak decay
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.long)
+    q, k, v, g, beta = synth.gdr_inputs(1, int(cu[-1]), 2, K, V, torch.float32, seed=K + V, g_scale=0.01)
+    h0 = torch.randn(len(lens), 2, K, V, generator=torch.Generator().manual_seed(6))
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta, initial_state=h0, cu_seqlens=cu)
+    o, s = gd.fused_recurrent_gated_delta_rule(*_to(device, q, k, v, g, beta), initial_state=h0.to(device),
+                                               output_final_state=True, cu_seqlens=cu.to(device))
+    assert _errors(o, want_o)[0] <= FP32_TOL and _errors(s, want_s)[0] <= FP32_TOL
