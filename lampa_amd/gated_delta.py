@@ -23,6 +23,7 @@ import warnings
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 from . import _capi
 from ._capi import check, ptr, require_cuda, stream_of
@@ -246,7 +247,7 @@ def _recurrent_launch(q, k, v, g, beta, scale, initial_state, output_final_state
     if cu_seqlens is not None:
         _sequence_bounds(cu_seqlens, B, T)
     o = torch.empty_like(v)
-    ht = torch.empty((n_seq, HV, K, V), dtype=torch.float32, device=q.device) if output_final_state else None
+    ht = g.new_empty((n_seq, HV, K, V)) if output_final_state else None
     cu = None if cu_seqlens is None else cu_seqlens.to(device=q.device, dtype=torch.int64).contiguous()
     h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
     fn = _capi.lib().lampa_gdr_recurrent_headwise_fwd if headwise else _capi.lib().lampa_gdr_recurrent_fwd
@@ -540,10 +541,8 @@ class _GatedDelta(torch.autograd.Function):
     @staticmethod
     def forward(ctx, launcher, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm,
                 differentiable, grad_mode):
-        require_cuda(q, k, v, g, beta, initial_state)
         ctx.g_dtype, ctx.beta_dtype = g.dtype, beta.dtype
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
+        q, k, v, g, beta = _operands(q, k, v, g, beta, initial_state)
         ctx.differentiable = differentiable
         ctx.kept = None
         ctx.set_materialize_grads(False)
@@ -598,10 +597,36 @@ class _GatedDelta(torch.autograd.Function):
         return (None, dq, dk, dv, dg.to(ctx.g_dtype), dbeta.to(ctx.beta_dtype), None, dh0, None, None, None, None, None)
 
 
+_functorch_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+
+
+def _direct(*tensors) -> bool:
+    """Whether a call may go to its launcher without an autograd function around it, which costs 5 of the 17 us of a call on a
+    few tokens: no gradient can be asked for, and nothing looks on that would have to see the function (tracing, compilation,
+    vmap and the other functorch transforms, forward-mode gradients, tensor subclasses)."""
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) is not torch.Tensor or (grad and t.requires_grad) or _functorch_wrapped(t)):
+            return False
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+                or torch._C._are_functorch_transforms_active() or _forward_ad._current_level >= 0)
+
+
+def _operands(q, k, v, g, beta, initial_state):
+    """The tensors as the launchers read them: on the GPU, contiguous, g and beta in fp32."""
+    require_cuda(q, k, v, g, beta, initial_state)
+    return (q.contiguous(), k.contiguous(), v.contiguous(), g.to(torch.float32).contiguous(),
+            beta.to(torch.float32).contiguous())
+
+
 def _check_shapes(q, k, v, g, beta, what, headwise_beta_ok=False):
     """g and beta are per (token, value head): [B, T, HV]. The reference's token-serial kernel also takes a headwise
     beta [B, T, HV, V] (``gated_delta_rule_ori.py:444-447,515``), and so does ``fused_recurrent_gated_delta_rule`` here;
     the chunk operator has no such form (the reference asserts ``len(beta.shape) == 3`` there)."""
+    qs, vs, gs = q.shape, v.shape, g.shape
+    if (len(qs) == 4 and k.shape == qs and len(vs) == 4 and vs[0] == qs[0] and vs[1] == qs[1] and vs[2] % qs[2] == 0
+            and gs == vs[:3] and beta.shape == gs):
+        return
     if q.dim() != 4 or k.shape != q.shape or v.dim() != 4 or v.shape[:2] != q.shape[:2]:
         raise ValueError(f"{what}: expected q, k [B, T, H, K] and v [B, T, HV, V], got {tuple(q.shape)}, "
                          f"{tuple(k.shape)}, {tuple(v.shape)}")
@@ -656,6 +681,8 @@ def chunk_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g:
         scale = k.shape[-1] ** -0.5
     l2norm = L2_CHUNK if use_qk_l2norm_in_kernel else L2_NONE
     launcher = _chunk_launch_any_head if _chunk_path_supported(q, v) else _recurrent_launch
+    if _direct(q, k, v, g, beta, initial_state, cu_seqlens):
+        return launcher(*_operands(q, k, v, g, beta, initial_state), scale, initial_state, output_final_state, cu_seqlens, l2norm)
     o, final_state = _GatedDelta.apply(launcher, q, k, v, g, beta, scale, initial_state, output_final_state,
                                        cu_seqlens, l2norm, True, torch.is_grad_enabled())
     return o.to(q.dtype), final_state
@@ -678,5 +705,8 @@ def fused_recurrent_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.
         beta = torch.ones_like(g)
     _check_shapes(q, k, v, g, beta, "fused_recurrent_gated_delta_rule", headwise_beta_ok=True)
     l2norm = L2_RECURRENT if use_qk_l2norm_in_kernel else L2_NONE
+    if _direct(q, k, v, g, beta, initial_state, cu_seqlens):
+        return _recurrent_launch(*_operands(q, k, v, g, beta, initial_state), scale, initial_state, output_final_state,
+                                 cu_seqlens, l2norm)
     return _GatedDelta.apply(_recurrent_launch, q, k, v, g, beta, scale, initial_state, output_final_state,
                              cu_seqlens, l2norm, False, torch.is_grad_enabled())

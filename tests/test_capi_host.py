@@ -534,3 +534,21 @@ def test_bench_reads_the_traffic_table_of_the_committed_profile():
             text = open(os.path.join(prof, name)).read()
             assert re.search(r"^commit: [0-9a-f]{7,40}\b", text, flags=re.M), name
             assert "rocprofv3" in text, name
+
+
+def test_calls_that_go_to_their_launcher_directly():
+    # without an autograd function around it only where none could be missed: no gradients, no transform or trace looking on
+    from lampa_amd import gated_delta as gd
+    from torch.autograd import forward_ad
+
+    x, leaf = torch.zeros(2, 3), torch.zeros(2, 3, requires_grad=True)
+    assert gd._direct(x, None, x) and not gd._direct(x, leaf)
+    with torch.no_grad():
+        assert gd._direct(x, leaf)
+    assert not gd._direct(torch.nn.Parameter(x, requires_grad=False))
+    with forward_ad.dual_level():
+        assert not gd._direct(x)
+    seen = []
+    torch.func.vmap(lambda y: (seen.append(gd._direct(x)), y)[1])(x)
+    torch.jit.trace(lambda y: (seen.append(gd._direct(x)), y + 1)[1], (x,), check_trace=False)
+    assert seen == [False, False] and gd._direct(x)
