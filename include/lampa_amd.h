@@ -406,8 +406,9 @@ int lampa_hgdn_step(const void* q, const void* k, const void* v, const float* g,
 /* Several tokens of the hierarchical rule in one launch: tokens tok0 .. n_tok - 1 of every sequence, on the level states
  * after its first tok0 tokens (the remainder of hattention_prefill, models/hattention/kernel.py:467-575, behind the whole
  * chunks). q, k [B, n_tok, H, K]; v, o [B, n_tok, HV, V]; g, beta fp32 [B, n_tok, HV]; lam [B, n_tok, HV, L]; only rows
- * tok0 .. of them are read or written; states fp32 [B, HV, K, V, L] updated in place. K <= 128, L <= 32 and enough levels for
- * n_tok tokens. */
+ * tok0 .. of them are read or written; states fp32 [B, HV, K, V, L] updated in place: every level is written, and with L <= 17
+ * only levels that hold tokens are read (the others may be uninitialised). K <= 128, L <= 32 and enough levels for n_tok
+ * tokens. */
 int lampa_hgdn_tail(const void* q, const void* k, const void* v, const float* g, const float* beta, const void* lam,
                     int lam_dtype, float lam_div, float* states, void* o, int B, int n_tok, int tok0, int H, int HV, int K,
                     int V, int L, int dtype, float scale, int l2norm, void* stream);

@@ -462,19 +462,27 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
 }
 
 // ---- the tokens behind the whole chunks, in one launch -----------------------------------------------------------------
-// A wavefront owns one value column of one (sequence, value head): lane = state row (two rows for K > 64), the row's LM level
-// values in registers from the first token to the last, so a token costs no barrier, no LDS and no pass over the states.
-// Sums over the rows (k^T S_l for the levels > 0, the output, the two norms) are exchanges between lanes: 16 levels at a time
-// are halved four times until a lane holds one level's sum over its group of 16 lanes (`wave_sums16`), and go back to all
-// lanes as scalars. What bounds it is that serial chain per token (B * HV * V wavefronts, two per compute unit at 8 heads of
-// 64 columns); the next token's values are loaded while this one is worked on.
+// A wavefront owns one value column of one (sequence, value head), in one of two layouts. What bounds both is the serial chain
+// of a token (B * HV * V wavefronts, two per compute unit at 8 heads of 64 columns).
+//
+// hgdn_tail_kernel (up to 17 levels, sequences of up to 65 536 tokens): lane = (row group, level), a lane holds a quarter of
+// the rows of one level > 0. All levels take a token's transition at once: k^T S_l is a lane's own sum over its rows and two
+// register swaps over the row groups, the update a multiply and an fma per row. Level 0, the last token alone, is never
+// stored: it enters the output as a scalar and the state of the level it cascades into as one fma per row; the levels
+// between are summed over 16 lanes (DPP) every second token. k, q (normalised, fp32), the decays, the weights and v of 32
+// tokens are staged in LDS by the workgroup's four waves, so a token waits for no load. Levels that hold no token yet are
+// not read, and written as the zeros they are.
+// hgdn_tail_rows_kernel (more levels): lane = state row (two rows for K > 64), the row's LM level values in registers. Sums
+// over the rows (k^T S_l for the levels > 0, the output, the two norms) are exchanges between lanes: 16 levels at a time are
+// halved four times until a lane holds one level's sum over its group of 16 lanes (`wave_sums16`), and go back to all lanes
+// as scalars; the next token's values are loaded while this one is worked on.
 // A prefill of 15 000 tokens (24 behind its whole chunks, 8 heads of 64 x 64): 708 us with a launch of the single-token kernel
-// and its copies per token, 210 us with this kernel (54 us of them its own), 188 us (37) since no load is converted on
-// the spot under a condition.
+// and its copies per token, 188 us with the rows kernel (its own 38), TAIL_FIGURES.
 #define HGS_TAIL_LEVELS 17  // levels of the narrow instantiation: sequences up to 65 536 tokens
 #define HGS_TAIL_WAVES 4
 #define HGS_DPP_ROR8 0x128
 #define HGS_DPP_HALF_MIRROR 0x141
+#define HGS_DPP_MIRROR 0x140
 
 __device__ __forceinline__ float hgs_fold32(float a, float b) {  // lanes < 32: both halves of a, lanes >= 32: of b
   const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
@@ -516,7 +524,7 @@ __device__ __forceinline__ float hgs_lane(float x, int n) {
 
 template <typename T, int LM, int ROWS>
 __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
-    hgdn_tail_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
+    hgdn_tail_rows_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                      const float* __restrict__ g, const float* __restrict__ beta, const void* __restrict__ lam,
                      int lam_dtype, float lam_div, float* __restrict__ states, T* __restrict__ o, int n_tok, int tok0, int H,
                      int HV, int K, int V, int L, float scale, int l2norm) {
@@ -665,6 +673,172 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
   }
 }
 
+#define HGS_TAIL_BATCH 32  // tokens staged at a time
+
+template <typename T, int RP>
+__global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
+    hgdn_tail_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
+                     const float* __restrict__ g, const float* __restrict__ beta, const void* __restrict__ lam,
+                     int lam_dtype, float lam_div, float* __restrict__ states, T* __restrict__ o, int n_tok, int tok0, int H,
+                     int HV, int K, int V, int L, float scale, int l2norm) {
+  constexpr int KP = 4 * RP, NB = HGS_TAIL_BATCH, TPW = NB / HGS_TAIL_WAVES, NR = KP / 64;
+  __shared__ __align__(16) float s_k[NB][KP], s_q[NB][KP];
+  __shared__ float s_lam[NB][HGS_TAIL_LEVELS], s_v[NB][HGS_TAIL_WAVES];
+  __shared__ float4 s_sc[NB];  // e^g, beta, k . q
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int rg = lane >> 4, level = 1 + (lane & 15);
+  const int j = min((int)blockIdx.y * HGS_TAIL_WAVES + wave, V - 1);  // (waves past V work on the last column, storing nothing)
+  const bool live = (int)blockIdx.y * HGS_TAIL_WAVES + wave < V;
+  const int b = blockIdx.x / HV, hv = blockIdx.x % HV, h = hv / (HV / H);
+  float* col = states + (((size_t)b * HV + hv) * K * V + j) * L;  // row i: col + i * V * L
+  // (loads come from clamped addresses without conditions on the lane and are masked where they are used)
+  const bool filled = level < L && tok0 > 0 && ((tok0 - 1) >> (level - 1)) & 1;  // tokens in this lane's level
+  float S[RP], prev[RP];  // prev: the k of the token before (first token: level 0 as it was)
+#pragma unroll
+  for (int r = 0; r < RP; ++r) {
+    const size_t at = (size_t)min(rg * RP + r, K - 1) * V * L;
+    S[r] = col[at + min(level, L - 1)];
+    prev[r] = col[at];
+  }
+#pragma unroll
+  for (int r = 0; r < RP; ++r) {
+    S[r] = filled && rg * RP + r < K ? S[r] : 0.0f;
+    prev[r] = tok0 > 0 && rg * RP + r < K ? prev[r] : 0.0f;
+  }
+  float prev_v = 1.0f;  // beta v of the token before
+  auto stage = [&](int t0) __attribute__((always_inline)) {  // tokens t0 .. t0 + NB - 1, TPW of them by each wave
+    T kr[TPW][NR], qr[TPW][NR];
+    uint32_t lr[TPW];
+    float gr[TPW], br[TPW];
+    T vr[TPW];
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      const size_t tok = (size_t)b * n_tok + min(t0 + wave * TPW + i, n_tok - 1);
+#pragma unroll
+      for (int x = 0; x < NR; ++x) {
+        const int e = min(lane + 64 * x, K - 1);
+        kr[i][x] = k[(tok * H + h) * K + e];
+        qr[i][x] = q[(tok * H + h) * K + e];
+      }
+      const size_t li = (tok * HV + hv) * L + min(lane, L - 1);
+      lr[i] = lam_dtype == GDR_FP32 ? reinterpret_cast<const uint32_t*>(lam)[li] : reinterpret_cast<const uint16_t*>(lam)[li];
+      gr[i] = g[tok * HV + hv];
+      br[i] = beta[tok * HV + hv];
+      vr[i] = v[(tok * HV + hv) * V + min((int)blockIdx.y * HGS_TAIL_WAVES + min(lane, HGS_TAIL_WAVES - 1), V - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      const int at = wave * TPW + i;
+      float kf[NR], qf[NR], ks = 0.0f, qs = 0.0f, kq = 0.0f;
+#pragma unroll
+      for (int x = 0; x < NR; ++x) {
+        kf[x] = lane + 64 * x < K ? GdrElem<T>::to_float(kr[i][x]) : 0.0f;
+        qf[x] = lane + 64 * x < K ? GdrElem<T>::to_float(qr[i][x]) : 0.0f;
+        ks = __builtin_fmaf(kf[x], kf[x], ks);
+        qs = __builtin_fmaf(qf[x], qf[x], qs);
+      }
+      float rq = scale, rk = 1.0f;
+      if (l2norm == GDR_L2_CHUNK) {
+        rq = scale / __fsqrt_rn(wave_sum_all(qs) + 1e-6f);
+        rk = 1.0f / __fsqrt_rn(wave_sum_all(ks) + 1e-6f);
+      } else if (l2norm == GDR_L2_RECURRENT) {
+        rq = scale / (__fsqrt_rn(wave_sum_all(qs)) + 1e-6f);
+        rk = 1.0f / (__fsqrt_rn(wave_sum_all(ks)) + 1e-6f);
+      }
+#pragma unroll
+      for (int x = 0; x < NR; ++x) {
+        kf[x] *= rk;
+        qf[x] *= rq;
+        kq = __builtin_fmaf(kf[x], qf[x], kq);
+        s_k[at][lane + 64 * x] = kf[x];
+        s_q[at][lane + 64 * x] = qf[x];
+      }
+      kq = wave_sum_all(kq);
+      float lam_l = lam_dtype == GDR_FP32   ? __uint_as_float(lr[i])
+                    : lam_dtype == GDR_BF16 ? __uint_as_float(lr[i] << 16)
+                                            : (float)__builtin_bit_cast(_Float16, (uint16_t)lr[i]);
+      if (lam_div != 1.0f) {  // lambda / scale, rounded to lambda's own type as the element-wise division would
+        lam_l = __fdiv_rn(lam_l, lam_div);
+        lam_l = lam_dtype == GDR_FP32 ? lam_l : lam_dtype == GDR_BF16 ? (float)(__bf16)lam_l : (float)(_Float16)lam_l;
+      }
+      if (lane < HGS_TAIL_LEVELS) s_lam[at][lane] = lane < L ? lam_l : 0.0f;
+      if (lane < HGS_TAIL_WAVES) s_v[at][lane] = GdrElem<T>::to_float(vr[i]);
+      if (lane == 0) s_sc[at] = make_float4(__expf(gr[i]), br[i], kq, 0.0f);
+    }
+  };
+  for (int t0 = tok0; t0 < n_tok; t0 += NB) {
+    if (t0 > tok0) __syncthreads();  // (the batch before has been read)
+    stage(t0);
+    __syncthreads();
+    const int n = min(NB, n_tok - t0);
+    for (int i = 0; i < n; ++i) {
+      const int t = t0 + i;
+      float kk[RP], qq[RP];
+#pragma unroll
+      for (int r = 0; r < RP; r += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&s_k[i][rg * RP + r]), y = *reinterpret_cast<const f32x4*>(&s_q[i][rg * RP + r]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { kk[r + e] = x[e]; qq[r + e] = y[e]; }
+      }
+      const float4 sc = s_sc[i];
+      const float lam_l = s_lam[i][level], lam_0 = s_lam[i][0], bv = sc.y * s_v[i][wave];
+      // cascade: after t tokens the levels below z = 1 + (trailing zero bits of t) are full and go into level z
+      const int z = t == 0 ? 0 : 1 + __builtin_ctz(t);
+      if (z > 1) {
+#pragma unroll
+        for (int r = 0; r < RP; ++r) {
+          float x = level < z ? S[r] : 0.0f;
+          x += dpp_f32<GDR_DPP_QUAD_XOR1, 0xF>(0.0f, x);
+          x += dpp_f32<GDR_DPP_QUAD_XOR2, 0xF>(0.0f, x);
+          x += dpp_f32<HGS_DPP_HALF_MIRROR, 0xF>(0.0f, x);
+          x += dpp_f32<HGS_DPP_MIRROR, 0xF>(0.0f, x);
+          S[r] = level < z ? 0.0f : level == z ? S[r] + x : S[r];
+        }
+      }
+      const float into = level == z ? prev_v : 0.0f;
+      if (t == tok0) {  // (level 0 as it came may hold anything)
+#pragma unroll
+        for (int r = 0; r < RP; ++r) S[r] = level == z ? S[r] + prev[r] : S[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < RP; ++r) S[r] = __builtin_fmaf(prev[r], into, S[r]);
+      }
+      float d0 = 0.0f, d1 = 0.0f;
+#pragma unroll
+      for (int r = 0; r < RP; r += 2) {
+        d0 = __builtin_fmaf(kk[r], S[r], d0);
+        d1 = __builtin_fmaf(kk[r + 1], S[r + 1], d1);
+      }
+      float d = d0 + d1;
+      d = hgs_fold32(d, d);
+      d = hgs_fold16(d, d);
+      const float c = -sc.y * d;
+      float y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+      for (int r = 0; r < RP; ++r) {
+        S[r] = sc.x * __builtin_fmaf(kk[r], c, S[r]);
+        prev[r] = kk[r];
+        if (r & 1) y1 = __builtin_fmaf(qq[r], S[r], y1);
+        else y0 = __builtin_fmaf(qq[r], S[r], y0);
+      }
+      prev_v = bv;
+      const float y = wave_sum_all(lam_l * (y0 + y1)) + lam_0 * (bv * sc.z);
+      if (lane == 0 && live) o[(((size_t)b * n_tok + t) * HV + hv) * V + j] = GdrElem<T>::from_float(y);
+    }
+  }
+  if (!live) return;
+#pragma unroll
+  for (int r = 0; r < RP; ++r) {
+    const int i = rg * RP + r;
+    if (i < K && level < L) col[(size_t)i * V * L + level] = S[r];
+  }
+  // level 0, the last token alone: a row per lane (the last batch is still in LDS)
+  const int last = (n_tok - 1 - tok0) % NB;
+#pragma unroll
+  for (int x = 0; x < NR; ++x)
+    if (lane + 64 * x < K) col[(size_t)(lane + 64 * x) * V * L] = s_k[last][lane + 64 * x] * prev_v;
+}
+
 // Tokens tok0 .. n_tok - 1 of every sequence on the level states after its first tok0 tokens: q, k [B, n_tok, H, K],
 // v, o [B, n_tok, HV, V], g, beta [B, n_tok, HV], lam [B, n_tok, HV, L], states [B, HV, K, V, L] updated in place.
 extern "C" int lampa_hgdn_tail(const void* q, const void* k, const void* v, const float* g, const float* beta,
@@ -682,25 +856,27 @@ extern "C" int lampa_hgdn_tail(const void* q, const void* k, const void* v, cons
     if (1 + __builtin_ctz(t) >= L) return LAMPA_ERR_INVALID;
   hipStream_t s = (hipStream_t)stream;
   LAMPA_PROF(s, "start");
-#define HGS_TAIL(TT, LM, RR)                                                                                               \
-  hipLaunchKernelGGL((hgdn_tail_kernel<TT, LM, RR>), dim3(B * HV, (V + HGS_TAIL_WAVES - 1) / HGS_TAIL_WAVES),              \
-                     dim3(64 * HGS_TAIL_WAVES), 0, s, (const TT*)q, (const TT*)k, (const TT*)v, g, beta, lam, lam_dtype,   \
-                     lam_div, states, (TT*)o, n_tok, tok0, H, HV, K, V, L, scale, l2norm)
-#define HGS_TAIL_ROWS(TT, LM)         \
-  do {                                \
-    if (K <= 64) HGS_TAIL(TT, LM, 1); \
-    else HGS_TAIL(TT, LM, 2);         \
+#define HGS_TAIL(KERNEL)                                                                                                   \
+  hipLaunchKernelGGL((KERNEL), dim3(B * HV, (V + HGS_TAIL_WAVES - 1) / HGS_TAIL_WAVES), dim3(64 * HGS_TAIL_WAVES), 0, s,   \
+                     (const TT*)q, (const TT*)k, (const TT*)v, g, beta, lam, lam_dtype, lam_div, states, (TT*)o, n_tok,    \
+                     tok0, H, HV, K, V, L, scale, l2norm)
+#define HGS_TAIL_CASE(TYPE)                                                      \
+  do {                                                                           \
+    typedef TYPE TT;                                                             \
+    if (L <= HGS_TAIL_LEVELS) {                                                  \
+      if (K <= 64) HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 16>);                  \
+      else HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 32>);                          \
+    } else {                                                                     \
+      if (K <= 64) HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA HGS_LMAX HGS_COMMA 1>); \
+      else HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA HGS_LMAX HGS_COMMA 2>);   \
+    }                                                                            \
   } while (0)
-#define HGS_TAIL_CASE(TT)                                          \
-  do {                                                             \
-    if (L <= HGS_TAIL_LEVELS) HGS_TAIL_ROWS(TT, HGS_TAIL_LEVELS);  \
-    else HGS_TAIL_ROWS(TT, HGS_LMAX);                              \
-  } while (0)
+#define HGS_COMMA ,
   if (dtype == GDR_BF16) HGS_TAIL_CASE(__bf16);
   else if (dtype == GDR_FP16) HGS_TAIL_CASE(_Float16);
   else HGS_TAIL_CASE(float);
 #undef HGS_TAIL_CASE
-#undef HGS_TAIL_ROWS
+#undef HGS_COMMA
 #undef HGS_TAIL
   LAMPA_PROF(s, "hgdn_tail_kernel");
   return lampa_launch_status();

@@ -59,12 +59,22 @@ class HState(object):
 
     def __init__(self, base: int, htype: HType, hstruct: HStruct, shape: Tuple[int, ...], dtype: torch.dtype,
                  device: torch.device) -> None:
+        self._fill(base, htype, hstruct, shape, dtype, device, torch.zeros)
+
+    @classmethod
+    def _of(cls, base, htype, hstruct, shape, dtype, device, make) -> "HState":
+        """A state whose tensor comes from ``make`` (``torch.empty``: a kernel writes all of it)."""
+        state = cls.__new__(cls)
+        state._fill(base, htype, hstruct, shape, dtype, device, make)
+        return state
+
+    def _fill(self, base, htype, hstruct, shape, dtype, device, make) -> None:
         if htype != HType.WEAK or base != 2 or hstruct != HStruct.GDELTA:
             raise NotImplementedError
         self.base, self.htype, self.hstruct = base, htype, hstruct
         self.shape, self.dtype, self.device = tuple(shape), dtype, device
         self.max_num_levels = self.shape[-1]
-        self.states = torch.zeros(self.shape, dtype=self.dtype, device=self.device)
+        self.states = make(self.shape, dtype=self.dtype, device=self.device)
         self._counts = [0] * self.max_num_levels  # host integers; ``counts`` shows them as the reference's tensor
 
     @property
@@ -231,8 +241,14 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     if initial_state is None:  # hattention_prefill, kernel.py:467-575
         require_cuda(q, k, v, g, l, beta)
         k, v, g, l, beta = _rows_of(B, T, k=(k, H, K), v=(v, HV, V), g=(g, HV), l=(l, HV, L), beta=(beta, HV))
-        hstate = HState(2, HType.WEAK, HStruct.GDELTA, (B, HV, K, V, L), torch.float32, q.device)
         T0 = T - T % 64
+        Vp = 64 if V <= 64 else 128
+        padded = T0 > 0 and (K, V) != (64, Vp)
+        one = T0 + 1 == T and B * HV * V * L >= ONE_TOKEN_STEP[T0 > 0]  # a single token, by the step kernel
+        # (the tail kernel writes every level and reads those that hold tokens, so nothing has to be zeroed in front of it)
+        fills = T0 < T and not one and K <= TAIL_MAX_K and L <= TAIL_FILLS_LEVELS and not padded
+        hstate = HState._of(2, HType.WEAK, HStruct.GDELTA, (B, HV, K, V, L), torch.float32, q.device,
+                            torch.empty if fills else torch.zeros)
         if T0 < T:  # (the tail kernel reads the whole tensors)
             q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
             g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
@@ -240,8 +256,6 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         if T0:
             _check_chunk_shapes(T0, K, V, L)
             cut = lambda x: x[:, :T0]
-            Vp = 64 if V <= 64 else 128
-            padded = (K, V) != (64, Vp)
             states = torch.zeros(B, HV, 64, Vp, L, dtype=torch.float32, device=q.device) if padded else hstate.states
             o = _ForwardOnly.apply(cut(q), cut(k), cut(v), cut(g), cut(l), cut(beta), scale, lam_div, states, T)
             if padded:  # (the padded rows and columns of the states are zero)
@@ -249,7 +263,7 @@ def chunk_h_gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
             hstate._set_counts(T0)
         else:
             o = torch.empty_like(v)
-        if T0 + 1 == T and B * HV * V * L >= ONE_TOKEN_STEP[T0 > 0]:
+        if one:
             if T0 == 0:
                 return _step(hstate, q, k, v, g, l, beta, scale, lam_div, token_dim=True), hstate
             o[:, T0] = _step(hstate, *(x[:, T0] for x in (q, k, v, g, l, beta)), scale, lam_div)
@@ -293,6 +307,7 @@ def _rows_of(B: int, T: int, **tensors):
 # a chunk 114 / 158 us at 2^16, 166 / 158 at 2^17, 269 / 216 at 2^18.
 ONE_TOKEN_STEP = 2 ** 15, 2 ** 17
 
+TAIL_FILLS_LEVELS = 17  # up to so many levels ``lampa_hgdn_tail`` writes every level and reads only those that hold tokens
 TAIL_MAX_K = 128  # ``lampa_hgdn_tail`` holds a state column in two registers per lane and level at most
 
 

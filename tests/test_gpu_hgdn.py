@@ -373,3 +373,29 @@ def test_single_token_by_the_step_and_by_the_tail_kernel(device, T, K, V, monkey
     assert o.shape == v.shape and torch.equal(s.counts, s2.counts)
     assert torch.allclose(s.states, s2.states, rtol=1e-5, atol=1e-6)
     assert torch.allclose(o.float(), o2.float(), rtol=2 ** -7, atol=1e-5)          # one rounding to bf16 of sums that differ
+
+
+@pytest.mark.parametrize("B,T,t0,HV,K,V,L", [(2, 127, 64, 2, 64, 64, 15), (1, 70, 6, 3, 100, 5, 17), (1, 33, 0, 1, 128, 4, 8)])
+def test_tail_reads_only_the_levels_that_hold_tokens(device, B, T, t0, HV, K, V, L):
+    # whole batches of staged tokens, one over, and a partial one; levels without tokens may hold anything and come back zero
+    import ctypes
+    from lampa_amd import _capi
+    from lampa_amd._capi import ptr
+    gen = torch.Generator().manual_seed(T)
+    q, k = (torch.randn(B, T, HV, K, generator=gen) for _ in range(2))
+    v, lam = torch.randn(B, T, HV, V, generator=gen), torch.randn(B, T, HV, L, generator=gen)
+    g, beta = -0.2 * torch.rand(B, T, HV, generator=gen), torch.rand(B, T, HV, generator=gen)
+    want_o, want_s, want_c = oh.recurrent_c_state(q, k, v, g, beta, lam, scale=0.3)
+    states = torch.full((B, HV, K, V, L), float("nan"), device=device)
+    if t0:
+        _, s0, c0 = oh.recurrent_c_state(*(x[:, :t0].contiguous() for x in (q, k, v, g, beta, lam)), scale=0.3)
+        held = [level for level in range(L) if c0.tolist()[level]]
+        states[..., held] = s0[..., held].float().to(device)
+    args = [x.to(device) for x in (q, k, v, g, beta, lam)]
+    o = torch.empty_like(args[2])
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _capi.lib().lampa_hgdn_tail(*(ptr(x) for x in args), 2, 1.0, ptr(states), ptr(o), B, T, t0, HV, HV, K, V, L, 2, 0.3,
+                                       1, stream) == 0
+    assert (states.cpu() - want_s).abs().max() <= 2e-5 * want_s.abs().max()
+    assert (states[..., [level for level in range(L) if not want_c.tolist()[level]]] == 0).all()
+    assert (o[:, t0:].cpu() - want_o[:, t0:]).abs().max() <= 2e-5 * want_o.abs().max()
