@@ -477,7 +477,8 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
 // halved four times until a lane holds one level's sum over its group of 16 lanes (`wave_sums16`), and go back to all lanes
 // as scalars; the next token's values are loaded while this one is worked on.
 // A prefill of 15 000 tokens (24 behind its whole chunks, 8 heads of 64 x 64): 708 us with a launch of the single-token kernel
-// and its copies per token, 188 us with the rows kernel (its own 38), TAIL_FIGURES.
+// and its copies per token, 188 us with the rows kernel (its own 38),
+// 173 us with this one (25).
 #define HGS_TAIL_LEVELS 17  // levels of the narrow instantiation: sequences up to 65 536 tokens
 #define HGS_TAIL_WAVES 4
 #define HGS_DPP_ROR8 0x128
