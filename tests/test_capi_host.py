@@ -552,3 +552,19 @@ def test_calls_that_go_to_their_launcher_directly():
     torch.func.vmap(lambda y: (seen.append(gd._direct(x)), y)[1])(x)
     torch.jit.trace(lambda y: (seen.append(gd._direct(x)), y + 1)[1], (x,), check_trace=False)
     assert seen == [False, False] and gd._direct(x)
+
+
+@pytest.mark.parametrize("chunks,heads,want", [([235], 6, 42), ([94], 8, 24), ([938], 8, 64), ([47, 3, 0], 8, 13),
+                                               ([188] * 8, 8, 64), ([8000], 8, 128), ([1], 300, 1), ([20] * 70, 8, 70)])
+def test_segments_of_a_training_step(chunks, heads, want):
+    # one round of the walk where four-chunk segments would leave a second one half empty, else two; one segment a sequence
+    # at least (the balanced plan deals them out) and no more than there are runs of four chunks
+    assert gd_train(chunks, heads) == want
+
+
+def gd_train(chunks, heads):
+    from lampa_amd import gated_delta as gd
+
+    kind, total = gd._train_segmentation(chunks, heads, 256)
+    assert kind == "balanced"
+    return total
