@@ -74,6 +74,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 #define HG_CW 6                  // chain waves
 #define HG_LPW 2                 // levels per chain wave
+#define HG_SCAN_WAVES 4          // waves of the scan over the segments
 #define HG_NLV (HG_CW * HG_LPW)  // inter-chunk levels: sequences of up to 2^12 chunks
 #define HG_INTRA 7               // levels 0..6 live inside a chunk
 
@@ -510,15 +511,15 @@ __device__ __forceinline__ void slab_add(float* p, int lane, const f32x16* S) {
 // The carry chain after chunk cs (index in its sequence): the levels below the lowest clear bit z of cs are all
 // occupied; they and the new state already in s_acc are summed, in level order, and become level z. One barrier
 // per level (uniform over the workgroup); a wave that owns none of the levels only takes part in the barriers.
-template <int KT>
+template <int KT, int CW = HG_CW, int LPW = HG_LPW>
 __device__ __forceinline__ void hg_merge(int cs, int lvl0, int wave, bool chain, int lane, float* s_acc,
                                          f32x16 (*S)[KT / 32]) {
   const int z = __builtin_ctz(~cs);
   for (int j = lvl0; j < z; ++j) {
     if (chain) {
 #pragma unroll
-      for (int slot = 0; slot < HG_LPW; ++slot)
-        if (slot * HG_CW + wave == j) {
+      for (int slot = 0; slot < LPW; ++slot)
+        if (slot * CW + wave == j) {
           slab_add<KT>(s_acc, lane, S[slot]);
 #pragma unroll
           for (int km = 0; km < KT / 32; ++km) S[slot][km] = zero16();
@@ -528,8 +529,8 @@ __device__ __forceinline__ void hg_merge(int cs, int lvl0, int wave, bool chain,
   }
   if (chain) {
 #pragma unroll
-    for (int slot = 0; slot < HG_LPW; ++slot)
-      if (slot * HG_CW + wave == z) slab_load<KT>(s_acc, lane, S[slot]);
+    for (int slot = 0; slot < LPW; ++slot)
+      if (slot * CW + wave == z) slab_load<KT>(s_acc, lane, S[slot]);
   }
 }
 
@@ -765,76 +766,107 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
 }
 
 // ---- scan over the segments --------------------------------------------------------------------------------------
-// grid (VT/32, n_seq, HV), HG_CW waves. Segments hold G = 2^p chunks, so at a segment's first chunk only levels >= p
-// can be occupied; they are carried from segment to segment with the segment's composite map of the plain rule
-// (S -> d S + M' S; its N is the sum of everything the segment's own chunks contribute) and merged by the same carry
-// chain. Xinit[seg][level] receives every occupied level's state at the segment's first chunk.
+// grid (VT/32, n_seq, HV), HG_SCAN_WAVES waves of three levels each. Segments hold G = 2^p chunks, so at a segment's first
+// chunk only levels >= p can be occupied; they are carried from segment to segment with the segment's composite map of the
+// plain rule (S -> d S + M' S; its N is the sum of everything the segment's own chunks contribute) and merged by the same
+// carry chain. Xinit[seg][level] receives every occupied level's state at the segment's first chunk.
+// The kernel runs beside the prep kernel, whose workgroups of four waves fill every CU, and has to fit where one of them
+// ends: one wave per SIMD. With six waves of two levels (two SIMDs with two waves each) its workgroups waited until no more
+// of prep's were left: 133 us beside it for what takes 20 alone, the call 414 us; so 40 us, and 405 (15 segments of 64 chunks,
+// 8 heads of 64 x 64).
 template <int KT, int VT>
-__global__ void __launch_bounds__(64 * HG_CW)
+__global__ void __launch_bounds__(64 * HG_SCAN_WAVES, 2)
     hgdn_scan_kernel(const GdrPlanView pv, const unsigned char* __restrict__ Mcomp, const unsigned char* __restrict__ Ncomp,
                      const float* __restrict__ Dcomp, float* __restrict__ Xinit, int HV, int p) {
-  constexpr int NKS = KT / 16, M_BYTES = KT * KT * 2, N_BYTES = KT * 32 * 4;
+  constexpr int NKS = KT / 16, NM = (KT / 32) * NKS, M_BYTES = KT * KT * 2, N_BYTES = KT * 32 * 4;
+  constexpr int LPW = HG_NLV / HG_SCAN_WAVES;
+  static_assert(LPW == 3, "LEVELS");
   __shared__ __align__(16) float s_acc[KT * 32];
   const int vslab = blockIdx.x, seq = blockIdx.y, hv = blockIdx.z;
   const int seg0 = pv.seq_seg0[seq], nseg = pv.seq_nseg[seq];
   const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63;
-  f32x16 S[HG_LPW][KT / 32];
+  f32x16 S[LPW][KT / 32];
 #pragma unroll
-  for (int slot = 0; slot < HG_LPW; ++slot)
+  for (int slot = 0; slot < LPW; ++slot)
 #pragma unroll
     for (int km = 0; km < KT / 32; ++km) S[slot][km] = zero16();
-  // composite of the coming segment: loaded one step ahead (two register sets that swap roles)
-  constexpr int NM = (KT / 32) * NKS, NPT = KT / 32;
-  bf16x8 mA[NM], mB[NM];
-  f32x4 nA[NPT], nB[NPT];
-  float dA = 0.0f, dB = 0.0f;
-  auto issue = [&](int i, bf16x8* m, f32x4* n, float& d) __attribute__((always_inline)) {
-    const size_t sh = (size_t)(seg0 + max(0, min(i, nseg - 2))) * HV + hv;
-    const bf16x8* M = reinterpret_cast<const bf16x8*>(Mcomp + sh * M_BYTES);
+  // The workgroup's waves need all of a segment's M' and each a part of its N: they load both together, SCAN_DEPTH segments
+  // ahead into register sets that are fixed per step of an unrolled round, and hand M' around in LDS.
+  constexpr int PIECES = M_BYTES / 16, NT = 64 * HG_SCAN_WAVES, SCAN_DEPTH = 2;
+  constexpr int LEVELS = 1 + (1 << HG_SCAN_WAVES) + (1 << 2 * HG_SCAN_WAVES);
+  static_assert(M_BYTES == N_BYTES && PIECES == 2 * NT, "two pieces of each per thread");
+  __shared__ f32x4 s_m[2][PIECES];
+  const int piece[2] = {tid, tid + NT};
+  struct Set {
+    f32x4 m[2], n[2];
+    float d;
+  };
+  Set set[SCAN_DEPTH];
+  const int n_apply = nseg - 1;
+  auto issue = [&](int i, Set& x) __attribute__((always_inline)) {
+    const size_t sh = (size_t)(seg0 + max(0, min(i, n_apply - 1))) * HV + hv;
+    const f32x4* M = reinterpret_cast<const f32x4*>(Mcomp + sh * M_BYTES);
     const f32x4* N = reinterpret_cast<const f32x4*>(Ncomp + (sh * (VT / 32) + vslab) * N_BYTES);
 #pragma unroll
-    for (int f = 0; f < NM; ++f) m[f] = M[f * 64 + lane];
-#pragma unroll
-    for (int j = 0; j < NPT; ++j) n[j] = N[tid + 64 * HG_CW * j];
-    d = Dcomp[sh];
-  };
-  auto step = [&](int i, const bf16x8* m, const f32x4* n, float d, bf16x8* m2, f32x4* n2, float& d2)
-                  __attribute__((always_inline)) {
-    const int seg = seg0 + i, cs = i << p;
-#pragma unroll
-    for (int slot = 0; slot < HG_LPW; ++slot) {
-      const int lvl = slot * HG_CW + wave;
-      if ((cs >> lvl) & 1)
-        slab_store<KT>(Xinit + ((((size_t)seg * HG_NLV + lvl) * HV + hv) * (VT / 32) + vslab) * (KT * 32), lane, S[slot]);
+    for (int u = 0; u < 2; ++u) {
+      x.m[u] = M[piece[u]];
+      x.n[u] = N[piece[u]];
     }
-    if (i == nseg - 1) return;
-    issue(i + 1, m2, n2, d2);
+    x.d = Dcomp[sh];
+  };
+  auto store = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int slot = 0; slot < HG_LPW; ++slot) {
-      const int lvl = slot * HG_CW + wave;
-      if (!((cs >> lvl) & 1)) continue;
-      bf16x8 Sb[NKS];
+    for (int slot = 0; slot < LPW; ++slot)
+      if (((i << p) >> (slot * HG_SCAN_WAVES + wave)) & 1)
+        slab_store<KT>(Xinit + ((((size_t)(seg0 + i) * HG_NLV + slot * HG_SCAN_WAVES + wave) * HV + hv) * (VT / 32) + vslab) * (KT * 32),
+                     lane, S[slot]);
+  };
+  auto step = [&](int i, Set& x) __attribute__((always_inline)) {
+    const int cs = i << p;
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) Sb[ks] = acc_to_operand(S[slot][ks / 2], 8 * (ks % 2));
+    for (int u = 0; u < 2; ++u) s_m[i & 1][piece[u]] = x.m[u];
+    const f32x4 n0 = x.n[0], n1 = x.n[1];
+    const float d = x.d;
+    store(i);
+    issue(i + SCAN_DEPTH, x);
+    lds_barrier();  // M' is in LDS; the level that took the last carry has read s_acc
+    reinterpret_cast<f32x4*>(s_acc)[piece[0]] = n0;
+    reinterpret_cast<f32x4*>(s_acc)[piece[1]] = n1;
+    if ((cs >> wave) & LEVELS) {  // (one of this wave's levels is occupied)
+      bf16x8 m[NM];
 #pragma unroll
-      for (int km = 0; km < KT / 32; ++km) {
+      for (int f = 0; f < NM; ++f) m[f] = __builtin_bit_cast(bf16x8, s_m[i & 1][f * 64 + lane]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) S[slot][km][r] *= d;
+      for (int slot = 0; slot < LPW; ++slot) {
+        if (!((cs >> (slot * HG_SCAN_WAVES + wave)) & 1)) continue;
+        bf16x8 Sb[NKS];
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) S[slot][km] = mfma32(m[km * NKS + ks], Sb[ks], S[slot][km]);
+        for (int ks = 0; ks < NKS; ++ks) Sb[ks] = acc_to_operand(S[slot][ks / 2], 8 * (ks % 2));
+#pragma unroll
+        for (int km = 0; km < KT / 32; ++km) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) S[slot][km][r] *= d;
+#pragma unroll
+          for (int ks = 0; ks < NKS; ++ks) S[slot][km] = mfma32(m[km * NKS + ks], Sb[ks], S[slot][km]);
+        }
       }
     }
-    lds_barrier();  // the level that took the last carry has read s_acc
-#pragma unroll
-    for (int j = 0; j < NPT; ++j) reinterpret_cast<f32x4*>(s_acc)[tid + 64 * HG_CW * j] = n[j];
     lds_barrier();
-    hg_merge<KT>(cs + (1 << p) - 1, p, wave, true, lane, s_acc, S);
+    hg_merge<KT, HG_SCAN_WAVES, LPW>(cs + (1 << p) - 1, p, wave, true, lane, s_acc, S);
   };
-  if (nseg > 1) issue(0, mA, nA, dA);
-  for (int i = 0; i < nseg; i += 2) {
-    step(i, mA, nA, dA, mB, nB, dB);
-    if (i + 1 < nseg) step(i + 1, mB, nB, dB, mA, nA, dA);
+  if (n_apply > 0) {
+#pragma unroll
+    for (int u = 0; u < SCAN_DEPTH; ++u) issue(u, set[u]);
+    int i = 0;
+    for (; i + SCAN_DEPTH <= n_apply; i += SCAN_DEPTH) {
+#pragma unroll
+      for (int u = 0; u < SCAN_DEPTH; ++u) step(i + u, set[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < SCAN_DEPTH - 1; ++u)
+      if (i + u < n_apply) step(i + u, set[u]);
   }
+  if (nseg > 0) store(nseg - 1);
 }
 
 // ---- host side ------------------------------------------------------------------------------------------------
@@ -966,7 +998,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
     } else {
       composites();
     }
-    hipLaunchKernelGGL((hgdn_scan_kernel<KT, VT>), dim3(VT / 32, n_seq, HV), dim3(64 * HG_CW), 0, cs, pv, Mc, Nm, Dc, Xi,
+    hipLaunchKernelGGL((hgdn_scan_kernel<KT, VT>), dim3(VT / 32, n_seq, HV), dim3(64 * HG_SCAN_WAVES), 0, cs, pv, Mc, Nm, Dc, Xi,
                        HV, p);
     LAMPA_PROF(s, "hgdn_scan_kernel");
     if (overlap && hipEventRecord(ev_join, side) != hipSuccess) return LAMPA_ERR_LAUNCH;
