@@ -4,8 +4,9 @@
 // every lane keeps the K state rows of its column in registers, so the three contractions of a step (S^T k, the
 // rank-one update and S^T q) are per-lane loops with no cross-lane traffic; k_t and q_t are loaded one element per
 // lane, normalised with a wave reduction and broadcast with v_readlane.
-// gdr_recurrent_split_kernel (further down): 32 columns per wave, the state rows of a column split over the two halves
-// of the wave -- fewer instructions per token and wave, for launches of few waves.
+// gdr_recurrent_split_kernel (further down, what nearly all launches take): 16 columns per wave, the state rows of a column
+// split over eight lanes, the token's operands staged in LDS by the waves of a workgroup together. The first one serves sizes
+// and alignments that cannot be staged in 16-byte pieces, head-wise beta, and a few tokens of very many sequences.
 //
 // Replaces fused_recurrent_gated_delta_rule_fwd_kernel, models/hattention/gated_delta_rule_ori.py:372-464
 // (state layout [N, HV, K, V] fp32; grouped value heads HV >= H).  It is also the fp32 mode of the chunk operator and
@@ -131,7 +132,7 @@ __global__ void __launch_bounds__(64) gdr_recurrent_kernel(const T* __restrict__
 }
 
 // ---- the same recurrence with the state rows of a column split over eight lanes ---------------------------------------
-// For launches of few waves. A wave owns 16 value columns of one (sequence, value head): lane = (column pair, row group), a
+// A wave owns 16 value columns of one (sequence, value head): lane = (column pair, row group), a
 // lane keeps KT / 8 state rows of two columns, and the partial sums of S^T k and of S^T q meet over eight neighbouring lanes
 // (three DPP additions each, no LDS). One wave per SIMD is bound by the instructions of a step, four cycles each, and by the
 // dependent chain S^T k -> d -> S; the four waves of a CU, by the LDS reads of the token's k and q: with two columns to a lane
