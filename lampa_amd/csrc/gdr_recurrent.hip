@@ -544,7 +544,8 @@ static int gdr_recurrent_launch(const void* q, const void* k, const void* v, con
 //    would wait for its load), and every memory operation of a step is unconditional (under a condition it becomes a branch,
 //    after which the compiler no longer counts the operations in flight and drains them).
 // Before, with M through LDS, 32 columns per workgroup of four waves and three launches, 32 us of a call of 8 192 x 4 x 32 x 32
-// tokens; now 5 + 10. (All rows on one wave up to K = 32: 7 + 15; eight steps of maps ahead instead of four: 8 + 16.)
+// tokens in 128 segments; now 5 + 10. (All rows on one wave up to K = 32: 7 + 15; eight steps of maps ahead instead of four:
+// 8 + 16.) In the 256 segments that the operator makes of it 8 + 14, for 14 + 13 instead of 16 + 20 in the two other passes.
 typedef float rs_f32x4 __attribute__((ext_vector_type(4)));
 template <int KT>
 struct RsScanShape {

@@ -772,7 +772,7 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
 // carry chain. Xinit[seg][level] receives every occupied level's state at the segment's first chunk.
 // The kernel runs beside the prep kernel, whose workgroups of four waves fill every CU, and has to fit where one of them
 // ends: one wave per SIMD. With six waves of two levels (two SIMDs with two waves each) its workgroups waited until no more
-// of prep's were left: 133 us beside it for what takes 20 alone, the call 414 us; so 40 us, and 405 (15 segments of 64 chunks,
+// of prep's were left: 133 us beside it for what takes 20 alone, the call 414 us; so 31 to 73, and 405 (15 segments of 64 chunks,
 // 8 heads of 64 x 64).
 template <int KT, int VT>
 __global__ void __launch_bounds__(64 * HG_SCAN_WAVES, 2)
