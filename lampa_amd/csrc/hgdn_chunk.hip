@@ -447,7 +447,7 @@ __global__ void __launch_bounds__(256)
           acc = mfma32(frag_load(s_PL, 2 * tm + ks, lane), ld_kappa_tr(s_v, SV, 32 * vt, 16 * ks, lane), acc);
       float* out = Oi + ch * (64 * VT) + 32 * vt + ln;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) out[(32 * tm + acc_row(r, hh)) * VT] = acc[r];
+      for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(acc[r], &out[(32 * tm + acc_row(r, hh)) * VT]);
     } else {
       const int f = task - 2 * NU, which = f / (2 * NKS), g = f % (2 * NKS);  // fragment (tm, ks) = (g / NKS, g % NKS)
       const bf16x8 fr = ld_kappa(which == 0 ? s_w : s_qt, SK, 32 * (g / NKS) + ln, 16 * (g % NKS), hh);
@@ -556,8 +556,11 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
   // Output of a chunk: every wave of the workgroup sums eight rows of the chain waves' partial tiles and the intra-chunk
   // part (read one chunk ahead), rounds and stores them -- lane = (row, four columns).
   const int orow = 8 * wave + (lane >> 3), ocol = 4 * (lane & 7);
+  // (non-temporal, as prep stores it: each value is read once, and the records, which the slabs share, stay in the caches.
+  // 60 032 x 8 x 64 x 64: the stores 404 -> 402 us, the loads as well 400; 15 000 the same)
   auto oi_load = [&](int c) __attribute__((always_inline)) {
-    return *reinterpret_cast<const f32x4*>(Oi + ((size_t)uniform(c) * HV + hv) * (64 * VT) + orow * VT + 32 * vslab + ocol);
+    return __builtin_nontemporal_load(
+        reinterpret_cast<const f32x4*>(Oi + ((size_t)uniform(c) * HV + hv) * (64 * VT) + orow * VT + 32 * vslab + ocol));
   };
   auto out_rows = [&](int tok0, int len, f32x4 a) __attribute__((always_inline)) {
 #pragma unroll
