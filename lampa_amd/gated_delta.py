@@ -126,40 +126,19 @@ def _default_segmentation(chunks_per_seq, n_value_heads: int, slots: int, per_cu
     return "lengths", lens
 
 
-def _train_segmentation(chunks_per_seq, n_value_heads: int, cus: int):
-    """Segments of a training step, as ``_default_segmentation`` returns them: no shorter than four chunks, as even as they
-    come. A CU holds one workgroup of the backward's walk and two of the other segment kernels, so there are two rounds of the
-    walk where the call has that many segments; where it has less than 1.6 rounds, one round of longer ones is faster than two
-    of which the second is half empty (a round costs the walk about two chunks more than its longest segment has; above 1.6
-    the other kernels' longer segments cost as much). Kernels of a step against those on the forward's own segments, us:
-    14 983 x 6 x 64 x 64 (354 workgroups) 159 -> 137, six events of 20 000 x 4 (324) 141 -> 124, 2 x 5 000 x 8 (320)
-    144 -> 121, 60 000 x 8 (two full rounds, even) 414 -> 402, 2 x 20 000 x 8 297 -> 293, eight events of 96 000 x 8
-    598 -> 593 (one round: 666)."""
-    total = sum((n + 3) // 4 for n in chunks_per_seq)
-    one = max(1, len(chunks_per_seq), cus // n_value_heads)
-    if total * n_value_heads <= 1.6 * cus:
-        return "balanced", max(1, min(total, one))
-    rounds = max(2, -(-sum(chunks_per_seq) * n_value_heads // (cus * MAX_CHUNKS_PER_SEGMENT)))
-    return "balanced", max(1, min(total, max(len(chunks_per_seq), rounds * cus // n_value_heads)))
-
-
-_TRAIN_HEADS = 64, 64, 0  # K and V of the training kernels; the third entry asks ``_plan`` for a training step's segments
-
-
 def _plan(cu_host, device, n_value_heads: int, head_dims):
     """Host + device copies of the chunk/segment tables for these sequence boundaries (cached)."""
-    kind, arg, train = "cps", CHUNKS_PER_SEGMENT, head_dims == _TRAIN_HEADS
+    kind, arg = "cps", CHUNKS_PER_SEGMENT
     per_cu = 2 if max(head_dims) <= 64 else 1  # workgroups of the segment kernels a CU holds (LDS, registers)
     # (everything the tables depend on: dealing out the segments of a packed call costs more than its launches)
-    key = (tuple(cu_host), device, n_value_heads, per_cu, arg, MAX_CHUNKS_PER_SEGMENT, LONG_SEGMENT_FACTOR, train)
+    key = (tuple(cu_host), device, n_value_heads, per_cu, arg, MAX_CHUNKS_PER_SEGMENT, LONG_SEGMENT_FACTOR)
     hit = _plan_cache.get(key)
     if hit is not None:
         return hit
     if not arg:
         cus = torch.cuda.get_device_properties(device).multi_processor_count
         chunks_per_seq = [(b - a + 63) // 64 for a, b in zip(cu_host[:-1], cu_host[1:])]
-        kind, arg = (_train_segmentation(chunks_per_seq, n_value_heads, cus) if train else
-                     _default_segmentation(chunks_per_seq, n_value_heads, per_cu * cus, per_cu))
+        kind, arg = _default_segmentation(chunks_per_seq, n_value_heads, per_cu * cus, per_cu)
     lib = _capi.lib()
     cu = (ctypes.c_int64 * len(cu_host))(*cu_host)
     n_seq = len(cu_host) - 1
@@ -442,7 +421,7 @@ def _chunk_train_forward(q, k, v, head, g, beta, scale, initial_state, output_fi
     cu_host = _sequence_bounds(cu_seqlens, B, T)
     n_seq = len(cu_host) - 1
     kept = _Kept()
-    kept.plan = _plan(cu_host, q.device, HV, _TRAIN_HEADS)
+    kept.plan = _plan(cu_host, q.device, HV, (64, 64))
     plan_host, plan_dev = kept.plan
     lib, host_ptr = _capi.lib(), ctypes.c_void_p(plan_host.data_ptr())
     n_saved = check(lib.lampa_gdr_train_saved_bytes(host_ptr, HV), "lampa_gdr_train_saved_bytes")

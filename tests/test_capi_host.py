@@ -554,17 +554,26 @@ def test_calls_that_go_to_their_launcher_directly():
     assert seen == [False, False] and gd._direct(x)
 
 
-@pytest.mark.parametrize("chunks,heads,want", [([235], 6, 42), ([94], 8, 24), ([938], 8, 64), ([47, 3, 0], 8, 13),
-                                               ([188] * 8, 8, 64), ([8000], 8, 128), ([1], 300, 1), ([20] * 70, 8, 70)])
-def test_segments_of_a_training_step(chunks, heads, want):
-    # one round of the walk where four-chunk segments would leave a second one half empty, else two; one segment a sequence
-    # at least (the balanced plan deals them out) and no more than there are runs of four chunks
-    assert gd_train(chunks, heads) == want
-
-
-def gd_train(chunks, heads):
+@pytest.mark.parametrize("T,H,K,V", [(14983, 6, 16, 32), (60000, 8, 64, 64), (500, 4, 32, 32)])
+def test_a_training_step_is_cut_as_the_call_without_gradients(monkeypatch, T, H, K, V):
+    # the composites of a call round M' once per segment, so other segments are other outputs: a forward that keeps what the
+    # backward pass needs has to ask for the plan that the chunk kernels of its (padded) heads ask for without gradients
     from lampa_amd import gated_delta as gd
 
-    kind, total = gd._train_segmentation(chunks, heads, 256)
-    assert kind == "balanced"
-    return total
+    asked = []
+
+    class Stop(Exception):
+        pass
+
+    def plan(*args):
+        asked.append(args)
+        raise Stop
+
+    monkeypatch.setattr(gd, "_plan", plan)
+    q = k = torch.empty(1, T, H, 64, dtype=torch.bfloat16, device="meta")
+    g = torch.empty(1, T, H, device="meta")
+    for call in (lambda: gd._chunk_launch(q, k, q, g, g, 0.125, None, False, None, gd.L2_CHUNK),
+                 lambda: gd._chunk_train_forward(q, k, q, (K, V), g, g, 0.125, None, False, None, gd.L2_CHUNK)):
+        with pytest.raises(Stop):
+            call()
+    assert asked[0] == asked[1]

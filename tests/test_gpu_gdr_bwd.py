@@ -460,3 +460,19 @@ def test_values_that_are_not_finite_stay_out_of_earlier_gradients(device, token,
     for a, b in zip(got[:5], want[:5]):
         assert torch.equal(a[:, :end], b[:, :end])
     assert torch.equal(got[5], want[5])
+
+
+@pytest.mark.parametrize("T,lens,H,dtype", [(14983, None, 6, torch.float16), (20000, None, 8, torch.bfloat16),
+                                            (None, [5000, 0, 7001], 4, torch.bfloat16)])
+def test_forward_of_a_training_step_gives_the_bits_of_the_plain_call(device, T, lens, H, dtype):
+    """Outputs and final states of a forward that keeps what the backward pass needs: those of the call without gradients (the
+    same segments, so M' is rounded at the same places), where a segment's states live on into the next ones."""
+    cu = None if lens is None else torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), device=device)
+    (q, k, v, g, beta, _), _ = _inputs(1, T or sum(lens), H, H, 64, 64, dtype, H, unit=False, g_scale=0.05)
+    args = [x.to(device) for x in (q, k, v, g, beta)]
+    call = lambda: gd.chunk_gated_delta_rule(*args, output_final_state=True, cu_seqlens=cu, use_qk_l2norm_in_kernel=True)
+    o, s = call()
+    for x in args:
+        x.requires_grad_(True)
+    ot, st = call()
+    assert ot.requires_grad and torch.equal(o, ot) and torch.equal(s, st)
