@@ -565,14 +565,22 @@ __global__ void __launch_bounds__(64 * RsScanShape<KT>::NT)
                             int maxg, int W) {
   constexpr int NT = RsScanShape<KT>::NT, DEPTH = RsScanShape<KT>::DEPTH;
   __shared__ rs_f32x4 s_x[2][NT][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g4 = lane >> 4, j16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g4 = lane >> 4, j16 = lane & 15;
   const int hv = blockIdx.z, seq = blockIdx.y / maxg, grp = blockIdx.y - seq * maxg;
   const int seg0 = seq_seg0[seq], seg1 = seq_seg0[seq + 1];
   const int p0 = seg0 + grp * gs, cnt = min(gs, seg1 - p0);  // this group's segments
   if (cnt <= 0 || (COMPOSE && p0 + gs >= seg1)) return;       // (no one asks for the map of a sequence's last group)
   const int lead = COMPOSE ? 0 : grp, n_apply = lead + (COMPOSE ? cnt : cnt - 1);
-  // Lanes past V shadow the last column, rows past K the last rows of the same place in their run of four: they load, compute
-  // and store the same as those. What they feed into a product is met by a zero of M.
+  // A row tile wholly past K (K = 36 .. 48, 68 .. 112): zeros for the products of the other waves, and their barriers. It may
+  // not shadow rows of another tile as the lanes below do: a wave sums its own columns first, so it would store other last
+  // bits to the same place, with no order between the two.
+  if (16 * wave >= K) {
+    s_x[0][wave][lane] = s_x[1][wave][lane] = rs_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p = 0; p < n_apply; ++p) lds_barrier();
+    return;
+  }
+  // Lanes past V shadow the last column, rows past K the last rows of the same place in their run of four, all in the same
+  // wave: they load, compute and store the same as those. What they feed into a product is met by a zero of M.
   const int col = min((int)blockIdx.x * 16 + j16, V - 1);
   const bool is_m = COMPOSE && col < K;  // (a column of M: no additive term, starts from I)
   const int ncol = COMPOSE ? max(col - K, 0) : col;

@@ -639,3 +639,24 @@ def test_recurrent_scan_in_groups_of_segments(device, K, V, lens):
     o, s = gd.fused_recurrent_gated_delta_rule(*_to(device, q, k, v, g, beta), initial_state=h0.to(device),
                                                output_final_state=True, cu_seqlens=cu.to(device))
     assert _errors(o, want_o)[0] <= FP32_TOL and _errors(s, want_s)[0] <= FP32_TOL
+
+
+@pytest.mark.parametrize("K", [20, 36, 48, 64, 68, 96, 112])
+def test_recurrent_segments_give_the_same_bits_every_time(device, K):
+    # the scan over the segments where row tiles of 16 are partly or wholly past K (one writer per row, whatever the waves'
+    # order): outputs, final states and the token-serial gradients, which scan twice
+    T, V = 4000, 40
+    q, k, v, g, beta = _to(device, *synth.gdr_inputs(1, T, 2, K, V, torch.float32, seed=K, g_scale=0.01))
+    h0 = torch.randn(1, 2, K, V, generator=torch.Generator().manual_seed(1)).to(device)
+    do = torch.randn(1, T, 2, V, generator=torch.Generator().manual_seed(2)).to(device)
+
+    def run():
+        leaves = [x.detach().clone().requires_grad_(True) for x in (q, k, v, g, beta, h0)]
+        o, s = gd.chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], output_final_state=True, allow_fp32=True)
+        return (o, s, *torch.autograd.grad((o, s), leaves, (do, torch.ones_like(s))))
+
+    first = run()
+    for _ in range(5):
+        assert all(torch.equal(a, b) for a, b in zip(first, run()))
+    want_o, want_s = og.recurrent_c(*(x.cpu() for x in (q, k, v, g, beta)), initial_state=h0.cpu())
+    assert _errors(first[0], want_o)[0] <= FP32_TOL and _errors(first[1], want_s)[0] <= FP32_TOL
