@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
                                const float* __restrict__ g, const float* __restrict__ beta, T* __restrict__ o,
                                const float* __restrict__ h0, float* __restrict__ ht,
                                const int64_t* __restrict__ cu_seqlens, int64_t t_len, int H, int HV, int K, int V,
-                               float scale, int l2norm, const int32_t* __restrict__ ht_map) {
+                               float scale, int l2norm, const int32_t* __restrict__ ht_map, float lazy_span) {
   constexpr int RG = 8, WCOLS = 128 / RG;       // row groups and columns of a wave
   constexpr int NT = 64 * WAVES, COLS = WCOLS * WAVES;
   constexpr int RP = KT / RG;                   // state rows per lane
@@ -278,8 +278,8 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
     // the decay from the run's start up to token j, and c_j goes into the token's scalars instead (a multiply per state
     // element and token less); the state is brought back to scale after the run. (Runs as long as the group, 16 to 64 tokens,
     // cost nothing less and up to 2.5 times the error against 64 bits, from the rounding of the longer sums in e^.) A group
-    // with more than e^60 of decay (or growth) in one of its runs, where 1 / c_j would leave the fp32 range, takes the direct
-    // form. c_run: of lane 8 r + 7, the decay over run r.
+    // with more than e^lazy_span of decay (or growth) in one of its runs takes the direct form: beyond e^60 1 / c_j would leave
+    // the fp32 range; below zero every group does. c_run: of lane 8 r + 7, the decay over run r.
     float c_run = 1.0f;
     bool lazy = false;
     auto commit = [&](int64_t t0, int buf) __attribute__((always_inline)) {
@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
       cum += (lane & 7) >= 2 ? up2 : 0.0f;
       const float up4 = dpp_f32<GDR_DPP_ROW_SHR(4), 0xF>(0.0f, cum);
       cum += (lane & 7) >= 4 ? up4 : 0.0f;
-      lazy = __ballot(!(rec_run_sum<8>(fabsf(g_use)) <= 60.0f)) == 0;  // (false for a NaN as well)
+      lazy = __ballot(!(rec_run_sum<8>(fabsf(g_use)) <= lazy_span)) == 0;  // (false for a NaN as well)
       const float c_tok = expf(lazy ? cum : g_tok), rc_tok = lazy ? expf(-cum) : 1.0f;
       c_run = c_tok;
 #pragma unroll
@@ -477,14 +477,17 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
 }
 
 // Launch of the split kernel over `n_seq` runs of tokens; V: all the wave's columns (COMPOSITE: K + the value width).
+// lazy_form: whether groups of tokens may apply their decays lazily (see commit).
 template <typename T, bool COMPOSITE>
 static void gdr_split_launch(const void* q, const void* k, const void* v, const float* g, const float* beta, void* o,
                              const float* h0, float* ht, const int64_t* cu, int n_seq, int64_t t_len, int H, int HV, int K,
-                             int V, float scale, int l2norm, const int32_t* ht_map, hipStream_t s) {
+                             int V, float scale, int l2norm, const int32_t* ht_map, hipStream_t s,
+                             bool lazy_form = true) {
 #define GDR_REC_SPLIT(KT, WAVES)                                                                                         \
   hipLaunchKernelGGL((gdr_recurrent_split_kernel<T, KT, WAVES, COMPOSITE>),                                              \
                      dim3((V + 16 * WAVES - 1) / (16 * WAVES), n_seq * HV), dim3(64 * WAVES), 0, s, (const T*)q,         \
-                     (const T*)k, (const T*)v, g, beta, (T*)o, h0, ht, cu, t_len, H, HV, K, V, scale, l2norm, ht_map)
+                     (const T*)k, (const T*)v, g, beta, (T*)o, h0, ht, cu, t_len, H, HV, K, V, scale, l2norm, ht_map,   \
+                     lazy_form ? 60.0f : -1.0f)
 #define GDR_REC_SPLIT_K(WAVES)                  \
   do {                                          \
     if (K <= 16) GDR_REC_SPLIT(16, WAVES);      \
@@ -508,8 +511,15 @@ static int gdr_recurrent_launch(const void* q, const void* k, const void* v, con
   // as many sequences 37 against 44, a quarter 26 against 24; at K = 16, 32 and 128 the split form is faster throughout).
   const int64_t waves = (int64_t)((V + 31) / 32) * n_seq * HV, tokens = cu ? t_len / n_seq : t_len;
   const bool few_of_many = K > 32 && K <= 64 && tokens <= 2 && waves > 4096;
+  // Launches of more than 2 048 waves of 32 columns take the direct form, the state times each token's own e^g as the lane-per-
+  // column kernel has it. The lazy one takes ratios of decays from e^ of their sums: against 64 bits (64 tokens, K 16 to 128) its
+  // states are 3.3 times as far off at e^-0.8 a token, 1.4 times at e^-0.24, 0.84 times at e^-0.04, and 5.9 times at e^-2.4; the
+  // direct form's, 1.00 times. It costs a multiply per state element and token (fp32: 512 x 64 x 8 x 32 x 32 83 -> 87 us,
+  // 128 x 64 x 8 x 128 x 128 182 -> 198, 1 024 x 64 x 8 x 64 x 64 383 -> 411; a lane per column 135, 285, 474). Smaller launches
+  // are bound by the chain of a step; the two row groups that they took before were lazy over 8 to 64 tokens, and further off.
   if (K % 4 == 0 && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) & 15) == 0 && !few_of_many) {
-    gdr_split_launch<T, false>(q, k, v, g, beta, o, h0, ht, cu, n_seq, t_len, H, HV, K, V, scale, l2norm, nullptr, s);
+    gdr_split_launch<T, false>(q, k, v, g, beta, o, h0, ht, cu, n_seq, t_len, H, HV, K, V, scale, l2norm, nullptr, s,
+                               waves <= 2048);
     LAMPA_PROF(s, "gdr_recurrent_split_kernel");
     return lampa_launch_status();
   }
