@@ -191,7 +191,10 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
   constexpr int RG = 8, WCOLS = 128 / RG;       // row groups and columns of a wave
   constexpr int NT = 64 * WAVES, COLS = WCOLS * WAVES;
   constexpr int RP = KT / RG;                   // state rows per lane
-  constexpr int G = KT <= 64 ? 32 : 16;         // tokens per group
+  // Tokens per group. A workgroup of two waves (V <= 32) stages as much of k and q as one of four: with 32 tokens at K = 64 it
+  // held 47 KB, three were all that a CU had room for, and 1 024 took two rounds (128 x 8 x 64 x 32 fp32, 64 tokens 48 us, one
+  // 11; with 16 tokens 33 and 8.3).
+  constexpr int G = KT < 64 || (KT == 64 && WAVES > 2) ? 32 : 16;
   constexpr int P = KT / 4;                     // 4-element pieces of a row of k
   constexpr int ROW4 = (2 * KT + 4) / 4;        // 16-byte pieces per token in LDS: k | q, padded against conflicts
   constexpr int PIECES = (G * P + NT - 1) / NT; // pieces of k (and of q) per thread and group
@@ -203,6 +206,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
   __shared__ float4 s_sc[2][G + 2];
   __shared__ float s_v[2][(G + 2) * COLS];
   __shared__ T s_o[COMPOSITE ? 1 : G * COLS];  // o of a group, stored behind its last step
+  static_assert(KT > 64 || (sizeof(s_kq) + sizeof(s_sc) + sizeof(s_v) + sizeof(s_o)) * 8 / WAVES <= 160 * 1024, "eight waves to a CU");
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rg = lane % RG, cl = WCOLS * wave + 2 * (lane / RG);
   const int wcol = (int)blockIdx.x * COLS, col = wcol + cl;  // the first of this lane's two columns
   const int seq = blockIdx.y / HV, hv = blockIdx.y % HV;
