@@ -131,10 +131,10 @@ __global__ void __launch_bounds__(64) gdr_recurrent_kernel(const T* __restrict__
   }
 }
 
-// ---- the same recurrence with the state rows of a column split over eight lanes ---------------------------------------
+// ---- the same recurrence with the state rows of a column split over eight or four lanes -------------------------------
 // A wave owns 16 value columns of one (sequence, value head): lane = (column pair, row group), a
 // lane keeps KT / 8 state rows of two columns, and the partial sums of S^T k and of S^T q meet over eight neighbouring lanes
-// (three DPP additions each, no LDS). One wave per SIMD is bound by the instructions of a step, four cycles each, and by the
+// (three DPP additions each, no LDS); narrow heads have KT / 4 rows of one column to a lane (see NC). One wave per SIMD is bound by the instructions of a step, four cycles each, and by the
 // dependent chain S^T k -> d -> S; the four waves of a CU, by the LDS reads of the token's k and q: with two columns to a lane
 // those are KT / 8 values of each where a lane with one column reads twice as many. What is not the recurrence leaves the
 // step: the waves of a workgroup, which own neighbouring columns of the same head, load a group of tokens ahead, widen q, k
@@ -143,9 +143,7 @@ __global__ void __launch_bounds__(64) gdr_recurrent_kernel(const T* __restrict__
 // are applied as factors on the sums, not on the vectors. K a multiple of 4, q and k 16-byte aligned.
 // Against two row groups, 32 columns and a workgroup per wave (us, 64 tokens, states in and out): 16 x 8 x 64 x 64 bf16
 // 32.8 -> 20.7 (one token 8.0 -> 5.8), 32 x 4 x 128 x 128 110 -> 32, 128 x 8 x 64 x 64 82 -> 54, 40 x 6 x 32 x 64 fp32
-// 20.8 -> 16.3, 128 x 6 x 16 x 64 22.5 -> 16.6, but 128 x 8 x 16 x 32 17.9 -> 19.4; against a lane per column, where that was
-// taken before: 512 x 8 x 32 x 32 187 -> 73, 128 x 8 x 128 x 128 355 -> 159, 1 024 x 8 x 64 x 64 608 -> 357. (Groups of 16 or
-// 64 tokens at K = 16, four row groups of 32 columns a wave: slower.)
+// 20.8 -> 16.3, 128 x 8 x 16 x 32 17.5 -> 16.1. (Groups of 16 or 64 tokens at K = 16, four row groups of 32 columns a wave: slower.)
 // x summed over aligned runs of N lanes, in every lane
 template <int N>
 __device__ __forceinline__ float rec_run_sum(float x) {
@@ -188,9 +186,15 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
                                const float* __restrict__ h0, float* __restrict__ ht,
                                const int64_t* __restrict__ cu_seqlens, int64_t t_len, int H, int HV, int K, int V,
                                float scale, int l2norm, const int32_t* __restrict__ ht_map, float lazy_span) {
-  constexpr int RG = 8, WCOLS = 128 / RG;       // row groups and columns of a wave
+  // Heads of 16 rows, and of 32 where a workgroup has two waves, give a lane a quarter of the rows of one column: with two
+  // columns of two or four rows the sums over the lanes were the larger part of a step (64 tokens: 128 x 8 x 16 x 32 fp32
+  // 18.7 -> 16.2 us, 64 x 8 x 16 x 128 29.1 -> 25.7, 128 x 8 x 32 x 32 22.9 -> 20.4). At K = 32 with four waves it is slower
+  // (one token, 128 x 8 x 32 x 128 15.6 -> 17.1: a lane with one column reads twice as much of k and q from LDS).
+  constexpr int NC = KT == 16 || (KT == 32 && WAVES == 2) ? 1 : 2;  // columns of a lane
+  constexpr int RG = 4 * NC, WCOLS = 16;        // row groups and columns of a wave
   constexpr int NT = 64 * WAVES, COLS = WCOLS * WAVES;
   constexpr int RP = KT / RG;                   // state rows per lane
+  constexpr int CHAINS = NC == 1 && RP >= 8 ? 2 : 1;  // sums a lane adds its rows in (two, where one would be of eight: the error)
   // Tokens per group. A workgroup of two waves (V <= 32) stages as much of k and q as one of four: with 32 tokens at K = 64 it
   // held 47 KB, three were all that a CU had room for, and 1 024 took two rounds (128 x 8 x 64 x 32 fp32, 64 tokens 48 us, one
   // 11; with 16 tokens 33 and 8.3).
@@ -207,8 +211,8 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
   __shared__ float s_v[2][(G + 2) * COLS];
   __shared__ T s_o[COMPOSITE ? 1 : G * COLS];  // o of a group, stored behind its last step
   static_assert(KT > 64 || (sizeof(s_kq) + sizeof(s_sc) + sizeof(s_v) + sizeof(s_o)) * 8 / WAVES <= 160 * 1024, "eight waves to a CU");
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rg = lane % RG, cl = WCOLS * wave + 2 * (lane / RG);
-  const int wcol = (int)blockIdx.x * COLS, col = wcol + cl;  // the first of this lane's two columns
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rg = lane % RG, cl = WCOLS * wave + NC * (lane / RG);
+  const int wcol = (int)blockIdx.x * COLS, col = wcol + cl;  // (the first of) this lane's columns
   const int seq = blockIdx.y / HV, hv = blockIdx.y % HV;
   const int h = hv / (HV / H);
   const int64_t bos = cu_seqlens ? cu_seqlens[seq] : seq * t_len;
@@ -216,22 +220,23 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
 
   const int v_dim = COMPOSITE ? V - K : V;  // width of a row of v
   const bool even = V % 2 == 0 && ((reinterpret_cast<uintptr_t>(h0) | reinterpret_cast<uintptr_t>(ht)) & 7) == 0;  // columns in pairs
-  float S[2][RP];  // rows rg * RP + r
+  float S[NC][RP];  // rows rg * RP + r
 #pragma unroll
   for (int r = 0; r < RP; ++r) {
     const int i = rg * RP + r;
     if constexpr (COMPOSITE) {
-      S[0][r] = (i == col && i < K) ? 1.0f : 0.0f;
-      S[1][r] = (i == col + 1 && i < K) ? 1.0f : 0.0f;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) S[c][r] = (i == col + c && i < K) ? 1.0f : 0.0f;
     } else {
       const float* at = h0 + (((int64_t)seq * HV + hv) * K + i) * V + col;
       float2 x = make_float2(0.0f, 0.0f);
       if (h0 && i < K && col < V) {
-        if (even) x = *reinterpret_cast<const float2*>(at);
+        if (NC == 1) x.x = at[0];
+        else if (even) x = *reinterpret_cast<const float2*>(at);
         else x = make_float2(at[0], col + 1 < V ? at[1] : 0.0f);
       }
       S[0][r] = x.x;
-      S[1][r] = x.y;
+      if constexpr (NC == 2) S[NC - 1][r] = x.y;
     }
   }
   if (bos < eos) {
@@ -339,7 +344,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
     struct Operands {
       float4 sc;
       float kk[RP], qq[COMPOSITE ? 1 : RP];
-      float2 v;
+      float v[NC];
     };
     auto read_row = [&](const float* p, float* to) __attribute__((always_inline)) {
       if constexpr (RP == 2) {
@@ -358,16 +363,21 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
       const float* kr = reinterpret_cast<const float*>(&s_kq[buf][j * ROW4]) + rg * RP;
       read_row(kr, x.kk);
       if constexpr (!COMPOSITE) read_row(kr + KT, x.qq);
-      x.v = *reinterpret_cast<const float2*>(&s_v[buf][j * COLS + cl]);
+      if constexpr (NC == 2) {
+        const float2 v2 = *reinterpret_cast<const float2*>(&s_v[buf][j * COLS + cl]);
+        x.v[0] = v2.x; x.v[NC - 1] = v2.y;
+      } else {
+        x.v[0] = s_v[buf][j * COLS + cl];
+      }
     };
     fetch(bos);
     commit(bos, 0);
     lds_barrier();
-    // o of a group goes through LDS (row groups 0 and 1 write the first of two tokens, 2 and 3 the second) and leaves behind
+    // o of a group goes through LDS (the first NC row groups write the first of two tokens, the next the second) and leaves behind
     // the commit of the next group: stored token by token, the wait for that group's loads would be one for the stores too,
     // 2 us a group.
-    const int o_tok = (rg >> 1) & 1;
-    T* const so = s_o + o_tok * COLS + cl + (rg & 1);
+    const int o_tok = (rg / NC) & 1;
+    T* const so = s_o + o_tok * COLS + cl + rg % NC;
     auto flush = [&](int64_t t0, int n_tok) __attribute__((always_inline)) {
       if constexpr (!COMPOSITE) {
         const int c = WCOLS * wave + lane % WCOLS, j0 = lane / WCOLS;  // this wave's columns, four tokens at a time
@@ -392,37 +402,41 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
       auto run_group = [&](auto lazy_tag) __attribute__((always_inline)) {
         constexpr bool LAZY = decltype(lazy_tag)::value;
         auto step = [&](const Operands& x) __attribute__((always_inline)) {
-          float d[2], dk[2], out[2];
+          float d[NC], dk[NC], out[NC];
           const float4 sc = x.sc;
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            d[c] = S[c][0] * x.kk[0];
+          for (int c = 0; c < NC; ++c) {
+            float part[CHAINS];
 #pragma unroll
-            for (int r = 1; r < RP; ++r) d[c] = __builtin_fmaf(S[c][r], x.kk[r], d[c]);
+            for (int r = 0; r < RP; ++r)
+              part[r % CHAINS] = r < CHAINS ? S[c][r] * x.kk[r] : __builtin_fmaf(S[c][r], x.kk[r], part[r % CHAINS]);
+            d[c] = CHAINS == 2 ? part[0] + part[CHAINS - 1] : part[0];
           }
 #pragma unroll
-          for (int c = 0; c < 2; ++c) d[c] = rec_run_sum<RG>(d[c]);
+          for (int c = 0; c < NC; ++c) d[c] = rec_run_sum<RG>(d[c]);
           // S <- e^g S, then d = beta (v - S^T k), S <- S + k d^T, o = S^T q, with k = k_raw / |k|; in the lazy form on
           // S / c_j, where the decay is part of the scalars
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            const float vc = c ? x.v.y : x.v.x;
-            const float dc = LAZY ? sc.w * (vc - sc.x * d[c]) : sc.w * (vc - sc.z * sc.x * d[c]);
+          for (int c = 0; c < NC; ++c) {
+            const float dc = LAZY ? sc.w * (x.v[c] - sc.x * d[c]) : sc.w * (x.v[c] - sc.z * sc.x * d[c]);
             dk[c] = LAZY ? dc * sc.z : dc * sc.x;
           }
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
+          for (int c = 0; c < NC; ++c) {
+            float part[CHAINS];
 #pragma unroll
             for (int r = 0; r < RP; ++r) {
               S[c][r] = __builtin_fmaf(x.kk[r], dk[c], LAZY ? S[c][r] : sc.z * S[c][r]);
-              if constexpr (!COMPOSITE) out[c] = r == 0 ? S[c][0] * x.qq[0] : __builtin_fmaf(S[c][r], x.qq[r], out[c]);
+              if constexpr (!COMPOSITE)
+                part[r % CHAINS] = r < CHAINS ? S[c][r] * x.qq[r] : __builtin_fmaf(S[c][r], x.qq[r], part[r % CHAINS]);
             }
+            if constexpr (!COMPOSITE) out[c] = CHAINS == 2 ? part[0] + part[CHAINS - 1] : part[0];
           }
           if constexpr (COMPOSITE) return 0.0f;
           else {
 #pragma unroll
-            for (int c = 0; c < 2; ++c) out[c] = rec_run_sum<RG>(out[c]);
-            return (rg & 1 ? out[1] : out[0]) * sc.y;
+            for (int c = 0; c < NC; ++c) out[c] = rec_run_sum<RG>(out[c]);
+            return (rg % NC ? out[NC - 1] : out[0]) * sc.y;
           }
         };
         Operands xa, xb;
@@ -439,15 +453,15 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
             __builtin_amdgcn_sched_barrier(0);
             const float ob = step(xb);
             if constexpr (!COMPOSITE) {
-              if (rg < 4) so[j * COLS] = GdrElem<T>::from_float(o_tok ? ob : oa);
+              if (rg < 2 * NC) so[j * COLS] = GdrElem<T>::from_float(o_tok ? ob : oa);
             }
           }
           if constexpr (LAZY) {
             const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c_run), run + 7));
 #pragma unroll
             for (int r = 0; r < RP; ++r) {  // back to scale: S = c_last (S / c_last)
-              S[0][r] *= c;
-              S[1][r] *= c;
+#pragma unroll
+              for (int x = 0; x < NC; ++x) S[x][r] *= c;
             }
           }
         }
@@ -470,10 +484,10 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
       const int i = rg * RP + r;
       float* at = ht + (((int64_t)out_row * HV + hv) * K + i) * V + col;
       if (i < K && col < V) {
-        if (even) *reinterpret_cast<float2*>(at) = make_float2(S[0][r], S[1][r]);
+        if (NC == 2 && even) *reinterpret_cast<float2*>(at) = make_float2(S[0][r], S[NC - 1][r]);
         else {
           at[0] = S[0][r];
-          if (col + 1 < V) at[1] = S[1][r];
+          if (NC == 2 && col + 1 < V) at[1] = S[NC - 1][r];
         }
       }
     }
