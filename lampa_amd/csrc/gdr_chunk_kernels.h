@@ -1689,8 +1689,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         for (int e = 0; e < 4; ++e) {
           const float ks_ = SCALED ? acc[4 * b4 + e] : ek[4 * tm + b4][e] * acc[4 * b4 + e];
           // (training form: selected, not multiplied away, so that a v that is not finite stays out of M' and with it out
-          // of the gradients of the tokens before it)
-          const float v_ = KEEP ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e]) : vmask * (float)vv[4 * tm + b4][e];
+          // of the gradients of the tokens before it; so with SKIP_M, where it would reach M, and through M the other value
+          // columns behind the segment, only as long as M lives on)
+          const float v_ = KEEP || SKIP_M ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e]) : vmask * (float)vv[4 * tm + b4][e];
           acc[4 * b4 + e] = be[4 * tm + b4][e] * (v_ - ks_);
         }
       Rb[2 * tm + 0] = acc_to_op<OT>(acc, 0);
@@ -1754,7 +1755,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       // Columns of M that have become zero stay zero, whatever chunks follow: a wave whose columns all have only takes part
       // in the barriers from there on and leaves the LDS and the matrix cores, which bound this pass at the wide heads, to
       // the columns of N. The result is the same to the bit (a k, g or beta of a later chunk that is not finite reaches
-      // every column of N, and through N what comes after the segment). With decays of e^-0.8 a token a segment's M has
+      // every column of N, and through N what comes after the segment; a v, its own column of N alone). With decays of e^-0.8 a token a segment's M has
       // left the fp32 range after three chunks, with e^-0.24 after eight, with e^-0.04 after 47; looked at only once the
       // decays' own product has. 16 packed events of 520 000 tokens, 8 x 128 x 128, e^-0.8: pass 890 -> 691 us,
       // call 2 166 -> 2 000; no change where M lives on. Heads up to

@@ -689,3 +689,23 @@ def test_large_launches_are_as_exact_as_a_lane_per_column(device, B, T, H, K, V,
     off = lambda got: [float((x.double() - y).norm()) for x, y in zip(got, want)]
     lane = off(run(beta[..., None].expand_as(v).contiguous()))
     assert all(a <= 1.05 * b for a, b in zip(off(run(beta)), lane))
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 128, torch.float16), (128, 64, torch.bfloat16), (128, 128, torch.bfloat16)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_v_of_wide_heads_that_is_not_finite_stays_in_its_column(device, K, V, dtype, value, monkeypatch):
+    # early and late in a segment of four chunks (the map of a segment with strong decays has become zero by then), with
+    # decays that carry over many segments (head 0) and not over one (head 1): every other column keeps its bits
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 4)
+    T = 64 * 4 * 11 - 9
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 2, K, V, dtype, seed=K + V, g_scale=0.01)
+    g[:, :, 1] *= 160
+    args = _to(device, q, k, v, g, beta)
+    o, s = gd.chunk_gated_delta_rule(*args, output_final_state=True)
+    others = [c for c in range(V) if c != 5]
+    for at in (256 + 3, 256 + 200):
+        bad = args[2].clone()
+        bad[0, at, :, 5] = value
+        o1, s1 = gd.chunk_gated_delta_rule(args[0], args[1], bad, *args[3:], output_final_state=True)
+        assert not torch.isfinite(o1[0, at + 1:, 0, 5]).any() and not torch.isfinite(s1[0, 0, :, 5]).any()
+        assert torch.equal(o1[..., others], o[..., others]) and torch.equal(s1[..., others], s[..., others])
