@@ -1236,7 +1236,6 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         lds_barrier();  // the o tile of the last chunk is complete
         stager_flush(tk_p, ln_p);
       }
-      if constexpr (CUTS) lds_barrier();  // (the chain waves' notes on their columns, below)
     }
     return;
   }
@@ -1513,6 +1512,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   const int vslab = PASS_B ? wave : (is_m ? 0 : wave - KT / 32);
   const int col = 32 * vslab + ln;  // value column (unused for M slabs)
   const float vmask = is_m ? 0.0f : 1.0f;
+  const unsigned vkeep = uniform(is_m ? 0 : -1);
 
   f32x16 S[KT / 32];
   bool walked = false;
@@ -1572,6 +1572,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       issue(0, rm[0], rn[0], rd[0]);
       issue(1, rm[1], rn[1], rd[1]);
       int from = max(0, uniform(gdr_leading_cuts(dl, nst, lane)) - 1);
+      // (the decays' scalar loads stay in front of the branch: the compiler moves them behind it, a memory latency more in
+      // front of the first step; 15 000 tokens x 6 heads where nothing cuts off: pass 24.7 -> 25.0 us)
+      asm volatile("" : "+s"(rd[0]), "+s"(rd[1]));
       if (from > 0 && h0) {
         float probe = 0.0f;
 #pragma unroll
@@ -1632,7 +1635,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       for (int ks = 0; ks < KT / 16; ++ks) fk[tm * (KT / 16) + ks] = SWZ ? op_ld_kappa_swz<OT>(tx.k, SK, 32 * tm + ln, 16 * ks, hh)
                                         : op_ld_kappa<OT>(tx.k, SK, 32 * tm + ln, 16 * ks, hh);
   };
-  bool gone = false;  // (M) this wave's columns are zero
+  bool faded = false;  // the decays' product is zero (of a wide head: has been)
+  bool gone = false;   // (M) this wave's columns are zero
   auto m_is_zero = [&]() __attribute__((always_inline)) {
     unsigned any = 0;
 #pragma unroll
@@ -1643,7 +1647,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   };
   if (nc > 0) lds_barrier();  // tiles (c0) are ready
   if constexpr (EARLY_K) load_k_rows(tiles(0));
-  for (int c = c0; c < c1; ++c) {
+  int c = c0;
+  for (; c < c1 && !(SKIP_M && gone); ++c) {
     const GdrTilesT<OT> tl = tiles((c - c0) & 1);
     if constexpr (PASS_B && !OWN_Q) lds_barrier();  // Qb(c) (the chain waves only take part)
     const int c_nx = uniform(min(c + 1, c1 - 1));
@@ -1691,7 +1696,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
           // (training form: selected, not multiplied away, so that a v that is not finite stays out of M' and with it out
           // of the gradients of the tokens before it; so with SKIP_M, where it would reach M, and through M the other value
           // columns behind the segment, only as long as M lives on)
-          const float v_ = KEEP || SKIP_M ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e]) : vmask * (float)vv[4 * tm + b4][e];
+          const float v_ = SKIP_M ? op_elem_keep<OT>(vv[4 * tm + b4], e, vkeep)
+                           : KEEP ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e])
+                                  : vmask * (float)vv[4 * tm + b4][e];
           acc[4 * b4 + e] = be[4 * tm + b4][e] * (v_ - ks_);
         }
       Rb[2 * tm + 0] = acc_to_op<OT>(acc, 0);
@@ -1760,13 +1767,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       // decays' own product has. 16 packed events of 520 000 tokens, 8 x 128 x 128, e^-0.8: pass 890 -> 691 us,
       // call 2 166 -> 2 000; no change where M lives on. Heads up to
       // 64 x 64 are bound by the chain of a chunk and gain nothing (the loop's second exit cost them registers: 127 -> 144 us).
-      if (is_m && uniform(__float_as_int(dtot)) == 0) {
-        gone = m_is_zero();
-        if (gone) {
-          for (int left = c1 - c - 1; left > 0; --left) lds_barrier();  // B(c + 1) ..
-          break;
-        }
-      }
+      faded |= uniform(__float_as_int(dtot)) == 0;
+      if (is_m && faded) gone = m_is_zero();
     }
     if constexpr (PASS_B) {
       if constexpr (!EARLY_Q) {  // batch: Q rows, P fragments, output factors
@@ -1832,23 +1834,27 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   if constexpr (STAGER_FLUSH) {
     if (nc > 0) lds_barrier();  // the o tile of the last chunk is complete (the stagers write it out)
   }
+  if constexpr (SKIP_M) {
+    for (; c < c1; ++c) lds_barrier();  // B(c)
+  } else if constexpr (CUTS) {
+    faded = uniform(__float_as_int(dtot)) == 0;
+  }
   // epilogue; the opaque zero keeps the compiler from computing all these addresses before the loop
   int late = 0;
   asm volatile("" : "+v"(late));
   if constexpr (CUTS) {
     // A segment whose M is zero and whose N is finite hands N on whatever finite state it starts from: its decay is
     // stored as -0 (gdr_d_cut), which those who walk the composites look for. Every wave notes what it knows of its own
-    // columns, wave 0 stores the decay.
-    if (nc > 0) {
-      bool fine = false;
-      if (uniform(__float_as_int(dtot)) == 0) {
-        float probe = 0.0f;  // 0 x every entry: NaN unless all are finite
+    // columns, wave 0 stores the decay. Looked at only where the decays' product has left the fp32 range, which all chain
+    // waves see at the same chunk; the stagers may have ended, a barrier does not wait for waves that have. (With a note and
+    // a barrier in every segment, 9 000 tokens x 6 x 128 x 128 where none does: pass 25.0 us; so 23.9, without any look 23.7.)
+    if (faded) {
+      float probe = 0.0f;  // 0 x every entry: NaN unless all are finite
 #pragma unroll
-        for (int km = 0; km < KT / 32; ++km)
+      for (int km = 0; km < KT / 32; ++km)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(S[km][r], 0.0f, probe);
-        fine = is_m ? gone || m_is_zero() : __ballot(!(probe == 0.0f)) == 0;
-      }
+        for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(S[km][r], 0.0f, probe);
+      const bool fine = is_m ? gone || m_is_zero() : __ballot(!(probe == 0.0f)) == 0;
       float* note = tiles(0).misc + 8;
       if (lane == 0) note[wave] = fine ? 0.0f : 1.0f;
       lds_barrier();
@@ -2121,15 +2127,57 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
     for (int q4 = 0; q4 < 4; ++q4) n[q4] = N[(wave * 4 + q4) * 64 + lane];
     d = (top ? Dout : Dsrc)[sh];
   };
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d) issue(max(0, min(d, last)), rm[d], rn[d], rd[d]);
-
   // Strong decays: a group whose maps all cut off what lies before them is its last map (60 000 tokens x 8 heads:
-  // 7.9 -> 5.5 us).
-  bool cut = false;
-  if constexpr (MODE == SCAN_GROUP && !REV) {
-    cut = gdr_leading_cuts(Dsrc[(size_t)(item0 + min(lane, nsteps)) * HV + hv], G, lane) >= G;
-    if (cut) {
+  // 7.9 -> 5.5 us). The look at the decays must not hold up a walk that it does not shorten: their load is issued in front of
+  // the maps', so that it is waited for alone, and the maps' loads stay in order and in front of the branch; the group that is
+  // cut off leaves by itself. (Looked at behind the maps' loads, with one way through the loop for both: 9 000 tokens x 6 x
+  // 128 x 128 where nothing cuts off 13.8 us, 8.3 where all do; so 13.55 and 7.85; 13.3 without the look.)
+  constexpr bool LOOK = MODE == SCAN_GROUP && !REV;
+  const float d_look = LOOK ? Dsrc[(size_t)(item0 + min(lane, nsteps)) * HV + hv] : 0.0f;
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    if constexpr (LOOK) __builtin_amdgcn_sched_barrier(0);
+    issue(max(0, min(d, last)), rm[d], rn[d], rd[d]);
+  }
+
+  auto store_composite = [&](float dprod) __attribute__((always_inline)) {
+    const size_t gh = (size_t)(MODE == SCAN_PIECES ? seg0 + j : seq * gmax + j) * HV + hv;
+    if (is_pm) {
+      unsigned char* out = Mout + gh * M_BYTES;
+      const int mcol = 32 * vn + ln, ks = mcol >> 4, c16 = mcol & 15;
+      const int hs = (c16 >> 2) & 1, slot = 4 * (c16 >> 3) + (c16 & 3);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 32 * wave + acc_row(r, hh);
+        const float val = S[r] - (row == mcol ? dprod : 0.0f);
+        *reinterpret_cast<OT*>(out + ((size_t)((wave * NKS + ks) * 64 + 32 * hs + (row & 31))) * 16 + 2 * slot) = (OT)val;
+      }
+      if (vn == 0 && tid == 0) Dout[gh] = dprod;
+    } else {
+      f32x4* out = reinterpret_cast<f32x4*>(Nout + (gh * (VT / 32) + nblk) * N_BYTES);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        f32x4 t;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = S[4 * q4 + e];
+        out[(wave * 4 + q4) * 64 + lane] = t;
+      }
+    }
+  };
+  if constexpr (LOOK) {
+    __builtin_amdgcn_sched_barrier(0);
+    const bool cut = gdr_leading_cuts(d_look, G, lane) >= G;
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) asm volatile("" : "+s"(rd[d]));
+    if (__builtin_expect(cut, 0)) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {  // (loads that only the walk uses would be moved behind the branch)
+#pragma unroll
+        for (int f = 0; f < NM; ++f) asm volatile("" ::"v"(rm[d][f]));
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) asm volatile("" ::"v"(rn[d][q4]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
       const f32x4* N = reinterpret_cast<const f32x4*>(Nsrc + (((size_t)(item0 + nsteps) * HV + hv) * (VT / 32) + nblk) * N_BYTES);
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
@@ -2137,6 +2185,8 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[4 * q4 + e] = is_pm ? 0.0f : t[e];
       }
+      store_composite(-0.0f);
+      return;
     }
   }
 
@@ -2212,34 +2262,9 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
       for (int u = 0; u < LONG; ++u) step(p0 + u, rm[u % DEPTH], rn[u % DEPTH], rd[u % DEPTH]);
     }
   }
-  for (; !cut && p0 <= nsteps; p0 += DEPTH) {
+  for (; p0 <= nsteps; p0 += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) step(p0 + d, rm[d], rn[d], rd[d]);
   }
-  if constexpr (COMPOSE) dprod = cut ? -0.0f : __builtin_fabsf(dprod);
-
-  if (COMPOSE) {  // exactly G maps were applied (G is a multiple of DEPTH): store the composite
-    const size_t gh = (size_t)(MODE == SCAN_PIECES ? seg0 + j : seq * gmax + j) * HV + hv;
-    if (is_pm) {
-      unsigned char* out = Mout + gh * M_BYTES;
-      const int mcol = 32 * vn + ln, ks = mcol >> 4, c16 = mcol & 15;
-      const int hs = (c16 >> 2) & 1, slot = 4 * (c16 >> 3) + (c16 & 3);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = 32 * wave + acc_row(r, hh);
-        const float val = S[r] - (row == mcol ? dprod : 0.0f);
-        *reinterpret_cast<OT*>(out + ((size_t)((wave * NKS + ks) * 64 + 32 * hs + (row & 31))) * 16 + 2 * slot) = (OT)val;
-      }
-      if (vn == 0 && tid == 0) Dout[gh] = dprod;
-    } else {
-      f32x4* out = reinterpret_cast<f32x4*>(Nout + (gh * (VT / 32) + nblk) * N_BYTES);
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        f32x4 t;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) t[e] = S[4 * q4 + e];
-        out[(wave * 4 + q4) * 64 + lane] = t;
-      }
-    }
-  }
+  if (COMPOSE) store_composite(__builtin_fabsf(dprod));  // exactly G maps were applied (G is a multiple of DEPTH)
 }

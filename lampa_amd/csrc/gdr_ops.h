@@ -23,6 +23,20 @@ struct OpVec {
   typedef T x2 __attribute__((ext_vector_type(2)));
 };
 
+// Element e of x (a compile-time constant) widened, or zero where `keep` (all bits or none, the same in the whole wave) is
+// none: for bf16 in the one instruction that widens it.
+template <typename T>
+__device__ __forceinline__ float op_elem_keep(typename OpVec<T>::x4 x, int e, unsigned keep) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  const unsigned pair = __builtin_bit_cast(u32x2, x)[e / 2];
+  if constexpr (__is_same(T, __bf16)) {
+    const unsigned bytes = keep ? 0x01000c0cu : 0x0c0c0c0cu;  // bytes 1, 0 of the pair in front of two zeros
+    return __uint_as_float(e & 1 ? pair & (keep & 0xffff0000u) : __builtin_amdgcn_perm(pair, pair, bytes));
+  } else {
+    return (float)__builtin_bit_cast(typename OpVec<T>::x2, pair & keep)[e & 1];
+  }
+}
+
 // 8 accumulator registers [base, base + 8) of a lane, rounded to T: the lane's share of an MFMA operand whose 16-wide
 // contraction step covers accumulator rows 16 (base / 8) .. + 15 in slot order (see acc_to_operand in gdr_common.h).
 // Read as the B operand it is (rows of the accumulator tile = contraction, lane's column = operand column); read as

@@ -709,3 +709,18 @@ def test_v_of_wide_heads_that_is_not_finite_stays_in_its_column(device, K, V, dt
         o1, s1 = gd.chunk_gated_delta_rule(args[0], args[1], bad, *args[3:], output_final_state=True)
         assert not torch.isfinite(o1[0, at + 1:, 0, 5]).any() and not torch.isfinite(s1[0, 0, :, 5]).any()
         assert torch.equal(o1[..., others], o[..., others]) and torch.equal(s1[..., others], s[..., others])
+
+
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128)])
+def test_growth_without_bound_behind_a_map_that_has_become_zero(device, K, V, monkeypatch):
+    # a log-decay of plus infinity in the last chunk of a segment, where the decays' product and the segment's M are zero: it
+    # is not taken for a segment that cuts off the past, nothing behind it is finite, what lies before and the other head are
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 8)
+    T = 64 * 8 * 10
+    args = _to(device, *synth.gdr_inputs(1, T, 2, K, V, torch.bfloat16, seed=K, g_scale=1.6))
+    o, s = gd.chunk_gated_delta_rule(*args, output_final_state=True)
+    at, start = 64 * 8 + 64 * 7 + 5, 64 * 8 + 64 * 7
+    args[3][0, at, 0] = float("inf")
+    o1, s1 = gd.chunk_gated_delta_rule(*args, output_final_state=True)
+    assert torch.equal(o1[:, :start], o[:, :start]) and torch.equal(o1[:, :, 1], o[:, :, 1]) and torch.equal(s1[:, 1], s[:, 1])
+    assert not torch.isfinite(o1[0, start + 64:, 0]).any() and not torch.isfinite(s1[0, 0]).any()
