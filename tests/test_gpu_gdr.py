@@ -724,3 +724,28 @@ def test_growth_without_bound_behind_a_map_that_has_become_zero(device, K, V, mo
     o1, s1 = gd.chunk_gated_delta_rule(*args, output_final_state=True)
     assert torch.equal(o1[:, :start], o[:, :start]) and torch.equal(o1[:, :, 1], o[:, :, 1]) and torch.equal(s1[:, 1], s[:, 1])
     assert not torch.isfinite(o1[0, start + 64:, 0]).any() and not torch.isfinite(s1[0, 0]).any()
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (36, 64, torch.float32), (64, 130, torch.float16)])
+@pytest.mark.parametrize("lens", ["one", "two", "one long"])
+def test_few_tokens_of_very_many_sequences(device, K, V, dtype, lens):
+    # more than 4 096 waves of 32 columns at 32 < K <= 64: up to two tokens a sequence (on average: also where one sequence has
+    # most of them, and others none) go to the kernel with a lane per column; with states in and out
+    H, HV = 4, 8
+    n = 4096 // (HV * -(-V // 32)) + 1
+    packed = lens == "one long"
+    tokens = [1, 0] * (n // 2) + [n // 2] if packed else [1 if lens == "one" else 2] * n
+    n, cu = len(tokens), torch.tensor([0] + list(np.cumsum(tokens)), dtype=torch.long)
+    B, T = (1, int(cu[-1])) if packed else (n, tokens[0])
+    q, k, _, _, _ = synth.gdr_inputs(B, T, H, K, V, dtype, seed=K, g_scale=0.2)
+    _, _, v, g, beta = synth.gdr_inputs(B, T, HV, K, V, dtype, seed=V, g_scale=0.2)
+    h0 = torch.randn(n, HV, K, V, generator=torch.Generator().manual_seed(2))
+    where = {"cu_seqlens": cu} if packed else {}
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta, initial_state=h0, l2=og.L2_RECURRENT, **where)
+    where = {x: y.to(device) for x, y in where.items()}
+    o, s = gd.fused_recurrent_gated_delta_rule(*_to(device, q, k, v, g, beta), initial_state=h0.to(device),
+                                               output_final_state=True, use_qk_l2norm_in_kernel=True, **where)
+    assert _errors(s, want_s)[0] <= FP32_TOL
+    # (fp32 arithmetic, o rounded once: half a unit in the last place of the largest value)
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
+    assert (o.float().cpu() - want_o.float()).abs().max() <= FP32_TOL + ulp * want_o.abs().max()
