@@ -1696,7 +1696,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
           // (training form: selected, not multiplied away, so that a v that is not finite stays out of M' and with it out
           // of the gradients of the tokens before it; so with SKIP_M, where it would reach M, and through M the other value
           // columns behind the segment, only as long as M lives on)
-          const float v_ = SKIP_M ? op_elem_keep<OT>(vv[4 * tm + b4], e, vkeep)
+          const float v_ = SKIP_M ? (__is_same(OT, __bf16) ? 1.0f : vmask) * op_elem_keep<OT>(vv[4 * tm + b4], e, vkeep)
                            : KEEP ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e])
                                   : vmask * (float)vv[4 * tm + b4][e];
           acc[4 * b4 + e] = be[4 * tm + b4][e] * (v_ - ks_);
@@ -1762,13 +1762,14 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       // Columns of M that have become zero stay zero, whatever chunks follow: a wave whose columns all have only takes part
       // in the barriers from there on and leaves the LDS and the matrix cores, which bound this pass at the wide heads, to
       // the columns of N. The result is the same to the bit (a k, g or beta of a later chunk that is not finite reaches
-      // every column of N, and through N what comes after the segment; a v, its own column of N alone). With decays of e^-0.8 a token a segment's M has
-      // left the fp32 range after three chunks, with e^-0.24 after eight, with e^-0.04 after 47; looked at only once the
-      // decays' own product has. 16 packed events of 520 000 tokens, 8 x 128 x 128, e^-0.8: pass 890 -> 691 us,
-      // call 2 166 -> 2 000; no change where M lives on. Heads up to
-      // 64 x 64 are bound by the chain of a chunk and gain nothing (the loop's second exit cost them registers: 127 -> 144 us).
+      // every column of N, and through N what comes after the segment; a v, its own column of N alone). With decays of e^-0.8
+      // a token a segment's M has left the fp32 range after three chunks, with e^-0.24 after eight, with e^-0.04 after 47;
+      // looked at only once the decays' own product has. 16 packed events of 520 000 tokens, 8 x 128 x 128, e^-0.8: pass
+      // 890 -> 691 us, call 2 166 -> 2 000. Where M lives on, calls of 25 080 tokens x 5 heads take 0.6 us less (64 x 128) to
+      // 1 us more (128 x 64, of 98: other registers; as a branch of which the compiler does not know that the whole wave takes
+      // it, 2 us). Heads up to 64 x 64 are bound by the chain of a chunk and gain nothing.
       faded |= uniform(__float_as_int(dtot)) == 0;
-      if (is_m && faded) gone = m_is_zero();
+      if (uniform(is_m) && faded) gone = m_is_zero();
     }
     if constexpr (PASS_B) {
       if constexpr (!EARLY_Q) {  // batch: Q rows, P fragments, output factors
