@@ -5,8 +5,9 @@
 // rank-one update and S^T q) are per-lane loops with no cross-lane traffic; k_t and q_t are loaded one element per
 // lane, normalised with a wave reduction and broadcast with v_readlane.
 // gdr_recurrent_split_kernel (further down, what nearly all launches take): 16 columns per wave, the state rows of a column
-// split over eight lanes, the token's operands staged in LDS by the waves of a workgroup together. The first one serves sizes
-// and alignments that cannot be staged in 16-byte pieces, head-wise beta, and a few tokens of very many sequences.
+// split over eight or four lanes, the token's operands staged in LDS by the waves of a workgroup together. The first one serves
+// sizes and alignments that cannot be staged in 16-byte pieces, head-wise beta, and one or two tokens each of very many
+// sequences at 32 < K <= 64.
 //
 // Replaces fused_recurrent_gated_delta_rule_fwd_kernel, models/hattention/gated_delta_rule_ori.py:372-464
 // (state layout [N, HV, K, V] fp32; grouped value heads HV >= H).  It is also the fp32 mode of the chunk operator and

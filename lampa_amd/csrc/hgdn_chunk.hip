@@ -783,7 +783,7 @@ __global__ void __launch_bounds__(64 * HG_SCAN_WAVES, 2)
                      const float* __restrict__ Dcomp, float* __restrict__ Xinit, int HV, int p) {
   constexpr int NKS = KT / 16, NM = (KT / 32) * NKS, M_BYTES = KT * KT * 2, N_BYTES = KT * 32 * 4;
   constexpr int LPW = HG_NLV / HG_SCAN_WAVES;
-  static_assert(LPW == 3, "LEVELS");
+  static_assert(LPW == 3, "LEVELS holds the bits of a wave's three levels");
   __shared__ __align__(16) float s_acc[KT * 32];
   const int vslab = blockIdx.x, seq = blockIdx.y, hv = blockIdx.z;
   const int seg0 = pv.seq_seg0[seq], nseg = pv.seq_nseg[seq];
@@ -1024,8 +1024,9 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
 // power of two (or at least the longest sequence's chunk count: one segment per sequence); every sequence may hold at
 // most 2^12 chunks, every sequence length must be a multiple of 64 and L must cover 7 + the number of chunk-index bits
 // of the longest sequence.
-// level_states (nullable): fp32 [n_seq, HV, K, V, L], ZEROED by the caller; receives the occupied levels' states after
-// the last token of every sequence (the reference's HState.states); needs sequences of equal length, a multiple of 64.
+// level_states (nullable): fp32 [n_seq, HV, K, V, L]; receives the occupied levels' states after the last token of every
+// sequence (the reference's HState.states); needs sequences of equal length, a multiple of 64. The other levels are neither
+// read nor written: a caller that reads them zeroes them.
 extern "C" int lampa_hgdn_chunk_fwd(const void* q, const void* k, const void* v, const float* g, const float* beta,
                                     const void* lam, int lam_dtype, float lam_div, void* o, float* level_states,
                                     const int32_t* plan_host, const int32_t* plan_dev, int H, int HV, int K, int V, int L,

@@ -472,14 +472,14 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
 // between are summed over 16 lanes (DPP) every second token. k, q (normalised, fp32), the decays, the weights and v of 32
 // tokens are staged in LDS by the workgroup's four waves, so a token waits for no load. Levels that hold no token yet are
 // not read, and written as the zeros they are.
-// hgdn_tail_rows_kernel (more levels): lane = state row (two rows for K > 64), the row's LM level values in registers. Sums
+// hgdn_tail_rows_kernel (more levels): lane = state row (two rows for K > 64), the row's 32 level values in registers. Sums
 // over the rows (k^T S_l for the levels > 0, the output, the two norms) are exchanges between lanes: 16 levels at a time are
 // halved four times until a lane holds one level's sum over its group of 16 lanes (`wave_sums16`), and go back to all lanes
 // as scalars; the next token's values are loaded while this one is worked on.
 // A prefill of 15 000 tokens (24 behind its whole chunks, 8 heads of 64 x 64): 708 us with a launch of the single-token kernel
 // and its copies per token, 188 us with the rows kernel (its own 38),
 // 173 us with this one (25).
-#define HGS_TAIL_LEVELS 17  // levels of the narrow instantiation: sequences up to 65 536 tokens
+#define HGS_TAIL_LEVELS 17  // level 0 and one for each of 16 lanes: sequences up to 65 536 tokens
 #define HGS_TAIL_WAVES 4
 #define HGS_DPP_ROR8 0x128
 #define HGS_DPP_HALF_MIRROR 0x141
@@ -523,7 +523,7 @@ __device__ __forceinline__ float hgs_lane(float x, int n) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), n));
 }
 
-template <typename T, int LM, int ROWS>
+template <typename T, int ROWS>
 __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
     hgdn_tail_rows_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                      const float* __restrict__ g, const float* __restrict__ beta, const void* __restrict__ lam,
@@ -537,6 +537,7 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
   // Loads come from clamped addresses without conditions on the lane, and are converted and masked where they are used: a
   // conditional load that is converted on the spot is a branch with a wait for memory inside (one per value: four round
   // trips per token, and one per level at either end).
+  constexpr int LM = HGS_LMAX;
   float S[ROWS][LM];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r)
@@ -868,8 +869,8 @@ extern "C" int lampa_hgdn_tail(const void* q, const void* k, const void* v, cons
       if (K <= 64) HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 16>);                  \
       else HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 32>);                          \
     } else {                                                                     \
-      if (K <= 64) HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA HGS_LMAX HGS_COMMA 1>); \
-      else HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA HGS_LMAX HGS_COMMA 2>);   \
+      if (K <= 64) HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA 1>);              \
+      else HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA 2>);                      \
     }                                                                            \
   } while (0)
 #define HGS_COMMA ,

@@ -176,8 +176,8 @@ def _segment_tokens(tokens: int, n_value_heads: int, K: int, V: int) -> int:
     """Segment length of the segmented token-serial operator, a multiple of 32 (the kernel's groups of tokens): two waves
     of 16 value columns per SIMD in the output pass; one per SIMD where that leaves heads wider than 32 fewer than 128 tokens
     a segment (their maps are the larger part then). Measured against all lengths from 16 to 1 024, fp32, us with this rule
-    / best: 8 192 x 4 x 32 x 32 53 / 51, 1 000 x 4 x 32 x 32 27 / 27, 30 000 x 8 x 32 x 32 148 / 148, 3 000 x 8 x 64 x 64
-    76 / 76, 8 192 x 4 x 64 x 64 93 / 93, 30 000 x 8 x 64 x 64 410 / 410, 2 x 8 192 x 4 x 128 x 128 499 / 447."""
+    / best: 8 192 x 4 x 32 x 32 48 / 47, 1 000 x 4 x 32 x 32 27 / 27, 30 000 x 8 x 32 x 32 145 / 140, 3 000 x 8 x 64 x 64
+    76 / 75, 8 192 x 4 x 64 x 64 96 / 93, 30 000 x 8 x 64 x 64 400 / 400, 2 x 8 192 x 4 x 128 x 128 470 / 450."""
     work = tokens * n_value_heads * -(-V // 16)
     seg_len = -(-work // 2048 // 32) * 32
     if K > 32 and seg_len < 128:

@@ -308,7 +308,7 @@ def _rows_of(B: int, T: int, **tensors):
 ONE_TOKEN_STEP = 2 ** 15, 2 ** 17
 
 TAIL_FILLS_LEVELS = 17  # up to so many levels ``lampa_hgdn_tail`` writes every level and reads only those that hold tokens
-TAIL_MAX_K = 128  # ``lampa_hgdn_tail`` holds a state column in two registers per lane and level at most
+TAIL_MAX_K = 128  # ``lampa_hgdn_tail`` holds a state column in registers: of one level 32 rows a lane, of all levels two
 
 
 def _tail(hstate: HState, q, k, v, g, l, beta, o, t0: int, scale, lam_div) -> None:
