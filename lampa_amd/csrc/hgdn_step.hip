@@ -471,7 +471,10 @@ extern "C" int lampa_hgdn_step(const void* q, const void* k, const void* v, cons
 // stored: it enters the output as a scalar and the state of the level it cascades into as one fma per row; the levels
 // between are summed over 16 lanes (DPP) every second token. k, q (normalised, fp32), the decays, the weights and v of 32
 // tokens are staged in LDS by the workgroup's four waves, so a token waits for no load. Levels that hold no token yet are
-// not read, and written as the zeros they are.
+// not read, and written as the zeros they are. RP, the rows of a lane: 4, 8, 16 or 32 as K asks. (With 16 rows for every
+// K <= 64 and the loads of empty levels in front of the first token, many sequences of two or three tokens were slower than
+// with the rows kernel: 128 x 2 tokens, 4 heads of 16 x 32, 34.3 us there, 47.6 so, 34.2 now; 4 of 32 x 64 78.7, 90.0, 66.5;
+// 8 of 64 x 64 234, 174, 161.)
 // hgdn_tail_rows_kernel (more levels): lane = state row (two rows for K > 64), the row's 32 level values in registers. Sums
 // over the rows (k^T S_l for the levels > 0, the output, the two norms) are exchanges between lanes: 16 levels at a time are
 // halved four times until a lane holds one level's sum over its group of 16 lanes (`wave_sums16`), and go back to all lanes
@@ -683,7 +686,7 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
                      const float* __restrict__ g, const float* __restrict__ beta, const void* __restrict__ lam,
                      int lam_dtype, float lam_div, float* __restrict__ states, T* __restrict__ o, int n_tok, int tok0, int H,
                      int HV, int K, int V, int L, float scale, int l2norm) {
-  constexpr int KP = 4 * RP, NB = HGS_TAIL_BATCH, TPW = NB / HGS_TAIL_WAVES, NR = KP / 64;
+  constexpr int KP = 4 * RP, NB = HGS_TAIL_BATCH, TPW = NB / HGS_TAIL_WAVES, NR = KP > 64 ? KP / 64 : 1;
   __shared__ __align__(16) float s_k[NB][KP], s_q[NB][KP];
   __shared__ float s_lam[NB][HGS_TAIL_LEVELS], s_v[NB][HGS_TAIL_WAVES];
   __shared__ float4 s_sc[NB];  // e^g, beta, k . q
@@ -697,15 +700,19 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
   const bool filled = level < L && tok0 > 0 && ((tok0 - 1) >> (level - 1)) & 1;  // tokens in this lane's level
   float S[RP], prev[RP];  // prev: the k of the token before (first token: level 0 as it was)
 #pragma unroll
-  for (int r = 0; r < RP; ++r) {
-    const size_t at = (size_t)min(rg * RP + r, K - 1) * V * L;
-    S[r] = col[at + min(level, L - 1)];
-    prev[r] = col[at];
-  }
+  for (int r = 0; r < RP; ++r) S[r] = prev[r] = 0.0f;
+  if (tok0 > 0) {  // (else no level holds a token)
 #pragma unroll
-  for (int r = 0; r < RP; ++r) {
-    S[r] = filled && rg * RP + r < K ? S[r] : 0.0f;
-    prev[r] = tok0 > 0 && rg * RP + r < K ? prev[r] : 0.0f;
+    for (int r = 0; r < RP; ++r) {
+      const size_t at = (size_t)min(rg * RP + r, K - 1) * V * L;
+      S[r] = col[at + min(level, L - 1)];
+      prev[r] = col[at];
+    }
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {
+      S[r] = filled && rg * RP + r < K ? S[r] : 0.0f;
+      prev[r] = rg * RP + r < K ? prev[r] : 0.0f;
+    }
   }
   float prev_v = 1.0f;  // beta v of the token before
   auto stage = [&](int t0) __attribute__((always_inline)) {  // tokens t0 .. t0 + NB - 1, TPW of them by each wave
@@ -752,8 +759,10 @@ __global__ void __launch_bounds__(64 * HGS_TAIL_WAVES)
         kf[x] *= rk;
         qf[x] *= rq;
         kq = __builtin_fmaf(kf[x], qf[x], kq);
-        s_k[at][lane + 64 * x] = kf[x];
-        s_q[at][lane + 64 * x] = qf[x];
+        if (KP >= 64 || lane < KP) {
+          s_k[at][lane + 64 * x] = kf[x];
+          s_q[at][lane + 64 * x] = qf[x];
+        }
       }
       kq = wave_sum_all(kq);
       float lam_l = lam_dtype == GDR_FP32   ? __uint_as_float(lr[i])
@@ -866,7 +875,9 @@ extern "C" int lampa_hgdn_tail(const void* q, const void* k, const void* v, cons
   do {                                                                           \
     typedef TYPE TT;                                                             \
     if (L <= HGS_TAIL_LEVELS) {                                                  \
-      if (K <= 64) HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 16>);                  \
+      if (K <= 16) HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 4>);                   \
+      else if (K <= 32) HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 8>);              \
+      else if (K <= 64) HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 16>);             \
       else HGS_TAIL(hgdn_tail_kernel<TT HGS_COMMA 32>);                          \
     } else {                                                                     \
       if (K <= 64) HGS_TAIL(hgdn_tail_rows_kernel<TT HGS_COMMA 1>);              \

@@ -399,3 +399,30 @@ def test_tail_reads_only_the_levels_that_hold_tokens(device, B, T, t0, HV, K, V,
     assert (states.cpu() - want_s).abs().max() <= 2e-5 * want_s.abs().max()
     assert (states[..., [level for level in range(L) if not want_c.tolist()[level]]] == 0).all()
     assert (o[:, t0:].cpu() - want_o[:, t0:]).abs().max() <= 2e-5 * want_o.abs().max()
+
+
+@pytest.mark.parametrize("K", [1, 15, 16, 17, 32, 33])
+@pytest.mark.parametrize("T,t0", [(2, 0), (3, 0), (40, 7)])
+def test_tail_of_narrow_heads(device, K, T, t0):
+    # a lane's rows at their edges (4 up to K = 16, 8 up to 32, 16 beyond), from an empty state -- not read -- and from a held one
+    import ctypes
+    from lampa_amd import _capi
+    from lampa_amd._capi import ptr
+    B, HV, V, L = 3, 2, 6, 7
+    gen = torch.Generator().manual_seed(K)
+    q, k = (torch.randn(B, T, HV, K, generator=gen) for _ in range(2))
+    v, lam = torch.randn(B, T, HV, V, generator=gen), torch.randn(B, T, HV, L, generator=gen)
+    g, beta = -0.2 * torch.rand(B, T, HV, generator=gen), torch.rand(B, T, HV, generator=gen)
+    want_o, want_s, _ = oh.recurrent_c_state(q, k, v, g, beta, lam, scale=0.3)
+    states = torch.full((B, HV, K, V, L), float("nan"), device=device)
+    if t0:
+        _, s0, c0 = oh.recurrent_c_state(*(x[:, :t0].contiguous() for x in (q, k, v, g, beta, lam)), scale=0.3)
+        held = [level for level in range(L) if c0.tolist()[level]]
+        states[..., held] = s0[..., held].float().to(device)
+    args = [x.to(device) for x in (q, k, v, g, beta, lam)]
+    o = torch.empty_like(args[2])
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _capi.lib().lampa_hgdn_tail(*(ptr(x) for x in args), 2, 1.0, ptr(states), ptr(o), B, T, t0, HV, HV, K, V, L, 2, 0.3,
+                                       1, stream) == 0
+    assert (states.cpu() - want_s).abs().max() <= 2e-5 * want_s.abs().max()
+    assert (o[:, t0:].cpu() - want_o[:, t0:]).abs().max() <= 2e-5 * want_o.abs().max()
