@@ -107,7 +107,7 @@ struct HgPrepSmem {
   static_assert(6 * 1024 + HG_INTRA * 64 * 4 <= 64 * SK * 2, "fragments + lambda fit in the k tile");
 };
 
-template <typename T, int KT, int VT>
+template <typename T, int KT, int VT, bool FAR>
 __global__ void __launch_bounds__(256)
     hgdn_prep_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                      const void* __restrict__ lam, int lam_dtype, float lam_div,
@@ -447,7 +447,11 @@ __global__ void __launch_bounds__(256)
           acc = mfma32(frag_load(s_PL, 2 * tm + ks, lane), ld_kappa_tr(s_v, SV, 32 * vt, 16 * ks, lane), acc);
       float* out = Oi + ch * (64 * VT) + 32 * vt + ln;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(acc[r], &out[(32 * tm + acc_row(r, hh)) * VT]);
+      for (int r = 0; r < 16; ++r) {
+        float* at = &out[(32 * tm + acc_row(r, hh)) * VT];
+        if constexpr (FAR) __builtin_nontemporal_store(acc[r], at);
+        else *at = acc[r];
+      }
     } else {
       const int f = task - 2 * NU, which = f / (2 * NKS), g = f % (2 * NKS);  // fragment (tm, ks) = (g / NKS, g % NKS)
       const bf16x8 fr = ld_kappa(which == 0 ? s_w : s_qt, SK, 32 * (g / NKS) + ln, 16 * (g % NKS), hh);
@@ -534,7 +538,7 @@ __device__ __forceinline__ void hg_merge(int cs, int lvl0, int wave, bool chain,
   }
 }
 
-template <typename T, int KT, int VT>
+template <typename T, int KT, int VT, bool FAR>
 __global__ void __launch_bounds__(64 * (HG_CW + 2))
     hgdn_walk_kernel(const GdrPlanView pv, const int32_t* __restrict__ chunk_tok0, const int32_t* __restrict__ chunk_len,
                      const T* __restrict__ k, int H, const unsigned char* __restrict__ wrec, const unsigned char* __restrict__ Ub_in,
@@ -556,11 +560,10 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
   // Output of a chunk: every wave of the workgroup sums eight rows of the chain waves' partial tiles and the intra-chunk
   // part (read one chunk ahead), rounds and stores them -- lane = (row, four columns).
   const int orow = 8 * wave + (lane >> 3), ocol = 4 * (lane & 7);
-  // (non-temporal, as prep stores it: each value is read once, and the records, which the slabs share, stay in the caches.
-  // 60 032 x 8 x 64 x 64: the stores 404 -> 402 us, the loads as well 400; 15 000 the same)
   auto oi_load = [&](int c) __attribute__((always_inline)) {
-    return __builtin_nontemporal_load(
-        reinterpret_cast<const f32x4*>(Oi + ((size_t)uniform(c) * HV + hv) * (64 * VT) + orow * VT + 32 * vslab + ocol));
+    const f32x4* at = reinterpret_cast<const f32x4*>(Oi + ((size_t)uniform(c) * HV + hv) * (64 * VT) + orow * VT + 32 * vslab + ocol);
+    if constexpr (FAR) return __builtin_nontemporal_load(at);
+    else return *at;
   };
   auto out_rows = [&](int tok0, int len, f32x4 a) __attribute__((always_inline)) {
 #pragma unroll
@@ -941,9 +944,13 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, false, false, __bf16>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_a) != hipSuccess ||
-        hipFuncSetAttribute((const void*)hgdn_prep_kernel<T, KT, VT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)hgdn_prep_kernel<T, KT, VT, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             smem_p) != hipSuccess ||
-        hipFuncSetAttribute((const void*)hgdn_walk_kernel<T, KT, VT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)hgdn_prep_kernel<T, KT, VT, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            smem_p) != hipSuccess ||
+        hipFuncSetAttribute((const void*)hgdn_walk_kernel<T, KT, VT, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            smem_w) != hipSuccess ||
+        hipFuncSetAttribute((const void*)hgdn_walk_kernel<T, KT, VT, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             smem_w) != hipSuccess)
       return LAMPA_ERR_LAUNCH;
     attr_set = true;
@@ -988,7 +995,12 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   };
   if (pieces) composites();
   if (!fork()) return LAMPA_ERR_LAUNCH;
-  hipLaunchKernelGGL((hgdn_prep_kernel<T, KT, VT>), dim3(chunks, HV), dim3(256), smem_p, s, (const T*)q, (const T*)k,
+  // The intra-chunk part goes past the caches (stored and loaded with the non-temporal hint) where it is larger than they are:
+  // each value is read once, and the records, which the slabs share, stay there (8 x 64 x 64, us without / with the hint:
+  // 60 032 tokens 402.8 / 396.7, 40 000 333.0 / 330.4, 25 024 219.0 / 215.4). Below that it would only come back from
+  // further away (15 040 tokens, 31 MB, 138.9 / 139.4, 8 x 2 048 122.7 / 124.0, 64 x 64 36.6 / 37.3).
+  const bool far = (int64_t)chunks * HV * (64 * VT * 4) > (48ll << 20);
+  hipLaunchKernelGGL((far ? hgdn_prep_kernel<T, KT, VT, true> : hgdn_prep_kernel<T, KT, VT, false>), dim3(chunks, HV), dim3(256), smem_p, s, (const T*)q, (const T*)k,
                      (const T*)v, lam, lam_dtype, lam_div, pv.chunk_tok0, pv.chunk_len, tf, rec, Ubw, Oi, hstates, chunks_per_seq, H, HV, L,
                      scale, l2norm);
   LAMPA_PROF(s, "hgdn_prep_kernel");
@@ -1010,7 +1022,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
     if (hipStreamWaitEvent(s, ev_join, 0) != hipSuccess) return LAMPA_ERR_LAUNCH;
     hold.unlock();
   }
-  hipLaunchKernelGGL((hgdn_walk_kernel<T, KT, VT>), dim3(segs, HV, VT / 32), dim3(64 * (HG_CW + 2)), smem_w, s, pv,
+  hipLaunchKernelGGL((far ? hgdn_walk_kernel<T, KT, VT, true> : hgdn_walk_kernel<T, KT, VT, false>), dim3(segs, HV, VT / 32), dim3(64 * (HG_CW + 2)), smem_w, s, pv,
                      pv.chunk_tok0, pv.chunk_len, (const T*)k, H, rec, Ubw, Oi, split ? (const float*)Xi : (const float*)nullptr, (T*)o,
                      hstates, L, HV);
   LAMPA_PROF(s, "hgdn_walk_kernel");
