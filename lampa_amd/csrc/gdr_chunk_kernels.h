@@ -1566,7 +1566,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
     };
     if (nst > 0) {
       // (strong decays: the walk starts at the last map of a run of maps that cut off what lies before them; 60 000 tokens x
-      // 8 heads at e^-0.8 a token: pass 60.1 -> 57.2 us, call 130 -> 124, and 39.7 -> 39.3 for 6 007 tokens where none does)
+      // 8 heads at e^-0.8 a token: pass 60.1 -> 57.2 us, call 131 -> 124.5; 6 007 tokens where none does 39.6 -> 38.7)
       const int pl = min(lane, nst - 1);
       const float dl = (pl < lead ? Dgrp : Dcomp)[(size_t)(pl < lead ? seq * gmax + pl : item0 + (pl - lead)) * HV + hv];
       issue(0, rm[0], rn[0], rd[0]);
