@@ -2,6 +2,7 @@
 // The kernels (and the description of the algorithm) are in gdr_chunk_kernels.h.
 #include "gdr_chunk_kernels.h"
 #include "gdr_train.h"
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -9,14 +10,16 @@ struct GdrWorkspace {
   int64_t off_t, off_m, off_n, off_d, off_sinit, off_gm, off_gn, off_gd, max_groups, bytes;
 };
 
-static GdrWorkspace gdr_workspace(int64_t chunks, int64_t segs, int HV, int K, int V) {
+// kept: the records are kept elsewhere (training form)
+static GdrWorkspace gdr_workspace(int64_t chunks, int64_t segs, int HV, int K, int V, bool kept = false) {
   GdrWorkspace w;
   int64_t off = 0;
-  w.off_t = off;     off += lampa_align_up(chunks * HV * (int64_t)REC_BYTES, 256);
+  w.off_t = off;     off += kept ? 0 : lampa_align_up(chunks * HV * (int64_t)REC_BYTES, 256);
   w.off_m = off;     off += lampa_align_up(segs * HV * (int64_t)K * K * 2, 256);
   w.off_n = off;     off += lampa_align_up(segs * HV * (int64_t)K * V * 4, 256);
   w.off_d = off;     off += lampa_align_up(segs * HV * 4, 256);
-  w.off_sinit = off; off += lampa_align_up((segs + 1) * HV * (int64_t)K * V * 4, 256);  // + a spare slot (scan)
+  // the segments' initial states + a spare slot (scan); before the scan the chunks' edges (GDR_EDGE_*) and a spare row
+  w.off_sinit = off; off += lampa_align_up(std::max((segs + 1) * HV * (int64_t)K * V, (chunks + 1) * HV) * 4, 256);
   // two-level scan: composites of the groups of GDR_SCAN_GROUP segments
   w.max_groups = segs / GDR_SCAN_GROUP + 2;
   w.off_gm = off;    off += lampa_align_up(w.max_groups * HV * (int64_t)K * K * 2, 256);
@@ -45,6 +48,11 @@ extern "C" int64_t lampa_gdr_chunk_workspace_bytes(int64_t total_chunks, int64_t
   return gdr_workspace(total_chunks, n_segments, HV, K, V).bytes;
 }
 
+// chunks of the longest segment
+static int gdr_max_chunks(const int32_t* plan_host) {
+  return plan_host[plan_host[PLAN_OFF_SEG_NCHUNKS] + plan_host[plan_host[PLAN_OFF_SEG_ORDER]]];
+}
+
 // Buffers of the training form (gdr_train.h), or none.
 struct GdrKeep {
   unsigned char *rec, *states, *mt;
@@ -56,9 +64,9 @@ struct GdrKeep {
 template <typename T, int KT, int VT, bool KEEP = false>
 static int gdr_chunk_launch(const void* q, const void* k, const void* v, const float* g, const float* beta, void* o,
                             const float* h0, float* ht, const GdrPlanView pv, int n_seq, int chunks, int segs, int max_nseg,
-                            int H, int HV, float scale, int l2norm, unsigned char* ws, hipStream_t s,
+                            int max_chunks, int H, int HV, float scale, int l2norm, unsigned char* ws, hipStream_t s,
                             const GdrKeep kp = GdrKeep{}) {
-  const GdrWorkspace w = gdr_workspace(KEEP ? 0 : chunks, segs, HV, KT, VT);  // (KEEP: the records are kept elsewhere)
+  const GdrWorkspace w = gdr_workspace(chunks, segs, HV, KT, VT, KEEP);
   unsigned char* tf = KEEP ? kp.rec : ws + w.off_t;
   unsigned char* Mc = ws + w.off_m;
   unsigned char* Nc = ws + w.off_n;
@@ -85,13 +93,14 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
   }
   hold.unlock();
   LAMPA_PROF(s, "start");
+  float* edge = segs > n_seq && max_chunks >= GDR_EDGE_NC ? Si : nullptr;  // the chunks' edges, for the composite pass
   if (chunks > 0) {
     hipLaunchKernelGGL((gdr_local_kernel<T, T, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g, beta,
-                       pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, kp.positive_g);
+                       pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, kp.positive_g, edge);
     LAMPA_PROF(s, "gdr_local_kernel");
     if (segs > n_seq) {
       hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
-                         (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, Mc, Nc, Dc,
+                         (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)Si, Mc, Nc, Dc,
                          (T*)nullptr, (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
                          (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, kp.mt, VT);
       LAMPA_PROF(s, "gdr_segment_kernel<composite>");
@@ -155,7 +164,7 @@ extern "C" int lampa_gdr_chunk_fwd(const void* q, const void* k, const void* v, 
   int max_nseg = 0;
   for (int i = 0; i < n_seq; ++i) max_nseg = plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] > max_nseg ? plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] : max_nseg;
 #define GDR_CASE(TT, KK, VV)                                                                                       \
-  return gdr_chunk_launch<TT, KK, VV>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, H, HV, scale, \
+  return gdr_chunk_launch<TT, KK, VV>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, gdr_max_chunks(plan_host), H, HV, scale, \
                                       l2norm, ws, s)
   if (dtype == GDR_BF16) {
     if (K == 32 && V == 32) GDR_CASE(__bf16, 32, 32);
@@ -192,7 +201,7 @@ extern "C" int64_t lampa_gdr_train_saved_bytes(const int32_t* plan_host, int HV)
 }
 extern "C" int64_t lampa_gdr_train_workspace_bytes(const int32_t* plan_host, int HV) {
   if (!plan_host || HV < 1) return LAMPA_ERR_INVALID;
-  return gdr_workspace(0, plan_host[PLAN_N_SEGMENTS], HV, 64, 64).bytes;
+  return gdr_workspace(plan_host[PLAN_TOTAL_CHUNKS], plan_host[PLAN_N_SEGMENTS], HV, 64, 64, true).bytes;
 }
 
 // As lampa_gdr_chunk_fwd for q, k, v of 64 columns; the rows of o are V <= 64 columns, a multiple of 8 (K, V: the heads before
@@ -221,8 +230,8 @@ extern "C" int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const voi
     return LAMPA_ERR_INVALID;
   }
   if (dtype == GDR_BF16)
-    return gdr_chunk_launch<__bf16, 64, 64, true>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, H, HV, scale,
+    return gdr_chunk_launch<__bf16, 64, 64, true>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, gdr_max_chunks(plan_host), H, HV, scale,
                                                   l2norm, (unsigned char*)workspace, (hipStream_t)stream, kp);
-  return gdr_chunk_launch<_Float16, 64, 64, true>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, H, HV, scale,
+  return gdr_chunk_launch<_Float16, 64, 64, true>(q, k, v, g, beta, o, h0, ht, pv, n_seq, chunks, segs, max_nseg, gdr_max_chunks(plan_host), H, HV, scale,
                                                   l2norm, (unsigned char*)workspace, (hipStream_t)stream, kp);
 }

@@ -92,6 +92,35 @@ __device__ __forceinline__ int gdr_leading_cuts(float d, int n, int lane) {
   return open ? __builtin_ctzll(open) : 64;
 }
 
+// Edge of a chunk and head: its total log-decay (units of log 2), where the map of every token is a contraction times its
+// decay -- no positive log-decay, 0 <= beta |k|^2 <= 2 for the key as the operator uses it, all of it finite -- and infinity
+// elsewhere: chunks of finite edges leave at most 2^(sum of the edges) of any state, whatever their keys.
+//
+// The composite pass starts where the edges behind sum up to GDR_EDGE_REACH: nothing is left there of M and of the sources in
+// front. With beta up to 2^14 and beta |k|^2 <= 2 a write is below 2^8 |v|, the state of 128 chunks below 2^21 |v|, and 2^-208 of
+// that below the fp32 range up to |v| = 2^38 (M = 0, by which the scan forgets a state, is found at 2^-149). At e^-0.8 a token a
+// segment's last three chunks are walked, at e^-0.24 ten, at e^-0.04 all. us of the composite pass / the call before and after:
+// 60 000 tokens x 8 heads x 64 x 64 at e^-0.8 45.7 -> 25.7 / 125.5 -> 112, at e^-0.24 126 -> 117.6; 16 packed events of 520 000
+// tokens, 8 x 128 x 128 689 -> 241 / 2 005 -> 1 590; at e^-0.04 131.7 -> 132.0 and 290.5 -> 292.3, the price of the look.
+#define GDR_EDGE_BETA 16384.0f
+#define GDR_EDGE_REACH -208.0f
+// Chunks left out that pay for looking at their v; chunks of a segment that pay for the look at its edges (15 000 tokens x 8 x
+// 128 x 64 at e^-0.04, segments of seven: 93.1 -> 94.8 us) and that two loads a lane cover.
+#define GDR_EDGE_MIN 2
+#define GDR_EDGE_NC 8
+#define GDR_EDGE_NC_MAX 128
+
+// How many of the nc <= GDR_EDGE_NC_MAX chunks of one head a composite leaves out (edges: that of its first chunk). Not made
+// uniform here: with the count in a scalar register the passes that keep the raw k tile take 167 registers instead of 157
+// (15 000 tokens, hierarchical prefill: 172.5 -> 178 us).
+__device__ __forceinline__ int gdr_chunks_left_out(const float* edges, int HV, int nc, int lane) {
+  const float edge = edges[max(nc - 1 - lane, 0) * HV], far = edges[max(nc - 65 - lane, 0) * HV];
+  const float past = wave_inclusive_scan(lane < nc ? edge : 0.0f);  // lane i: the last i + 1 chunks
+  const unsigned long long reach = __ballot(past <= GDR_EDGE_REACH);
+  const int left = nc - 1 - (reach ? __builtin_ctzll(reach) : nc);
+  return left < GDR_EDGE_MIN || __ballot(!(edge <= 0.0f && far <= 0.0f)) ? 0 : left;
+}
+
 __device__ __forceinline__ bf16x8 frag_load(const unsigned char* base, int frag, int lane) {
   return *reinterpret_cast<const bf16x8*>(base + (size_t)frag * 1024 + lane * 16);
 }
@@ -225,7 +254,7 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
                                                           const int32_t* __restrict__ chunk_tok0,
                                                           const int32_t* __restrict__ chunk_len,
                                                           unsigned char* __restrict__ rec, int n_chunks, int H, int HV,
-                                                          int l2norm, int32_t* positive_g) {
+                                                          int l2norm, int32_t* positive_g, float* __restrict__ edge) {
   using X8 = typename OpVec<T>::x8;    // input fragments (the K K^T products run in the input type)
   using O8 = typename OpVec<OT>::x8;   // record elements
   using O2 = typename OpVec<OT>::x2;
@@ -328,12 +357,12 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
       if (tt == 1) {  // A21^T: rows j (tile 0), columns i (tile 1): A_ij = ra_i ca_j (k_i.k_j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) a21t[r] = accA[1][r] * cola_t * rowc[r / 4][r % 4];
-      } else {        // diagonal blocks: rows i, columns j, strictly lower
+      } else {        // diagonal blocks: rows i, columns j, strictly lower (and the diagonal, for the edge)
         float* blk = tt == 0 ? s_A11 : s_A22;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int il = acc_row(r, hh);
-          blk[il * SB + ln] = il > ln ? accA[tt][r] * cola * rowa[r / 4][r % 4] : 0.0f;
+          blk[il * SB + ln] = il >= ln ? accA[tt][r] * cola * rowa[r / 4][r % 4] : 0.0f;
         }
       }
     }
@@ -361,12 +390,17 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
         for (int r = 0; r < 16; ++r) {
           const int il = acc_row(r, hh);
           blk[il * SB + ln] = accA[tt][r] * (br4[r / 4][r % 4] * rr4[r / 4][r % 4] * rc) *
-                              safe_exp2(il > ln ? gr4[r / 4][r % 4] - gc : 1.0f);
+                              safe_exp2(il >= ln ? gr4[r / 4][r % 4] - gc : 1.0f);
         }
       }
     }
   }
   lds_fence();
+  if (edge) {  // the diagonal holds beta_i |rk_i k_i|^2 (see GDR_EDGE_*); no row of the substitution reads it
+    const float diag = s_Ad[hh * (32 * SB) + ln * (SB + 1)];
+    const bool tame = !rising && !__ballot(!(diag >= 0.0f && diag <= 2.0f && __builtin_fabsf(bz) <= GDR_EDGE_BETA));
+    if (lane == 0) edge[(size_t)chunk * HV + hv] = tame ? g_last : __builtin_inff();
+  }
   // ---- the four 16x16 diagonal blocks by forward substitution: lane 16 b + c owns column c of block b (block b = rows
   //      and columns 16 (b % 2) .. + 15 of the 32x32 diagonal block b / 2), fp32 throughout
   {
@@ -699,9 +733,19 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
     map = seg * gmax + piece;
   }
   const int c1 = c0 + nc;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
+  // Composite pass: chunks that what comes behind them in the segment leaves nothing of are left out (GDR_EDGE_*; `Sinit` holds
+  // the edges).
+  constexpr bool EDGES = !PASS_B;
+  int left = 0;
+  if constexpr (EDGES) {
+    if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
+      left = gdr_chunks_left_out(Sinit + (size_t)c0 * HV + hv, HV, nc, lane);
+    c0 += left;
+    nc -= left;
+  }
   // (the per-chunk tables are separate restrict parameters: read through the view they could alias the kernel's
   // stores, would be fetched with vector loads and would sit in the same queue as the stagers' prefetches)
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
   // Segments that cut off what lies before them are found (see the end of the kernel), in the composite pass of the plain rule.
   constexpr bool CUTS = !PASS_B && SCALED_K;
   constexpr bool SKIP_M = CUTS && KT + VT > 128;
@@ -1514,6 +1558,63 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   const float vmask = is_m ? 0.0f : 1.0f;
   const unsigned vkeep = uniform(is_m ? 0 : -1);
 
+  unsigned* const wild = reinterpret_cast<unsigned*>(tiles(0).misc + 24);  // a byte per value column
+  if (EDGES && left > 0 && uniform(is_m)) {
+    // M is zero, and the waves of its columns look at the v of the chunks left out instead, some beside each chunk that is
+    // walked: a column with a value that is not finite is none of N either, as where all chunks are walked. That traffic (a
+    // quarter of what the chunks' tiles would be) is what the pass then takes its time for. The waves leave by themselves: a
+    // way back into the recurrence would cost its loop 100 spilled registers.
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    constexpr int PPR = VT / 8, STEP = 2 * KT / PPR, LOADS = 64 / STEP;  // 16-byte pieces of a row, rows a load, loads a chunk
+    const int tok0 = chunk_tok0[uniform(c0 - left)], rs = HV * VT;
+    const T* vb = v + ((size_t)tok0 * HV + hv) * VT;
+    const int off = (tid / PPR) * rs + 8 * (tid % PPR);
+    const int part = (left + nc) / (nc + 1);
+    u16x2 top[4] = {};
+    if (tid < VT / 4) wild[tid] = 0;
+    int x = 0;
+    for (int c = 0; c <= nc; ++c) {
+      for (const int end = min(x + part, left); x < end; ++x) {
+        uint4 raw[LOADS];
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u)
+          raw[u] = *reinterpret_cast<const uint4*>(vb + (size_t)(64 * x + u * STEP) * rs + off);
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) {
+          top[0] = __builtin_elementwise_max(top[0], __builtin_bit_cast(u16x2, raw[u].x & 0x7fff7fffu));
+          top[1] = __builtin_elementwise_max(top[1], __builtin_bit_cast(u16x2, raw[u].y & 0x7fff7fffu));
+          top[2] = __builtin_elementwise_max(top[2], __builtin_bit_cast(u16x2, raw[u].z & 0x7fff7fffu));
+          top[3] = __builtin_elementwise_max(top[3], __builtin_bit_cast(u16x2, raw[u].w & 0x7fff7fffu));
+        }
+      }
+      if (c == nc) {
+        const unsigned short limit = __is_same(T, _Float16) ? 0x7c00 : 0x7f80;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          atomicOr(&wild[2 * (tid % PPR) + h], (top[2 * h][0] >= limit ? 1u : 0u) | (top[2 * h][1] >= limit ? 1u << 8 : 0u) |
+                                                   (top[2 * h + 1][0] >= limit ? 1u << 16 : 0u) |
+                                                   (top[2 * h + 1][1] >= limit ? 1u << 24 : 0u));
+      }
+      lds_barrier();  // tiles (c0) are ready, then B(c0) .. B(c1 - 1)
+    }
+    const size_t at = ((size_t)map * HV + hv) * (KT * KT * 2);
+    const bool pairs = PIECES && gmax > 0;
+    const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int y = 16 * tid; y < (pairs ? 2 : 1) * KT * KT * 2; y += 16 * 2 * KT) {
+      *reinterpret_cast<f32x4*>(Mcomp + (pairs ? 2 : 1) * at + y) = none;
+      if constexpr (KEEP) *reinterpret_cast<f32x4*>(keep + at + y) = none;  // (map = seg)
+    }
+    float sum = CUTS ? 0.0f : 1.0f;
+    if constexpr (CUTS) {  // (the notes on N, see the end)
+      lds_barrier();
+#pragma unroll
+      for (int w = KT / 32; w < NSLAB; ++w) sum += tiles(0).misc[8 + w];
+    }
+    if (tid == 0) Dcomp[(size_t)map * HV + hv] = sum == 0.0f ? -0.0f : 0.0f;
+    return;
+  }
+
   f32x16 S[KT / 32];
   bool walked = false;
   if constexpr (PASS_B && KT == 64) if (gmax > 0) {
@@ -1839,6 +1940,12 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
     for (; c < c1; ++c) lds_barrier();  // B(c)
   } else if constexpr (CUTS) {
     faded = uniform(__float_as_int(dtot)) == 0;
+  }
+  if (EDGES && left > 0 && reinterpret_cast<const unsigned char*>(wild)[col]) {
+#pragma unroll
+    for (int km = 0; km < KT / 32; ++km)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[km][r] = __builtin_nanf("");
   }
   // epilogue; the opaque zero keeps the compiler from computing all these addresses before the loop
   int late = 0;

@@ -958,10 +958,12 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   LAMPA_PROF(s, "start");
   if (chunks == 0) return LAMPA_OK;
   // (the hierarchical kernels keep bf16 operands whatever the input type)
-  hipLaunchKernelGGL((gdr_local_kernel<T, __bf16, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g,
-                     beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, (int32_t*)nullptr);
-  LAMPA_PROF(s, "gdr_local_kernel");
+  // The chunks' edges lie where the scan writes behind the composites: 12 K V >= 49 152 floats a segment and head, of at most
+  // 4 096 chunks.
   const bool split = segs > n_seq;
+  hipLaunchKernelGGL((gdr_local_kernel<T, __bf16, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g,
+                     beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, (int32_t*)nullptr, split ? Xi : nullptr);
+  LAMPA_PROF(s, "gdr_local_kernel");
   // The composites of pieces fill the chip and run in front of the prep kernel. What follows them, and the composites of
   // whole segments, need T only, like the prep kernel, and are latency bound on a few workgroups: they run on a second
   // stream (default priority) beside the prep kernel and join before the walk.
@@ -987,7 +989,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
     // (only a sequence's last segment can be shorter than 2^p chunks, and its composite is not needed)
     hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, false, __bf16>), dim3(pieces ? segs * pieces : segs, HV),
                        dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, cs, (const T*)q, (const T*)k, (const T*)v, g,
-                       beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)nullptr, pieces ? ws + w.off_pm : Mc,
+                       beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)Xi, pieces ? ws + w.off_pm : Mc,
                        pieces ? ws + w.off_pn : Nm, pieces ? (float*)(ws + w.off_pd) : Dc, (T*)nullptr, (float*)nullptr, H, HV,
                        scale, l2norm, (const unsigned char*)nullptr, (const unsigned char*)nullptr, (const float*)nullptr,
                        (const float*)nullptr, pieces, (unsigned char*)nullptr, VT);

@@ -749,3 +749,41 @@ def test_few_tokens_of_very_many_sequences(device, K, V, dtype, lens):
     # (fp32 arithmetic, o rounded once: half a unit in the last place of the largest value)
     ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
     assert (o.float().cpu() - want_o.float()).abs().max() <= FP32_TOL + ulp * want_o.abs().max()
+
+
+@pytest.mark.parametrize("K,V,dtype,cps", [(64, 64, torch.bfloat16, 9), (64, 64, torch.float16, 70), (32, 32, torch.bfloat16, 8),
+                                           (64, 128, torch.bfloat16, 9), (128, 64, torch.float16, 8),
+                                           (128, 128, torch.bfloat16, 66)])
+def test_composites_start_where_earlier_chunks_no_longer_count(device, K, V, dtype, cps, monkeypatch):
+    # Segments whose last two (head 0) or four (head 1) chunks decay by more than the fp32 range, of which the composite pass
+    # walks no others; head 2 has next to no decay, head 3 one in its second half. Then a v, at either end of the chunks
+    # left out and in those that are walked, or a k that is not finite: its column, or its head, is none behind it. Then a token
+    # that is no contraction, for which every chunk is walked.
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
+    T = 64 * cps * 3 - 9
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 4, K, V, dtype, seed=K + V, g_scale=0.02)
+    g[:, :, 0] *= 90
+    g[:, :, 1] *= 35
+    g[:, T // 2:, 3] *= 50
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta)
+    args = _to(device, q, k, v, g, beta)
+    o, s = gd.chunk_gated_delta_rule(*args, output_final_state=True)
+    _assert_bf16_close(o, want_o, "o")
+    _assert_bf16_close(s, want_s, "state")
+    for row in (0, 64 * (cps - 4) - 1, 64 * (cps - 2) - 1, 64 * cps - 1):
+        for value, col in ((float("inf"), 5), (float("nan"), V - 1)):
+            bad = args[2].clone()
+            bad[0, row, :2, col] = value
+            o1, s1 = gd.chunk_gated_delta_rule(args[0], args[1], bad, *args[3:], output_final_state=True)
+            assert not torch.isfinite(o1[0, row + 1:, :2, col]).any() and not torch.isfinite(s1[0, :2, :, col]).any()
+            assert torch.equal(o1[:, :, 2:], o[:, :, 2:]) and torch.equal(s1[:, 2:], s[:, 2:])
+    bad = args[1].clone()
+    bad[0, 70, :2, 3] = float("inf")
+    o2, s2 = gd.chunk_gated_delta_rule(args[0], bad, *args[2:], output_final_state=True)
+    assert not torch.isfinite(o2[0, 128:, :2]).any() and not torch.isfinite(s2[0, :2]).any()
+    beta2 = beta.clone()
+    beta2[0, 70, :] = 2.5
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta2)
+    o3, s3 = gd.chunk_gated_delta_rule(*args[:4], beta2.to(device), output_final_state=True)
+    _assert_bf16_close(o3, want_o, "o")
+    _assert_bf16_close(s3, want_s, "state")
