@@ -86,7 +86,8 @@ struct HgRec {
   static constexpr int QF = WF + 2 * NKS * 1024;        // Q~ fragments  [2][NKS] KiB
   static constexpr int DK = QF + 2 * NKS * 1024;        // e^{gamma_last - gamma_i} rk_i, fp32 [64]
   static constexpr int LT = DK + 256;                   // lambda_i[7 + j], fp32 [HG_NLV][64]
-  static constexpr int MISC = LT + HG_NLV * 256;        // e^{gamma_last}
+  // e^{gamma_last}, 0 if the chunk has a finite edge (GDR_EDGE_*) and finite lambda
+  static constexpr int MISC = LT + HG_NLV * 256;
   static constexpr int BYTES = MISC + 256;
   static constexpr int PIECES = BYTES / 16;
 };
@@ -103,7 +104,8 @@ struct HgPrepSmem {
   static constexpr int OFF_P = OFF_T + 3 * 32 * ST * 2;
   static constexpr int OFF_LAM = OFF_K + 6 * 1024;           // levels 0..6, written once the k tile is done with
   static constexpr int OFF_F = OFF_P + 6 * 1024;             // gamma, beta, rk, qsc, qs, dk, bek
-  static constexpr int BYTES = OFF_F + 7 * 64 * 4;           // 51.25 KiB at K = V = 64: three workgroups per CU
+  static constexpr int OFF_WILD = OFF_F + 7 * 64 * 4;        // per wave: not all of its lambda are finite
+  static constexpr int BYTES = OFF_WILD + 16;                // 51.27 KiB at K = V = 64: three workgroups per CU
   static_assert(6 * 1024 + HG_INTRA * 64 * 4 <= 64 * SK * 2, "fragments + lambda fit in the k tile");
 };
 
@@ -114,7 +116,8 @@ __global__ void __launch_bounds__(256)
                      const int32_t* __restrict__ chunk_tok0,
                      const int32_t* __restrict__ chunk_len, const unsigned char* __restrict__ tmat,
                      unsigned char* __restrict__ wrec, unsigned char* __restrict__ Ub_out, float* __restrict__ Oi,
-                     float* __restrict__ hstates, int chunks_per_seq, int H, int HV, int L, float scale, int l2norm) {
+                     float* __restrict__ hstates, const float* __restrict__ edge, int chunks_per_seq, int H, int HV, int L,
+                     float scale, int l2norm) {
   using SM = HgPrepSmem<KT, VT>;
   using REC = HgRec<KT>;
   constexpr int SK = SM::SK, SV = SM::SV, ST = SM::ST, NKS = KT / 16;
@@ -135,6 +138,7 @@ __global__ void __launch_bounds__(256)
   float* s_qs = s_gamma + 256;   // scale e^{gamma_i} rq_i
   float* s_dk = s_gamma + 320;   // e^{gamma_last - gamma_i} rk_i
   float* s_bek = s_gamma + 384;  // beta_i e^{gamma_i} rk_i
+  float* s_wild = reinterpret_cast<float*>(smem + SM::OFF_WILD);
 
   const int chunk = blockIdx.x, hv = blockIdx.y;
   const int h = hv / (HV / H);
@@ -260,7 +264,6 @@ __global__ void __launch_bounds__(256)
       s_dk[row] = dk;
       s_bek[row] = bek;
       reinterpret_cast<float*>(rec + REC::DK)[row] = dk;
-      if (row == 0) reinterpret_cast<float*>(rec + REC::MISC)[0] = __builtin_amdgcn_exp2f(g_last);
     }
     // lambda, transposed ([level][row]): the inter-chunk levels go to the record
     if (lam_div != 1.0f) {  // lambda / scale, rounded to lambda's own type as the element-wise division would
@@ -270,6 +273,11 @@ __global__ void __launch_bounds__(256)
         lv[j] = lam_dtype == GDR_FP32 ? x : lam_dtype == GDR_BF16 ? (float)(__bf16)x : (float)(_Float16)x;
       }
     }
+    float probe = 0.0f;  // 0 x every weight: NaN unless all are finite
+#pragma unroll
+    for (int j = 0; j < NLAM; ++j) probe = __builtin_fmaf(lv[j], 0.0f, probe);
+    const bool wild = __ballot(!(probe == 0.0f)) != 0;
+    if (lane == 0) s_wild[wave] = wild ? 1.0f : 0.0f;
     float* lt = reinterpret_cast<float*>(rec + REC::LT);
 #pragma unroll
     for (int j = 0; j < NLAM; ++j) {
@@ -282,6 +290,10 @@ __global__ void __launch_bounds__(256)
       if (HG_INTRA + idx / 64 >= L) lt[idx] = 0.0f;
   }
   __syncthreads();
+  if (tid == 0) {
+    const float wild = (edge[ch] <= 0.0f ? 0.0f : 1.0f) + ((s_wild[0] + s_wild[1]) + (s_wild[2] + s_wild[3]));
+    *reinterpret_cast<f32x4*>(rec + REC::MISC) = f32x4{__builtin_amdgcn_exp2f(s_gamma[63]), wild, 0.0f, 0.0f};
+  }
 
   auto t_frag = [&](int tm, int ks) {  // A operand of T: rows 32 tm + ln, contraction step ks (tokens 16 ks ..)
     const int blk = tm == 0 ? 0 : (ks < 2 ? 1 : 2);
@@ -514,16 +526,17 @@ __device__ __forceinline__ void slab_add(float* p, int lane, const f32x16* S) {
 
 // The carry chain after chunk cs (index in its sequence): the levels below the lowest clear bit z of cs are all
 // occupied; they and the new state already in s_acc are summed, in level order, and become level z. One barrier
-// per level (uniform over the workgroup); a wave that owns none of the levels only takes part in the barriers.
+// per level (uniform over the workgroup); a wave that owns none of the levels only takes part in the barriers. gone: levels
+// that are zero.
 template <int KT, int CW = HG_CW, int LPW = HG_LPW>
 __device__ __forceinline__ void hg_merge(int cs, int lvl0, int wave, bool chain, int lane, float* s_acc,
-                                         f32x16 (*S)[KT / 32]) {
+                                         f32x16 (*S)[KT / 32], const bool* gone = nullptr) {
   const int z = __builtin_ctz(~cs);
   for (int j = lvl0; j < z; ++j) {
     if (chain) {
 #pragma unroll
       for (int slot = 0; slot < LPW; ++slot)
-        if (slot * CW + wave == j) {
+        if (slot * CW + wave == j && !(gone && gone[slot])) {
           slab_add<KT>(s_acc, lane, S[slot]);
 #pragma unroll
           for (int km = 0; km < KT / 32; ++km) S[slot][km] = zero16();
@@ -667,6 +680,24 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
     if (Xinit && ((cs0 >> lvl) & 1))
       slab_load<KT>(Xinit + ((((size_t)seg * HG_NLV + lvl) * HV + hv) * (VT / 32) + vslab) * (KT * 32), lane, S[slot]);
   }
+  // A level whose state has decayed to zero adds nothing to the output and stays zero: it is passed by until it is merged
+  // anew, at chunks of finite edges and weights. Looked at only where the decays' product since then has left the fp32 range.
+  bool part_filled = true;  // this wave's partial tile is not zero
+  int age[HG_LPW];  // an upper bound of that product's exponent
+  bool gone[HG_LPW];
+  auto is_zero = [&](const f32x16* x) __attribute__((always_inline)) {
+    unsigned any = 0;
+#pragma unroll
+    for (int km = 0; km < KT / 32; ++km)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) any |= __float_as_uint(x[km][r]) << 1;
+    return __ballot(any != 0) == 0;
+  };
+#pragma unroll
+  for (int slot = 0; slot < HG_LPW; ++slot) {
+    gone[slot] = is_zero(S[slot]);
+    age[slot] = 0;
+  }
   f32x4 oi_cur = oi_load(c0);
   for (int c = c0; c < c1; ++c) {
     const int cs = cs0 + (c - c0);
@@ -677,12 +708,17 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
     const __bf16* s_kt = reinterpret_cast<const __bf16*>(smem + SM::OFF_KT) + ((c - c0) & 1) * (64 * SM::SK);
     const float* s_dk = reinterpret_cast<const float*>(rec + REC::DK);
     const float* s_lt = reinterpret_cast<const float*>(rec + REC::LT);
-    const float dec = reinterpret_cast<const float*>(rec + REC::MISC)[0];
+    const float* misc = reinterpret_cast<const float*>(rec + REC::MISC);
+    const float dec = misc[0];
+    const bool tame = uniform(__float_as_int(misc[1])) == 0;
+    const int dec_exp = (uniform(__float_as_int(dec)) >> 23) - 126;
+    bool active = false;
     f32x16 O[2] = {zero16(), zero16()};
 #pragma unroll
     for (int slot = 0; slot < HG_LPW; ++slot) {
       const int lvl = slot * HG_CW + wave;
-      if (!((cs >> lvl) & 1)) continue;
+      if (!((cs >> lvl) & 1) || (gone[slot] && tame)) continue;
+      active = true;
       // The fragments of a stage are read from LDS as one batch ahead of its MFMAs (lds_fence() pins that order; left
       // alone the compiler fetches each fragment right before its MFMA and pays the LDS latency every time), and the
       // two accumulation chains of a stage are interleaved.
@@ -741,8 +777,11 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
       for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
         for (int km = 0; km < KT / 32; ++km) S[slot][km] = mfma32(fr[km * 4 + ks], Zb[ks], S[slot][km]);
+      age[slot] = max(age[slot] + dec_exp, -4096);
+      gone[slot] = false;
     }
-    {
+    if (active || part_filled) {
+      part_filled = active;
       float* part = s_part + wave * 64 * SP;
 #pragma unroll
       for (int tm = 0; tm < 2; ++tm)
@@ -751,7 +790,19 @@ __global__ void __launch_bounds__(64 * (HG_CW + 2))
     }
     lds_barrier();  // M0(c)
     out_rows(tok0, len, oi_cur);
-    if (c + 1 < c1) hg_merge<KT>(cs, 0, wave, true, lane, s_acc, S);
+    if (c + 1 < c1) {
+      // (here, not behind the state's products: there the test costs 17 spilled registers)
+#pragma unroll
+      for (int slot = 0; slot < HG_LPW; ++slot)
+        if (age[slot] < -150 && !gone[slot]) gone[slot] = is_zero(S[slot]);
+      hg_merge<KT>(cs, 0, wave, true, lane, s_acc, S, gone);
+#pragma unroll
+      for (int slot = 0; slot < HG_LPW; ++slot)
+        if (slot * HG_CW + wave == __builtin_ctz(~cs)) {
+          age[slot] = 0;
+          gone[slot] = false;
+        }
+    }
     oi_cur = oi_next;
   }
   // the level states after the sequence's last token (before any carry): level 7 + j for the occupied inter-chunk levels
@@ -877,7 +928,7 @@ __global__ void __launch_bounds__(64 * HG_SCAN_WAVES, 2)
 
 // ---- host side ------------------------------------------------------------------------------------------------
 struct HgWorkspace {
-  int64_t off_t, off_m, off_n, off_d, off_rec, off_nc, off_oi, off_x, off_pm, off_pn, off_pd, bytes;
+  int64_t off_t, off_m, off_n, off_d, off_rec, off_nc, off_oi, off_x, off_pm, off_pn, off_pd, off_e, bytes;
 };
 
 // Segment composites: one workgroup per (segment, head) walks its chunks one after the other, 3.4 us each, and the plan's
@@ -910,6 +961,7 @@ static HgWorkspace hg_workspace(int64_t chunks, int64_t segs, int HV, int K, int
   w.off_pm = off;  off += lampa_align_up(pieces * HV * (int64_t)K * K * 4, 256);  // M' in two 16-bit parts
   w.off_pn = off;  off += lampa_align_up(pieces * HV * (int64_t)K * V * 4, 256);
   w.off_pd = off;  off += lampa_align_up(pieces * HV * 4, 256);
+  w.off_e = off;   off += lampa_align_up(chunks * HV * 4, 256);  // the chunks' edges (GDR_EDGE_*)
   w.bytes = off > 0 ? off : 256;
   return w;
 }
@@ -935,6 +987,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   unsigned char* Ubw = ws + w.off_nc;
   float* Oi = (float*)(ws + w.off_oi);
   float* Xi = (float*)(ws + w.off_x);
+  float* edge = (float*)(ws + w.off_e);
   constexpr int smem_a = GdrSegSmem<KT, VT, false, false>::BYTES, smem_p = HgPrepSmem<KT, VT>::BYTES,
                 smem_w = HgWalkSmem<KT>::BYTES;
   static bool attr_set_dev[64];  // the attribute belongs to the device's copy of the kernel
@@ -958,11 +1011,9 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   LAMPA_PROF(s, "start");
   if (chunks == 0) return LAMPA_OK;
   // (the hierarchical kernels keep bf16 operands whatever the input type)
-  // The chunks' edges lie where the scan writes behind the composites: 12 K V >= 49 152 floats a segment and head, of at most
-  // 4 096 chunks.
   const bool split = segs > n_seq;
   hipLaunchKernelGGL((gdr_local_kernel<T, __bf16, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g,
-                     beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, (int32_t*)nullptr, split ? Xi : nullptr);
+                     beta, pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, (int32_t*)nullptr, edge);
   LAMPA_PROF(s, "gdr_local_kernel");
   // The composites of pieces fill the chip and run in front of the prep kernel. What follows them, and the composites of
   // whole segments, need T only, like the prep kernel, and are latency bound on a few workgroups: they run on a second
@@ -989,7 +1040,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
     // (only a sequence's last segment can be shorter than 2^p chunks, and its composite is not needed)
     hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, false, __bf16>), dim3(pieces ? segs * pieces : segs, HV),
                        dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, cs, (const T*)q, (const T*)k, (const T*)v, g,
-                       beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)Xi, pieces ? ws + w.off_pm : Mc,
+                       beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)edge, pieces ? ws + w.off_pm : Mc,
                        pieces ? ws + w.off_pn : Nm, pieces ? (float*)(ws + w.off_pd) : Dc, (T*)nullptr, (float*)nullptr, H, HV,
                        scale, l2norm, (const unsigned char*)nullptr, (const unsigned char*)nullptr, (const float*)nullptr,
                        (const float*)nullptr, pieces, (unsigned char*)nullptr, VT);
@@ -1003,7 +1054,7 @@ static int hg_launch(const void* q, const void* k, const void* v, const float* g
   // further away (15 040 tokens, 31 MB, 138.9 / 139.4, 8 x 2 048 122.7 / 124.0, 64 x 64 36.6 / 37.3).
   const bool far = (int64_t)chunks * HV * (64 * VT * 4) > (48ll << 20);
   hipLaunchKernelGGL((far ? hgdn_prep_kernel<T, KT, VT, true> : hgdn_prep_kernel<T, KT, VT, false>), dim3(chunks, HV), dim3(256), smem_p, s, (const T*)q, (const T*)k,
-                     (const T*)v, lam, lam_dtype, lam_div, pv.chunk_tok0, pv.chunk_len, tf, rec, Ubw, Oi, hstates, chunks_per_seq, H, HV, L,
+                     (const T*)v, lam, lam_dtype, lam_div, pv.chunk_tok0, pv.chunk_len, tf, rec, Ubw, Oi, hstates, (const float*)edge, chunks_per_seq, H, HV, L,
                      scale, l2norm);
   LAMPA_PROF(s, "hgdn_prep_kernel");
   if (split) {

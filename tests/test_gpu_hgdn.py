@@ -426,3 +426,36 @@ def test_tail_of_narrow_heads(device, K, T, t0):
                                        1, stream) == 0
     assert (states.cpu() - want_s).abs().max() <= 2e-5 * want_s.abs().max()
     assert (o[:, t0:].cpu() - want_o[:, t0:]).abs().max() <= 2e-5 * want_o.abs().max()
+
+
+@pytest.mark.parametrize("V,dtype,cps,chunks", [(64, torch.bfloat16, None, 21), (128, torch.float16, 16, 41), (64, torch.bfloat16, 64, 130)])
+def test_levels_that_have_decayed_to_zero(device, V, dtype, cps, chunks, monkeypatch):
+    """Decays that take a level's state out of the fp32 range after one, three or no chunks, or in the second half only: the
+    walk passes such levels by. Then a weight of every level, or a key, that is not finite in a chunk whose levels are passed by:
+    what the weights and the states say is none."""
+    monkeypatch.setattr(hgdn, "CHUNKS_PER_SEGMENT", cps)
+    T = 64 * chunks
+    q, k, v, g, beta, lam = _inputs(1, T, 4, 64, V, dtype, seed=chunks, g_scale=0.02)
+    g[:, :, 0] *= 120
+    g[:, :, 1] *= 40
+    g[:, T // 2:, 3] *= 50
+    want = _want(q, k, v, g, beta, lam)
+    run = lambda k, lam: hgdn.chunk_h_gated_delta_rule(*(x.to(device) for x in (q, k, v, g, lam, beta)), output_final_state=True,
+                                                       use_qk_l2norm_in_kernel=True)
+    o, state = run(k, lam)
+    max_abs, mean_rel = _errors(o, want)
+    assert max_abs <= MAX_ABS and mean_rel <= MEAN_REL, f"{max_abs:.3e} {mean_rel:.3e}"
+    assert torch.isfinite(state.states).all()
+    t = 64 * 15 + 7  # (levels 7 .. 10 hold tokens there)
+    bad = lam.clone()
+    bad[0, t, :, 10] = float("nan")
+    o1, _ = run(k, bad)
+    assert torch.isnan(o1[0, t]).all()
+    o1[0, t] = o[0, t]
+    assert torch.equal(o1, o)
+    bad = k.clone()
+    bad[0, T - 70] = float("inf")
+    o2, state2 = run(bad, lam)
+    assert torch.equal(o2[0, :T - 128], o[0, :T - 128]) and not torch.isfinite(o2[0, T - 64:]).any()
+    occupied = [0, 1, 2, 3, 4, 5, 6] + [7 + j for j in range(12) if (chunks - 1) >> j & 1]
+    assert not torch.isfinite(state2.states[..., occupied[7:]]).any()
