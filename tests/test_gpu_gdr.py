@@ -787,3 +787,35 @@ def test_composites_start_where_earlier_chunks_no_longer_count(device, K, V, dty
     o3, s3 = gd.chunk_gated_delta_rule(*args[:4], beta2.to(device), output_final_state=True)
     _assert_bf16_close(o3, want_o, "o")
     _assert_bf16_close(s3, want_s, "state")
+
+
+@pytest.mark.parametrize("K,V,lens", [(16, 32, [2500]), (32, 32, [1500, 1700]), (36, 20, [3000]), (64, 64, [6000]), (128, 16, [9000])])
+def test_recurrent_scan_behind_maps_without_a_past(device, K, V, lens):
+    # Long sequences whose groups of segments have zero maps (head 0: the scan starts behind the last of them), maps with next to
+    # no decay (head 1) or either in one half of the sequence; then a v and an initial state that are not finite: their
+    # columns are none from there on, whatever the decays.
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.long)
+    T, n = int(cu[-1]), len(lens)
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 4, K, V, torch.float32, seed=K, g_scale=0.02)
+    g[:, :, 0] *= 150
+    g[:, : T // 2, 2] *= 150
+    g[:, T // 2:, 3] *= 150
+    h0 = torch.randn(n, 4, K, V, generator=torch.Generator().manual_seed(2))
+    args = _to(device, q, k, v, g, beta)
+    run = lambda v, h0: gd.fused_recurrent_gated_delta_rule(args[0], args[1], v, *args[3:], initial_state=h0.to(device),
+                                                            output_final_state=True, cu_seqlens=cu.to(device))
+    o, s = run(args[2], h0)
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta, initial_state=h0, cu_seqlens=cu)
+    assert _errors(o, want_o)[0] <= FP32_TOL and _errors(s, want_s)[0] <= FP32_TOL
+    bad = args[2].clone()
+    bad[0, 40, :, 3] = float("inf")
+    o1, s1 = run(bad, h0)
+    keep = [c for c in range(V) if c != 3]
+    assert not torch.isfinite(o1[0, 41:lens[0], :, 3]).any() and not torch.isfinite(s1[0, :, :, 3]).any()
+    assert torch.equal(o1[..., keep], o[..., keep]) and torch.equal(s1[..., keep], s[..., keep])
+    bad = h0.clone()
+    bad[n - 1, :, 1, 5] = float("nan")
+    o2, s2 = run(args[2], bad)
+    keep = [c for c in range(V) if c != 5]
+    assert torch.isnan(o2[0, T - lens[-1]:, :, 5]).all() and torch.isnan(s2[n - 1, :, :, 5]).all()
+    assert torch.equal(o2[..., keep], o[..., keep]) and torch.equal(s2[..., keep], s[..., keep])
