@@ -76,7 +76,8 @@ struct GbWalkSmem {
 static_assert(GbWalkSmem::BYTES <= 163840, "LDS of a CU");
 struct GbSourceSmem {
   static constexpr int OFF_P = 2 * GbSet<false>::BYTES;
-  static constexpr int BYTES = OFF_P + 3 * GB_TRI;
+  static constexpr int OFF_NOTE = OFF_P + 3 * GB_TRI;  // a byte per value column, q, the two waves of N'
+  static constexpr int BYTES = OFF_NOTE + 80;
 };
 static_assert(GbSourceSmem::BYTES <= 81920, "two workgroups per CU");
 
@@ -529,13 +530,15 @@ __device__ __forceinline__ void gb_zero_upper(unsigned char* smem, int tid) {
 // ---- source pass: every segment's N' (the walk from a zero gradient, no gradients written) --------------------------------
 // Grid segments x heads (long segments first), eight waves: 0, 1 the gradient of the state (32 value columns each), 4-6 the
 // tiles of P, 2 and 3 / 4-7 stage the next chunk into the other set of tiles. Two barriers per chunk, two workgroups per CU (80 KB
-// of LDS, 128 registers). 52 - 57 us, by card, at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the products).
+// of LDS, 128 registers). 52 - 57 us, by card, at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the
+// products), and 39 at e^-0.8 a token, where three of a segment's 15 chunks are walked and the q and dO of the others looked at (half
+// of its traffic then); with the walk that starts at the next segment (197 -> 190) the training step 370 -> 352.
 template <typename T>
 __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
     gdrb_source_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ dout,
                        const unsigned char* __restrict__ recs, const GdrPlanView pv, const int32_t* __restrict__ chunk_tok0,
                        const int32_t* __restrict__ chunk_len, unsigned char* __restrict__ Nr, int H, int HV, float scale,
-                       int l2norm) {
+                       int l2norm, const float* __restrict__ edges, const float* __restrict__ Dc, float* __restrict__ Dr) {
   using OT = T;
   extern __shared__ __align__(16) unsigned char smem[];
   unsigned char* const b_p = smem + GbSourceSmem::OFF_P;
@@ -552,12 +555,54 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
   // chunk earlier still
   auto set_of = [&](int c) { return gb_tiles<OT, false>(smem, (cl - c) & 1); };
   gb_zero_upper<OT, false>(smem, tid);
+  // Chunks at the segment's end that those in front of them leave nothing of are left out, as in the forward's composites, after
+  // a look at their q and dO: a q that is not finite is in all of N', a dO in its column.
+  unsigned* const note = reinterpret_cast<unsigned*>(smem + GbSourceSmem::OFF_NOTE);
+  int left = 0;
+  if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
+    left = uniform(gdr_chunks_left_out<true>(edges + (size_t)c0 * HV + hv, HV, nc, lane));
+  const int ct = cl - left;  // the chunk the walk starts at
+  if (left > 0) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    if (tid < 20) note[tid] = 0;
+    u16x2 top_q = {0, 0}, top_d[4] = {};
+    const int row = tid >> 3, part = tid & 7;  // (a thread a 16-byte piece of the chunk's 64 rows)
+    const T* qp = q + ((size_t)tok_of(ct + 1) * H + h) * 64 + 8 * part;
+    const T* dp = dout + ((size_t)tok_of(ct + 1) * HV + hv) * 64 + 8 * part;
+    const int rows = 64 * (left - 1) + len_last;
+    for (int x = 0; x < left; x += 4) {
+      uint4 rq[4], rd[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const size_t r = min(64 * (x + u) + row, rows - 1);
+        rq[u] = *reinterpret_cast<const uint4*>(qp + r * H * 64);
+        rd[u] = *reinterpret_cast<const uint4*>(dp + r * HV * 64);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t a[4] = {rq[u].x, rq[u].y, rq[u].z, rq[u].w}, d[4] = {rd[u].x, rd[u].y, rd[u].z, rd[u].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          top_q = __builtin_elementwise_max(top_q, __builtin_bit_cast(u16x2, a[e] & 0x7fff7fffu));
+          top_d[e] = __builtin_elementwise_max(top_d[e], __builtin_bit_cast(u16x2, d[e] & 0x7fff7fffu));
+        }
+      }
+    }
+    const unsigned short limit = __is_same(T, _Float16) ? 0x7c00 : 0x7f80;
+    lds_barrier();
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      atomicOr(&note[2 * part + e], (top_d[2 * e][0] >= limit ? 1u : 0u) | (top_d[2 * e][1] >= limit ? 1u << 8 : 0u) |
+                                        (top_d[2 * e + 1][0] >= limit ? 1u << 16 : 0u) | (top_d[2 * e + 1][1] >= limit ? 1u << 24 : 0u));
+    if (top_q[0] >= limit || top_q[1] >= limit) note[16] = 1;
+    // (read behind the walk's barriers)
+  }
   if (wave < 2) {
     GbChain<OT> ch;
     ch.G[0] = zero16();
     ch.G[1] = zero16();
     if (nc > 0) lds_barrier();  // (0) the tiles of the first chunk are complete
-    for (int c = cl; c >= c0; --c) {
+    for (int c = ct; c >= c0; --c) {
       const GbTiles<OT> t = set_of(c);
       ch.state_rows(t, nullptr, wave, lane, hh, ln);
       lds_barrier();  // (1) P is complete
@@ -565,6 +610,26 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
       ch.update(t, scale, wave, lane, hh);
       lds_barrier();  // (2) the tiles of chunk c have been read, those of chunk c - 1 are complete
     }
+    if (left > 0 && (note[16] || reinterpret_cast<const unsigned char*>(note)[32 * wave + ln])) {
+#pragma unroll
+      for (int km = 0; km < 2; ++km)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ch.G[km][r] = __builtin_nanf("");
+    }
+    // A segment without M (the forward's mark) and with a finite N' hands N' on whatever finite gradient comes from behind it
+    const float dc = Dc[(size_t)seg * HV + hv];
+    float dr = __builtin_fabsf(dc);
+    if (gdr_d_cut(dc)) {
+      float probe = 0.0f;
+#pragma unroll
+      for (int km = 0; km < 2; ++km)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(ch.G[km][r], 0.0f, probe);
+      if (lane == 0) note[18 + wave] = __ballot(!(probe == 0.0f)) != 0;
+      lds_barrier();  // (of the two waves that are left)
+      if (!(note[18] | note[19])) dr = -0.0f;
+    }
+    if (tid == 0) Dr[(size_t)seg * HV + hv] = dr;
     // N' in accumulator order, as the forward composites keep N
     f32x4* out = reinterpret_cast<f32x4*>(Nr + (((size_t)seg * HV + hv) * 2 + wave) * GDR_STATE_BYTES);
 #pragma unroll
@@ -585,11 +650,11 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
       c = uniform(max(c, c0));
       st.issue(dout, nullptr, rec_of(c), nullptr, tok_of(c), len_of(c), HV, hv, bt);
     };
-    issue(cl);
-    st.stage(set_of(cl), len_of(cl), bt);
-    issue(cl - 1);
+    issue(ct);
+    st.stage(set_of(ct), len_of(ct), bt);
+    issue(ct - 1);
     lds_barrier();  // (0)
-    for (int c = cl; c >= c0; --c) {
+    for (int c = ct; c >= c0; --c) {
       if (c > c0) st.stage(set_of(c - 1), len_of(c - 1), bt);
       issue(c - 2);
       lds_barrier();  // (1)
@@ -609,11 +674,11 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
       st.stage_q(set_of(c), len_of(c), l2norm, gt);
       if (wave == 7) sf.stage(set_of(c), lane);
     };
-    issue(cl);
-    stage(cl);
-    issue(cl - 1);
+    issue(ct);
+    stage(ct);
+    issue(ct - 1);
     lds_barrier();  // (0)
-    for (int c = cl; c >= c0; --c) {
+    for (int c = ct; c >= c0; --c) {
       const GbTiles<OT> t = set_of(c);
       if (wave < 7) {
         f32x16 p = gb_pair<OT>(t.k, jt, t.q, it, ln, hh);
@@ -701,8 +766,15 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
     const int seg0 = pv.seq_seg0[seq], last = seg0 + pv.seq_nseg[seq] - 1, behind = last - seg;
     const int lead = gmax > 0 ? behind / GDR_SCAN_GROUP : 0, nst = lead + behind - lead * GDR_SCAN_GROUP;
     const int slab = wave & 1, km = (wave >> 1) & 1;
+    // (from a gradient of zero behind the sequence; a given one may not be finite)
+    int from = 0;
+    if (nst > 1 && !dht) {
+      const int pl = min(lane, nst - 1);
+      const size_t at = (size_t)(pl < lead ? seq * gmax + pl : last - lead * GDR_SCAN_GROUP - (pl - lead)) * HV + hv;
+      from = max(0, uniform(gdr_leading_cuts((pl < lead ? Dgrp : Dc)[at], nst, lane)) - 1);
+    }
     if (wave >= 4) {
-      for (int p = 0; p < nst; ++p) lds_barrier();
+      for (int p = from; p < nst; ++p) lds_barrier();
       lds_barrier();
       lds_barrier();
     } else {
@@ -742,9 +814,9 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
         S = acc;
       };
       if (nst > 0) {
-        walk_issue(0, rm[0], rn[0], rd[0]);
-        walk_issue(1, rm[1], rn[1], rd[1]);
-        for (int p = 0; p < nst; p += 2) {
+        walk_issue(from, rm[0], rn[0], rd[0]);
+        walk_issue(from + 1, rm[1], rn[1], rd[1]);
+        for (int p = from; p < nst; p += 2) {
           walk_step(p, rm[0], rn[0], rd[0]);
           walk_issue(p + 2, rm[0], rn[0], rd[0]);
           if (p + 1 < nst) walk_step(p + 1, rm[1], rn[1], rd[1]);
@@ -1190,7 +1262,7 @@ __global__ void __launch_bounds__(GB_WALK_THREADS, 3)
 
 // ---- host ----------------------------------------------------------------------------------------------------------
 struct GbWorkspace {
-  int64_t nr, gm, gn, gd, max_groups, bytes;
+  int64_t nr, gm, gn, gd, dr, max_groups, bytes;
 };
 static GbWorkspace gb_workspace(int64_t segs, int HV) {
   GbWorkspace w;
@@ -1201,6 +1273,7 @@ static GbWorkspace gb_workspace(int64_t segs, int HV) {
   w.gm = take(w.max_groups * HV * (int64_t)GDR_STATE_BYTES);
   w.gn = take(w.max_groups * HV * 2 * (int64_t)GDR_STATE_BYTES);
   w.gd = take(w.max_groups * HV * 4);
+  w.dr = take(segs * HV * 4);
   w.bytes = off;
   return w;
 }
@@ -1237,19 +1310,21 @@ static int gb_run(const void* q, const void* k, const void* v, const void* dout,
   float* Gd = (float*)(ws + w.gd);
   const unsigned char *recs = saved + sv.off_rec, *states = saved + sv.off_states, *Mt = saved + sv.off_mt;
   const float* Dc = (const float*)(saved + sv.off_d);
+  float* Dr = (float*)(ws + w.dr);
   LAMPA_PROF(s, "start");
   if (segs > n_seq) {
     hipLaunchKernelGGL((gdrb_source_kernel<T>), dim3(segs * HV), dim3(GB_SOURCE_THREADS), GbSourceSmem::BYTES, s, (const T*)q,
-                       (const T*)k, (const T*)dout, recs, pv, pv.chunk_tok0, pv.chunk_len, Nr, H, HV, scale, l2norm);
+                       (const T*)k, (const T*)dout, recs, pv, pv.chunk_tok0, pv.chunk_len, Nr, H, HV, scale, l2norm,
+                       (const float*)(saved + sv.off_e), Dc, Dr);
     LAMPA_PROF(s, "gdrb_source_kernel");
     if (gmax > 0) {
       hipLaunchKernelGGL((gdr_scan2_kernel<T, 64, 64, 4, SCAN_GROUP, true>), dim3(4 * gmax, n_seq, HV), dim3(128), 0, s, pv, Mt,
-                         Nr, Dc, (const float*)nullptr, (float*)nullptr, Gm, Gn, Gd, HV, 0, gmax);
+                         Nr, (const float*)Dr, (const float*)nullptr, (float*)nullptr, Gm, Gn, Gd, HV, 0, gmax);
       LAMPA_PROF(s, "gdr_scan2_kernel<group, reversed>");
     }
   }
   hipLaunchKernelGGL((gdrb_walk_kernel<T>), dim3(segs * HV), dim3(GB_WALK_THREADS), GbWalkSmem::BYTES, s, (const T*)q,
-                     (const T*)k, (const T*)v, (const T*)dout, recs, states, pv, pv.chunk_tok0, pv.chunk_len, Mt, Dc, Nr, Gm, Gn,
+                     (const T*)k, (const T*)v, (const T*)dout, recs, states, pv, pv.chunk_tok0, pv.chunk_len, Mt, (const float*)Dr, Nr, Gm, Gn,
                      Gd, gmax, dht, (T*)dq, (T*)dk, (T*)dv, dg, dbeta, dh0, H, HV, scale, l2norm, Kw, Vw);
   LAMPA_PROF(s, "gdrb_walk_kernel");
   return lampa_launch_status();

@@ -56,7 +56,7 @@ static int gdr_max_chunks(const int32_t* plan_host) {
 // Buffers of the training form (gdr_train.h), or none.
 struct GdrKeep {
   unsigned char *rec, *states, *mt;
-  float* d;
+  float *d, *edge;
   int32_t* positive_g;
   int o_width;
 };
@@ -93,14 +93,15 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
   }
   hold.unlock();
   LAMPA_PROF(s, "start");
-  float* edge = segs > n_seq && max_chunks >= GDR_EDGE_NC ? Si : nullptr;  // the chunks' edges, for the composite pass
+  float* const edges = KEEP ? kp.edge : Si;
+  float* edge = segs > n_seq && max_chunks >= GDR_EDGE_NC ? edges : nullptr;  // (of shorter segments no one asks for them)
   if (chunks > 0) {
     hipLaunchKernelGGL((gdr_local_kernel<T, T, KT>), dim3(gdr_local_grid(chunks, HV)), dim3(64), 0, s, (const T*)k, g, beta,
                        pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, kp.positive_g, edge);
     LAMPA_PROF(s, "gdr_local_kernel");
     if (segs > n_seq) {
       hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
-                         (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)Si, Mc, Nc, Dc,
+                         (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)edges, Mc, Nc, Dc,
                          (T*)nullptr, (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
                          (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, kp.mt, VT);
       LAMPA_PROF(s, "gdr_segment_kernel<composite>");
@@ -191,6 +192,7 @@ GdrSaved gdr_saved_layout(int64_t chunks, int64_t segs, int HV) {
   v.off_states = off; off += lampa_align_up(chunks * HV * (int64_t)GDR_STATE_BYTES, 256);
   v.off_mt = off;     off += lampa_align_up(segs * HV * (int64_t)GDR_STATE_BYTES, 256);
   v.off_d = off;      off += lampa_align_up(segs * HV * 4, 256);
+  v.off_e = off;      off += lampa_align_up((chunks + 1) * HV * 4, 256);
   v.bytes = off > 0 ? off : 256;
   return v;
 }
@@ -224,7 +226,7 @@ extern "C" int lampa_gdr_chunk_fwd_train(const void* q, const void* k, const voi
   for (int i = 0; i < n_seq; ++i) max_nseg = plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] > max_nseg ? plan_host[plan_host[PLAN_OFF_SEQ_NSEG] + i] : max_nseg;
   const GdrSaved sv = gdr_saved_layout(chunks, segs, HV);
   unsigned char* sp = (unsigned char*)saved;
-  GdrKeep kp{sp + sv.off_rec, sp + sv.off_states, sp + sv.off_mt, (float*)(sp + sv.off_d), nullptr, V};
+  GdrKeep kp{sp + sv.off_rec, sp + sv.off_states, sp + sv.off_mt, (float*)(sp + sv.off_d), (float*)(sp + sv.off_e), nullptr, V};
   if (positive_g_host && hipHostGetDevicePointer((void**)&kp.positive_g, positive_g_host, 0) != hipSuccess) {
     (void)hipGetLastError();
     return LAMPA_ERR_INVALID;

@@ -113,8 +113,11 @@ __device__ __forceinline__ int gdr_leading_cuts(float d, int n, int lane) {
 // How many of the nc <= GDR_EDGE_NC_MAX chunks of one head a composite leaves out (edges: that of its first chunk). Not made
 // uniform here: with the count in a scalar register the passes that keep the raw k tile take 167 registers instead of 157
 // (15 000 tokens, hierarchical prefill: 172.5 -> 178 us).
+// BACK: the chunks at the segment's end, which those in front of them leave nothing of where a gradient is walked back.
+template <bool BACK = false>
 __device__ __forceinline__ int gdr_chunks_left_out(const float* edges, int HV, int nc, int lane) {
-  const float edge = edges[max(nc - 1 - lane, 0) * HV], far = edges[max(nc - 65 - lane, 0) * HV];
+  const float edge = edges[(BACK ? min(lane, nc - 1) : max(nc - 1 - lane, 0)) * HV];
+  const float far = edges[(BACK ? min(64 + lane, nc - 1) : max(nc - 65 - lane, 0)) * HV];
   const float past = wave_inclusive_scan(lane < nc ? edge : 0.0f);  // lane i: the last i + 1 chunks
   const unsigned long long reach = __ballot(past <= GDR_EDGE_REACH);
   const int left = nc - 1 - (reach ? __builtin_ctzll(reach) : nc);
@@ -2240,8 +2243,8 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
   // the maps', so that it is waited for alone, and the maps' loads stay in order and in front of the branch; the group that is
   // cut off leaves by itself. (Looked at behind the maps' loads, with one way through the loop for both: 9 000 tokens x 6 x
   // 128 x 128 where nothing cuts off 13.8 us, 8.3 where all do; so 13.55 and 7.85; 13.3 without the look.)
-  constexpr bool LOOK = MODE == SCAN_GROUP && !REV;
-  const float d_look = LOOK ? Dsrc[(size_t)(item0 + min(lane, nsteps)) * HV + hv] : 0.0f;
+  constexpr bool LOOK = MODE == SCAN_GROUP;
+  const float d_look = LOOK ? Dsrc[(size_t)(REV ? item0 - min(lane, nsteps) : item0 + min(lane, nsteps)) * HV + hv] : 0.0f;
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) {
     if constexpr (LOOK) __builtin_amdgcn_sched_barrier(0);
@@ -2286,7 +2289,8 @@ __global__ void __launch_bounds__(64 * (KT / 32)) gdr_scan2_kernel(const GdrPlan
         for (int q4 = 0; q4 < 4; ++q4) asm volatile("" ::"v"(rn[d][q4]));
       }
       __builtin_amdgcn_sched_barrier(0);
-      const f32x4* N = reinterpret_cast<const f32x4*>(Nsrc + (((size_t)(item0 + nsteps) * HV + hv) * (VT / 32) + nblk) * N_BYTES);
+      const int at = REV ? item0 - nsteps : item0 + nsteps;
+      const f32x4* N = reinterpret_cast<const f32x4*>(Nsrc + (((size_t)at * HV + hv) * (VT / 32) + nblk) * N_BYTES);
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
         const f32x4 t = N[(wave * 4 + q4) * 64 + lane];

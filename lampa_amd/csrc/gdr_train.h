@@ -1,6 +1,6 @@
 // What the training form of the chunk forward keeps for the backward pass (K = V = 64): the records of the chunks, the
 // state in front of every chunk (16-bit operand fragments of the two 32-column slabs) and every segment's transposed M'
-// (16-bit A-operand fragments) and decay.
+// (16-bit A-operand fragments) and decay, and the chunks' edges (GDR_EDGE_*; written where a segment has GDR_EDGE_NC chunks).
 #pragma once
 #include "common.h"
 #include "gdr_plan.h"
@@ -11,7 +11,7 @@
 static inline bool gdr_train_width(int n) { return n >= 8 && n <= 64 && n % 8 == 0; }
 
 struct GdrSaved {
-  int64_t off_rec, off_states, off_mt, off_d, bytes;
+  int64_t off_rec, off_states, off_mt, off_d, off_e, bytes;
 };
 GdrSaved gdr_saved_layout(int64_t chunks, int64_t segs, int HV);
 

@@ -476,3 +476,32 @@ def test_forward_of_a_training_step_gives_the_bits_of_the_plain_call(device, T, 
         x.requires_grad_(True)
     ot, st = call()
     assert ot.requires_grad and torch.equal(o, ot) and torch.equal(s, st)
+
+
+@pytest.mark.parametrize("dtype,cps,T", [(torch.bfloat16, 9, 64 * 9 * 3 - 9), (torch.float16, 9, 64 * 9 * 25), (torch.bfloat16, 66, 64 * 66 * 2 + 700)])
+def test_sources_end_where_later_chunks_no_longer_count(device, dtype, cps, T, monkeypatch):
+    """Segments whose first two (head 0) or four (head 1) chunks decay by more than the fp32 range, of which the pass for the
+    segments' own gradients walks no others (and the walk over the segments behind starts at the next one); head 2 has next to
+    no decay, head 3 one in its first half. Then a dO or a q that is not finite at either end of the chunks left out: none of
+    the gradients that it belongs to in front of it are."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
+    (q, k, v, g, beta, do), _ = _inputs(1, T, 4, 4, 64, 64, dtype, seed=cps, unit=False, g_scale=0.02)
+    g[:, :, 0] *= 90
+    g[:, :, 1] *= 35
+    g[:, : T // 2, 3] *= 50
+    got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, True)
+    want = ob.backward_manual(q, k, v, g, beta, do, l2=og.L2_CHUNK)
+    _check(got[:5], want[:5], dtype, chunked=True)
+    assert all(torch.isfinite(x).all() for x in got[:5])
+    seg = 64 * cps  # (of the second segment)
+    for row in (seg + 64 * 2, seg + 64 * 4 + 3, 2 * seg - 1):
+        bad = do.clone()
+        bad[0, row, :2, 40] = float("inf")
+        nan = _gpu_grads(device, q, k, v, g, beta, bad, None, None, None, True)
+        assert not torch.isfinite(nan[2][0, :row, :2, 40]).any()
+        assert all(torch.equal(a[:, :, 2:], b[:, :, 2:]) for a, b in zip(nan[:5], got[:5]))
+        bad = q.clone()
+        bad[0, row, :2, 3] = float("nan")
+        nan = _gpu_grads(device, bad, k, v, g, beta, do, None, None, None, True)
+        assert not torch.isfinite(nan[2][0, : row // 64 * 64, :2]).any()
+        assert all(torch.equal(a[:, :, 2:], b[:, :, 2:]) for a, b in zip(nan[:5], got[:5]))
