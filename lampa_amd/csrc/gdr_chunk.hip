@@ -84,6 +84,8 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
   if (!attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_a) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP, false>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, smem_a) != hipSuccess ||
         hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, true, false, T, 32, KEEP>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem_b) != hipSuccess ||
         hipFuncSetAttribute((const void*)gdr_segment_kernel<T, KT, VT, true, false, T, CWN>,
@@ -100,7 +102,8 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
                        pv.chunk_tok0, pv.chunk_len, tf, chunks, H, HV, l2norm, kp.positive_g, edge);
     LAMPA_PROF(s, "gdr_local_kernel");
     if (segs > n_seq) {
-      hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
+      hipLaunchKernelGGL((edge ? gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP>
+                               : gdr_segment_kernel<T, KT, VT, false, true, T, 32, KEEP, false>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, false>::WAVES), smem_a, s,
                          (const T*)q, (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, (const float*)edges, Mc, Nc, Dc,
                          (T*)nullptr, (float*)nullptr, H, HV, scale, l2norm, (const unsigned char*)nullptr,
                          (const unsigned char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0, kp.mt, VT);
