@@ -819,3 +819,35 @@ def test_recurrent_scan_behind_maps_without_a_past(device, K, V, lens):
     keep = [c for c in range(V) if c != 5]
     assert torch.isnan(o2[0, T - lens[-1]:, :, 5]).all() and torch.isnan(s2[n - 1, :, :, 5]).all()
     assert torch.equal(o2[..., keep], o[..., keep]) and torch.equal(s2[..., keep], s[..., keep])
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (64, 128, torch.float16), (32, 32, torch.bfloat16),
+                                       (128, 64, torch.bfloat16), (128, 128, torch.float16)])
+def test_states_behind_segments_without_a_past(device, K, V, dtype, monkeypatch):
+    # Packed sequences of one to ten segments: every segment of head 0 cuts off its past, those of a sequence's first half
+    # (head 2) or second half (head 3) do, none of head 1. Then with initial states, then a v that is not finite: its column is
+    # none from there on.
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 4)
+    lens = [64 * 4 * 6 - 9, 64 * 4 * 2, 100, 64 * 4 * 9 + 1]
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.long)
+    T = int(cu[-1])
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 4, K, V, dtype, seed=K + V, g_scale=0.02)
+    g[:, :, 0] *= 90
+    for a, b in zip(cu[:-1].tolist(), cu[1:].tolist()):
+        g[:, a:(a + b) // 2, 2] *= 90
+        g[:, (a + b) // 2:b, 3] *= 90
+    h0 = torch.randn(len(lens), 4, K, V, generator=torch.Generator().manual_seed(2))
+    args = _to(device, q, k, v, g, beta)
+    for init in (None, h0):
+        given = None if init is None else init.to(device)
+        run = lambda v: gd.chunk_gated_delta_rule(args[0], args[1], v, *args[3:], initial_state=given, output_final_state=True,
+                                                  cu_seqlens=cu.to(device))
+        o, s = run(args[2])
+        want_o, want_s = og.recurrent_c(q, k, v, g, beta, initial_state=init, cu_seqlens=cu)
+        _assert_bf16_close(o, want_o, "o")
+        _assert_bf16_close(s, want_s, "state")
+        bad = args[2].clone()
+        bad[0, 40, :, 3] = float("inf")
+        o1, s1 = run(bad)
+        assert not torch.isfinite(o1[0, 41:lens[0], :, 3]).any() and not torch.isfinite(s1[0, :, :, 3]).any()
+        assert torch.equal(o1[0, lens[0]:], o[0, lens[0]:]) and torch.equal(s1[1:], s[1:])
