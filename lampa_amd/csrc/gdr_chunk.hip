@@ -134,16 +134,15 @@ static int gdr_chunk_launch(const void* q, const void* k, const void* v, const f
                        pv, Mc, Nc, Dc, h0, Si, HV, segs);
     LAMPA_PROF(s, "gdr_scan_kernel");
   }
-  const unsigned char* Nw = two_level && !walk_in_output ? nullptr : Nc;  // (a leaf pass leaves the state of every segment)
   const int narrow = gdr_narrow_output.load();
   if (!KEEP && CWN == 16 && (narrow == 2 || (narrow == 1 && KT + VT > 128)))
     hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true, false, T, CWN>), dim3(segs * HV),
                        dim3(64 * GdrSegShape<KT, VT, true, CWN>::WAVES), smem_n, s, (const T*)q, (const T*)k, (const T*)v, g, beta,
-                       pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, (unsigned char*)Nw, Dc, (T*)o, ht, H, HV, scale, l2norm,
+                       pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, Nc, Dc, (T*)o, ht, H, HV, scale, l2norm,
                        (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states, KEEP ? kp.o_width : VT);
   else
   hipLaunchKernelGGL((gdr_segment_kernel<T, KT, VT, true, false, T, 32, KEEP>), dim3(segs * HV), dim3(64 * GdrSegShape<KT, VT, true>::WAVES), smem_b, s, (const T*)q,
-                     (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, (unsigned char*)Nw, Dc, (T*)o, ht, H, HV, scale,
+                     (const T*)k, (const T*)v, g, beta, pv, pv.chunk_tok0, pv.chunk_len, tf, Si, Mc, Nc, Dc, (T*)o, ht, H, HV, scale,
                      l2norm, (const unsigned char*)Gm, (const unsigned char*)Gn, (const float*)Gd, h0, walk_in_output ? gmax : 0, kp.states, KEEP ? kp.o_width : VT);
   LAMPA_PROF(s, "gdr_segment_kernel<output>");
   return lampa_launch_status();

@@ -821,14 +821,16 @@ def test_recurrent_scan_behind_maps_without_a_past(device, K, V, lens):
     assert torch.equal(o2[..., keep], o[..., keep]) and torch.equal(s2[..., keep], s[..., keep])
 
 
-@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (64, 128, torch.float16), (32, 32, torch.bfloat16),
-                                       (128, 64, torch.bfloat16), (128, 128, torch.float16)])
-def test_states_behind_segments_without_a_past(device, K, V, dtype, monkeypatch):
-    # Packed sequences of one to ten segments: every segment of head 0 cuts off its past, those of a sequence's first half
+@pytest.mark.parametrize("K,V,dtype,cps,chunks", [
+    (64, 64, torch.bfloat16, 4, [24, 8, 2, 37]), (64, 128, torch.float16, 4, [24, 8, 2, 37]), (32, 32, torch.bfloat16, 4, [24, 8, 2, 37]),
+    (128, 64, torch.bfloat16, 4, [24, 8, 2, 37]), (128, 128, torch.float16, 4, [24, 8, 2, 37]), (128, 64, torch.float16, 3, [72, 3, 30]),
+    (32, 32, torch.bfloat16, 3, [219]), (128, 128, torch.bfloat16, 2, [49, 1])])
+def test_states_behind_segments_without_a_past(device, K, V, dtype, cps, chunks, monkeypatch):
+    # Packed sequences of one segment to more than the 64 that are looked at: every segment of head 0 cuts off its past, those of a sequence's first half
     # (head 2) or second half (head 3) do, none of head 1. Then with initial states, then a v that is not finite: its column is
     # none from there on.
-    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 4)
-    lens = [64 * 4 * 6 - 9, 64 * 4 * 2, 100, 64 * 4 * 9 + 1]
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
+    lens = [64 * n - 9 * (n % 2) for n in chunks]
     cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.long)
     T = int(cu[-1])
     q, k, v, g, beta = synth.gdr_inputs(1, T, 4, K, V, dtype, seed=K + V, g_scale=0.02)
