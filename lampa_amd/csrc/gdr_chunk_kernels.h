@@ -93,7 +93,8 @@ __device__ __forceinline__ int gdr_leading_cuts(float d, int n, int lane) {
 }
 // The state that segment `seg` starts from, `size` floats in the slabs of the scan below (null: zero). Without an initial
 // state, behind maps that all cut off what lies before them, that is N of the last one, and the scan passes by such segments:
-// the call on 16 packed events of 520 000 tokens, 8 x 128 x 128, at e^-0.8 a token 1 600 -> 1 562 us; where nothing cuts off (4 x
+// the call on 16 packed events of 520 000 tokens, 8 x 128 x 128, at e^-0.8 a token 1 600 -> 1 562 us (scan 45 -> 6, output pass
+// 1 028 -> 1 060, to which the scan's copy came from the caches and N comes from HBM); where nothing cuts off (4 x
 // 14 803 tokens, 4 x 128 x 64, e^-0.04) 133.1 -> 132.9, the look being beside the first loads in both passes.
 __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv, int seg, int hv, int HV, int size,
                                                           const float* Sinit, const unsigned char* Ncomp, const float* Dcomp,
