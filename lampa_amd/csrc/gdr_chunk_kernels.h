@@ -1634,7 +1634,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       if constexpr (KEEP) *reinterpret_cast<f32x4*>(keep + at + y) = none;  // (map = seg)
     }
     float sum = CUTS ? 0.0f : 1.0f;
-    if constexpr (CUTS) {  // (the notes on N, see the end)
+    if constexpr (CUTS) {  // (the notes on N, which its waves leave wherever chunks are left out, see the end)
       lds_barrier();
 #pragma unroll
       for (int w = KT / 32; w < NSLAB; ++w) sum += tiles(0).misc[8 + w];
@@ -1975,6 +1975,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   } else if constexpr (CUTS) {
     faded = uniform(__float_as_int(dtot)) == 0;
   }
+  // (the waves of M wait for the notes below wherever chunks were left out, also where the decays' product has not become zero:
+  // at the smallest subnormal it stays what it is under every factor above a half)
+  if constexpr (CUTS && EDGES) faded |= uniform(left) > 0;
   if (EDGES && left > 0 && reinterpret_cast<const unsigned char*>(wild)[col]) {
 #pragma unroll
     for (int km = 0; km < KT / 32; ++km)
@@ -1987,8 +1990,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   if constexpr (CUTS) {
     // A segment whose M is zero and whose N is finite hands N on whatever finite state it starts from: its decay is
     // stored as -0 (gdr_d_cut), which those who walk the composites look for. Every wave notes what it knows of its own
-    // columns, wave 0 stores the decay. Looked at only where the decays' product has left the fp32 range, which all chain
-    // waves see at the same chunk; the stagers may have ended, a barrier does not wait for waves that have. (With a note and
+    // columns, wave 0 (or, where chunks were left out, the waves of M above) stores the decay. Looked at only there and where the
+    // decays' product has left the fp32 range, which all chain waves see at the same chunk; the stagers may have ended, a barrier does not wait for waves that have. (With a note and
     // a barrier in every segment, 9 000 tokens x 6 x 128 x 128 where none does: pass 25.0 us; so 23.9, without any look 23.7.)
     if (faded) {
       float probe = 0.0f;  // 0 x every entry: NaN unless all are finite

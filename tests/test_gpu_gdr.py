@@ -853,3 +853,33 @@ def test_states_behind_segments_without_a_past(device, K, V, dtype, cps, chunks,
         o1, s1 = run(bad)
         assert not torch.isfinite(o1[0, 41:lens[0], :, 3]).any() and not torch.isfinite(s1[0, :, :, 3]).any()
         assert torch.equal(o1[0, lens[0]:], o[0, lens[0]:]) and torch.equal(s1[1:], s[1:])
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (64, 64, torch.float16), (32, 32, torch.bfloat16), (128, 128, torch.float16)])
+def test_chunks_left_out_where_the_decays_product_stays_subnormal(device, K, V, dtype, monkeypatch):
+    # A segment of three chunks with next to no decay, one of 2^-90, one of 2^-58.5 and 61 of 2^-0.99 each: together 2^-208.9, but
+    # multiplied one after the other in fp32 the decays stay at 2^-149. A v in front that is not finite: its column of N is none,
+    # so the map is no cut, and the column stays none behind the next segment, which cuts off what is finite.
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 66)
+    T = 64 * 66 * 3
+    edges = [-90.0, -58.5] + [-0.99] * 61
+    product = np.float32(1.0)
+    for edge in edges:
+        product = np.float32(product * np.float32(2.0 ** edge))
+    assert product == np.float32(2.0 ** -149)
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 2, K, V, dtype, seed=K)
+    g[:] = -100 * np.log(2.0) / 64
+    g[:, :64 * 3] = -1e-4
+    for c, edge in enumerate(edges):
+        g[:, 64 * (3 + c):64 * (4 + c)] = edge * np.log(2.0) / 64
+    args = _to(device, q, k, v, g, beta)
+    o, s = gd.chunk_gated_delta_rule(*args, output_final_state=True)
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta)
+    _assert_bf16_close(o, want_o, "o")
+    _assert_bf16_close(s, want_s, "state")
+    bad = args[2].clone()
+    bad[0, 70, :, 5] = float("inf")
+    o1, s1 = gd.chunk_gated_delta_rule(args[0], args[1], bad, *args[3:], output_final_state=True)
+    assert not torch.isfinite(o1[0, 71:, :, 5]).any() and not torch.isfinite(s1[0, :, :, 5]).any()
+    keep = [c for c in range(V) if c != 5]
+    assert torch.equal(o1[..., keep], o[..., keep]) and torch.equal(s1[..., keep], s[..., keep])
