@@ -560,7 +560,7 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
   unsigned* const note = reinterpret_cast<unsigned*>(smem + GbSourceSmem::OFF_NOTE);
   int left = 0;
   if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
-    left = uniform(gdr_chunks_left_out<true>(edges + (size_t)c0 * HV + hv, HV, nc, lane));
+    left = uniform(gdr_chunks_left_out<T, true>(edges + (size_t)c0 * HV + hv, HV, nc, lane));
   const int ct = cl - left;  // the chunk the walk starts at
   if (left > 0) {
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));

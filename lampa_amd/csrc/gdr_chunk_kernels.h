@@ -113,14 +113,13 @@ __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv,
 // decay -- no positive log-decay, 0 <= beta |k|^2 <= 2 for the key as the operator uses it, all of it finite -- and infinity
 // elsewhere: chunks of finite edges leave at most 2^(sum of the edges) of any state, whatever their keys.
 //
-// The composite pass starts where the edges behind sum up to GDR_EDGE_REACH: nothing is left there of M and of the sources in
-// front. With beta up to 2^14 and beta |k|^2 <= 2 a write is below 2^8 |v|, the state of 128 chunks below 2^21 |v|, and 2^-208 of
-// that below the fp32 range up to |v| = 2^38 (M = 0, by which the scan forgets a state, is found at 2^-149). At e^-0.8 a token a
-// segment's last three chunks are walked, at e^-0.24 ten, at e^-0.04 all. us of the composite pass / the call before and after:
-// 60 000 tokens x 8 heads x 64 x 64 at e^-0.8 45.7 -> 25.7 / 125.5 -> 112, at e^-0.24 126 -> 117.6; 16 packed events of 520 000
-// tokens, 8 x 128 x 128 689 -> 241 / 2 005 -> 1 590; at e^-0.04 131.7 -> 132.0 and 290.5 -> 292.3, the price of the look.
-#define GDR_EDGE_BETA 16384.0f
-#define GDR_EDGE_REACH -208.0f
+// The composite pass starts where the edges behind sum up to gdr_edge_reach: nothing is left there of M and of the sources in
+// front. With beta up to 2 and beta |k|^2 <= 2 a write is below 2 |v|, the state of 128 chunks below 2^14 |v|, of the largest v of
+// bf16 below 2^142, of fp16 below 2^30, and 2^-292 or 2^-208 of that is below the fp32 range. (2^-208 for bf16 as well, which holds
+// for v up to 2^44: 60 000 tokens x 8 at e^-0.8 a token 111.3 us instead of 112.0, at e^-0.24 121.4 instead of 125.5.)
+#define GDR_EDGE_BETA 2.0f
+template <typename T>
+__device__ constexpr float gdr_edge_reach() { return __is_same(T, _Float16) ? -208.0f : -292.0f; }
 // Chunks left out that pay for looking at their v; chunks of a segment that pay for the look at its edges (15 000 tokens x 8 x
 // 128 x 64 at e^-0.04, segments of seven: 93.1 -> 94.8 us) and that two loads a lane cover.
 #define GDR_EDGE_MIN 2
@@ -131,12 +130,12 @@ __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv,
 // uniform here: with the count in a scalar register the passes that keep the raw k tile take 167 registers instead of 157
 // (15 000 tokens, hierarchical prefill: 172.5 -> 178 us).
 // BACK: the chunks at the segment's end, which those in front of them leave nothing of where a gradient is walked back.
-template <bool BACK = false>
+template <typename T, bool BACK = false>
 __device__ __forceinline__ int gdr_chunks_left_out(const float* edges, int HV, int nc, int lane) {
   const float edge = edges[(BACK ? min(lane, nc - 1) : max(nc - 1 - lane, 0)) * HV];
   const float far = edges[(BACK ? min(64 + lane, nc - 1) : max(nc - 65 - lane, 0)) * HV];
   const float past = wave_inclusive_scan(lane < nc ? edge : 0.0f);  // lane i: the last i + 1 chunks
-  const unsigned long long reach = __ballot(past <= GDR_EDGE_REACH);
+  const unsigned long long reach = __ballot(past <= gdr_edge_reach<T>());
   const int left = nc - 1 - (reach ? __builtin_ctzll(reach) : nc);
   return left < GDR_EDGE_MIN || __ballot(!(edge <= 0.0f && far <= 0.0f)) ? 0 : left;
 }
@@ -762,7 +761,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   int left = 0;
   if constexpr (EDGES) {
     if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
-      left = gdr_chunks_left_out(Sinit + (size_t)c0 * HV + hv, HV, nc, lane);
+      left = gdr_chunks_left_out<T>(Sinit + (size_t)c0 * HV + hv, HV, nc, lane);
     c0 += left;
     nc -= left;
   }

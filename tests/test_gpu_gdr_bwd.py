@@ -480,14 +480,15 @@ def test_forward_of_a_training_step_gives_the_bits_of_the_plain_call(device, T, 
 
 @pytest.mark.parametrize("dtype,cps,T", [(torch.bfloat16, 9, 64 * 9 * 3 - 9), (torch.float16, 9, 64 * 9 * 25), (torch.bfloat16, 66, 64 * 66 * 2 + 700)])
 def test_sources_end_where_later_chunks_no_longer_count(device, dtype, cps, T, monkeypatch):
-    """Segments whose first two (head 0) or four (head 1) chunks decay by more than the fp32 range, of which the pass for the
+    """Segments whose first two (head 0) or four (head 1; of fp16 three) chunks decay by more than the fp32 range and the range of the
+    sources together, of which the pass for the
     segments' own gradients walks no others (and the walk over the segments behind starts at the next one); head 2 has next to
     no decay, head 3 one in its first half. Then a dO or a q that is not finite at either end of the chunks left out: none of
     the gradients that it belongs to in front of it are."""
     monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
     (q, k, v, g, beta, do), _ = _inputs(1, T, 4, 4, 64, 64, dtype, seed=cps, unit=False, g_scale=0.02)
-    g[:, :, 0] *= 90
-    g[:, :, 1] *= 35
+    g[:, :, 0] *= 110
+    g[:, :, 1] *= 55
     g[:, : T // 2, 3] *= 50
     got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, True)
     want = ob.backward_manual(q, k, v, g, beta, do, l2=og.L2_CHUNK)
@@ -505,3 +506,22 @@ def test_sources_end_where_later_chunks_no_longer_count(device, dtype, cps, T, m
         nan = _gpu_grads(device, bad, k, v, g, beta, do, None, None, None, True)
         assert not torch.isfinite(nan[2][0, : row // 64 * 64, :2]).any()
         assert all(torch.equal(a[:, :, 2:], b[:, :, 2:]) for a, b in zip(nan[:5], got[:5]))
+
+
+@pytest.mark.parametrize("q_exp,do_exp,edge", [(0, 115, -70), (60, 60, -72)])
+def test_large_sources_behind_strong_decays(device, q_exp, do_exp, edge, monkeypatch):
+    """Three chunks of 2^edge that write nothing in front of q and dO whose products are large, no dO before these: what is left
+    of them there is small, but within the fp32 range."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 12)
+    T, seg = 64 * 24, 64 * 12
+    (q, k, v, g, beta, do), _ = _inputs(1, T, 2, 2, 64, 64, torch.bfloat16, seed=3, unit=True, g_scale=1e-4)
+    q[:, seg:] *= 2.0 ** q_exp
+    do *= 2.0 ** do_exp
+    do[:, :seg + 64 * 3] = 0
+    beta[:, seg:seg + 64 * 3] = 0
+    g[:, seg:seg + 64 * 3] = edge * 0.6931471805599453 / 64
+    got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, False)
+    want = ob.backward_manual(q, k, v, g, beta, do)
+    for a, b in zip(got[1:3], want[1:3]):  # dk, dv of the segment in front
+        a, b = a[:, :seg].cpu().double(), b[:, :seg]
+        assert 0 < b.abs().max() < 2.0 ** -80 and (a - b).norm() <= 2e-2 * b.norm()

@@ -459,3 +459,16 @@ def test_levels_that_have_decayed_to_zero(device, V, dtype, cps, chunks, monkeyp
     assert torch.equal(o2[0, :T - 128], o[0, :T - 128]) and not torch.isfinite(o2[0, T - 64:]).any()
     occupied = [0, 1, 2, 3, 4, 5, 6] + [7 + j for j in range(12) if (chunks - 1) >> j & 1]
     assert not torch.isfinite(state2.states[..., occupied[7:]]).any()
+
+
+@pytest.mark.parametrize("V", [64, 128])
+def test_large_values_in_front_of_strong_decays(device, V):
+    """Three chunks of 2^-73 at the end of a segment behind v of the size 2^122, nothing written from there on: what the next
+    segment reads is small, but within the fp32 range."""
+    q, k, v, g, beta, lam = _inputs(1, 64 * 18, 2, 64, V, torch.bfloat16, seed=V, g_scale=1e-4)
+    v[:, :64 * 13] *= 2.0 ** 122
+    beta[:, 64 * 13:] = 0
+    g[:, 64 * 13:64 * 16] = -73 * 0.6931471805599453 / 64
+    want = _want(q, k, v, g, beta, lam)[:, 64 * 16:].double()
+    got = _run(device, q, k, v, g, beta, lam, 16)[:, 64 * 16:].cpu().double()
+    assert 0 < want.abs().max() < 2.0 ** -80 and (got - want).norm() <= 2e-2 * want.norm()
