@@ -76,7 +76,7 @@ struct GbWalkSmem {
 static_assert(GbWalkSmem::BYTES <= 163840, "LDS of a CU");
 struct GbSourceSmem {
   static constexpr int OFF_P = 2 * GbSet<false>::BYTES;
-  static constexpr int OFF_NOTE = OFF_P + 3 * GB_TRI;  // a byte per value column, q, the two waves of N'
+  static constexpr int OFF_NOTE = OFF_P + 3 * GB_TRI;  // the waves' largest q and dO, the two waves of N'
   static constexpr int BYTES = OFF_NOTE + 80;
 };
 static_assert(GbSourceSmem::BYTES <= 81920, "two workgroups per CU");
@@ -531,7 +531,7 @@ __device__ __forceinline__ void gb_zero_upper(unsigned char* smem, int tid) {
 // Grid segments x heads (long segments first), eight waves: 0, 1 the gradient of the state (32 value columns each), 4-6 the
 // tiles of P, 2 and 3 / 4-7 stage the next chunk into the other set of tiles. Two barriers per chunk, two workgroups per CU (80 KB
 // of LDS, 128 registers). 52 - 57 us, by card, at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the
-// products), and 39 at e^-0.8 a token, where three of a segment's 15 chunks are walked and the q and dO of the others looked at (half
+// products), and 39 at e^-0.8 a token, where four of a segment's 15 chunks are walked and the q and dO of the others looked at (half
 // of its traffic then); with the walk that starts at the next segment (197 -> 190) the training step 370 -> 352.
 template <typename T>
 __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
@@ -555,20 +555,19 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
   // chunk earlier still
   auto set_of = [&](int c) { return gb_tiles<OT, false>(smem, (cl - c) & 1); };
   gb_zero_upper<OT, false>(smem, tid);
-  // Chunks at the segment's end that those in front of them leave nothing of are left out, as in the forward's composites, after
-  // a look at their q and dO: a q that is not finite is in all of N', a dO in its column.
-  unsigned* const note = reinterpret_cast<unsigned*>(smem + GbSourceSmem::OFF_NOTE);
+  // Chunks at the segment's end that those in front of them leave nothing of are left out, as in the forward's composites, where a
+  // look at their q and dO finds the sources scale q dO small enough: 128 chunks of these add up to less than 2^13 times the largest,
+  // 2^127 of bf16 (so that nothing overflows either), 2^58 of fp16. With larger ones, or any that is not finite, all are walked.
+  float* const note = reinterpret_cast<float*>(smem + GbSourceSmem::OFF_NOTE);
   int left = 0;
   if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
     left = uniform(gdr_chunks_left_out<T, true>(edges + (size_t)c0 * HV + hv, HV, nc, lane));
-  const int ct = cl - left;  // the chunk the walk starts at
   if (left > 0) {
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    if (tid < 20) note[tid] = 0;
-    u16x2 top_q = {0, 0}, top_d[4] = {};
+    u16x2 top_q = {0, 0}, top_d = {0, 0};
     const int row = tid >> 3, part = tid & 7;  // (a thread a 16-byte piece of the chunk's 64 rows)
-    const T* qp = q + ((size_t)tok_of(ct + 1) * H + h) * 64 + 8 * part;
-    const T* dp = dout + ((size_t)tok_of(ct + 1) * HV + hv) * 64 + 8 * part;
+    const T* qp = q + ((size_t)tok_of(cl - left + 1) * H + h) * 64 + 8 * part;
+    const T* dp = dout + ((size_t)tok_of(cl - left + 1) * HV + hv) * 64 + 8 * part;
     const int rows = 64 * (left - 1) + len_last;
     for (int x = 0; x < left; x += 4) {
       uint4 rq[4], rd[4];
@@ -584,19 +583,25 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           top_q = __builtin_elementwise_max(top_q, __builtin_bit_cast(u16x2, a[e] & 0x7fff7fffu));
-          top_d[e] = __builtin_elementwise_max(top_d[e], __builtin_bit_cast(u16x2, d[e] & 0x7fff7fffu));
+          top_d = __builtin_elementwise_max(top_d, __builtin_bit_cast(u16x2, d[e] & 0x7fff7fffu));
         }
       }
     }
-    const unsigned short limit = __is_same(T, _Float16) ? 0x7c00 : 0x7f80;
+    constexpr bool HALF = __is_same(T, _Float16);
+    auto size_of = [](u16x2 top) {  // the largest of the wave (a NaN counts as infinity)
+      const unsigned short x = min(max(top[0], top[1]), (unsigned short)(HALF ? 0x7c00 : 0x7f80));
+      return wave_inclusive_max((float)__builtin_bit_cast(T, x));
+    };
+    const float wave_q = size_of(top_q), wave_d = size_of(top_d);
+    if (lane == 63) { note[wave] = wave_q; note[8 + wave] = wave_d; }
     lds_barrier();
+    float big_q = note[0], big_d = note[8];
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
-      atomicOr(&note[2 * part + e], (top_d[2 * e][0] >= limit ? 1u : 0u) | (top_d[2 * e][1] >= limit ? 1u << 8 : 0u) |
-                                        (top_d[2 * e + 1][0] >= limit ? 1u << 16 : 0u) | (top_d[2 * e + 1][1] >= limit ? 1u << 24 : 0u));
-    if (top_q[0] >= limit || top_q[1] >= limit) note[16] = 1;
-    // (read behind the walk's barriers)
+    for (int w = 1; w < 8; ++w) { big_q = fmaxf(big_q, note[w]); big_d = fmaxf(big_d, note[8 + w]); }
+    const float norm_q = l2norm == GDR_L2_NONE ? 8.0f * big_q : big_q <= 0x1p60f ? 1.0f : __builtin_inff();
+    if (!(__builtin_fabsf(scale) * norm_q * big_d <= (HALF ? 0x1p45f : 0x1p114f))) left = 0;
   }
+  const int ct = uniform(cl - left);  // the chunk the walk starts at
   if (wave < 2) {
     GbChain<OT> ch;
     ch.G[0] = zero16();
@@ -610,12 +615,6 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
       ch.update(t, scale, wave, lane, hh);
       lds_barrier();  // (2) the tiles of chunk c have been read, those of chunk c - 1 are complete
     }
-    if (left > 0 && (note[16] || reinterpret_cast<const unsigned char*>(note)[32 * wave + ln])) {
-#pragma unroll
-      for (int km = 0; km < 2; ++km)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) ch.G[km][r] = __builtin_nanf("");
-    }
     // A segment without M (the forward's mark) and with a finite N' hands N' on whatever finite gradient comes from behind it
     const float dc = Dc[(size_t)seg * HV + hv];
     float dr = __builtin_fabsf(dc);
@@ -625,9 +624,9 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
       for (int km = 0; km < 2; ++km)
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(ch.G[km][r], 0.0f, probe);
-      if (lane == 0) note[18 + wave] = __ballot(!(probe == 0.0f)) != 0;
+      if (lane == 0) note[16 + wave] = __ballot(!(probe == 0.0f)) ? 1.0f : 0.0f;
       lds_barrier();  // (of the two waves that are left)
-      if (!(note[18] | note[19])) dr = -0.0f;
+      if (note[16] + note[17] == 0.0f) dr = -0.0f;
     }
     if (tid == 0) Dr[(size_t)seg * HV + hv] = dr;
     // N' in accumulator order, as the forward composites keep N

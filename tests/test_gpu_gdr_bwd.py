@@ -525,3 +525,18 @@ def test_large_sources_behind_strong_decays(device, q_exp, do_exp, edge, monkeyp
     for a, b in zip(got[1:3], want[1:3]):  # dk, dv of the segment in front
         a, b = a[:, :seg].cpu().double(), b[:, :seg]
         assert 0 < b.abs().max() < 2.0 ** -80 and (a - b).norm() <= 2e-2 * b.norm()
+
+
+@pytest.mark.parametrize("dtype,q_exp,do_exp,scale", [(torch.bfloat16, 70, 60, 1.0), (torch.bfloat16, 0, 100, 2.0 ** 40)])
+def test_sources_that_overflow_behind_strong_decays(device, dtype, q_exp, do_exp, scale, monkeypatch):
+    """Products of q, dO and the scale beyond the fp32 range behind three chunks of 2^-100: the gradients in front of these are
+    none, as where every chunk is walked."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 12)
+    T, seg = 64 * 24, 64 * 12
+    (q, k, v, g, beta, do), _ = _inputs(1, T, 2, 2, 64, 64, dtype, seed=3, unit=True, g_scale=1e-4)
+    q[:, seg:] *= 2.0 ** q_exp
+    do *= 2.0 ** do_exp
+    do[:, :seg + 64 * 3] = 0
+    g[:, seg:seg + 64 * 3] = -100 * 0.6931471805599453 / 64
+    got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, False, scale=scale)
+    assert not torch.isfinite(got[2][:, :seg]).any()
