@@ -531,7 +531,7 @@ __device__ __forceinline__ void gb_zero_upper(unsigned char* smem, int tid) {
 // Grid segments x heads (long segments first), eight waves: 0, 1 the gradient of the state (32 value columns each), 4-6 the
 // tiles of P, 2 and 3 / 4-7 stage the next chunk into the other set of tiles. Two barriers per chunk, two workgroups per CU (80 KB
 // of LDS, 128 registers). 52 - 57 us, by card, at 60 000 tokens x 8 heads (74 us with one set of tiles and the staging between the
-// products), and 39 at e^-0.8 a token, where four of a segment's 15 chunks are walked and the q and dO of the others looked at (half
+// products), and 39 at e^-0.8 a token, where three of a segment's 15 chunks are walked and the q and dO of the others looked at (half
 // of its traffic then); with the walk that starts at the next segment (197 -> 190) the training step 370 -> 352.
 template <typename T>
 __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
@@ -557,11 +557,11 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
   gb_zero_upper<OT, false>(smem, tid);
   // Chunks at the segment's end that those in front of them leave nothing of are left out, as in the forward's composites, where a
   // look at their q and dO finds the sources scale q dO small enough: 128 chunks of these add up to less than 2^13 times the largest,
-  // 2^127 of bf16 (so that nothing overflows either), 2^58 of fp16. With larger ones, or any that is not finite, all are walked.
+  // 2^58. With larger ones, or any that is not finite, all are walked.
   float* const note = reinterpret_cast<float*>(smem + GbSourceSmem::OFF_NOTE);
   int left = 0;
   if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
-    left = uniform(gdr_chunks_left_out<T, true>(edges + (size_t)c0 * HV + hv, HV, nc, lane));
+    left = uniform(gdr_chunks_left_out<true>(edges + (size_t)c0 * HV + hv, HV, nc, lane));
   if (left > 0) {
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     u16x2 top_q = {0, 0}, top_d = {0, 0};
@@ -599,7 +599,7 @@ __global__ void __launch_bounds__(GB_SOURCE_THREADS, 4)
 #pragma unroll
     for (int w = 1; w < 8; ++w) { big_q = fmaxf(big_q, note[w]); big_d = fmaxf(big_d, note[8 + w]); }
     const float norm_q = l2norm == GDR_L2_NONE ? 8.0f * big_q : big_q <= 0x1p60f ? 1.0f : __builtin_inff();
-    if (!(__builtin_fabsf(scale) * norm_q * big_d <= (HALF ? 0x1p45f : 0x1p114f))) left = 0;
+    if (!(__builtin_fabsf(scale) * norm_q * big_d <= 0x1p45f)) left = 0;
   }
   const int ct = uniform(cl - left);  // the chunk the walk starts at
   if (wave < 2) {

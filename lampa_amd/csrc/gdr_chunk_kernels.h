@@ -113,13 +113,13 @@ __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv,
 // decay -- no positive log-decay, 0 <= beta |k|^2 <= 2 for the key as the operator uses it, all of it finite -- and infinity
 // elsewhere: chunks of finite edges leave at most 2^(sum of the edges) of any state, whatever their keys.
 //
-// The composite pass starts where the edges behind sum up to gdr_edge_reach: nothing is left there of M and of the sources in
-// front. With beta up to 2 and beta |k|^2 <= 2 a write is below 2 |v|, the state of 128 chunks below 2^14 |v|, of the largest v of
-// bf16 below 2^142, of fp16 below 2^30, and 2^-292 or 2^-208 of that is below the fp32 range. (2^-208 for bf16 as well, which holds
-// for v up to 2^44: 60 000 tokens x 8 at e^-0.8 a token 111.3 us instead of 112.0, at e^-0.24 121.4 instead of 125.5.)
+// The composite pass starts where the edges behind sum up to GDR_EDGE_REACH: nothing is left there of M and of the sources in
+// front. With beta up to 2 and beta |k|^2 <= 2 a write is below 2 |v|, the state of 128 chunks below 2^14 |v|, and 2^-208 of that
+// below the fp32 range up to |v| = 2^44 (every fp16). A column of the value with a larger one in front is worked out token by
+// token (gdr_serial_slab).
 #define GDR_EDGE_BETA 2.0f
-template <typename T>
-__device__ constexpr float gdr_edge_reach() { return __is_same(T, _Float16) ? -208.0f : -292.0f; }
+#define GDR_EDGE_REACH -208.0f
+#define GDR_EDGE_LARGE 0x5580  // bits of the bf16 2^44
 // Chunks left out that pay for looking at their v; chunks of a segment that pay for the look at its edges (15 000 tokens x 8 x
 // 128 x 64 at e^-0.04, segments of seven: 93.1 -> 94.8 us) and that two loads a lane cover.
 #define GDR_EDGE_MIN 2
@@ -130,12 +130,12 @@ __device__ constexpr float gdr_edge_reach() { return __is_same(T, _Float16) ? -2
 // uniform here: with the count in a scalar register the passes that keep the raw k tile take 167 registers instead of 157
 // (15 000 tokens, hierarchical prefill: 172.5 -> 178 us).
 // BACK: the chunks at the segment's end, which those in front of them leave nothing of where a gradient is walked back.
-template <typename T, bool BACK = false>
+template <bool BACK = false>
 __device__ __forceinline__ int gdr_chunks_left_out(const float* edges, int HV, int nc, int lane) {
   const float edge = edges[(BACK ? min(lane, nc - 1) : max(nc - 1 - lane, 0)) * HV];
   const float far = edges[(BACK ? min(64 + lane, nc - 1) : max(nc - 65 - lane, 0)) * HV];
   const float past = wave_inclusive_scan(lane < nc ? edge : 0.0f);  // lane i: the last i + 1 chunks
-  const unsigned long long reach = __ballot(past <= gdr_edge_reach<T>());
+  const unsigned long long reach = __ballot(past <= GDR_EDGE_REACH);
   const int left = nc - 1 - (reach ? __builtin_ctzll(reach) : nc);
   return left < GDR_EDGE_MIN || __ballot(!(edge <= 0.0f && far <= 0.0f)) ? 0 : left;
 }
@@ -663,6 +663,55 @@ __device__ __forceinline__ bf16x8 ld_kappa_tr(const __bf16* arr, int stride, int
   return out;
 }
 
+// N of a segment, 32 value columns, token by token in fp32 (S: a wave's accumulator tiles). For columns that hold values beyond
+// GDR_EDGE_LARGE in front of strong decays: rare, and as slow as it is short (60 000 tokens x 8 with such a value in every
+// segment, 64 x 64 104 -> 710 us, 128 x 128 226 -> 1 790; in every column the same).
+// k, v, g, beta: the segment's first token; tmat: its first record; col: this lane's value column.
+template <typename T, int KT>
+__device__ __forceinline__ void gdr_serial_slab(const T* k, const T* v, const float* g, const float* beta, const unsigned char* tmat,
+                                                int tokens, int kstride, int vstride, int HV, int hh, f32x16* S) {
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  struct Token {
+    T4 k[KT / 8];
+    float v, g, beta, rk;
+  };
+  auto fetch = [&](int t, Token& x) __attribute__((always_inline)) {
+    t = min(t, tokens - 1);
+    const T* row = k + (size_t)t * kstride + 4 * hh;
+#pragma unroll
+    for (int i = 0; i < KT / 8; ++i) x.k[i] = *reinterpret_cast<const T4*>(row + 8 * i);  // rows 8 i + 4 hh .. + 3
+    x.v = (float)v[(size_t)t * vstride];
+    x.g = g[(size_t)t * HV];
+    x.beta = beta[(size_t)t * HV];
+    x.rk = reinterpret_cast<const float*>(tmat + (size_t)(t / GDR_C) * HV * REC_BYTES + T_BYTES)[128 + t % GDR_C];
+  };
+#pragma unroll
+  for (int km = 0; km < KT / 32; ++km) S[km] = zero16();
+  Token cur, next;
+  fetch(0, cur);
+#pragma unroll 1
+  for (int t = 0; t < tokens; ++t) {
+    fetch(t + 1, next);
+    const float dec = __builtin_amdgcn_exp2f(1.44269504f * cur.g);
+    float dot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < KT / 8; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = dec * S[i / 4][4 * (i % 4) + e];
+        S[i / 4][4 * (i % 4) + e] = x;
+        dot = __builtin_fmaf((float)cur.k[i][e], x, dot);
+      }
+    dot += __shfl_xor(dot, 32);
+    const float u = cur.beta * (cur.v - cur.rk * dot) * cur.rk;
+#pragma unroll
+    for (int i = 0; i < KT / 8; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[i / 4][4 * (i % 4) + e] += (float)cur.k[i][e] * u;
+    cur = next;
+  }
+}
+
 // KEEP (training form, K = V = 64, see gdr_train.h): PASS_A also maps the last segment of a sequence and stores M' once
 // more in the fragment order of its transpose; PASS_B stores the state in front of every chunk -- the operand fragments
 // the chain waves hold anyway, 8 KiB per chunk and head in 1 KiB runs. o's rows are then o_width <= VT elements (a multiple
@@ -758,12 +807,16 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, hh = lane >> 5, ln = lane & 31;
   // Composite pass: chunks that what comes behind them in the segment leaves nothing of are left out (GDR_EDGE_*; `Sinit` holds
   // the edges).
-  int left = 0;
+  // (The chunks of a segment follow one another and only its last one may be shorter: with the first one's token, fetched beside
+  // the edges, no table entry has to be fetched behind the look.)
+  int left = 0, first_tok = 0, last_len = 0;
   if constexpr (EDGES) {
+    if (nc > 0) { first_tok = chunk_tok0[c0]; last_len = chunk_len[c1 - 1]; }
     if (nc >= GDR_EDGE_NC && nc <= GDR_EDGE_NC_MAX)
-      left = gdr_chunks_left_out<T>(Sinit + (size_t)c0 * HV + hv, HV, nc, lane);
+      left = gdr_chunks_left_out(Sinit + (size_t)c0 * HV + hv, HV, nc, lane);
     c0 += left;
     nc -= left;
+    first_tok += GDR_C * left;
   }
   // (the per-chunk tables are separate restrict parameters: read through the view they could alias the kernel's
   // stores, would be fetched with vector loads and would sit in the same queue as the stagers' prefetches)
@@ -1233,8 +1286,10 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       typename Raw8<T>::type* const rkB = SCALED ? rk1_ : rk0_;
       // the chunks' table entries live in scalar registers and are fetched a chunk period before their first use
       const int ca = uniform(c0), cb = uniform(min(c0 + 1, cl)), cc = uniform(min(c0 + 2, cl));
-      const int tk0 = chunk_tok0[ca], ln0 = chunk_len[ca], tk1 = chunk_tok0[cb], ln1 = chunk_len[cb];
-      int ln_c = ln0, ln_c1 = ln1, tk_c2 = chunk_tok0[cc], ln_c2 = chunk_len[cc];  // of chunks c, c + 1, c + 2 (clamped)
+      auto tok_of = [&](int c) { return EDGES ? uniform(first_tok + GDR_C * (c - c0)) : chunk_tok0[c]; };
+      auto len_of = [&](int c) { return EDGES ? uniform(c == cl ? last_len : GDR_C) : chunk_len[c]; };
+      const int tk0 = tok_of(ca), ln0 = len_of(ca), tk1 = tok_of(cb), ln1 = len_of(cb);
+      int ln_c = ln0, ln_c1 = ln1, tk_c2 = tok_of(cc), ln_c2 = len_of(cc);  // of chunks c, c + 1, c + 2 (clamped)
       int tk_c = tk0, tk_c1 = tk1, tk_p = 0, ln_p = 0;                              // (tk_p, ln_p: of chunk c - 1)
       // the o tile (rows of chunk `tok0`) -> HBM, 16-byte pieces, whole rows (non-temporal: o is not read again here)
       auto stager_flush = [&](int tok0, int len) __attribute__((always_inline)) {
@@ -1586,14 +1641,16 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   const unsigned vkeep = uniform(is_m ? 0 : -1);
 
   unsigned* const wild = reinterpret_cast<unsigned*>(tiles(0).misc + 24);  // a byte per value column
+  if (EDGES && tid == 0) tiles(0).misc[4] = left > 0 ? 1.0f : 0.0f;  // (for the end: no register holds it over the loop)
   if (EDGES && left > 0 && uniform(is_m)) {
     // M is zero, and the waves of its columns look at the v of the chunks left out instead, some beside each chunk that is
-    // walked: a column with a value that is not finite is none of N either, as where all chunks are walked. That traffic (a
-    // quarter of what the chunks' tiles would be) is what the pass then takes its time for. The waves leave by themselves: a
-    // way back into the recurrence would cost its loop 100 spilled registers.
+    // walked: a column with a value that is not finite is none of N either, as where all chunks are walked (note 1 or 3), and one
+    // with a value that is too large is worked out here (note 2). That traffic (a quarter of what the chunks' tiles would be)
+    // is what the pass then takes its time for. The waves leave by themselves: a way back into the recurrence would cost its
+    // loop 100 spilled registers.
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     constexpr int PPR = VT / 8, STEP = 2 * KT / PPR, LOADS = 64 / STEP;  // 16-byte pieces of a row, rows a load, loads a chunk
-    const int tok0 = chunk_tok0[uniform(c0 - left)], rs = HV * VT;
+    const int tok0 = uniform(first_tok - GDR_C * left), rs = HV * VT;
     const T* vb = v + ((size_t)tok0 * HV + hv) * VT;
     const int off = (tid / PPR) * rs + 8 * (tid % PPR);
     const int part = (left + nc) / (nc + 1);
@@ -1615,12 +1672,12 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         }
       }
       if (c == nc) {
-        const unsigned short limit = __is_same(T, _Float16) ? 0x7c00 : 0x7f80;
+        constexpr bool HALF = __is_same(T, _Float16);
+        auto note = [&](unsigned short x) { return x >= (HALF ? 0x7c00 : 0x7f80) ? 1u : !HALF && x >= GDR_EDGE_LARGE ? 2u : 0u; };
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          atomicOr(&wild[2 * (tid % PPR) + h], (top[2 * h][0] >= limit ? 1u : 0u) | (top[2 * h][1] >= limit ? 1u << 8 : 0u) |
-                                                   (top[2 * h + 1][0] >= limit ? 1u << 16 : 0u) |
-                                                   (top[2 * h + 1][1] >= limit ? 1u << 24 : 0u));
+          atomicOr(&wild[2 * (tid % PPR) + h], note(top[2 * h][0]) | note(top[2 * h][1]) << 8 | note(top[2 * h + 1][0]) << 16 |
+                                                   note(top[2 * h + 1][1]) << 24);
       }
       lds_barrier();  // tiles (c0) are ready, then B(c0) .. B(c1 - 1)
     }
@@ -1632,11 +1689,37 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       *reinterpret_cast<f32x4*>(Mcomp + (pairs ? 2 : 1) * at + y) = none;
       if constexpr (KEEP) *reinterpret_cast<f32x4*>(keep + at + y) = none;  // (map = seg)
     }
+    bool fine = true;
+    for (int slab = wave; slab < (__is_same(T, _Float16) ? 0 : VT / 32); slab += KT / 32) {
+      const bool large = reinterpret_cast<const unsigned char*>(wild)[32 * slab + ln] == 2;
+      if (__ballot(large) == 0) continue;
+      f32x16 N[KT / 32];
+      const size_t gi = (size_t)tok0 * HV + hv;
+      gdr_serial_slab<T, KT>(k + ((size_t)tok0 * H + h) * KT, v + gi * VT + 32 * slab + ln, g + gi, beta + gi,
+                             tmat + ((size_t)(c1 - nc - left) * HV + hv) * REC_BYTES, GDR_C * (left + nc - 1) + last_len, H * KT,
+                             HV * VT, HV, hh, N);
+      float probe = 0.0f;
+      f32x4* out = reinterpret_cast<f32x4*>(Ncomp + (((size_t)map * HV + hv) * (VT / 32) + slab) * (KT * 32 * 4));
+#pragma unroll
+      for (int km = 0; km < KT / 32; ++km)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          f32x4 t;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            t[e] = N[km][4 * q4 + e];
+            probe = __builtin_fmaf(t[e], 0.0f, probe);
+          }
+          if (large) out[(km * 4 + q4) * 64 + lane] = t;
+        }
+      fine &= __ballot(large && !(probe == 0.0f)) == 0;
+    }
     float sum = CUTS ? 0.0f : 1.0f;
     if constexpr (CUTS) {  // (the notes on N, which its waves leave wherever chunks are left out, see the end)
+      if (lane == 0) tiles(0).misc[8 + wave] = fine ? 0.0f : 1.0f;
       lds_barrier();
 #pragma unroll
-      for (int w = KT / 32; w < NSLAB; ++w) sum += tiles(0).misc[8 + w];
+      for (int w = 0; w < NSLAB; ++w) sum += tiles(0).misc[8 + w];
     }
     if (tid == 0) Dcomp[(size_t)map * HV + hv] = sum == 0.0f ? -0.0f : 0.0f;
     return;
@@ -1976,8 +2059,10 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   }
   // (the waves of M wait for the notes below wherever chunks were left out, also where the decays' product has not become zero:
   // at the smallest subnormal it stays what it is under every factor above a half)
-  if constexpr (CUTS && EDGES) faded |= uniform(left) > 0;
-  if (EDGES && left > 0 && reinterpret_cast<const unsigned char*>(wild)[col]) {
+  const bool shortened = EDGES && nc > 0 && uniform(__float_as_int(tiles(0).misc[4])) != 0;
+  if constexpr (CUTS && EDGES) faded |= shortened;
+  const int wild_v = EDGES && shortened ? reinterpret_cast<const unsigned char*>(wild)[col] : 0;
+  if (EDGES && (wild_v & 1)) {
 #pragma unroll
     for (int km = 0; km < KT / 32; ++km)
 #pragma unroll
@@ -2025,6 +2110,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
     // (a piece's M' is kept as pairs of value and remainder: gdr_scan2_kernel<PIECES>)
     unsigned char* out = Mcomp + ((size_t)map * HV + hv) * (KT * KT * 2) + late;
     if constexpr (PIECES) out += gmax > 0 ? ((size_t)map * HV + hv) * (KT * KT * 2) : 0;
+    // (`late` also keeps the comparisons with I from being held over the loop: 32 masks in scalar registers, most of them spilled)
     const int mcol = 32 * wave + ln, ks = mcol >> 4, c16 = mcol & 15;
     const int hs = (c16 >> 2) & 1, slot = 4 * (c16 >> 3) + (c16 & 3);
 #pragma unroll
@@ -2070,7 +2156,7 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         f32x4 t;
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[e] = S[km][4 * q4 + e];
-        reinterpret_cast<f32x4*>(out)[(km * 4 + q4) * 64 + lane] = t;
+        if (!EDGES || wild_v != 2) reinterpret_cast<f32x4*>(out)[(km * 4 + q4) * 64 + lane] = t;
       }
   }
   }  // (the 32-column chain wave)

@@ -755,15 +755,15 @@ def test_few_tokens_of_very_many_sequences(device, K, V, dtype, lens):
                                            (64, 128, torch.bfloat16, 9), (128, 64, torch.float16, 8),
                                            (128, 128, torch.bfloat16, 66)])
 def test_composites_start_where_earlier_chunks_no_longer_count(device, K, V, dtype, cps, monkeypatch):
-    # Segments whose last two (head 0) or four (head 1; of fp16 three) chunks decay by more than the fp32 range and the range
-    # of v together, of which the composite pass walks no others; head 2 has next to no decay, head 3 one in its second half. Then a
-    # v, at either end of the chunks left out and in those that are walked, or a k that is not finite: its column, or its head, is none behind it. Then a token
+    # Segments whose last two (head 0) or four (head 1) chunks decay by more than the fp32 range, of which the composite pass
+    # walks no others; head 2 has next to no decay, head 3 one in its second half. Then a v, at either end of the chunks
+    # left out and in those that are walked, or a k that is not finite: its column, or its head, is none behind it. Then a token
     # that is no contraction, for which every chunk is walked.
     monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
     T = 64 * cps * 3 - 9
     q, k, v, g, beta = synth.gdr_inputs(1, T, 4, K, V, dtype, seed=K + V, g_scale=0.02)
-    g[:, :, 0] *= 110
-    g[:, :, 1] *= 55
+    g[:, :, 0] *= 90
+    g[:, :, 1] *= 35
     g[:, T // 2:, 3] *= 50
     want_o, want_s = og.recurrent_c(q, k, v, g, beta)
     args = _to(device, q, k, v, g, beta)
@@ -855,12 +855,11 @@ def test_states_behind_segments_without_a_past(device, K, V, dtype, cps, chunks,
         assert torch.equal(o1[0, lens[0]:], o[0, lens[0]:]) and torch.equal(s1[1:], s[1:])
 
 
-@pytest.mark.parametrize("K,V", [(64, 64), (32, 32), (128, 128)])
-def test_chunks_left_out_where_the_decays_product_stays_subnormal(device, K, V, monkeypatch):
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (64, 64, torch.float16), (32, 32, torch.bfloat16), (128, 128, torch.float16)])
+def test_chunks_left_out_where_the_decays_product_stays_subnormal(device, K, V, dtype, monkeypatch):
     # A segment of three chunks with next to no decay, one of 2^-90, one of 2^-58.5 and 61 of 2^-0.99 each: together 2^-208.9, but
     # multiplied one after the other in fp32 the decays stay at 2^-149. A v in front that is not finite: its column of N is none,
-    # so the map is no cut, and the column stays none behind the next segment, which cuts off what is finite. (fp16: the edges that
-    # leave chunks of bf16 out multiply to zero.)
+    # so the map is no cut, and the column stays none behind the next segment, which cuts off what is finite.
     monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 66)
     T = 64 * 66 * 3
     edges = [-90.0, -58.5] + [-0.99] * 61
@@ -868,7 +867,7 @@ def test_chunks_left_out_where_the_decays_product_stays_subnormal(device, K, V, 
     for edge in edges:
         product = np.float32(product * np.float32(2.0 ** edge))
     assert product == np.float32(2.0 ** -149)
-    q, k, v, g, beta = synth.gdr_inputs(1, T, 2, K, V, torch.float16, seed=K)
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 2, K, V, dtype, seed=K)
     g[:] = -100 * np.log(2.0) / 64
     g[:, :64 * 3] = -1e-4
     for c, edge in enumerate(edges):
@@ -888,16 +887,35 @@ def test_chunks_left_out_where_the_decays_product_stays_subnormal(device, K, V, 
 
 @pytest.mark.parametrize("K,V,exponent,edge", [(64, 64, 115, -70), (64, 64, 122, -73), (32, 32, 122, -73), (64, 128, 122, -73),
                                                (128, 64, 115, -70), (128, 128, 122, -73)])
-def test_large_values_in_front_of_strong_decays(device, K, V, exponent, edge, monkeypatch):
-    # Three chunks of 2^edge behind v of the size 2^exponent, nothing written from there on: what is left is small, but within the
-    # fp32 range. (2e-2: the roundings to bf16 of an ordinary call's outputs.)
+@pytest.mark.parametrize("l2norm", [False, True])
+def test_large_values_in_front_of_strong_decays(device, K, V, exponent, edge, l2norm, monkeypatch):
+    # Three chunks of 2^edge at the end of a segment behind v of the size 2^exponent, nothing written from there to the next segment's
+    # end: what is left is small, but within the fp32 range. The same in the third, ragged segment. (2e-2: the roundings to bf16
+    # of an ordinary call's outputs.) Then such values in two columns only, one of them with a NaN as well.
     monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 12)
-    q, k, v, g, beta = synth.gdr_inputs(1, 64 * 15, 2, K, V, torch.bfloat16, seed=K, g_scale=1e-4)
-    v[:, :64 * 9] *= 2.0 ** exponent
-    beta[:, 64 * 9:] = 0
-    g[:, 64 * 9:64 * 12] = edge * np.log(2.0) / 64
-    want_o, want_s = og.recurrent_c(q, k, v, g, beta)
-    o, s = gd.chunk_gated_delta_rule(*_to(device, q, k, v, g, beta), output_final_state=True)
-    for got, want in ((o[:, 64 * 12:].cpu().double(), want_o[:, 64 * 12:].double()), (s.cpu().double(), want_s.double())):
-        assert 0 < want.abs().max() < 2.0 ** -80
+    seg, T = 64 * 12, 64 * 35 + 40
+    q, k, v, g, beta = synth.gdr_inputs(1, T, 2, K, V, torch.bfloat16, seed=K, g_scale=1e-4)
+    small = v.clone()
+    for at in (0, 2 * seg):
+        v[:, at:at + 64 * 9] *= 2.0 ** exponent
+        beta[:, at + 64 * 9:at + 2 * seg] = 0
+        g[:, at + 64 * 9:at + seg] = edge * np.log(2.0) / 64
+    args = _to(device, q, k, v, g, beta)
+    run = lambda v: gd.chunk_gated_delta_rule(args[0], args[1], v.to(device), *args[3:], output_final_state=True,
+                                              use_qk_l2norm_in_kernel=l2norm)
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta, l2=og.L2_CHUNK if l2norm else og.L2_NONE)
+    o, s = run(v)
+    for got, want in ((o[:, seg:2 * seg].cpu().double(), want_o[:, seg:2 * seg].double()), (s.cpu().double(), want_s.double())):
+        assert 0 < want.abs().max() < 2.0 ** -60
         assert (got - want).norm() <= 2e-2 * want.norm()
+    leaves = [x.clone().requires_grad_(True) for x in args]
+    ot, st = gd.chunk_gated_delta_rule(*leaves, output_final_state=True, use_qk_l2norm_in_kernel=l2norm)
+    assert torch.equal(ot[:, :2 * seg], o[:, :2 * seg])
+    mixed = small.clone()
+    mixed[..., 3], mixed[..., V - 1] = v[..., 3], v[..., V - 1]
+    mixed[0, 70, :, V - 1] = float("nan")
+    os_, _ = run(small)
+    om, _ = run(mixed)
+    assert torch.equal(om[:, :2 * seg, :, 3], o[:, :2 * seg, :, 3]) and torch.isnan(om[:, seg:2 * seg, :, V - 1]).all()
+    keep = [c for c in range(V) if c not in (3, V - 1)]
+    assert torch.equal(om[:, seg:2 * seg][..., keep], os_[:, seg:2 * seg][..., keep])

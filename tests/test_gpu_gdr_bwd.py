@@ -480,15 +480,14 @@ def test_forward_of_a_training_step_gives_the_bits_of_the_plain_call(device, T, 
 
 @pytest.mark.parametrize("dtype,cps,T", [(torch.bfloat16, 9, 64 * 9 * 3 - 9), (torch.float16, 9, 64 * 9 * 25), (torch.bfloat16, 66, 64 * 66 * 2 + 700)])
 def test_sources_end_where_later_chunks_no_longer_count(device, dtype, cps, T, monkeypatch):
-    """Segments whose first two (head 0) or four (head 1; of fp16 three) chunks decay by more than the fp32 range and the range of the
-    sources together, of which the pass for the
+    """Segments whose first two (head 0) or four (head 1) chunks decay by more than the fp32 range, of which the pass for the
     segments' own gradients walks no others (and the walk over the segments behind starts at the next one); head 2 has next to
     no decay, head 3 one in its first half. Then a dO or a q that is not finite at either end of the chunks left out: none of
     the gradients that it belongs to in front of it are."""
     monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", cps)
     (q, k, v, g, beta, do), _ = _inputs(1, T, 4, 4, 64, 64, dtype, seed=cps, unit=False, g_scale=0.02)
-    g[:, :, 0] *= 110
-    g[:, :, 1] *= 55
+    g[:, :, 0] *= 90
+    g[:, :, 1] *= 35
     g[:, : T // 2, 3] *= 50
     got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, True)
     want = ob.backward_manual(q, k, v, g, beta, do, l2=og.L2_CHUNK)
