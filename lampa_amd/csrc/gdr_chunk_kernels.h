@@ -415,11 +415,8 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
     }
   }
   lds_fence();
-  if (edge) {  // the diagonal holds beta_i |rk_i k_i|^2 (see GDR_EDGE_*); no row of the substitution reads it
-    const float diag = s_Ad[hh * (32 * SB) + ln * (SB + 1)];
-    const bool tame = !rising && !__ballot(!(diag >= 0.0f && diag <= 2.0f && __builtin_fabsf(bz) <= GDR_EDGE_BETA));
-    if (lane == 0) edge[(size_t)chunk * HV + hv] = tame ? g_last : __builtin_inff();
-  }
+  // the diagonal holds beta_i |rk_i k_i|^2 (see GDR_EDGE_*; looked at last); no row of the substitution reads it
+  const float diag = s_Ad[hh * (32 * SB) + ln * (SB + 1)];
   // ---- the four 16x16 diagonal blocks by forward substitution: lane 16 b + c owns column c of block b (block b = rows
   //      and columns 16 (b % 2) .. + 15 of the 32x32 diagonal block b / 2), fp32 throughout
   {
@@ -550,6 +547,10 @@ __global__ void __launch_bounds__(64, 4) gdr_local_kernel(const T* __restrict__ 
       const int row = acc_row(r0, hh) + (odd ? 1 : 0);
       *reinterpret_cast<O2*>(out + T_OFF_21 / 2 + row * 32 + (ln & ~1)) = pk;
     }
+  }
+  if (edge) {
+    const bool tame = !rising && !__ballot(!(diag >= 0.0f && diag <= 2.0f && __builtin_fabsf(bz) <= GDR_EDGE_BETA));
+    if (lane == 0) edge[(size_t)chunk * HV + hv] = tame ? g_last : __builtin_inff();
   }
 }
 
@@ -822,7 +823,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   // stores, would be fetched with vector loads and would sit in the same queue as the stagers' prefetches)
   // Segments that cut off what lies before them are found (see the end of the kernel), in the composite pass of the plain rule.
   constexpr bool CUTS = !PASS_B && SCALED_K;
-  constexpr bool SKIP_M = CUTS && KT + VT > 128;
+  // SKIP_M, see below, has little left to skip where the edges are looked at, and there it costs the loop registers: 60 000 tokens
+  // x 8 x 128 x 128 at e^-0.04 a token 115.4 us with both, 108.2 with the edges alone, 107.6 with SKIP_M alone.
+  constexpr bool V_OUT = CUTS && KT + VT > 128, SKIP_M = V_OUT && !EDGES;
 
   if (wave >= NSLAB) {
     // ================================================ stager ================================================
@@ -1824,10 +1827,13 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
       for (int km = 0; km < KT / 32; ++km) S[km] = zero16();
     }
   } else {
+    // (opaque, or the comparisons are kept for the epilogue: 32 masks over the loop, in registers that the training form lacks)
+    int own = 32 * wave + ln;
+    if constexpr (EDGES && KT + VT <= 128 && SCALED) asm volatile("" : "+v"(own));
 #pragma unroll
     for (int km = 0; km < KT / 32; ++km)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) S[km][r] = (is_m && 32 * km + acc_row(r, hh) == 32 * wave + ln) ? 1.0f : 0.0f;
+      for (int r = 0; r < 16; ++r) S[km][r] = (is_m && 32 * km + acc_row(r, hh) == own) ? 1.0f : 0.0f;
   }
 
   GDR_Q_BUFFERS(0);
@@ -1911,9 +1917,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
         for (int e = 0; e < 4; ++e) {
           const float ks_ = SCALED ? acc[4 * b4 + e] : ek[4 * tm + b4][e] * acc[4 * b4 + e];
           // (training form: selected, not multiplied away, so that a v that is not finite stays out of M' and with it out
-          // of the gradients of the tokens before it; so with SKIP_M, where it would reach M, and through M the other value
-          // columns behind the segment, only as long as M lives on)
-          const float v_ = SKIP_M ? (__is_same(OT, __bf16) ? 1.0f : vmask) * op_elem_keep<OT>(vv[4 * tm + b4], e, vkeep)
+          // of the gradients of the tokens before it; so with the wide heads, where it would reach M, and through M the other value
+          // columns behind the segment, only as long as M lives on, or where it lies in chunks that are walked)
+          const float v_ = V_OUT ? (__is_same(OT, __bf16) ? 1.0f : vmask) * op_elem_keep<OT>(vv[4 * tm + b4], e, vkeep)
                            : KEEP ? (is_m ? 0.0f : (float)vv[4 * tm + b4][e])
                                   : vmask * (float)vv[4 * tm + b4][e];
           acc[4 * b4 + e] = be[4 * tm + b4][e] * (v_ - ks_);
