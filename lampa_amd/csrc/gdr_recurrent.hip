@@ -651,13 +651,14 @@ __global__ void __launch_bounds__(64 * RsScanShape<KT>::NT)
   // Notes of the groups' maps, [HV][sequence][group][16 columns]: RS_FINITE, all entries are; RS_ZERO, those of M are zero. A
   // group behind maps that all are finite, the last of them without M (decays beyond the fp32 range), starts behind that one, on
   // the initial state as it is: 8 192 tokens x 4 at e^-0.8 a token, 32 x 32: scan 12.5 -> 7.5 us, call 45.8 -> 41.0, 64 x 64
-  // 92.9 -> 89.7; at e^-0.04, where no map is zero, 45.5 -> 45.9.
-  const int nb = (W + 15) / 16, n_notes = lead * nb;
-  const int* const seen = notes + ((int64_t)hv * (gridDim.y / maxg) + seq) * maxg * nb;
+  // 92.9 -> 89.7; at e^-0.04, where no map is zero, 45.5 -> 45.9. (Behind fewer than two groups there is nothing to leave out, and a
+  // word that no one writes is read in their place: the loads are unconditional.)
+  const int nb = (W + 15) / 16, n_notes = lead > 1 ? lead * nb : 1;
+  const int* const seen = lead > 1 ? notes + ((int64_t)hv * (gridDim.y / maxg) + seq) * maxg * nb : seq_seg0;
   int note[RS_NOTE_LOADS];
   if constexpr (!COMPOSE) {
 #pragma unroll
-    for (int x = 0; x < RS_NOTE_LOADS; ++x) note[x] = seen[min(lane + 64 * x, max(n_notes - 1, 0))];
+    for (int x = 0; x < RS_NOTE_LOADS; ++x) note[x] = seen[min(lane + 64 * x, n_notes - 1)];
   }
   auto store = [&](int64_t at, int width) __attribute__((always_inline)) {
     float* to = out + (at * HV + hv) * K * width + col;
@@ -800,7 +801,7 @@ int gdr_segment_scan(const float* mn, const float* h0, const int32_t* seq_seg0, 
   } while (0)
   LAMPA_PROF(s, "start");
   int gs = n_seg, maxg = 1;
-  int* notes = (int*)sinit;  // (read, not used, where there are no groups)
+  int* notes = nullptr;
   if (groups && n_seq <= GDR_SCAN_GROUP_SEQS && n_seg <= GDR_SCAN_GROUP_SEGS && n_seg >= 24 * n_seq) {
     gs = 1;
     while (2 * gs * gs * n_seq < n_seg) ++gs;
