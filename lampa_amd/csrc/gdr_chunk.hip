@@ -10,7 +10,7 @@ struct GdrWorkspace {
   int64_t off_t, off_m, off_n, off_d, off_sinit, off_gm, off_gn, off_gd, max_groups, bytes;
 };
 
-// kept: the records are kept elsewhere (training form)
+// kept: the records and the edges are kept elsewhere (training form)
 static GdrWorkspace gdr_workspace(int64_t chunks, int64_t segs, int HV, int K, int V, bool kept = false) {
   GdrWorkspace w;
   int64_t off = 0;
@@ -18,8 +18,8 @@ static GdrWorkspace gdr_workspace(int64_t chunks, int64_t segs, int HV, int K, i
   w.off_m = off;     off += lampa_align_up(segs * HV * (int64_t)K * K * 2, 256);
   w.off_n = off;     off += lampa_align_up(segs * HV * (int64_t)K * V * 4, 256);
   w.off_d = off;     off += lampa_align_up(segs * HV * 4, 256);
-  // the segments' initial states + a spare slot (scan); before the scan the chunks' edges (GDR_EDGE_*) and a spare row
-  w.off_sinit = off; off += lampa_align_up(std::max((segs + 1) * HV * (int64_t)K * V, (chunks + 1) * HV) * 4, 256);
+  // the segments' initial states + a spare slot (scan); before the scan the chunks' edges (GDR_EDGE_*)
+  w.off_sinit = off; off += lampa_align_up(std::max((segs + 1) * HV * (int64_t)K * V, kept ? 0 : chunks * HV) * 4, 256);
   // two-level scan: composites of the groups of GDR_SCAN_GROUP segments
   w.max_groups = segs / GDR_SCAN_GROUP + 2;
   w.off_gm = off;    off += lampa_align_up(w.max_groups * HV * (int64_t)K * K * 2, 256);
@@ -195,7 +195,7 @@ GdrSaved gdr_saved_layout(int64_t chunks, int64_t segs, int HV) {
   v.off_states = off; off += lampa_align_up(chunks * HV * (int64_t)GDR_STATE_BYTES, 256);
   v.off_mt = off;     off += lampa_align_up(segs * HV * (int64_t)GDR_STATE_BYTES, 256);
   v.off_d = off;      off += lampa_align_up(segs * HV * 4, 256);
-  v.off_e = off;      off += lampa_align_up((chunks + 1) * HV * 4, 256);
+  v.off_e = off;      off += lampa_align_up(chunks * HV * 4, 256);
   v.bytes = off > 0 ? off : 256;
   return v;
 }
