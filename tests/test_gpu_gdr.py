@@ -824,7 +824,8 @@ def test_recurrent_scan_behind_maps_without_a_past(device, K, V, lens):
 @pytest.mark.parametrize("K,V,dtype,cps,chunks", [
     (64, 64, torch.bfloat16, 4, [24, 8, 2, 37]), (64, 128, torch.float16, 4, [24, 8, 2, 37]), (32, 32, torch.bfloat16, 4, [24, 8, 2, 37]),
     (128, 64, torch.bfloat16, 4, [24, 8, 2, 37]), (128, 128, torch.float16, 4, [24, 8, 2, 37]), (128, 64, torch.float16, 3, [72, 3, 30]),
-    (32, 32, torch.bfloat16, 3, [219]), (128, 128, torch.bfloat16, 2, [49, 1])])
+    (32, 32, torch.bfloat16, 3, [219]), (128, 128, torch.bfloat16, 2, [49, 1]), (128, 128, torch.bfloat16, 2, [49]),
+    (128, 64, torch.float16, 2, [60, 60])])
 def test_states_behind_segments_without_a_past(device, K, V, dtype, cps, chunks, monkeypatch):
     # Packed sequences of one segment to more than the 64 that are looked at: every segment of head 0 cuts off its past, those of a sequence's first half
     # (head 2) or second half (head 3) do, none of head 1. Then with initial states, then a v that is not finite: its column is
@@ -885,13 +886,37 @@ def test_chunks_left_out_where_the_decays_product_stays_subnormal(device, K, V, 
     assert torch.equal(o1[..., keep], o[..., keep]) and torch.equal(s1[..., keep], s[..., keep])
 
 
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (64, 64, torch.float16), (32, 32, torch.bfloat16), (128, 128, torch.bfloat16)])
+@pytest.mark.parametrize("beta0", [3.0, 2.0])
+def test_tokens_that_are_no_contraction_keep_what_lies_before_them(device, K, V, dtype, beta0, monkeypatch):
+    # Five chunks at a segment's end whose log-decays sum up to 2^-320 and whose tokens all map one direction by 1 - beta0: with 3 they
+    # take the decay back and hand the row on as it was, with 2 (a reflection) nothing is left. (2e-2, of fp16 2.5e-3: the roundings
+    # of an ordinary call's outputs.)
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 12)
+    q, k, v, g, beta = synth.gdr_inputs(1, 64 * 15, 2, K, V, dtype, seed=K, g_scale=1e-3)
+    end = slice(64 * 7, 64 * 12)
+    k[:, end] = 0
+    k[:, end, :, 5] = 1
+    v[:, end] = 0
+    beta[:, end] = beta0
+    beta[:, 64 * 12:] = 0
+    g[:, end] = -np.log(2.0)
+    want_o, want_s = og.recurrent_c(q, k, v, g, beta)
+    o, s = gd.chunk_gated_delta_rule(*_to(device, q, k, v, g, beta), output_final_state=True)
+    bound = 2e-2 if dtype == torch.bfloat16 else 2.5e-3
+    for got, want in ((o[:, 64 * 12:].cpu().double(), want_o[:, 64 * 12:].double()), (s.cpu().double(), want_s.double())):
+        assert (want.abs().max() > 1e-3) == (beta0 == 3.0)
+        assert (got - want).norm() <= bound * want.norm() + 1e-30
+
+
 @pytest.mark.parametrize("K,V,exponent,edge", [(64, 64, 115, -70), (64, 64, 122, -73), (32, 32, 122, -73), (64, 128, 122, -73),
-                                               (128, 64, 115, -70), (128, 128, 122, -73)])
+                                               (128, 64, 115, -70), (128, 128, 122, -73), (64, 64, 43, -50), (128, 128, 43, -50)])
 @pytest.mark.parametrize("l2norm", [False, True])
 def test_large_values_in_front_of_strong_decays(device, K, V, exponent, edge, l2norm, monkeypatch):
     # Three chunks of 2^edge at the end of a segment behind v of the size 2^exponent, nothing written from there to the next segment's
     # end: what is left is small, but within the fp32 range. The same in the third, ragged segment. (2e-2: the roundings to bf16
-    # of an ordinary call's outputs.) Then such values in two columns only, one of them with a NaN as well.
+    # of an ordinary call's outputs. 2^43 and 2^-150: of values that are walked.) Then such values in two columns only, one of them
+    # with a NaN as well.
     monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 12)
     seg, T = 64 * 12, 64 * 35 + 40
     q, k, v, g, beta = synth.gdr_inputs(1, T, 2, K, V, torch.bfloat16, seed=K, g_scale=1e-4)

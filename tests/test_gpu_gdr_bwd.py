@@ -539,3 +539,41 @@ def test_sources_that_overflow_behind_strong_decays(device, dtype, q_exp, do_exp
     g[:, seg:seg + 64 * 3] = -100 * 0.6931471805599453 / 64
     got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, False, scale=scale)
     assert not torch.isfinite(got[2][:, :seg]).any()
+
+
+@pytest.mark.parametrize("beta0", [3.0, 2.0])
+def test_tokens_that_are_no_contraction_keep_the_gradient_behind_them(device, beta0, monkeypatch):
+    """Five chunks at a segment's start whose log-decays sum up to 2^-320 and whose tokens all map one direction by 1 - beta0: with 3
+    they take the decay back and hand the gradient of that row on as it was, with 2 nothing is left of it in front. (2e-2: the
+    roundings of an ordinary call's gradients.)"""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 12)
+    T, seg = 64 * 24, 64 * 12
+    (q, k, v, g, beta, do), _ = _inputs(1, T, 2, 2, 64, 64, torch.bfloat16, seed=5, unit=True, g_scale=1e-3)
+    start = slice(seg, seg + 64 * 5)
+    k[:, start] = 0
+    k[:, start, :, 5] = 1
+    beta[:, start] = beta0
+    g[:, start] = -0.6931471805599453
+    do[:, :seg + 64 * 5] = 0
+    got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, False)
+    want = ob.backward_manual(q, k, v, g, beta, do)
+    b = want[2][:, :seg]  # dv
+    assert (b.abs().max() > 1e-2) == (beta0 == 3.0)
+    assert (got[2][:, :seg].cpu().double() - b).norm() <= 2e-2 * b.norm() + 1e-30
+
+
+def test_sources_of_grouped_heads_with_chunks_left_out(device, monkeypatch):
+    """Two q / k heads of four value heads: the look at q of the chunks left out follows the group. A q of the second head that is
+    not finite leaves the first head's gradients alone."""
+    monkeypatch.setattr(gd, "CHUNKS_PER_SEGMENT", 9)
+    T, seg = 64 * 9 * 3 - 20, 64 * 9
+    (q, k, v, g, beta, do), _ = _inputs(1, T, 2, 4, 64, 64, torch.bfloat16, seed=7, unit=False, g_scale=2.0)
+    got = _gpu_grads(device, q, k, v, g, beta, do, None, None, None, True)
+    want = ob.backward_manual(q, k, v, g, beta, do, l2=og.L2_CHUNK)
+    _check(got[:5], want[:5], torch.bfloat16, chunked=True)
+    bad = q.clone()
+    bad[0, 2 * seg - 1, 1, 3] = float("nan")
+    nan = _gpu_grads(device, bad, k, v, g, beta, do, None, None, None, True)
+    assert not torch.isfinite(nan[2][0, : 2 * seg - 64, 2:]).any() and not torch.isfinite(nan[1][0, : 2 * seg - 64, 1]).any()
+    for i, heads in enumerate((1, 1, 2, 2, 2)):
+        assert torch.equal(nan[i][:, :, :heads], got[i][:, :, :heads])

@@ -472,3 +472,25 @@ def test_large_values_in_front_of_strong_decays(device, V):
     want = _want(q, k, v, g, beta, lam)[:, 64 * 16:].double()
     got = _run(device, q, k, v, g, beta, lam, 16)[:, 64 * 16:].cpu().double()
     assert 0 < want.abs().max() < 2.0 ** -80 and (got - want).norm() <= 2e-2 * want.norm()
+
+
+@pytest.mark.parametrize("V,dtype,cps,chunks,HV", [(64, torch.bfloat16, 16, 37, 4), (128, torch.float16, 16, 37, 2), (64, torch.bfloat16, 64, 130, 2)])
+def test_values_that_are_not_finite_in_chunks_left_out(device, V, dtype, cps, chunks, HV, monkeypatch):
+    """Composites of whole segments and of pieces (eight chunks each) whose last two or three chunks decay by more than the fp32
+    range: a v that is not finite, in the chunks left out or in the last one, is in its column of every later output, and in no
+    other where it was left out."""
+    monkeypatch.setattr(hgdn, "CHUNKS_PER_SEGMENT", cps)
+    q, k, v, g, beta, lam = _inputs(1, 64 * chunks, 1, 64, V, dtype, seed=V, HV=HV, g_scale=1.5)
+    run = lambda v: hgdn.chunk_h_gated_delta_rule(*(x.to(device) for x in (q, k, v, g, lam, beta)), use_qk_l2norm_in_kernel=True)[0]
+    o = run(v)
+    max_abs, mean_rel = _errors(o, _want(q, k, v, g, beta, lam))
+    assert max_abs <= MAX_ABS and mean_rel <= MEAN_REL, f"{max_abs:.3e} {mean_rel:.3e}"
+    piece = 64 * (cps if cps < 64 else 8)
+    keep = [c for c in range(V) if c != 5]
+    for row in (3, piece - 64 * 4 - 1, piece - 1):
+        bad = v.clone()
+        bad[0, row, :, 5] = float("inf")
+        o1 = run(bad)
+        assert not torch.isfinite(o1[0, row + 1:, :, 5]).any()
+        if row < piece - 64 * 3:
+            assert torch.equal(o1[0, piece:][..., keep], o[0, piece:][..., keep])
