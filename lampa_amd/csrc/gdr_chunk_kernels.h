@@ -796,8 +796,9 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   const int hv = gridDim.y > 1 ? blockIdx.y : bx % HV;
   const int h = hv / (HV / H);
   const int flags = pv.seg_flags[seg];
-  if (!PASS_B && !KEEP && (flags & SEG_LAST)) return;  // nothing follows the last segment of a sequence
   int c0 = pv.seg_chunk0[seg], nc = pv.seg_nchunks[seg], map = seg;  // map: where the composite goes
+  if constexpr (EDGES) asm volatile("" : "+s"(c0), "+s"(nc));  // (fetched beside the flags, not behind them: the look waits for them)
+  if (!PASS_B && !KEEP && (flags & SEG_LAST)) return;  // nothing follows the last segment of a sequence
   if (PIECES && gmax > 0) {
     const int piece = (int)blockIdx.x % gmax;
     nc /= gmax;
