@@ -247,8 +247,9 @@ def main():
         "kernel_over_twin": round(stage_us.get("gdr_segment_kernel<output>", float("nan")) / probe_us, 3),
         "note": "the output pass's loads and stores with no arithmetic (lampa_gdr_traffic_probe), 100 launches with "
                 "HIP events: the practical floor of that kernel on this memory system"}
-    # the same twin with the reads of the walk over the earlier composites that the output pass does before its first chunk
-    # (the second level of the two-level scan runs inside that kernel): the floor of the kernel as it is now
+    # the same twin with the reads of a whole walk over the earlier composites in front of the first chunk (the second level of the
+    # two-level scan runs inside the output pass): the floor of the kernel where no segment cuts off its past. At these inputs'
+    # decays every segment does, and the kernel reads one composite or none: its own floor is the twin above.
     n_seg_probe = (n_chunks_probe + cps_probe - 1) // cps_probe
     comp = torch.zeros((n_seg_probe + (n_seg_probe + 7) // 8) * H * 24576, dtype=torch.uint8, device=dev)
 
@@ -270,8 +271,9 @@ def main():
     roofline["memory_only_twin_with_walk"] = {
         "us": round(walk_us, 2), "bytes": walk_bytes, "GB/s": round(walk_bytes / (walk_us * 1e-6) / 1e9, 1),
         "kernel_over_twin": round(stage_us.get("gdr_segment_kernel<output>", float("nan")) / walk_us, 3),
-        "note": "the twin above plus the composites the kernel reads for the scan's second level before its first chunk "
-                "(lampa_gdr_traffic_probe_walk: per step and wave 8 KiB of M' and 8 KiB of N, two steps ahead)"}
+        "note": "the twin above plus the composites of a whole walk over the scan's second level before the first chunk "
+                "(lampa_gdr_traffic_probe_walk: per step and wave 8 KiB of M' and 8 KiB of N, two steps ahead), which the "
+                "kernel makes where no segment cuts off its past; at these inputs it starts behind the last one"}
     del rec, o_probe, comp
     # ---- per-step distribution (HIP events on the launch stream, one pair per step) and a cold variant that rotates
     #      among input sets totalling more than 512 MB, so that no step finds its inputs in the memory-side cache ----

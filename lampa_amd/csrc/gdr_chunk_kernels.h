@@ -93,9 +93,10 @@ __device__ __forceinline__ int gdr_leading_cuts(float d, int n, int lane) {
 }
 // The state that segment `seg` starts from, `size` floats in the slabs of the scan below (null: zero). Without an initial
 // state, behind maps that all cut off what lies before them, that is N of the last one, and the scan passes by such segments:
-// the call on 16 packed events of 520 000 tokens, 8 x 128 x 128, at e^-0.8 a token 1 600 -> 1 562 us (scan 45 -> 6, output pass
-// 1 028 -> 1 060, to which the scan's copy came from the caches and N comes from HBM); where nothing cuts off (4 x
-// 14 803 tokens, 4 x 128 x 64, e^-0.04) 133.1 -> 132.9, the look being beside the first loads in both passes.
+// the call on 16 packed events of 520 000 tokens, 8 x 128 x 128, at e^-0.8 a token 1 600 -> 1 562 us (scan 45 -> 6, whose traffic
+// falls from 190 to 13 MB; the output pass, which reads N instead of the scan's copy, moves the same 4.67 GB and takes 0.5 to 2 %
+// more, by box); where nothing cuts off (4 x 14 803 tokens, 4 x 128 x 64, e^-0.04) 133.1 -> 132.9, the look being beside the first
+// loads in both passes.
 __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv, int seg, int hv, int HV, int size,
                                                           const float* Sinit, const unsigned char* Ncomp, const float* Dcomp,
                                                           const float* h0, int lane) {
@@ -115,8 +116,14 @@ __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv,
 //
 // The composite pass starts where the edges behind sum up to GDR_EDGE_REACH: nothing is left there of M and of the sources in
 // front. With beta up to 2 and beta |k|^2 <= 2 a write is below 2 |v|, the state of 128 chunks below 2^14 |v|, and 2^-208 of that
-// below the fp32 range up to |v| = 2^44 (every fp16). A column of the value with a larger one in front is worked out token by
-// token (gdr_serial_slab).
+// below the fp32 range up to |v| = 2^44 (every fp16). A value column with a larger one in front is worked out token by token
+// (gdr_serial_slab).
+//
+// At e^-0.8 a token a segment's last three chunks are walked, at e^-0.24 ten, at e^-0.04 all. us of the composite pass / of the call
+// without the look and with it, in turn on one box: 60 000 tokens x 8 x 64 x 64 at e^-0.8 38.8 -> 18.8 (174 -> 96 MB) / 121.3 -> 110.4,
+// at e^-0.24 38.0 -> 27.3 / 127.9 -> 117.5; 16 packed events of 520 000 tokens, 8 x 128 x 128 706 -> 249 (2.26 -> 1.15 GB) / 1 972 ->
+// 1 504. At e^-0.04 the price of the look: the call 128.5 -> 129.5, 60 000 x 8 x 128 x 128 293.3 -> 295.2, x 32 x 32 104.9 -> 105.3,
+// the hierarchical prefill of 15 000 169.6 -> 171.6.
 #define GDR_EDGE_BETA 2.0f
 #define GDR_EDGE_REACH -208.0f
 #define GDR_EDGE_LARGE 0x5580  // bits of the bf16 2^44

@@ -650,8 +650,8 @@ __global__ void __launch_bounds__(64 * RsScanShape<KT>::NT)
   }
   // Notes of the groups' maps, [HV][sequence][group][16 columns]: RS_FINITE, all entries are; RS_ZERO, those of M are zero. A
   // group behind maps that all are finite, the last of them without M (decays beyond the fp32 range), starts behind that one, on
-  // the initial state as it is: 8 192 tokens x 4 at e^-0.8 a token, 32 x 32: scan 12.5 -> 7.5 us, call 45.8 -> 41.0, 64 x 64
-  // 92.9 -> 89.7; at e^-0.04, where no map is zero, 45.5 -> 45.9. (Behind fewer than two groups there is nothing to leave out, and a
+  // the initial state as it is: 8 192 tokens x 4 at e^-0.8 a token, 32 x 32: scan 12.5 -> 7.4 us, call 45.1 -> 40.0; at
+  // e^-0.04, where no map is zero, 45.7 -> 46.1, 64 x 64 93.1 -> 93.4. (Behind fewer than two groups there is nothing to leave out, and a
   // word that no one writes is read in their place: the loads are unconditional.)
   const int nb = (W + 15) / 16, n_notes = lead > 1 ? lead * nb : 1;
   const int* const seen = lead > 1 ? notes + ((int64_t)hv * (gridDim.y / maxg) + seq) * maxg * nb : seq_seg0;
