@@ -115,8 +115,8 @@ __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv,
 // elsewhere: chunks of finite edges leave at most 2^(sum of the edges) of any state, whatever their keys.
 //
 // The composite pass starts where the edges behind sum up to GDR_EDGE_REACH: nothing is left there of M and of the sources in
-// front. With beta up to 2 and beta |k|^2 <= 2 a write is below 2 |v|, the state of 128 chunks below 2^14 |v|, and 2^-208 of that
-// below the fp32 range up to |v| = 2^44 (every fp16). A value column with a larger one in front is worked out token by token
+// front. With beta up to 2^14 and beta |k|^2 <= 2 a write is below 2^8 |v|, the state of 128 chunks below 2^21 |v|, and 2^-208 of
+// that below the fp32 range up to |v| = 2^36 (every fp16). A value column with a larger one in front is worked out token by token
 // (gdr_serial_slab).
 //
 // At e^-0.8 a token a segment's last three chunks are walked, at e^-0.24 ten, at e^-0.04 all. us of the composite pass / of the call
@@ -124,9 +124,9 @@ __device__ __forceinline__ const float* gdr_segment_state(const GdrPlanView& pv,
 // at e^-0.24 38.0 -> 27.3 / 127.9 -> 117.5; 16 packed events of 520 000 tokens, 8 x 128 x 128 706 -> 249 (2.26 -> 1.15 GB) / 1 972 ->
 // 1 504. At e^-0.04 the price of the look: the call 128.5 -> 129.5, 60 000 x 8 x 128 x 128 293.3 -> 295.2, x 32 x 32 104.9 -> 105.3,
 // the hierarchical prefill of 15 000 169.6 -> 171.6.
-#define GDR_EDGE_BETA 2.0f
+#define GDR_EDGE_BETA 16384.0f
 #define GDR_EDGE_REACH -208.0f
-#define GDR_EDGE_LARGE 0x5580  // bits of the bf16 2^44
+#define GDR_EDGE_LARGE 0x5180  // bits of the bf16 2^36
 // Chunks left out that pay for looking at their v; chunks of a segment that pay for the look at its edges (15 000 tokens x 8 x
 // 128 x 64 at e^-0.04, segments of seven: 93.1 -> 94.8 us) and that two loads a lane cover.
 #define GDR_EDGE_MIN 2
@@ -832,7 +832,8 @@ __global__ void __launch_bounds__((64 * GdrSegShape<KT, VT, PASS_B, CW>::WAVES),
   // Segments that cut off what lies before them are found (see the end of the kernel), in the composite pass of the plain rule.
   constexpr bool CUTS = !PASS_B && SCALED_K;
   // SKIP_M, see below, has little left to skip where the edges are looked at, and there it costs the loop registers: 60 000 tokens
-  // x 8 x 128 x 128 at e^-0.04 a token 115.4 us with both, 108.2 with the edges alone, 107.6 with SKIP_M alone.
+  // x 8 x 128 x 128 at e^-0.04 a token 115.4 us with both, 108.2 with the edges alone, 107.6 with SKIP_M alone. (Of keys that are no
+  // contraction no chunk is left out, and with strong decays M is then walked to its segment's end also where it has become zero.)
   constexpr bool V_OUT = CUTS && KT + VT > 128, SKIP_M = V_OUT && !EDGES;
 
   if (wave >= NSLAB) {
